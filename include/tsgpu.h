@@ -84,13 +84,14 @@ typedef struct tsg_schedule {
  *                resolve launch's last workgroup (0 = separate commit launch)
  *   team_max     waves per item of latency-bound batches (1, 2, 4 or 8)
  *   team_waves   resident waves the team size is sized against
- *   prefetch_max batches of at most this many items get their neighbour
- *                lists computed ahead, window by window (0 = never)
+ *   prefetch_max batches of at most this many items count as latency-bound:
+ *                outside dependency order they get their neighbour lists
+ *                computed ahead, window by window (0 = never)
  *   ahead        1: a single-job run prepares each stage's content-independent
- *                work (random candidates, pick ranks, the neighbour lists of
- *                its leading latency-bound batches) during the previous
- *                stage on a second stream, in two buffer sets used in turn,
- *                when they fit in device memory; 2: one buffer set per stage,
+ *                work (random candidates, pick ranks, neighbour lists; with
+ *                flow 0 those of its leading latency-bound batches only)
+ *                during the previous stage on a second stream, in two
+ *                buffer sets used in turn, when they fit in device memory; 2: one buffer set per stage,
  *                every item's neighbour list, prepared as far ahead as the
  *                host has reached (when the stages fit, else as 1); 0: per
  *                window on the job stream
@@ -99,16 +100,17 @@ typedef struct tsg_schedule {
  *                instead of two launches per batch (0 = off)
  *   coop_max     batches of at most this many items (<= 16 * coop_wgs) go
  *                to that launch
- *   flow         1: with `ahead`, each stage's leading run of latency-bound
- *                new-pixel batches goes to one launch of persistent
- *                workgroups that resolve the items in order, each waiting
- *                only for the neighbours committed inside the run (per-pixel
- *                flags); 2: as 1, and the leading run of latency-bound redo
- *                batches too, reading neighbours not redone before them from
- *                a snapshot of the state taken as the stage opens; 0: one
- *                launch (or loop step) per batch
- *   flow_wgs     workgroups of that launch (0: as many as are resident)
- *   flow_team    waves per item in that launch (1, 2, 4 or 8)
+ *   flow         1 (or 2): with `ahead`, every stage runs in dependency order:
+ *                launches of persistent workgroups that resolve the stage's
+ *                items in order, redo items and new pixels alike, each
+ *                waiting only for those of its neighbours that an earlier
+ *                batch of the stage resolves (records posted per pixel); 0:
+ *                one launch (or loop step) per batch
+ *   flow_wgs     workgroups of such a launch (0: as many as are resident)
+ *   flow_team    there, least waves per item of a batch of at most
+ *                prefetch_max items (1, 2, 4 or 8; a small batch takes up to
+ *                team_max while its items fit team_waves waves); larger
+ *                batches take one wave per item
  *   defer        1: in a single-job run, a throughput-bound batch's commit is
  *                done by the next such batch's launch (its items read the
  *                previous batch's records from a second state array), so a
@@ -119,10 +121,9 @@ typedef struct tsg_schedule {
  *                take in turn (no wave waits for the slowest item of its
  *                workgroup); 0: one workgroup per 8 items (three resident
  *                per CU, where the persistent kernel's registers allow two)
- *   flow_head    leading items of each dependency-ordered run that go to a
- *                launch of their own, with teams of flow_head_team waves
- *                (the run's first items form its longest serial chain)
- *   flow_head_team  waves per item in that launch (1, 2, 4 or 8) */
+ *   flow_head    leading items of each such stage that take teams of
+ *                flow_head_team waves (they form its longest serial chain)
+ *   flow_head_team  waves per item of those (1, 2, 4 or 8) */
 typedef struct tsg_tuning {
     uint32_t small_max;
     uint32_t fuse_max;

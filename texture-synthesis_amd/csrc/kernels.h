@@ -113,9 +113,7 @@ struct PrefetchArgs {
     const uint32_t* bounds;       // batch b holds items [bounds[b], bounds[b + 1]) (nb + 1 entries)
     const uint32_t* bnres;        // and starts with bnres[b] resolved pixels
     uint32_t nb;
-    // items below redo_end redo resolved pixels: their dependency bits mark
-    // neighbours redone by an earlier batch (rank - locked below the item's
-    // batch start); the other items' bits mark pixels of mask_new
+    // items below redo_end redo resolved pixels and see no pixel of mask_new
     uint32_t redo_end, locked;
     const int32_t* offtab;
     uint32_t offtab_n;
@@ -123,34 +121,50 @@ struct PrefetchArgs {
     uint32_t item0, item1;
     int32_t* out_nbrs;            // [item - item0][k]
     uint32_t* out_cnt;
-    // optional: per item, bit j set when neighbour j is a pixel of mask_new
+    // optional: per item, bit j set when neighbour j is a pixel that an
+    // earlier batch of the stage resolves (rank - locked, its position in the
+    // work list, below the item's batch start); needs the batch table
     uint64_t* out_dep;            // [item - item0]
 };
 
-// A run of consecutive items [a.item0, a.item0 + n) of one segment (new
-// pixels, or redo items with state_old) in one launch of persistent
-// workgroups. Every item has its neighbour list
-// (a.pre_nbrs) and a dependency mask dep[item - a.pre_base]: bit j set when
-// neighbour j is a pixel committed by an earlier item of the run. Workgroups
-// take items in order from a ticket counter, wait until each dependency's
-// flag holds `epoch`, resolve, commit their item's pixel and publish it by
-// writing `epoch` into its flag. Items wait only on earlier items, which
-// running workgroups hold, so the run always drains. A wait longer than
-// spin_limit polls sets bit 2 of *overflow and ends every wait of the launch
-// (the results are then invalid and the host reports the failure).
+// A dependency-ordered run: consecutive items [a.item0, a.item0 + n) of one
+// stage in one launch of persistent workgroups, redo items and new pixels
+// alike. Every item has its neighbour list (a.pre_nbrs) and a dependency mask
+// dep[item - a.pre_base]: bit j set when neighbour j is a pixel that an
+// earlier batch of the stage resolves. Such a neighbour is read from the
+// stage's mail, every other one from a.state, which the run leaves as the
+// stage opened. Workgroups take items in order from a ticket counter; an item
+// waits until the mail of its dependencies carries the stage's tag, resolves
+// and posts its own pixel. Items wait only on earlier items, which running
+// workgroups hold, so the run always drains. A wait longer than spin_limit
+// polls sets bit 2 of *overflow and ends every wait of the launch (the
+// results are then invalid and the host reports the failure).
+//
+// Mail: two 64-bit words per output pixel, {colour | xy[23:0] << 32 | tag <<
+// 56} and {patch | xy[31:24] << 32 | map << 40 | tag << 56}. Each word is
+// stored and loaded whole (relaxed, device scope) and carries its own tag, so
+// a reader that sees the tag in both words has the record: no ordering
+// between words, no separate flag, and no release or acquire of anything else.
 struct FlowArgs {
-    uint32_t* ticket;
-    uint32_t ticket_base;         // counter value at the launch start
+    uint32_t* ticket;             // zero as the launch starts, used by this launch alone
     uint32_t n;
     const uint64_t* dep;
-    uint32_t* flag;               // per pixel: epoch of the run that committed it
-    uint32_t epoch;
+    unsigned long long* mail;
+    uint32_t tag;                 // 1..255, of this stage
     uint32_t spin_limit;
     uint32_t* overflow;
-    // a run of redo items: the state as the segment opened; neighbours
-    // without a dependency bit are read there (the run rewrites the live
-    // state), and commits touch neither mask nor score. Null: new pixels.
-    const uint4* state_old;
+};
+
+// The end of a stage run in dependency order: the records of its items
+// (mail) into the state, and, with `maps`, every resolved pixel recoloured
+// from that level (next_pyramid_level, ms.rs:687-700). Resolved-list
+// positions [q0, q1); those in [s0, s1) are the stage's items.
+struct StageEndArgs {
+    const uint32_t* rlist;
+    uint32_t q0, q1, s0, s1;
+    const unsigned long long* mail;
+    const MapDesc* maps;
+    uint4* state;
 };
 
 struct RandArgs {
@@ -390,11 +404,12 @@ hipError_t launch_resolve_coop(const BatchArgs& a, const uint32_t* bounds, const
 hipError_t launch_resolve_small(const BatchArgs& a, const uint32_t* bounds, const uint32_t* nres,
                                 uint32_t n_batches, bool guided, hipStream_t s);
 hipError_t launch_resolve(const BatchArgs& a, bool guided, hipStream_t s);
-// A dependency-ordered run (FlowArgs): wgs persistent workgroups of `team`
-// waves; wgs <= flow_max_wgs(team, guided). Consumes n + wgs tickets.
+// A dependency-ordered run (FlowArgs) with `team` waves per item (1, 2, 4 or
+// 8) on at most wgs persistent workgroups. flow_max_wgs: as many as are resident.
 uint32_t flow_max_wgs(uint32_t team, bool guided);
 hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t wgs, uint32_t team, bool guided,
                                hipStream_t s);
+hipError_t launch_stage_end(const StageEndArgs& a, hipStream_t s);
 // Tile bitmask (one u64 per 8x8 tile) of a one-byte-per-pixel mask.
 hipError_t launch_mask_tiles(const uint8_t* mask, uint32_t W, uint32_t H, uint32_t tiles_x, uint32_t tiles_y,
                              uint64_t* tiles, hipStream_t s);
@@ -409,7 +424,6 @@ hipError_t launch_commit(const CommitArgs& a, hipStream_t s);
 uint32_t persist_max_wgs(bool guided);
 hipError_t launch_resolve_persist(const BatchArgs& a, uint32_t wgs, bool guided, hipStream_t s);
 hipError_t launch_defer_flush(const DeferFlushArgs& a, hipStream_t s);
-hipError_t launch_state_snapshot(const uint32_t* rlist, uint32_t n, const uint4* state, uint4* old, hipStream_t s);
 hipError_t launch_recolor(const RecolorArgs& a, hipStream_t s);
 // separable resampling pass: vertical (u8 -> f32) and horizontal (f32 -> u8)
 hipError_t launch_resample_v(const uint32_t* src, uint32_t w, uint32_t h, float4* dst, uint32_t nh,

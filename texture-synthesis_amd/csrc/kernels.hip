@@ -1026,7 +1026,8 @@ __device__ __forceinline__ uint4 item_at_random(const BatchArgs& a, const MapDes
 // The neighbour weights (ms.rs:405-425, 1198-1203), from the neighbour
 // offsets alone: distances, their average over the 4k duplicated entries
 // summed in order, exp(-d / avg).
-__device__ __forceinline__ void item_geometry(const BatchArgs& a, int x, int y, uint32_t kf, WaveLds* L, int lane) {
+template <class Lds>
+__device__ __forceinline__ void item_geometry(const BatchArgs& a, int x, int y, uint32_t kf, Lds* L, int lane) {
     if (lane < (int)kf) {
         const int32_t o = L->nd[lane];
         const int nx = x + packed_dx(o), ny = y + packed_dy(o);
@@ -1069,13 +1070,13 @@ __device__ __forceinline__ void item_geometry(const BatchArgs& a, int x, int y, 
     wave_sync();
 }
 
-// old_state (redo runs): neighbours without a bit in `fresh` are read there.
+// held (dependency-ordered runs): lane j's neighbour record, already read.
 template <bool GUIDED>
 __device__ __forceinline__ uint32_t item_neighbours(const BatchArgs& a, const MapDesc* maps, uint32_t item,
                                                     uint32_t rel, int x, int y, uint32_t kf, uint32_t n_k0,
                                                     WaveLds* L, int lane, bool geo_done,
                                                     uint32_t& xy, uint32_t& ms, uint64_t& uniq,
-                                                    const uint4* old_state = nullptr, uint64_t fresh = 0) {
+                                                    const uint4* held = nullptr) {
     bool coh_valid = false;
     uint4 coh = make_uint4(0, 0, 0, 0);
     if (lane < (int)kf) {
@@ -1088,14 +1089,15 @@ __device__ __forceinline__ uint32_t item_neighbours(const BatchArgs& a, const Ma
         }
         uint32_t nflat = (uint32_t)ny * a.W + (uint32_t)nx;
         uint4 st;
-        if (a.state2) {
+        if (held) {
+            st = *held;
+        } else if (a.state2) {
             // deferred commit: the previous batch's records are still in state2
             const uint32_t sp = gld(a.stamp + nflat);
             const uint4 s0 = gld(a.state + nflat), s1 = gld(a.state2 + nflat);
             st = sp == a.serial - 1u ? s1 : s0;
         } else {
-            const uint4* src = (old_state && !((fresh >> lane) & 1ull)) ? old_state : a.state;
-            st = gld(src + nflat);
+            st = gld(a.state + nflat);
         }
         L->pat[lane] = st.x;
         if (GUIDED) L->gpat[lane] = gld(a.tg + nflat);
@@ -1133,9 +1135,9 @@ __device__ __forceinline__ uint32_t item_neighbours(const BatchArgs& a, const Ma
 
 // Leader: every candidate without pruning, find_best_match's sequential
 // rule, for NaN cost tables and the full-cost test hook.
-template <bool GUIDED>
+template <bool GUIDED, class Lds>
 __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t rel,
-                                           uint32_t kf, uint32_t n_coh, uint32_t n_c, WaveLds* L, const float* lut,
+                                           uint32_t kf, uint32_t n_coh, uint32_t n_c, const Lds* L, const float* lut,
                                            const float* glut, int slot, int lane, float& best, uint32_t& bidx) {
     const uint32_t slot4 = (uint32_t)slot * 4u;
     for (uint32_t base = 0; base < n_c; base += kWave) {
@@ -1219,8 +1221,9 @@ __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* ma
 // Leader: the winning candidate. Returns the result (lane 0), also written
 // to result[rel] unless a.result is null. xm: the winner's coordinate and
 // map word when the evaluation carried them (else they are read again).
+template <class Lds>
 __device__ __forceinline__ uint4 item_winner(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t rel,
-                                             uint32_t n_coh, const WaveLds* L, float best, uint32_t bidx, int lane,
+                                             uint32_t n_coh, const Lds* L, float best, uint32_t bidx, int lane,
                                              const uint2* xm = nullptr) {
     if (lane != 0) return make_uint4(0, 0, 0, 0);
     uint32_t cxy, cmap, patch;
@@ -1252,26 +1255,39 @@ __device__ __forceinline__ uint4 item_winner(const BatchArgs& a, const MapDesc* 
     return r;
 }
 
-// Resolves work item `item` of the batch starting at item0 against the state
-// frozen at the batch start (n_res resolved pixels); writes result[item -
-// item0]. Lt: the team's WaveLds (member q uses Lt + q); `valid` is false
-// for members of a team past the batch end, which still take the barriers.
-// Flow runs, leader: waits until every neighbour committed inside the run
-// (dependency bit set) has published its flag, then acquires at device scope
-// so that the team's state reads see those commits.
-__device__ __forceinline__ void flow_wait(const FlowArgs& f, const BatchArgs& a, uint32_t item, int x, int y,
-                                          uint32_t kf, const WaveLds* L, int lane) {
-    const uint64_t dep = f.dep[item - a.pre_base] & (kf >= 64u ? ~0ull : ((1ull << kf) - 1ull));
-    if (dep == 0) return;
-    uint32_t q = 0;
-    bool need = (dep >> lane) & 1ull;
-    if (need) {
-        const int32_t o = L->nd[lane];
-        q = (uint32_t)(y + packed_dy(o)) * a.W + (uint32_t)(x + packed_dx(o));
-    }
+// ---- mail of the dependency-ordered runs (FlowArgs) ----
+__device__ __forceinline__ void mail_post(const FlowArgs& f, uint32_t p, uint32_t colour, uint32_t xy, uint32_t map,
+                                          uint32_t patch) {
+    const unsigned long long tag = (unsigned long long)f.tag << 56;
+    const unsigned long long w0 = colour | (unsigned long long)(xy & 0xffffffu) << 32 | tag;
+    const unsigned long long w1 =
+        patch | (unsigned long long)(xy >> 24) << 32 | (unsigned long long)(map & 0xffffu) << 40 | tag;
+    __hip_atomic_store(f.mail + 2 * (size_t)p, w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(f.mail + 2 * (size_t)p + 1, w1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The state record that mail words hold.
+__device__ __forceinline__ uint4 mail_record(unsigned long long w0, unsigned long long w1) {
+    const uint32_t h0 = (uint32_t)(w0 >> 32), h1 = (uint32_t)(w1 >> 32);
+    const uint32_t map = (h1 >> 8) & 0xffffu;
+    return make_uint4((uint32_t)w0, (h0 & 0xffffffu) | (h1 << 24), map | (map << 16), (uint32_t)w1);
+}
+// Neighbour records of an item of a dependency-ordered run, lane j's in lane
+// j (`have`: the lane holds a neighbour, at pixel q): those without a bit in
+// `dep` from the state, the others from the mail once it carries the tag.
+__device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs& a, uint64_t dep, uint32_t q,
+                                              bool have, int lane) {
+    const bool mine = have && ((dep >> lane) & 1ull);
+    uint4 st = make_uint4(0, 0, 0, 0);
+    if (have && !mine) st = gld(a.state + q);
+    bool need = mine;
+    unsigned long long w0 = 0, w1 = 0;
     uint32_t polls = 0;
     for (;;) {
-        if (need) need = __hip_atomic_load(f.flag + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != f.epoch;
+        if (need) {
+            w0 = __hip_atomic_load(f.mail + 2 * (size_t)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            w1 = __hip_atomic_load(f.mail + 2 * (size_t)q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            need = (uint32_t)(w0 >> 56) != f.tag || (uint32_t)(w1 >> 56) != f.tag;
+        }
         if (__ballot(need) == 0ull) break;
         ++polls;
         if ((polls & 63u) == 0u) {
@@ -1285,14 +1301,84 @@ __device__ __forceinline__ void flow_wait(const FlowArgs& f, const BatchArgs& a,
         }
         __builtin_amdgcn_s_sleep(1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (mine) st = mail_record(w0, w1);
+    return st;
 }
 
+// This member's slice of the candidates, exact pruning: unique coherence
+// candidates [c0, c0 + ncs) of the list, then random ones [r0, r0 + nrs):
+// the coherence group alone first (it usually holds the winner and bounds the
+// rest), then the random ones 64 at a time. cxy, cms, uniq: item_neighbours'
+// coherence candidates; rpre: the member's first 64 random candidates.
+template <bool GUIDED, int FIRST_SH>
+__device__ __forceinline__ Best eval_slice(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t rel,
+                                           uint32_t kf, uint32_t n_coh, uint32_t n_k0, uint32_t cxy, uint32_t cms,
+                                           uint64_t uniq, uint32_t r0, uint32_t nrs, uint2 rpre, int member, int T,
+                                           bool lead, WaveLds* L, const float* lut, const float* glut, int slot,
+                                           int lane, unsigned long long* tb) {
+    const uint32_t n_u = (uint32_t)__popcll(uniq);
+    const uint32_t cper = (n_u + (uint32_t)T - 1) / (uint32_t)T;
+    const uint32_t c0 = min(n_u, (uint32_t)member * cper);
+    const uint32_t ncs = min(n_u, c0 + cper) - c0;
+    const uint32_t nv = ncs + nrs;
+    const uint32_t upos = bits_below(uniq);
+    const bool mine_u = ((uniq >> lane) & 1ull) && upos >= c0 && upos < c0 + ncs;
+    Best bst{FLT_MAX, kNone, 0u, 0u};
+    uint32_t g_lo = 0;
+    bool first = true;
+    while (g_lo < nv) {
+        // groups: the first kLead coherence candidates (a full evaluation of
+        // a few likely winners gives an early bound), the other coherence
+        // candidates, then the random ones 64 at a time
+        const uint32_t g_hi = g_lo < ncs ? (g_lo == 0 && ncs > 2 * kLead ? kLead : ncs)
+                                         : min(nv, g_lo + (uint32_t)kWave);
+        // coherence entries of the group
+        if (mine_u) {
+            const uint32_t v = upos - c0;
+            if (v >= g_lo && v < g_hi) {
+                L->act_xy[v - g_lo] = cxy;
+                L->act_ms[v - g_lo] = cms;
+                L->act_idx[v - g_lo] = (uint32_t)lane;
+            }
+        }
+        // random entries of the group
+        const uint32_t v = g_lo + (uint32_t)lane;
+        const uint32_t rr = v >= ncs ? v - ncs : 0u;
+        const uint32_t src = rr < (uint32_t)kWave ? rr : 0u;
+        const uint32_t pxy = (uint32_t)__shfl((int)rpre.x, (int)src);
+        const uint32_t pms = (uint32_t)__shfl((int)rpre.y, (int)src);
+        if (v < g_hi && v >= ncs) {
+            const uint32_t ci = n_k0 + r0 + rr;
+            uint32_t rxy, rms;
+            if (!a.ext_cands && rr < (uint32_t)kWave) {
+                rxy = pxy;
+                rms = pms | 0x80000000u;
+            } else {
+                cand_get(a, L, rel, item, n_coh, ci, rxy, rms);
+            }
+            L->act_xy[lane] = rxy;
+            L->act_ms[lane] = rms;
+            L->act_idx[lane] = ci;
+        }
+        wave_sync();
+        eval_group<GUIDED, FIRST_SH>(maps, a.n_maps, L, lut, glut, slot, lane, kf, g_hi - g_lo, bst,
+                                     tb);
+        if (lead && first) phase_clock(a, item, 4, lane);
+        first = false;
+        g_lo = g_hi;
+    }
+    return bst;
+}
+
+// Resolves work item `item` of the batch starting at item0 against the state
+// frozen at the batch start (n_res resolved pixels); writes result[item -
+// item0]. Lt: the team's WaveLds (member q uses Lt + q); `valid` is false
+// for members of a team past the batch end, which still take the barriers.
 // Returns the result in the leader's lane 0 (zero elsewhere).
 template <bool GUIDED, int FIRST_SH = 6, int KNN_U = 4>
 __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t item0, uint32_t n_res,
                               WaveLds* Lt, int member, int T, bool valid, const float* lut, const float* glut,
-                              int lane, const FlowArgs* flow = nullptr) {
+                              int lane) {
     uint4 res = make_uint4(0, 0, 0, 0);
     WaveLds* L = Lt + member;
     const int slot = lane % lut_copies<GUIDED>();
@@ -1326,8 +1412,7 @@ __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc*
     }
     // ---- 1. k nearest resolved neighbours (leader) ----
     // With a neighbour list computed ahead every member reads it and derives
-    // the weights at once (in a flow run, while the leader waits for the
-    // neighbours committed inside the run).
+    // the weights at once.
     const bool pre = valid && !a.ext_nbrs && !a.knn_only && a.pre_nbrs && item >= a.pre_base && item < a.pre_end;
     if (valid && lead) {
         const uint32_t kf0 = item_knn<KNN_U>(a, item, rel, x, y, n_res, L, lane);
@@ -1336,7 +1421,6 @@ __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc*
             L->t_bound = ~0ull;
         }
         if (pre && kf0) item_geometry(a, x, y, kf0, L, lane);
-        if (flow) flow_wait(*flow, a, item, x, y, kf0, L, lane);
     } else if (pre) {
         const uint32_t kf0 = gld(a.pre_cnt + (item - a.pre_base));
         if (lane < (int)kf0) L->nd[lane] = gld(a.pre_nbrs + (size_t)(item - a.pre_base) * a.k + lane);
@@ -1363,10 +1447,7 @@ __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc*
         // ---- 2. neighbour state, weights, coherence candidates (every member) ----
         uint32_t cxy, cms;
         uint64_t uniq;
-        const uint4* old_state = flow ? flow->state_old : nullptr;
-        const uint64_t fresh = old_state ? flow->dep[item - a.pre_base] : 0ull;
-        n_coh = item_neighbours<GUIDED>(a, maps, item, rel, x, y, kf, n_k0, L, lane, pre, cxy, cms, uniq, old_state,
-                                        fresh);
+        n_coh = item_neighbours<GUIDED>(a, maps, item, rel, x, y, kf, n_k0, L, lane, pre, cxy, cms, uniq);
         if (!a.ext_cands) {
             n_k0 = n_coh;
             n_c = n_coh + a.m;
@@ -1375,60 +1456,9 @@ __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc*
         exact = a.exact || a.ext_full_cost || a.lut_nan || !(L->avg > 0.0);
         if (!exact) {
             // ---- 3. this member's slice, exact pruning ----
-            // slice: unique coherence candidates [c0, c0 + ncs) then random ones
-            // [r0, r0 + nrs): the coherence group alone first (it usually holds
-            // the winner and bounds the rest), then the random ones 64 at a time.
-            const uint32_t n_u = (uint32_t)__popcll(uniq);
-            const uint32_t cper = (n_u + (uint32_t)T - 1) / (uint32_t)T;
-            const uint32_t c0 = min(n_u, (uint32_t)member * cper);
-            const uint32_t ncs = min(n_u, c0 + cper) - c0;
-            const uint32_t nv = ncs + nrs;
-            const uint32_t upos = bits_below(uniq);
-            const bool mine_u = ((uniq >> lane) & 1ull) && upos >= c0 && upos < c0 + ncs;
-            Best bst{FLT_MAX, kNone, 0u, 0u};
-            uint32_t g_lo = 0;
-            bool first = true;
-            while (g_lo < nv) {
-                // groups: the first kLead coherence candidates (a full evaluation of
-                // a few likely winners gives an early bound), the other coherence
-                // candidates, then the random ones 64 at a time
-                const uint32_t g_hi = g_lo < ncs ? (g_lo == 0 && ncs > 2 * kLead ? kLead : ncs)
-                                                 : min(nv, g_lo + (uint32_t)kWave);
-                // coherence entries of the group
-                if (mine_u) {
-                    const uint32_t v = upos - c0;
-                    if (v >= g_lo && v < g_hi) {
-                        L->act_xy[v - g_lo] = cxy;
-                        L->act_ms[v - g_lo] = cms;
-                        L->act_idx[v - g_lo] = (uint32_t)lane;
-                    }
-                }
-                // random entries of the group
-                const uint32_t v = g_lo + (uint32_t)lane;
-                const uint32_t rr = v >= ncs ? v - ncs : 0u;
-                const uint32_t src = rr < (uint32_t)kWave ? rr : 0u;
-                const uint32_t pxy = (uint32_t)__shfl((int)rpre.x, (int)src);
-                const uint32_t pms = (uint32_t)__shfl((int)rpre.y, (int)src);
-                if (v < g_hi && v >= ncs) {
-                    const uint32_t ci = n_k0 + r0 + rr;
-                    uint32_t rxy, rms;
-                    if (!a.ext_cands && rr < (uint32_t)kWave) {
-                        rxy = pxy;
-                        rms = pms | 0x80000000u;
-                    } else {
-                        cand_get(a, L, rel, item, n_coh, ci, rxy, rms);
-                    }
-                    L->act_xy[lane] = rxy;
-                    L->act_ms[lane] = rms;
-                    L->act_idx[lane] = ci;
-                }
-                wave_sync();
-                eval_group<GUIDED, FIRST_SH>(maps, a.n_maps, L, lut, glut, slot, lane, kf, g_hi - g_lo, bst,
-                                             T > 1 ? &Lt->t_bound : nullptr);
-                if (lead && first) phase_clock(a, item, 4, lane);
-                first = false;
-                g_lo = g_hi;
-            }
+            const Best bst = eval_slice<GUIDED, FIRST_SH>(a, maps, item, rel, kf, n_coh, n_k0, cxy, cms, uniq, r0, nrs,
+                                                          rpre, member, T, lead, L, lut, glut, slot, lane,
+                                                          T > 1 ? &Lt->t_bound : nullptr);
             if (lead) phase_clock(a, item, 5, lane);
             if (lane == 0) {
                 L->t_B = bst.B;
@@ -1716,47 +1746,415 @@ __global__ __launch_bounds__(kWave* kSmallWaves) void k_resolve_coop(BatchArgs a
     }
 }
 
-// A dependency-ordered run of new-pixel items (FlowArgs): one item per
-// workgroup at a time, the workgroup's waves as its team. Thread 0 is the
-// team leader's lane 0: it holds the item's result, commits the pixel and
-// publishes it with a device-scope release. a.result is not used.
+// ---- dependency-ordered runs (FlowArgs) ----
+
+// The members of the argument block that a dependency-ordered run has no use
+// for, as constants: no code for them is kept in its item loops.
+__device__ __forceinline__ void flow_args(BatchArgs& a) {
+    a.ext_nbrs = nullptr;
+    a.ext_cands = nullptr;
+    a.ext_full_cost = nullptr;
+    a.dbg_best = nullptr;
+    a.state2 = nullptr;
+    a.result = nullptr;
+    a.exact = 0;
+}
+
+// Pixel of the neighbour at (x + dx, y + dy); in tiling mode a ghost
+// neighbour is the pixel it copies (ms.rs:510-512, 1132-1136).
+__device__ __forceinline__ uint32_t nbr_flat(const BatchArgs& a, int x, int y, int32_t o) {
+    int nx = x + packed_dx(o), ny = y + packed_dy(o);
+    if (a.gmask) {
+        nx = nx < 0 ? nx + (int)a.W : (nx >= (int)a.W ? nx - (int)a.W : nx);
+        ny = ny < 0 ? ny + (int)a.H : (ny >= (int)a.H ? ny - (int)a.H : ny);
+    }
+    return __umul24((uint32_t)ny, a.W) + (uint32_t)nx;
+}
+
+// Hands a workgroup's waves the items of a run in order: tickets are taken
+// eight items at a time (one device-wide atomic per item would serialise on
+// its address), the next eight while the current ones run. A workgroup's
+// tickets must grow: were its waves to wait on items of a later ticket while
+// an earlier one of its own had yet to be handed out, no wave would be left
+// to run that one. So a ticket is taken only once the one before it is known.
+// A wave that takes an item waits for its ticket only; a slot is refilled
+// once all eight takers of its last ticket have read it.
+struct ItemQueue {
+    uint32_t next;       // items handed to this workgroup
+    uint32_t read[4];    // per slot: takers that have read it
+    unsigned long long slot[4];  // {ticket number + 1, first item} of tickets r, r + 4, ...
+};
+constexpr uint32_t kTicketItems = 8;
+
+__device__ __forceinline__ void queue_fetch(ItemQueue* q, const FlowArgs& f, uint32_t r) {
+    while (__hip_atomic_load(&q->read[r & 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < kTicketItems * (r >> 2))
+        __builtin_amdgcn_s_sleep(1);
+    const uint32_t t = atomicAdd(f.ticket, kTicketItems);
+    __hip_atomic_store(&q->slot[r & 3], (unsigned long long)(r + 1) << 32 | t, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ uint32_t queue_next(ItemQueue* q, const FlowArgs& f, int lane) {
+    uint32_t idx = 0;
+    if (lane == 0) {
+        const uint32_t n = atomicAdd(&q->next, 1u), r = n / kTicketItems, pos = n % kTicketItems;
+        if (n == 0) queue_fetch(q, f, 0);
+        unsigned long long v;
+        for (;;) {
+            v = __hip_atomic_load(&q->slot[r & 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if ((uint32_t)(v >> 32) == r + 1) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        atomicAdd(&q->read[r & 3], 1u);
+        if (pos == kTicketItems / 2) queue_fetch(q, f, r + 1);  // ticket r is known
+        idx = (uint32_t)v + pos;
+    }
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)idx);
+}
+
+// A run with one wave per item, for batches large enough to fill the chip:
+// persistent workgroups whose waves take items in order and evaluate them
+// with exact pruning, as k_resolve's do.
 template <bool GUIDED>
-__global__ __launch_bounds__(kWave* kWavesPerWG) void k_resolve_flow(BatchArgs a, FlowArgs f) {
+__global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(6))) void k_flow_wave(BatchArgs a,
+                                                                                                          FlowArgs f) {
     const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ MapDesc smaps[kMapCache];
-    __shared__ uint32_t s_idx;
+    __shared__ ItemQueue queue;
+    flow_args(a);
+    if (threadIdx.x == 0) {
+        queue.next = 0;
+        for (int q = 0; q < 4; ++q) queue.read[q] = 0, queue.slot[q] = 0;
+    }
     float *lut, *glut;
     const MapDesc* maps;
-    WaveLds* wls = setup_lds<GUIDED>(a, smem, lut, glut, smaps, maps);
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    const int T = (int)(blockDim.x / kWave);
+    WaveLds* wls = setup_lds<GUIDED>(a, smem, lut, glut, smaps, maps);  // ends with a barrier
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane0 = threadIdx.x % kWave;
+    WaveLds* L = wls + wave;
     for (;;) {
-        __syncthreads();
-        if (threadIdx.x == 0) s_idx = atomicAdd(f.ticket, 1u) - f.ticket_base;
-        __syncthreads();
-        const uint32_t idx = s_idx;
+        // an opaque lane index: the item's lane-dependent addresses are
+        // computed per item instead of held in registers across the loop
+        int lane = lane0;
+        asm volatile("" : "+v"(lane));
+        const uint32_t idx = queue_next(&queue, f, lane);
         if (idx >= f.n) break;
-        const uint32_t item = a.item0 + idx;
-        const uint32_t p = threadIdx.x == 0 ? a.work[item] : 0u;
-        const uint4 r = resolve_team<GUIDED>(a, maps, item, item, 0u, wls, wave, T, true, lut, glut, lane, &f);
-        if (threadIdx.x == 0) {
-            // Generator::update (ms.rs:334-377): the state record, published
-            // at once; the mask bit and the score are read only after the run
-            const MapDesc& md = maps[r.y & 0xffffu];
-            const uint32_t color = gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu));
-            a.state_w[p] = make_uint4(color, r.x, r.y & ~kFallbackBit, r.z);
-            __hip_atomic_store(f.flag + p, f.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            if (!f.state_old) {
-                // a new pixel enters the resolved mask and keeps its first score
-                const uint32_t px = p % a.W, py = p / a.W;
-                atomicOr((unsigned long long*)&a.mask_w[(py >> 3) * a.tiles_x + (px >> 3)],
-                         1ull << (((py & 7u) << 3) | (px & 7u)));
-                a.score_w[p] = __uint_as_float(r.w);
+        const uint32_t item = a.item0 + idx, rel = item - a.pre_base;
+        phase_clock(a, item, 0, lane);
+        const uint32_t flat = gld(a.work + item);
+        const uint32_t kf = gld(a.pre_cnt + rel);
+        int32_t o = 0;
+        if (lane < (int)kf) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
+        uint2 rpre = make_uint2(0, 0);
+        const uint2* rc = a.rcands + (size_t)(item - a.rc_base) * a.m;
+        if ((uint32_t)lane < a.m) rpre = gld(rc + lane);
+        const int x = (int)(flat % a.W), y = (int)(flat / a.W);
+        if (lane < (int)kf) L->nd[lane] = o;
+        uint4 r;
+        if (kf == 0) {
+            r = item_at_random(a, maps, item, 0, flat, lane);
+        } else {
+            wave_sync();
+            item_geometry(a, x, y, kf, L, lane);
+            const uint4 st = flow_records(f, a, f.dep[rel], lane < (int)kf ? nbr_flat(a, x, y, o) : 0u,
+                                          lane < (int)kf, lane);
+            phase_clock(a, item, 1, lane);
+            uint32_t cxy, cms;
+            uint64_t uniq;
+            const uint32_t n_coh = item_neighbours<GUIDED>(a, maps, item, 0, x, y, kf, 0, L, lane, true, cxy, cms,
+                                                           uniq, &st);
+            phase_clock(a, item, 2, lane);
+            if (!a.lut_nan && L->avg > 0.0) {
+                const Best b = eval_slice<GUIDED, 6>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, 0, a.m, rpre, 0,
+                                                     1, true, L, lut, glut, lane % lut_copies<GUIDED>(), lane, nullptr);
+                phase_clock(a, item, 5, lane);
+                const bool have = b.Bi != kNone;
+                const uint2 xm = make_uint2(b.xy, b.ms);
+                r = item_winner(a, maps, item, 0, n_coh, L, have ? b.B : FLT_MAX, have ? b.Bi : 0u, lane,
+                                have ? &xm : nullptr);
+            } else {
+                float best = FLT_MAX;
+                uint32_t bidx = 0;
+                item_exact<GUIDED>(a, maps, item, 0, kf, n_coh, n_coh + a.m, L, lut, glut, lane % lut_copies<GUIDED>(),
+                                   lane, best, bidx);
+                r = item_winner(a, maps, item, 0, n_coh, L, best, bidx, lane);
             }
-            phase_clock(a, item, 10, 0);
         }
+        if (lane == 0) {
+            // Generator::update (ms.rs:334-377), posted; a new pixel keeps its first score
+            const MapDesc& md = maps[r.y & 0xffffu];
+            const uint32_t colour = gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu));
+            mail_post(f, flat, colour, r.x, r.y & 0xffffu, r.z);
+            if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+        }
+        phase_clock(a, item, 6, lane);
+        wave_sync();
+    }
+    launch_span(a, t_start);
+}
+
+// What a team's members share of one item (two in turn: the members of the
+// next item's team write the other one before the slowest has read this).
+struct TeamLds {
+    double dist[kMaxK];
+    double avg;
+    unsigned long long best;  // least (cost bits << 32 | candidate index)
+    uint4 coh[kMaxK];
+    int32_t nd[kMaxK];
+    float w[kMaxK];
+    uint32_t pat[kMaxK];
+    uint32_t gpat[kMaxK];
+    uint32_t n_coh;
+    uint32_t next;            // the workgroup's next item
+};
+constexpr uint32_t kSlots = 8;  // coherence candidates (and random ones) of a member per round
+// words of a candidate's row of terms: rows 4 banks apart, so that eight
+// lanes' float4 reads of their rows cover the banks
+constexpr uint32_t kTermRow = kMaxK + 4;
+constexpr size_t kTeamWaveLds = 2 * kSlots * kTermRow * sizeof(float);
+
+// A run with a team of T waves per item (the workgroup), for batches too
+// small to fill the chip, where the dependency chain binds: an item's time
+// from its last dependency's mail to its own is what counts, not its work.
+// So everything that the dependencies do not decide is done before the wait
+// (weights, the random candidates' pixels and colours, the records of the
+// other neighbours), and after it every candidate is evaluated in full: one
+// round trip for the coherence candidates' pixels, during which the random
+// ones' terms are formed, one in-order sum per lane, one 64-bit minimum in
+// LDS. Pruning, duplicate removal and a leader's merge would each add a
+// dependent step that the idle lanes save nothing by. The winner's own lane
+// posts it.
+template <bool GUIDED, int T>
+__global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f) {
+    const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ MapDesc smaps[kMapCache];
+    __shared__ TeamLds team[2];
+    flow_args(a);
+    float *lut, *glut;
+    const MapDesc* maps;
+    if (threadIdx.x == 0) team[0].next = atomicAdd(f.ticket, 1u);
+    float* rows = reinterpret_cast<float*>(setup_lds<GUIDED>(a, smem, lut, glut, smaps, maps));  // ends with a barrier
+    constexpr int C = lut_copies<GUIDED>();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x % kWave;
+    rows += (size_t)wave * (2 * kSlots * kTermRow);
+    const uint32_t slot4 = (uint32_t)(lane % C) * 4u;
+    MapDesc m0{};
+    if (a.n_maps == 1) m0 = ld_uniform(maps);
+    const uint32_t rper = (a.m + T - 1) / T;
+    const uint32_t r0 = min(a.m, (uint32_t)wave * rper), nrs = min(a.m, r0 + rper) - r0;
+    uint32_t idx = team[0].next;
+    for (uint32_t turn = 0; idx < f.n; turn ^= 1u) {
+        TeamLds* L = &team[turn];
+        const uint32_t item = a.item0 + idx, rel = item - a.pre_base;
+        if (wave == 0) {
+            phase_clock(a, item, 0, lane);
+            if (lane == 0) {
+                team[turn ^ 1u].next = atomicAdd(f.ticket, 1u);
+                L->best = ~0ull;
+            }
+        }
+        const uint32_t flat = gld(a.work + item);
+        const uint32_t kf = gld(a.pre_cnt + rel);
+        const bool has = lane < (int)kf;
+        int32_t o = 0;
+        if (has) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
+        const uint2* rc = a.rcands + (size_t)(item - a.rc_base) * a.m;
+        const int x = (int)(flat % a.W), y = (int)(flat / a.W);
+        if (kf == 0) {
+            // no resolved neighbour: alike for every member
+            if (wave == 0) {
+                const uint4 r = item_at_random(a, maps, item, 0, flat, lane);
+                if (lane == 0) {
+                    const MapDesc& md = maps[r.y & 0xffffu];
+                    mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
+                    if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+                }
+            }
+            __syncthreads();
+            idx = team[turn ^ 1u].next;
+            continue;
+        }
+        const int dx = packed_dx(o), dy = packed_dy(o);
+        const uint32_t nq = has ? nbr_flat(a, x, y, o) : 0u;
+        // a candidate per lane: random ones in lanes 0..7, coherence ones in 8..15
+        const uint32_t sl = (uint32_t)lane & (kSlots - 1);
+        uint32_t sxy = 0, smap = 0, scol = 0, spatch = 0, sidx = 0;
+        bool son = false;
+        uint32_t gp = kOutsidePx;
+        if (GUIDED && has) gp = gld(a.tg + nq);
+        uint32_t px[kSlots], gpx[kSlots];
+        auto random_slots = [&](uint32_t q) {
+            // the round's random candidates: pixels of every neighbour, own colour
+            const uint32_t n = nrs > q * kSlots ? min(nrs - q * kSlots, kSlots) : 0u;
+            if (lane < (int)kSlots) {
+                son = sl < n;
+                if (son) {
+                    const uint2 r = gld(rc + r0 + q * kSlots + sl);
+                    sxy = r.x;
+                    smap = r.y;
+                }
+            }
+#pragma unroll
+            for (uint32_t c = 0; c < kSlots; ++c) {
+                px[c] = gpx[c] = kOutsidePx;
+                if (c < n) {
+                    const uint32_t cxy = (uint32_t)__builtin_amdgcn_readlane((int)sxy, (int)c);
+                    const uint32_t cm = (uint32_t)__builtin_amdgcn_readlane((int)smap, (int)c);
+                    if (has) {
+                        if (a.n_maps == 1) gather_xy<GUIDED>(m0, cxy, -dx, -dy, px[c], gpx[c]);
+                        else gather_xy<GUIDED>(maps[cm], cxy, -dx, -dy, px[c], gpx[c]);
+                    }
+                }
+            }
+            if (lane < (int)kSlots && son) {
+                const MapDesc& md = maps[smap];
+                const uint32_t f0 = (sxy >> 16) * md.w + (sxy & 0xffffu);
+                scol = gld(md.px + f0);
+                spatch = f0;
+            }
+            return n;
+        };
+        uint32_t n_r = random_slots(0);
+        if (wave == T - 1) {
+            // the weights, from the neighbour offsets alone
+            if (has) {
+                L->nd[lane] = o;
+                if (GUIDED) L->gpat[lane] = gp;
+            }
+            wave_sync();
+            item_geometry(a, x, y, kf, L, lane);
+        }
+        if (wave == 0) {
+            const uint4 st = flow_records(f, a, f.dep[rel], nq, has, lane);
+            phase_clock(a, item, 1, lane);
+            bool ok = false;
+            uint32_t cx = 0, cy = 0, cm = 0;
+            if (has) {
+                L->pat[lane] = st.x;
+                cx = (st.y & 0xffffu) - (uint32_t)dx;
+                cy = (st.y >> 16) - (uint32_t)dy;
+                cm = st.z >> 16;
+                ok = cm < a.n_maps && coord_ok(maps[cm], (int)cx, (int)cy);
+            }
+            const uint64_t om = __ballot(ok);
+            if (ok) L->coh[bits_below(om)] = make_uint4(cx | (cy << 16), cm, st.w, 0u);
+            if (lane == 0) L->n_coh = (uint32_t)__popcll(om);
+        }
+        __syncthreads();
+        const uint32_t n_coh = L->n_coh;
+        if (!a.lut_nan && L->avg > 0.0) {
+            if (wave == 0) phase_clock(a, item, 2, lane);
+            NbrRow row;
+            row.q = bytes_scaled<C>(has ? L->pat[lane] : 0u);
+            row.g = GUIDED ? bytes_scaled<C>(gp) : make_uint4(0, 0, 0, 0);
+            row.w = has ? L->w[lane] : 0.0f;
+            const uint32_t cper = (n_coh + T - 1) / T;
+            const uint32_t c0 = min(n_coh, (uint32_t)wave * cper), ncs = min(n_coh, c0 + cper) - c0;
+            // the lane's best candidate so far
+            unsigned long long bkey = ~0ull;
+            uint32_t bxy = 0, bmap = 0, bcol = 0, bpatch = 0;
+            for (uint32_t q = 0;;) {
+                const uint32_t n_c = ncs > q * kSlots ? min(ncs - q * kSlots, kSlots) : 0u;
+                if (lane >= (int)kSlots) {
+                    son = lane < (int)(2 * kSlots) && sl < n_c;
+                    if (son) {
+                        const uint4 e = L->coh[c0 + q * kSlots + sl];
+                        sxy = e.x;
+                        smap = e.y;
+                        spatch = e.z;
+                    }
+                }
+                sidx = lane < (int)kSlots ? n_coh + r0 + q * kSlots + sl : c0 + q * kSlots + sl;
+                uint32_t cpx[kSlots], cgpx[kSlots];
+#pragma unroll
+                for (uint32_t c = 0; c < kSlots; ++c) {
+                    cpx[c] = cgpx[c] = kOutsidePx;
+                    if (c < n_c) {
+                        const uint32_t cxy = (uint32_t)__builtin_amdgcn_readlane((int)sxy, (int)(kSlots + c));
+                        const uint32_t cm = (uint32_t)__builtin_amdgcn_readlane((int)smap, (int)(kSlots + c));
+                        if (has) {
+                            if (a.n_maps == 1) gather_xy<GUIDED>(m0, cxy, dx, dy, cpx[c], cgpx[c]);
+                            else gather_xy<GUIDED>(maps[cm], cxy, dx, dy, cpx[c], cgpx[c]);
+                        }
+                    }
+                }
+                if (lane >= (int)kSlots && son) {
+                    const MapDesc& md = maps[smap];
+                    scol = gld(md.px + (sxy >> 16) * md.w + (sxy & 0xffffu));
+                }
+                // terms: row c of the round's 16, one neighbour per lane
+#pragma unroll
+                for (uint32_t c = 0; c < kSlots; ++c)
+                    if (c < n_r && has) rows[c * kTermRow + lane] = term_at<GUIDED>(row, lut, glut, slot4, px[c], gpx[c]);
+#pragma unroll
+                for (uint32_t c = 0; c < kSlots; ++c)
+                    if (c < n_c && has)
+                        rows[(kSlots + c) * kTermRow + lane] = term_at<GUIDED>(row, lut, glut, slot4, cpx[c], cgpx[c]);
+                wave_sync();
+                if (son) {
+                    // the reference's sequential f32 sum, terms read ahead of the adds
+                    const float* tp = rows + (uint32_t)lane * kTermRow;
+                    float s = 0.0f;
+                    uint32_t j = 0;
+                    for (; j + 16 <= kf; j += 16) {
+                        const float4 q0 = *reinterpret_cast<const float4*>(tp + j);
+                        const float4 q1 = *reinterpret_cast<const float4*>(tp + j + 4);
+                        const float4 q2 = *reinterpret_cast<const float4*>(tp + j + 8);
+                        const float4 q3 = *reinterpret_cast<const float4*>(tp + j + 12);
+                        s = __fadd_rn(s, q0.x); s = __fadd_rn(s, q0.y); s = __fadd_rn(s, q0.z); s = __fadd_rn(s, q0.w);
+                        s = __fadd_rn(s, q1.x); s = __fadd_rn(s, q1.y); s = __fadd_rn(s, q1.z); s = __fadd_rn(s, q1.w);
+                        s = __fadd_rn(s, q2.x); s = __fadd_rn(s, q2.y); s = __fadd_rn(s, q2.z); s = __fadd_rn(s, q2.w);
+                        s = __fadd_rn(s, q3.x); s = __fadd_rn(s, q3.y); s = __fadd_rn(s, q3.z); s = __fadd_rn(s, q3.w);
+                    }
+                    for (; j < kf; ++j) s = __fadd_rn(s, tp[j]);
+                    // a cost the reference's search cannot take over its start
+                    // value counts as that value (find_best_match, ms.rs:1184-1224)
+                    const unsigned long long key =
+                        (unsigned long long)__float_as_uint(s < FLT_MAX ? s : FLT_MAX) << 32 | sidx;
+                    if (key < bkey) {
+                        bkey = key;
+                        bxy = sxy;
+                        bmap = smap;
+                        bcol = scol;
+                        bpatch = spatch;
+                    }
+                }
+                ++q;
+                if (q * kSlots >= nrs && q * kSlots >= ncs) break;
+                wave_sync();
+                n_r = random_slots(q);
+            }
+            if (wave == 0) phase_clock(a, item, 4, lane);
+            if (bkey != ~0ull) atomicMin(&L->best, bkey);
+            __syncthreads();
+            if (wave == 0) phase_clock(a, item, 5, lane);
+            const unsigned long long best = L->best;
+            if (bkey == best) {
+                // the winner's lane (indices differ): Generator::update
+                // (ms.rs:334-377), posted; a new pixel keeps its first score
+                const float cost = __uint_as_float((uint32_t)(best >> 32));
+                mail_post(f, flat, bcol, bxy, bmap, bpatch);
+                gst(a.item_score + item, cost);
+                if (item >= a.first_new) gst(a.score_w + flat, cost);
+            }
+        } else {
+            if (wave == 0) {
+                float best = FLT_MAX;
+                uint32_t bidx = 0;
+                item_exact<GUIDED>(a, maps, item, 0, kf, n_coh, n_coh + a.m, L, lut, glut, lane % C, lane, best, bidx);
+                const uint4 r = item_winner(a, maps, item, 0, n_coh, L, best, bidx, lane);
+                if (lane == 0) {
+                    const MapDesc& md = maps[r.y & 0xffffu];
+                    mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
+                    if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+                }
+            }
+            __syncthreads();
+        }
+        if (wave == 0) phase_clock(a, item, 6, lane);
+        idx = team[turn ^ 1u].next;
     }
     launch_span(a, t_start);
 }
@@ -1779,8 +2177,9 @@ __device__ __forceinline__ void prefetch_item(const PrefetchArgs& a, WaveLds* L,
         n_at = a.bnres[lo];
         bs = a.bounds[lo];
     }
-    const KnnView v{a.W,        a.H,      a.tiles_x, a.tiles_y, a.mask, a.rlist, a.offtab, a.offtab_n,
-                    a.mask_new, a.tile_min, a.rank, n_at};
+    const KnnView v{a.W,    a.H,      a.tiles_x,  a.tiles_y,
+                    a.mask, a.rlist,  a.offtab,   a.offtab_n,
+                    item < a.redo_end ? nullptr : a.mask_new, a.tile_min, a.rank, n_at};
     uint32_t iters, buffered;
     const uint32_t kf = knn_search(v, L, (int)(flat % a.W), (int)(flat / a.W), a.k, n_at, lane, iters, buffered);
     if (lane < (int)kf) gst(a.out_nbrs + (size_t)rel * a.k + lane, L->nd[lane]);
@@ -1790,13 +2189,8 @@ __device__ __forceinline__ void prefetch_item(const PrefetchArgs& a, WaveLds* L,
         if (lane < (int)kf) {
             const int32_t o = L->nd[lane];
             const int X = (int)(flat % a.W) + packed_dx(o), Y = (int)(flat / a.W) + packed_dy(o);
-            if (item < a.redo_end) {
-                // redone by an earlier batch of the segment
-                const uint32_t r = a.rank[(uint32_t)Y * a.W + (uint32_t)X];
-                d = r >= a.locked && r - a.locked < bs;
-            } else if (a.mask_new) {
-                d = px_set(a.mask_new, a.tiles_x, X, Y);
-            }
+            const uint32_t r = gld(a.rank + (uint32_t)Y * a.W + (uint32_t)X);
+            d = r >= a.locked && r - a.locked < bs;
         }
         const uint64_t dm = __ballot(d);
         if (lane == 0) a.out_dep[rel] = dm;
@@ -1968,12 +2362,26 @@ __global__ void k_defer_flush(DeferFlushArgs a) {
     }
 }
 
-// old[p] = state[p] for the first n pixels of the resolved list.
-__global__ void k_state_snapshot(const uint32_t* rlist, uint32_t n, const uint4* state, uint4* old) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t p = rlist[i];
-    old[p] = state[p];
+// StageEndArgs: the records of a dependency-ordered stage into the state,
+// recoloured from the next stage's level. One read of the mail (or of the
+// state), one colour gather and one 16-byte write per pixel: HBM-bound.
+__global__ void k_stage_end(StageEndArgs a) {
+    const uint32_t q = a.q0 + blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= a.q1) return;
+    const uint32_t p = gld(a.rlist + q);
+    const bool item = q >= a.s0 && q < a.s1;
+    uint4 st;
+    if (item) {
+        const unsigned long long* m = a.mail + 2 * (size_t)p;
+        st = mail_record(gld(m), gld(m + 1));
+    } else {
+        st = gld(a.state + p);
+    }
+    if (a.maps) {
+        const MapDesc md = a.maps[st.z & 0xffffu];
+        st.x = gld(md.px + (st.y >> 16) * md.w + (st.y & 0xffffu));
+    }
+    gst(a.state + p, st);
 }
 
 // next_pyramid_level (ms.rs:687-700): recolour every resolved pixel.
@@ -2481,6 +2889,25 @@ void set_launch_events(hipEvent_t start, hipEvent_t stop) {
     g_ev_stop = stop;
 }
 
+namespace {
+struct FlowKernel {
+    void (*fn)(BatchArgs, FlowArgs);
+    uint32_t threads;
+    size_t lds;
+};
+bool flow_kernel(uint32_t team, bool guided, FlowKernel* k) {
+    if (team == 1) {
+        *k = {guided ? k_flow_wave<true> : k_flow_wave<false>, (uint32_t)(kWave * kWavesPerWG), resolve_lds_bytes(guided)};
+        return true;
+    }
+    *k = {nullptr, kWave * team, lut_bytes(guided) + team * kTeamWaveLds};
+    if (team == 2) k->fn = guided ? k_flow_team<true, 2> : k_flow_team<false, 2>;
+    if (team == 4) k->fn = guided ? k_flow_team<true, 4> : k_flow_team<false, 4>;
+    if (team == 8) k->fn = guided ? k_flow_team<true, 8> : k_flow_team<false, 8>;
+    return k->fn != nullptr;
+}
+}  // namespace
+
 hipError_t configure_kernels() {
     for (const void* f : {(const void*)k_engine<true>, (const void*)k_engine<false>}) {
         const hipError_t e0 = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2508,12 +2935,13 @@ hipError_t configure_kernels() {
     e = hipFuncSetAttribute((const void*)k_resolve_coop<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)resolve_small_lds_bytes(false));
     if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)k_resolve_flow<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)resolve_lds_bytes(true));
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)k_resolve_flow<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)resolve_lds_bytes(false));
-    if (e != hipSuccess) return e;
+    for (uint32_t team : {1u, 2u, 4u, 8u})
+        for (bool guided : {false, true}) {
+            FlowKernel k;
+            if (!flow_kernel(team, guided, &k)) return hipErrorInvalidValue;
+            e = hipFuncSetAttribute((const void*)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
+            if (e != hipSuccess) return e;
+        }
     return hipFuncSetAttribute((const void*)k_resolve_small<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)resolve_small_lds_bytes(false));
 }
@@ -2697,10 +3125,6 @@ hipError_t launch_resolve_small(const BatchArgs& a, const uint32_t* bounds, cons
     return hipGetLastError();
 }
 
-size_t flow_lds_bytes(uint32_t team, bool guided) {
-    return lut_bytes(guided) + team * sizeof(WaveLds);
-}
-
 uint32_t persist_max_wgs(bool guided) {
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
@@ -2727,13 +3151,12 @@ hipError_t launch_resolve_persist(const BatchArgs& a, uint32_t wgs, bool guided,
 }
 
 uint32_t flow_max_wgs(uint32_t team, bool guided) {
-    if (team == 0 || team > (uint32_t)kWavesPerWG) return 0;
+    FlowKernel k;
+    if (!flow_kernel(team, guided, &k)) return 0;
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    const void* f = guided ? (const void*)k_resolve_flow<true> : (const void*)k_resolve_flow<false>;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kWave * team, flow_lds_bytes(team, guided)) !=
-        hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k.fn, (int)k.threads, k.lds) != hipSuccess)
         return 0;
     return (uint32_t)(per_cu * cus);
 }
@@ -2741,21 +3164,17 @@ uint32_t flow_max_wgs(uint32_t team, bool guided) {
 hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t wgs, uint32_t team, bool guided,
                                hipStream_t s) {
     if (f.n == 0) return hipSuccess;
-    if (team == 0 || team > (uint32_t)kWavesPerWG || (team & (team - 1)) != 0) return hipErrorInvalidValue;
-    if (wgs == 0 || !f.ticket || !f.dep || !f.flag || !f.overflow || f.epoch == 0 || f.spin_limit == 0)
+    FlowKernel k;
+    if (!flow_kernel(team, guided, &k)) return hipErrorInvalidValue;
+    if (wgs == 0 || !f.ticket || !f.dep || !f.mail || !f.overflow || f.tag == 0 || f.tag > 255 || f.spin_limit == 0)
         return hipErrorInvalidValue;
     // every item needs its neighbour list; test hooks are not supported
     if (!a.pre_nbrs || a.item0 < a.pre_base || a.item0 + f.n > a.pre_end || a.ext_nbrs || a.ext_cands ||
-        a.dbg_nbrs || a.dbg_best || a.knn_only || a.ext_full_cost || a.gmask)
+        a.dbg_nbrs || a.dbg_best || a.knn_only || a.ext_full_cost || a.exact)
         return hipErrorInvalidValue;
-    const uint32_t lds = (uint32_t)flow_lds_bytes(team, guided);
-    if (guided) {
-        hipExtLaunchKernelGGL(k_resolve_flow<true>, dim3(wgs), dim3(kWave * team), lds, s, g_ev_start, g_ev_stop, 0u,
-                              a, f);
-    } else {
-        hipExtLaunchKernelGGL(k_resolve_flow<false>, dim3(wgs), dim3(kWave * team), lds, s, g_ev_start, g_ev_stop,
-                              0u, a, f);
-    }
+    const uint32_t per = team == 1 ? kTicketItems : 1u, most = (f.n + per - 1) / per;
+    hipExtLaunchKernelGGL(k.fn, dim3(wgs < most ? wgs : most), dim3(k.threads), (uint32_t)k.lds, s, g_ev_start, g_ev_stop,
+                          0u, a, f);
     return hipGetLastError();
 }
 
@@ -2795,9 +3214,9 @@ hipError_t launch_defer_flush(const DeferFlushArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_state_snapshot(const uint32_t* rlist, uint32_t n, const uint4* state, uint4* old, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_state_snapshot, dim3((n + 255) / 256), dim3(256), 0, s, rlist, n, state, old);
+hipError_t launch_stage_end(const StageEndArgs& a, hipStream_t s) {
+    if (a.q1 <= a.q0) return hipSuccess;
+    hipLaunchKernelGGL(k_stage_end, dim3((a.q1 - a.q0 + 255) / 256), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

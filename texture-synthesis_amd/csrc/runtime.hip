@@ -6,7 +6,8 @@
 // stage seed, stage size, adaptive alpha and 256-entry cost tables
 // (ms.rs:786-858), picks the new pixels in the reference's order
 // (pick_random_unresolved, ms.rs:380-389), and enqueues Jacobi batches of
-// {k_resolve, k_commit} on one stream without waiting on the device.
+// {k_resolve, k_commit} on one stream without waiting on the device; a single
+// job's stages run in dependency order instead (flow_stage).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -626,7 +627,6 @@ struct tsg_job {
         bool done_recorded = false;
         int stage = -1;
         uint64_t n_open = 0, S_eff = 0;
-        uint64_t w_end = 0;    // end of the leading run of latency-bound batches
         uint64_t pre_end = 0;  // items [0, pre_end) have neighbour lists
     } ahead[8];
     bool ahead_on = false;
@@ -669,18 +669,18 @@ struct tsg_job {
     DBuf<uint32_t> pre_n;      // per window item: resolved count at its batch start
     DBuf<int32_t> pre_nbrs;    // per window item: k packed offsets
     DBuf<uint32_t> pre_cnt;
-    // dependency-ordered runs: per pixel the epoch of the run that committed
-    // it, the runs' ticket counter and its value as the next run starts
-    DBuf<uint32_t> flow_flag;
+    // stages in dependency order: two mail words per pixel, and ticket
+    // counters, one per launch (cleared together, used in turn)
+    DBuf<unsigned long long> mail;
     DBuf<uint32_t> flow_ticket;
-    DBuf<uint4> state_old;  // redo runs: the state as the redo segment opened
     // deferred commits: records of the last batches, their batch serials, and
     // three pending masks used in turn (serial % 3)
     DBuf<uint4> state2;
     DBuf<uint32_t> stamp;
     DBuf<uint64_t> pend;
     uint32_t serial = 2;
-    uint32_t flow_epoch = 0, flow_tickets = 0;
+    bool flow_on = false;           // this run's stages go in dependency order
+    uint32_t flow_tag = 0, flow_launches = 0;
     size_t small_used = 0;
     // host bookkeeping
     std::vector<uint32_t> unresolved;
@@ -904,6 +904,7 @@ constexpr int kKinds = 7;
 constexpr size_t kEngineRcBudget = 4u << 20;  // random-candidate chunk of a job under the engine
 constexpr uint64_t kPrefetchCap = 65536;       // items per prefetched kNN window
 constexpr uint32_t kFlowSpin = 1u << 18;       // polls of one dependency wait before a run gives up
+constexpr uint32_t kFlowTickets = 256;         // ticket counters of a job's dependency-ordered launches
 
 hipError_t next_event(tsg_job* j, hipEvent_t* e) {
     if (j->ev_next == j->ev_pool.size()) {
@@ -1017,14 +1018,15 @@ int wait_picks(tsg_job* j, int t) {
 }
 
 // Device bytes of the stage-ahead buffers: two sets sized for the largest
-// stage, or (deep) one set per stage.
+// stage, or (deep) one set per stage, and the mail of the stages run in
+// dependency order.
 uint64_t ahead_set_bytes(const tsg_job* j, uint64_t S) {
     return std::max<uint64_t>(1, S) * (j->prm.random_sample_locations * sizeof(uint2) + j->prm.nearest_neighbors * 4 + 16) +
            (uint64_t)j->tiles_x * j->tiles_y * 20;
 }
-uint64_t ahead_bytes(const tsg_job* j) { return 2 * ahead_set_bytes(j, stage_size(j, 0)); }
+uint64_t ahead_bytes(const tsg_job* j) { return 2 * ahead_set_bytes(j, stage_size(j, 0)) + j->N * 16; }
 uint64_t ahead_bytes_deep(const tsg_job* j) {
-    uint64_t b = 0;
+    uint64_t b = j->N * 16;
     for (int s = 0; s <= (int)j->prm.backtrack_stages; ++s) b += ahead_set_bytes(j, stage_size(j, s));
     return b;
 }
@@ -1086,7 +1088,7 @@ int ahead_stage(tsg_job* j) {
     }
     // the stage's batches (start item, resolved count at the start); the
     // neighbour lists of the items in the leading latency-bound batches
-    // (deep: of every item; the rest search in-kernel)
+    // (in dependency order, or deep: of every item; else the rest search in-kernel)
     std::vector<uint32_t> tab;  // bounds (nb + 1), then resolved counts (nb)
     std::vector<uint32_t> nres_b;
     uint64_t i = 0, nres = n_open, w_end = 0;
@@ -1103,7 +1105,7 @@ int ahead_stage(tsg_job* j) {
     const uint32_t nb = (uint32_t)nres_b.size();
     tab.push_back((uint32_t)S_eff);
     tab.insert(tab.end(), nres_b.begin(), nres_b.end());
-    const uint64_t pre_end = j->ahead_deep ? S_eff : w_end;
+    const uint64_t pre_end = j->ahead_deep || j->flow_on ? S_eff : w_end;
     if (pre_end) {
         HIP_TRY(A.n_at.reserve(tab.size()));
         HIP_TRY(j->ctx->staging_side.upload(A.n_at.p, tab.data(), tab.size() * 4, side));
@@ -1137,7 +1139,6 @@ int ahead_stage(tsg_job* j) {
     A.stage = t;
     A.n_open = n_open;
     A.S_eff = S_eff;
-    A.w_end = w_end;
     A.pre_end = pre_end;
     j->ahead_open = nres;
     j->ahead_next = t + 1;
@@ -1234,7 +1235,7 @@ int step_open_stage(tsg_job* j) {
     const uint32_t m = (uint32_t)j->prm.random_sample_locations;
     st.level = t == 0 ? 0u : (uint32_t)std::min(t, P - 1);
     const MapDesc* maps = j->maps.p + (size_t)st.level * nf;
-    if (st.level > 0) {
+    if (st.level > 0 && !j->flow_on) {  // in dependency order the last stage's end recoloured
         RecolorArgs ra{maps, j->rlist.p, (uint32_t)j->n_res, j->state.p};
         HIP_TRY(timed_launch(j, K_RECOLOR, j->n_res, [&] { return launch_recolor(ra, s); }));
     }
@@ -1512,11 +1513,114 @@ int step_finish(tsg_job* j) {
     return TSG_OK;
 }
 
-// Single job: with stage-ahead neighbour lists, each stage's leading run of
-// new-pixel batches goes to one dependency-ordered launch (k_resolve_flow);
-// other runs of small batches go to one single-workgroup launch; other
-// batches get one k_resolve launch, committing in its last workgroup when
-// the batch holds at most fuse_max items.
+// Progress of a run with a callback: called once batch end i1 of the open
+// stage is in the state, whenever the rounded overall percentage changes.
+struct Progress {
+    tsg_progress_fn cb;
+    void* user;
+    int last_pct = 0;
+    std::vector<uint8_t> snap;
+    bool due(const tsg_job* j, uint64_t i1) const {
+        return cb && pct(j, i1) != last_pct;
+    }
+    static int pct(const tsg_job* j, uint64_t i1) {
+        return (int)std::lround((double)(j->overall_cur + i1) / (double)std::max<uint64_t>(j->overall_total, 1) * 100.0);
+    }
+    int call(tsg_job* j, uint64_t i1) {
+        if (!due(j, i1)) return TSG_OK;
+        last_pct = pct(j, i1);
+        snap.resize(j->N * 4);
+        HIP_TRY(hipStreamSynchronize(j->ctx->stream));
+        std::vector<uint4> stv(j->N);
+        HIP_TRY(hipMemcpy(stv.data(), j->state.p, j->N * sizeof(uint4), hipMemcpyDeviceToHost));
+        for (size_t q = 0; q < j->N; ++q) memcpy(&snap[q * 4], &stv[q].x, 4);
+        cb(user, snap.data(), j->W, j->H, j->overall_cur + i1, j->overall_total, i1, j->step.S);
+        return TSG_OK;
+    }
+};
+
+// Waves per item of the batch of items [i0, i1) in a dependency-ordered
+// stage: a latency-bound batch (at most prefetch_max items) takes the largest
+// team that keeps the batch's items within team_waves waves, at least
+// flow_team, and the stage's first flow_head items take flow_head_team;
+// larger batches take a wave per item.
+uint32_t flow_team_of(const tsg_job* j, uint64_t i0, uint64_t i1) {
+    const tsg_tuning& u = j->tune;
+    if (i1 - i0 > u.prefetch_max) return 1;
+    if (i0 < u.flow_head) return u.flow_head_team;
+    return std::max(u.flow_team, team_for(i1 - i0, u.team_max, u.team_waves));
+}
+
+// The open stage in dependency order (k_flow_team, k_flow_wave): consecutive
+// batches of one team size go to one launch, redo items and new pixels alike;
+// the state stays as the stage opened until the stage's end writes its mail
+// into it, recoloured for the next stage. With a callback the launches also
+// end where it is due, and the items so far enter the state (no later item
+// reads them there: its own batch starts after them).
+int flow_stage(tsg_job* j, Progress& pr) {
+    hipStream_t s = j->ctx->stream;
+    tsg_job::Step& st = j->step;
+    BatchArgs& a = st.a;
+    int rc;
+    // one tag per stage: a pyramid has at most 16 levels, so a run at most 17 stages
+    ++j->flow_tag;
+    const uint32_t lock = (uint32_t)j->locked;
+    uint64_t q0 = 0;  // items below are in the state
+    while (st.i < st.S_eff) {
+        const uint64_t i0 = st.i;
+        uint64_t i1 = 0, b0 = 0, b1 = 0;
+        uint32_t team = 0;
+        bool due = false;
+        while (step_peek(j, b0, b1)) {
+            const uint32_t t = flow_team_of(j, b0, b1);
+            if (team && t != team) break;
+            team = t;
+            step_advance(j, b0, b1);
+            i1 = b1;
+            if ((due = pr.due(j, i1))) break;
+        }
+        const uint32_t most = flow_max_wgs(team, j->guided);
+        const uint32_t wgs = j->tune.flow_wgs ? std::min(j->tune.flow_wgs, most) : most;
+        if (j->flow_launches == kFlowTickets) {
+            HIP_TRY(hipMemsetAsync(j->flow_ticket.p, 0, kFlowTickets * 4, s));
+            j->flow_launches = 0;
+        }
+        const uint32_t n = (uint32_t)(i1 - i0);
+        const FlowArgs f{j->flow_ticket.p + j->flow_launches++, n, j->aset(st.t).dep.p, j->mail.p, j->flow_tag, kFlowSpin,
+                         j->overflow.p};
+        a.item0 = (uint32_t)i0;
+        a.item1 = (uint32_t)i1;
+        HIP_TRY(timed_launch(j, team == 1 ? K_RESOLVE : K_RUN, n,
+                             [&] { return launch_resolve_flow(a, f, wgs, team, j->guided, s); }));
+        if ((rc = ahead_poll(j, false))) return rc;
+        if (due) {
+            const StageEndArgs e{j->rlist.p, lock + (uint32_t)q0, lock + (uint32_t)i1, lock, lock + (uint32_t)st.S_eff,
+                                 j->mail.p, nullptr, j->state.p};
+            HIP_TRY(timed_launch(j, K_COMMIT, i1 - q0, [&] { return launch_stage_end(e, s); }));
+            q0 = i1;
+            if ((rc = pr.call(j, i1))) return rc;
+        }
+    }
+    // the next stage's level: its opening recolours every resolved pixel
+    const int P = (int)j->prm.backtrack_stages;
+    const uint32_t next = st.t < P ? (uint32_t)std::min(st.t + 1, P - 1) : 0u;
+    const StageEndArgs e{j->rlist.p,
+                         next ? 0u : lock,
+                         next ? (uint32_t)j->n_res : lock + (uint32_t)st.S_eff,
+                         lock,
+                         lock + (uint32_t)st.S_eff,
+                         j->mail.p,
+                         next ? j->maps.p + (size_t)next * j->filt.size() : nullptr,
+                         j->state.p};
+    HIP_TRY(timed_launch(j, K_COMMIT, st.S_eff, [&] { return launch_stage_end(e, s); }));
+    return TSG_OK;
+}
+
+// Single job: with stage-ahead neighbour lists, every stage runs in
+// dependency order (flow_stage). Else runs of small batches go to one
+// single-workgroup launch; other batches get one k_resolve launch,
+// committing in its last workgroup when the batch holds at most fuse_max
+// items.
 int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     hipStream_t s = j->ctx->stream;
     int rc;
@@ -1526,6 +1630,16 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     const bool deep_fits = j->prm.backtrack_stages + 1 <= 8 && ahead_bytes_deep(j) <= kAheadBudget;
     j->ahead_deep = j->tune.ahead >= 2 && !j->prm.tiling_mode && deep_fits;
     j->ahead_on = j->ahead_deep || (j->tune.ahead && !j->prm.tiling_mode && ahead_bytes(j) <= kAheadBudget);
+    // dependency order needs the stage-ahead neighbour lists
+    j->flow_on = j->ahead_on && j->tune.flow;
+    if (j->flow_on) {
+        HIP_TRY(j->mail.reserve(2 * j->N));
+        HIP_TRY(hipMemsetAsync(j->mail.p, 0, j->N * 16, s));
+        j->flow_tag = 0;
+        HIP_TRY(j->flow_ticket.reserve(kFlowTickets));
+        HIP_TRY(hipMemsetAsync(j->flow_ticket.p, 0, kFlowTickets * 4, s));
+        j->flow_launches = 0;
+    }
     if (j->ahead_on) {
         const uint64_t smax = std::max<uint64_t>(1, stage_size(j, 0));
         for (int q = 0; q < 2 && !j->ahead_deep; ++q) {
@@ -1548,31 +1662,8 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
         HIP_TRY(hipStreamWaitEvent(j->ctx->side, e, 0));
         if ((rc = ahead_stage(j))) return rc;
     }
-    // dependency-ordered runs need the stage-ahead neighbour lists
-    bool flow_on = j->ahead_on && j->tune.flow;
-    const uint32_t flow_team = j->tune.flow_team;
-    uint32_t flow_wgs = 0;
-    if (flow_on) {
-        const uint32_t mx = flow_max_wgs(flow_team, j->guided);
-        flow_wgs = j->tune.flow_wgs ? std::min(j->tune.flow_wgs, mx) : mx;
-        flow_on = flow_wgs > 0;
-    }
-    if (flow_on) {
-        if (j->flow_flag.n < j->N) {
-            HIP_TRY(j->flow_flag.alloc(j->N));
-            HIP_TRY(hipMemsetAsync(j->flow_flag.p, 0, j->N * 4, s));
-            j->flow_epoch = 0;
-        }
-        if (j->tune.flow >= 2 && j->state_old.n < j->N) HIP_TRY(j->state_old.alloc(j->N));
-    }
     // persistent single-wave batches
     const uint32_t persist_wgs = j->tune.persist ? persist_max_wgs(j->guided) : 0u;
-    if (flow_on && !j->flow_ticket.n) {
-        // the ticket counter of dependency-ordered runs
-        HIP_TRY(j->flow_ticket.alloc(1));
-        HIP_TRY(hipMemsetAsync(j->flow_ticket.p, 0, 4, s));
-        j->flow_tickets = 0;
-    }
     // deferred commits for throughput-bound batches (not in tiling mode,
     // whose commits also set ghost flags)
     const bool defer_on = j->tune.defer && !j->prm.tiling_mode;
@@ -1605,73 +1696,10 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
         j->serial += 2;  // no stamp names the batch before the next one
         return TSG_OK;
     };
-    int last_pct = 0;
-    std::vector<uint8_t> snap;
+    Progress pr{cb, user};
     auto progress = [&](uint64_t i1) -> int {
         if (int rc3 = flush_def()) return rc3;
-        int pct = (int)std::lround((double)(j->overall_cur + i1) / (double)std::max<uint64_t>(j->overall_total, 1) *
-                                   100.0);
-        if (pct == last_pct) return TSG_OK;
-        last_pct = pct;
-        snap.resize(j->N * 4);
-        HIP_TRY(hipStreamSynchronize(s));
-        std::vector<uint4> stv(j->N);
-        HIP_TRY(hipMemcpy(stv.data(), j->state.p, j->N * sizeof(uint4), hipMemcpyDeviceToHost));
-        for (size_t q = 0; q < j->N; ++q) memcpy(&snap[q * 4], &stv[q].x, 4);
-        cb(user, snap.data(), j->W, j->H, j->overall_cur + i1, j->overall_total, i1, j->step.S);
-        return TSG_OK;
-    };
-    // items [i0, end) of the open stage in one dependency-ordered launch;
-    // old: a redo run, which reads neighbours not redone before it from the
-    // state as the segment opened
-    auto flow_run = [&](uint64_t i0, uint64_t end, const uint4* old) -> int {
-        if (int rc3 = flush_def()) return rc3;
-        tsg_job::Step& st = j->step;
-        BatchArgs& a = st.a;
-        a.item0 = (uint32_t)i0;
-        a.item1 = (uint32_t)end;
-        a.n_res = (uint32_t)j->n_res;
-        if (++j->flow_epoch == 0) {
-            HIP_TRY(hipMemsetAsync(j->flow_flag.p, 0, j->N * 4, s));
-            j->flow_epoch = 1;
-        }
-        // the run's leading items (its longest serial chain) in a launch of
-        // their own with larger teams; the rest follow in stream order, under
-        // the same epoch, so their waits on the head are already satisfied
-        uint64_t h = 0;
-        const uint32_t head_wgs = j->tune.flow_head ? flow_max_wgs(j->tune.flow_head_team, j->guided) : 0u;
-        if (head_wgs && i0 + j->tune.flow_head < end) {
-            h = j->tune.flow_head;
-            const uint32_t nh = (uint32_t)h;
-            const uint32_t gh = std::min(head_wgs, nh);
-            const FlowArgs fh{j->flow_ticket.p, j->flow_tickets, nh, j->aset(st.t).dep.p, j->flow_flag.p,
-                              j->flow_epoch, kFlowSpin, j->overflow.p, old};
-            HIP_TRY(timed_launch(j, K_RUN, nh, [&] {
-                BatchArgs fa = a;
-                fa.item1 = (uint32_t)(i0 + h);
-                fa.result = nullptr;
-                return launch_resolve_flow(fa, fh, gh, j->tune.flow_head_team, j->guided, s);
-            }));
-            j->flow_tickets += nh + gh;
-        }
-        const uint32_t n = (uint32_t)(end - i0 - h);
-        const uint32_t g = std::min(flow_wgs, n);
-        const FlowArgs f{j->flow_ticket.p, j->flow_tickets, n, j->aset(st.t).dep.p, j->flow_flag.p,
-                         j->flow_epoch, kFlowSpin, j->overflow.p, old};
-        HIP_TRY(timed_launch(j, K_RUN, n, [&] {
-            BatchArgs fa = a;  // results stay in registers
-            fa.item0 = (uint32_t)(i0 + h);
-            fa.result = nullptr;
-            return launch_resolve_flow(fa, f, g, flow_team, j->guided, s);
-        }));
-        j->flow_tickets += n + g;
-        while (st.i < end) {
-            const uint64_t b0 = st.i, b1 = batch_end(j, b0, st.redo, st.S_eff);
-            step_advance(j, b0, b1);
-        }
-        if (st.i != end) return fail(TSG_ERR_DEVICE, "dependency-ordered run out of step");
-        if (cb) return progress(end);
-        return TSG_OK;
+        return pr.call(j, i1);
     };
     std::vector<uint32_t> sb_bounds, sb_nres;
     bool sb_coop = false;  // the pending run goes to the cooperative kernel
@@ -1710,25 +1738,9 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     while (!step_done(j)) {
         if ((rc = step_open_stage(j))) return rc;
         uint64_t i0, i1;
+        if (j->flow_on && (rc = flow_stage(j, pr))) return rc;
         while (step_peek(j, i0, i1)) {
             if ((rc = ahead_poll(j, false))) return rc;
-            tsg_job::Step& st = j->step;
-            const uint64_t flow_end = flow_on ? std::min<uint64_t>(j->aset(st.t).w_end, st.S_eff) : 0;
-            if (flow_on && j->tune.flow >= 2 && i0 == 0 && st.redo_eff > 0 && flow_end > 0) {
-                // the stage's leading redo batches: one run over a snapshot
-                // of the resolved pixels' state
-                if ((rc = flush_small())) return rc;
-                HIP_TRY(launch_state_snapshot(j->rlist.p, (uint32_t)j->n_res, j->state.p, j->state_old.p, s));
-                if ((rc = flow_run(0, std::min(flow_end, st.redo_eff), j->state_old.p))) return rc;
-                continue;
-            }
-            if (flow_on && i0 == st.redo_eff && flow_end > i0) {
-                // the stage's new-pixel batches with neighbour lists: one
-                // dependency-ordered run
-                if ((rc = flush_small())) return rc;
-                if ((rc = flow_run(i0, flow_end, nullptr))) return rc;
-                continue;
-            }
             if (step_wants_prefetch(j, i0, i1)) {
                 // earlier small batches read the previous window: launch them first
                 if ((rc = flush_small())) return rc;
@@ -1850,7 +1862,7 @@ size_t job_footprint(const tsg_job* j) {
     for (const tsg_job::Ahead& A : j->ahead)
         b += A.rc.n * sizeof(uint2) + A.nbrs.n * 4 + A.cnt.n * 4 + A.n_at.n * 4 + A.mend.n * 8 + A.mnew.n * 8 +
              A.tmin.n * 4 + A.dep.n * 8;
-    b += j->flow_flag.n * 4 + j->flow_ticket.n * 4 + j->state_old.n * sizeof(uint4);
+    b += j->mail.n * 8 + j->flow_ticket.n * 4;
     b += j->state2.n * sizeof(uint4) + j->stamp.n * 4 + j->pend.n * 8;
     b += j->st_part.n * 8 + j->st_part_n.n * 8 + j->eng.luts.n * 4;
     return b;
@@ -2782,14 +2794,17 @@ void tsg_tuning_default(tsg_tuning* t) {
     t->fuse_max = 0;
     t->team_max = 8;
     t->team_waves = 4096;
-    t->prefetch_max = 1024;  // autotuned: 26.3 ms against 27.2 ms at 2048
+    t->prefetch_max = 1024;
     // 2 (a set per stage, every neighbour list ahead) measured 27.2 ms against
     // 26.9 ms: the second stream's kernels wait for free slots behind the
     // latency-bound launches instead of filling them
     t->ahead = 1;
     t->coop_wgs = 0;  // a grid barrier costs more than the launches it saves (measured)
     t->coop_max = 0;
-    t->flow = 1;  // 38.9 -> 27.9 ms on that workload
+    // stages in dependency order: 21.7 -> 13.5 ms on that workload against
+    // dependency-ordered runs of the leading new-pixel batches alone, 7.1 ->
+    // 2.5 ms at 64^2, 51.5 -> 41.9 ms at 2048^2
+    t->flow = 1;
     t->flow_wgs = 0;
     t->flow_team = 4;
     // 1 measured 26.99 ms against 26.34 ms (1024^2) and 71.5 against 67.8 ms
@@ -2800,8 +2815,6 @@ void tsg_tuning_default(tsg_tuning* t) {
     // per-8-items launch measured 24.05 ms against 25.1 ms for the persistent
     // one, which its 128 VGPRs hold at two workgroups
     t->persist = 0;
-    // 25.6 ms against 26.1 ms (1024-item heads of 256..2048 measured alike;
-    // 4-wave heads 25.9, 2-wave heads 26.7)
     t->flow_head = 1024;
     t->flow_head_team = 8;
 }
