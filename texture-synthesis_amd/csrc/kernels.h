@@ -167,6 +167,30 @@ struct StageEndArgs {
     uint4* state;
 };
 
+// A stage's pick order (pick_random_unresolved, ms.rs:380-389): step q takes
+// entry idx = draw(seed + q, L0 - q) of the unresolved list, the list's last
+// entry takes its place and the list shrinks by one. The picks go to the
+// resolved list from position pos0 on, with their ranks, and into the tile
+// masks; the list left over goes to u1.
+struct PickArgs {
+    uint64_t seed;            // of step 0
+    uint32_t n, L0;           // steps; entries before the first
+    const uint32_t* u0;       // the list (null: entry i is pixel i)
+    uint32_t* u1;             // L0 - n entries
+    uint32_t* idx;            // [n] scratch
+    uint32_t* link;           // [n] scratch
+    uint32_t* head;           // [L0] scratch
+    uint32_t W, tiles_x, tiles;
+    uint32_t* rlist;
+    uint32_t* rank;
+    uint32_t pos0;
+    const uint64_t* open;     // resolved mask as the stage opens
+    uint64_t* mend;           // ... and as it ends
+    uint64_t* mnew;           // the picks
+    uint32_t* tile_min;       // least resolved-list position of each tile's picks
+};
+hipError_t launch_picks(const PickArgs& a, hipStream_t s);
+
 struct RandArgs {
     const MapDesc* maps;
     uint32_t n_maps;

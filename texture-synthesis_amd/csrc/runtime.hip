@@ -680,6 +680,11 @@ struct tsg_job {
     DBuf<uint64_t> pend;
     uint32_t serial = 2;
     bool flow_on = false;           // this run's stages go in dependency order
+    // their pick orders, on the device: the unresolved list (null: every
+    // pixel in order) before and after a stage's picks, and scratch
+    DBuf<uint32_t> unres[2], pick_idx, pick_link, pick_head;
+    const uint32_t* pick_list = nullptr;
+    uint64_t pick_left = 0;         // entries of the list
     uint32_t flow_tag = 0, flow_launches = 0;
     size_t small_used = 0;
     // host bookkeeping
@@ -879,6 +884,19 @@ int init_state(tsg_job* j) {
     return TSG_OK;
 }
 
+// The unresolved list of a run whose pick orders are drawn on the device.
+int picks_begin(tsg_job* j) {
+    j->pick_left = j->N0;
+    j->pick_list = nullptr;
+    if (j->N0 < j->N) {
+        // inpainting or random init: not every pixel in order
+        HIP_TRY(j->unres[0].reserve(j->N0));
+        HIP_TRY(j->ctx->staging.upload(j->unres[0].p, j->unresolved.data(), j->N0 * 4, j->ctx->stream));
+        j->pick_list = j->unres[0].p;
+    }
+    return TSG_OK;
+}
+
 // End of the batch starting at item i of stage t when n_res pixels are resolved.
 uint64_t batch_end_at(const tsg_job* j, int t, uint64_t i, uint64_t n_res, uint64_t redo, uint64_t S_eff) {
     uint64_t redo_eff = std::min<uint64_t>(redo, S_eff);
@@ -1018,15 +1036,15 @@ int wait_picks(tsg_job* j, int t) {
 }
 
 // Device bytes of the stage-ahead buffers: two sets sized for the largest
-// stage, or (deep) one set per stage, and the mail of the stages run in
-// dependency order.
+// stage, or (deep) one set per stage, and the mail and pick lists of the
+// stages run in dependency order.
 uint64_t ahead_set_bytes(const tsg_job* j, uint64_t S) {
     return std::max<uint64_t>(1, S) * (j->prm.random_sample_locations * sizeof(uint2) + j->prm.nearest_neighbors * 4 + 16) +
            (uint64_t)j->tiles_x * j->tiles_y * 20;
 }
-uint64_t ahead_bytes(const tsg_job* j) { return 2 * ahead_set_bytes(j, stage_size(j, 0)) + j->N * 16; }
+uint64_t ahead_bytes(const tsg_job* j) { return 2 * ahead_set_bytes(j, stage_size(j, 0)) + j->N * 36; }
 uint64_t ahead_bytes_deep(const tsg_job* j) {
-    uint64_t b = j->N * 16;
+    uint64_t b = j->N * 36;
     for (int s = 0; s <= (int)j->prm.backtrack_stages; ++s) b += ahead_set_bytes(j, stage_size(j, s));
     return b;
 }
@@ -1038,8 +1056,6 @@ int ahead_stage(tsg_job* j) {
     const int P = (int)j->prm.backtrack_stages;
     const int t = j->ahead_next;
     if (t > P) return TSG_OK;
-    int rc = wait_picks(j, t);
-    if (rc) return rc;
     tsg_job::Ahead& A = j->aset(t);
     hipStream_t side = j->ctx->side;
     const uint32_t nf = (uint32_t)j->filt.size();
@@ -1051,8 +1067,15 @@ int ahead_stage(tsg_job* j) {
     const uint64_t pss = (uint64_t)Pcg32::seed_from_u64(j->prm.seed + (uint64_t)ps).next_u32();
     const uint64_t n_open = j->ahead_open;
     const uint64_t redo = n_open - j->locked;
-    const std::vector<uint32_t>& picks = j->picks_keep[t];
-    const uint64_t S_eff = S > redo ? redo + picks.size() : S;
+    uint64_t n_new = 0;
+    if (j->flow_on) {
+        n_new = S > redo ? std::min(S - redo, j->pick_left) : 0;
+    } else {
+        int rc = wait_picks(j, t);
+        if (rc) return rc;
+        n_new = j->picks_keep[t].size();
+    }
+    const uint64_t S_eff = S > redo ? redo + n_new : S;
     const uint64_t redo_eff = std::min(redo, S_eff);
     if (A.done_recorded) HIP_TRY(hipStreamWaitEvent(side, A.done, 0));
     const size_t tiles = (size_t)j->tiles_x * j->tiles_y;
@@ -1068,23 +1091,59 @@ int ahead_stage(tsg_job* j) {
         HIP_TRY(A.tmin.reserve(tiles));
         if (!A.ready) HIP_TRY(hipEventCreateWithFlags(&A.ready, hipEventDisableTiming));
     }
-    // random candidates of every item (ms.rs:549-599: stage seed, item index, level maps)
+    // random candidates of every item (ms.rs:549-599: stage seed, item index,
+    // level maps); the first stage's on the job's stream, which has nothing
+    // else to run yet
     if (S_eff) {
+        hipStream_t rs = t == 0 && j->flow_on ? j->ctx->stream : side;
         RandArgs ra{j->maps.p + (size_t)level * nf, nf, pss, 0u, (uint32_t)S_eff, m, A.rc.p, j->overflow.p};
-        HIP_TRY(timed_launch_on(j, side, K_RAND, S_eff, [&] { return launch_rand(ra, side); }));
+        HIP_TRY(timed_launch_on(j, rs, K_RAND, S_eff, [&] { return launch_rand(ra, rs); }));
     }
     // picks into the resolved list, their ranks, the stage's picks as a mask
     // (with each tile's least rank) and the mask at the stage end
     const uint64_t* open_mask = t == 0 ? j->mask.p : j->aset(t - 1).mend.p;
-    HIP_TRY(hipMemcpyAsync(A.mend.p, open_mask, tiles * 8, hipMemcpyDeviceToDevice, side));
-    HIP_TRY(hipMemsetAsync(A.mnew.p, 0, tiles * 8, side));
-    HIP_TRY(hipMemsetAsync(A.tmin.p, 0xff, tiles * 4, side));
-    if (!picks.empty()) {
-        const uint32_t lo = (uint32_t)n_open, hi = (uint32_t)(n_open + picks.size());
-        HIP_TRY(j->ctx->staging_side.upload(j->rlist.p + n_open, picks.data(), picks.size() * 4, side));
-        HIP_TRY(launch_rank(j->rlist.p, lo, hi, j->rank.p, side));
-        HIP_TRY(launch_mask_or(j->rlist.p, lo, hi, j->W, j->tiles_x, A.mnew.p, A.tmin.p, side));
-        HIP_TRY(launch_mask_or(j->rlist.p, lo, hi, j->W, j->tiles_x, A.mend.p, nullptr, side));
+    if (j->flow_on) {
+        PickArgs pk{};
+        pk.seed = pss + redo;
+        pk.n = (uint32_t)n_new;
+        pk.L0 = (uint32_t)j->pick_left;
+        pk.u0 = j->pick_list;
+        if (n_new) {
+            DBuf<uint32_t>& rest = j->unres[j->pick_list == j->unres[0].p ? 1 : 0];
+            HIP_TRY(rest.reserve(std::max<uint64_t>(1, j->pick_left - n_new)));
+            HIP_TRY(j->pick_idx.reserve(j->N0));
+            HIP_TRY(j->pick_link.reserve(j->N0));
+            HIP_TRY(j->pick_head.reserve(j->N0));
+            pk.u1 = rest.p;
+            pk.idx = j->pick_idx.p;
+            pk.link = j->pick_link.p;
+            pk.head = j->pick_head.p;
+            j->pick_list = rest.p;
+            j->pick_left -= n_new;
+        }
+        pk.W = j->W;
+        pk.tiles_x = j->tiles_x;
+        pk.tiles = (uint32_t)tiles;
+        pk.rlist = j->rlist.p;
+        pk.rank = j->rank.p;
+        pk.pos0 = (uint32_t)n_open;
+        pk.open = open_mask;
+        pk.mend = A.mend.p;
+        pk.mnew = A.mnew.p;
+        pk.tile_min = A.tmin.p;
+        HIP_TRY(launch_picks(pk, side));
+    } else {
+        const std::vector<uint32_t>& picks = j->picks_keep[t];
+        HIP_TRY(hipMemcpyAsync(A.mend.p, open_mask, tiles * 8, hipMemcpyDeviceToDevice, side));
+        HIP_TRY(hipMemsetAsync(A.mnew.p, 0, tiles * 8, side));
+        HIP_TRY(hipMemsetAsync(A.tmin.p, 0xff, tiles * 4, side));
+        if (!picks.empty()) {
+            const uint32_t lo = (uint32_t)n_open, hi = (uint32_t)(n_open + picks.size());
+            HIP_TRY(j->ctx->staging_side.upload(j->rlist.p + n_open, picks.data(), picks.size() * 4, side));
+            HIP_TRY(launch_rank(j->rlist.p, lo, hi, j->rank.p, side));
+            HIP_TRY(launch_mask_or(j->rlist.p, lo, hi, j->W, j->tiles_x, A.mnew.p, A.tmin.p, side));
+            HIP_TRY(launch_mask_or(j->rlist.p, lo, hi, j->W, j->tiles_x, A.mend.p, nullptr, side));
+        }
     }
     // the stage's batches (start item, resolved count at the start); the
     // neighbour lists of the items in the leading latency-bound batches
@@ -1159,6 +1218,16 @@ int ahead_poll(tsg_job* j, bool block) {
         j->ahead_wanted = false;
         return TSG_OK;
     }
+    if (j->flow_on) {
+        // nothing to wait for; with a set per stage, every stage's at once:
+        // they fill the chip while the first stages' chains leave it idle
+        int rc;
+        do {
+            if ((rc = ahead_stage(j))) return rc;
+        } while (j->ahead_deep && j->ahead_next <= (int)j->prm.backtrack_stages);
+        j->ahead_wanted = false;
+        return TSG_OK;
+    }
     if (!block && !picks_available(j, j->ahead_next)) return TSG_OK;
     j->ahead_wanted = false;
     return ahead_stage(j);
@@ -1188,9 +1257,9 @@ int step_begin(tsg_job* j) {
         j->picks_keep.assign(P + 1, {});
         j->picks_ready.assign(P + 1, 0);
         j->pk_start_res = j->n_res;
-        j->pk_state = 1;
+        j->pk_state = j->flow_on ? 0 : 1;
     }
-    j->ctx->picks.submit(j);
+    if (!j->flow_on) j->ctx->picks.submit(j);
     j->lut_keep.assign(P + 1, std::vector<float>(512));
     j->small_used = 0;
     j->n_batches = 0;
@@ -1251,10 +1320,14 @@ int step_open_stage(tsg_job* j) {
     uint32_t lut_nan = 0;
     for (float v : j->lut_keep[t]) lut_nan |= (uint32_t)std::isnan(v);
     HIP_TRY(j->ctx->staging.upload(j->lut.p, j->lut_keep[t].data(), 512 * 4, s));
-    int rc = wait_picks(j, t);
-    if (rc) return rc;
+    if (!j->flow_on) {
+        int rc = wait_picks(j, t);
+        if (rc) return rc;
+    }
     st.S_eff = st.S;
-    if (st.S > st.redo) {
+    if (j->flow_on) {
+        st.S_eff = j->aset(t).S_eff;
+    } else if (st.S > st.redo) {
         st.S_eff = st.redo + j->picks_keep[t].size();
         if (!j->picks_keep[t].empty() && !j->ahead_on) {
             HIP_TRY(j->ctx->staging.upload(j->rlist.p + j->locked + st.redo, j->picks_keep[t].data(),
@@ -1273,8 +1346,9 @@ int step_open_stage(tsg_job* j) {
         if (A.stage != t || A.n_open != j->n_res || A.S_eff != st.S_eff)
             return fail(TSG_ERR_DEVICE, "stage-ahead buffers out of step");
         HIP_TRY(hipStreamWaitEvent(s, A.ready, 0));
-        j->ahead_wanted = true;
-        int rc2 = ahead_poll(j, false);
+        if (j->ahead_next <= P) j->ahead_wanted = true;
+        // in dependency order the stage's own launches go first
+        int rc2 = j->flow_on ? TSG_OK : ahead_poll(j, false);
         if (rc2) return rc2;
     }
     BatchArgs& a = st.a;
@@ -1624,15 +1698,22 @@ int flow_stage(tsg_job* j, Progress& pr) {
 int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     hipStream_t s = j->ctx->stream;
     int rc;
-    if ((rc = step_begin(j))) return rc;
     // content-independent work ahead on the side stream when the buffer
-    // sets fit the budget: one per stage (deep), else two of the largest stage
+    // sets fit the budget: one per stage (deep), else two of the largest
+    // stage. In dependency order a set per stage is also taken where it holds
+    // no more than the two would (at p = 0.5 it never does): the preparation
+    // then runs ahead of the stages without waiting for a set to come free.
+    const bool ahead_ok = j->tune.ahead && !j->prm.tiling_mode;
+    const bool two_fit = ahead_bytes(j) <= kAheadBudget;
     const bool deep_fits = j->prm.backtrack_stages + 1 <= 8 && ahead_bytes_deep(j) <= kAheadBudget;
-    j->ahead_deep = j->tune.ahead >= 2 && !j->prm.tiling_mode && deep_fits;
-    j->ahead_on = j->ahead_deep || (j->tune.ahead && !j->prm.tiling_mode && ahead_bytes(j) <= kAheadBudget);
+    j->ahead_deep = ahead_ok && deep_fits &&
+                    (j->tune.ahead >= 2 || (j->tune.flow && two_fit && ahead_bytes_deep(j) <= ahead_bytes(j)));
+    j->ahead_on = j->ahead_deep || (ahead_ok && two_fit);
     // dependency order needs the stage-ahead neighbour lists
     j->flow_on = j->ahead_on && j->tune.flow;
+    if ((rc = step_begin(j))) return rc;
     if (j->flow_on) {
+        if ((rc = picks_begin(j))) return rc;
         HIP_TRY(j->mail.reserve(2 * j->N));
         HIP_TRY(hipMemsetAsync(j->mail.p, 0, j->N * 16, s));
         j->flow_tag = 0;
@@ -1862,7 +1943,8 @@ size_t job_footprint(const tsg_job* j) {
     for (const tsg_job::Ahead& A : j->ahead)
         b += A.rc.n * sizeof(uint2) + A.nbrs.n * 4 + A.cnt.n * 4 + A.n_at.n * 4 + A.mend.n * 8 + A.mnew.n * 8 +
              A.tmin.n * 4 + A.dep.n * 8;
-    b += j->mail.n * 8 + j->flow_ticket.n * 4;
+    b += j->mail.n * 8 + j->flow_ticket.n * 4 + j->unres[0].n * 4 + j->unres[1].n * 4 + j->pick_idx.n * 4 +
+         j->pick_link.n * 4 + j->pick_head.n * 4;
     b += j->state2.n * sizeof(uint4) + j->stamp.n * 4 + j->pend.n * 8;
     b += j->st_part.n * 8 + j->st_part_n.n * 8 + j->eng.luts.n * 4;
     return b;
@@ -2211,6 +2293,8 @@ int batch_run_alone(tsg_batch* b) {
             A.tmin.release();
             A.dep.release();
         }
+        j->mail.release();
+        for (DBuf<uint32_t>* d : {&j->unres[0], &j->unres[1], &j->pick_idx, &j->pick_link, &j->pick_head}) d->release();
         g_pool_release = false;
         b->done.push_back(e);
     }
