@@ -21,7 +21,7 @@ struct BatchArgs {
     const uint32_t* work;    // stage work list: flat pixel of item i
     const uint32_t* rlist;   // resolved list (first n_res entries committed)
     uint32_t n_res;
-    const uint2* rcands;     // random candidates, item-major, m per item
+    const uint32_t* rcands;  // random candidates, item-major, m per item, rand_words() words each
     uint32_t rc_base;        // item index of rcands[0]
     uint32_t m;
     const int32_t* offtab;   // ring offsets (dx & 0xffff | dy << 16), canonical order
@@ -125,6 +125,7 @@ struct PrefetchArgs {
     // earlier batch of the stage resolves (rank - locked, its position in the
     // work list, below the item's batch start); needs the batch table
     uint64_t* out_dep;            // [item - item0]
+    uint32_t per_wave;            // with the batch table: items of a wave (set by the launcher)
 };
 
 // A dependency-ordered run: consecutive items [a.item0, a.item0 + n) of one
@@ -191,14 +192,18 @@ struct PickArgs {
 };
 hipError_t launch_picks(const PickArgs& a, hipStream_t s);
 
+// Words of a random candidate: x | y << 16, and its map unless there is but one.
+__host__ __device__ constexpr uint32_t rand_words(uint32_t n_maps) { return n_maps == 1 ? 1u : 2u; }
+
 struct RandArgs {
     const MapDesc* maps;
     uint32_t n_maps;
     uint64_t stage_seed;
     uint32_t item0, item1;
     uint32_t m;
-    uint2* out;              // [item - item0][m]
+    uint32_t* out;           // [item - item0][m], rand_words(n_maps) words each
     uint32_t* overflow;      // set when a rejection loop hits its bound
+    uint32_t masked;         // some map has a sample mask
 };
 
 struct CommitArgs {
@@ -314,7 +319,7 @@ struct QJob {
     const QPhase* phases;      // this launch's program
     uint32_t n_phases;
     uint32_t xcc;
-    uint2* rc;
+    uint32_t* rc;
     uint4* result;
     uint32_t* overflow;
     uint64_t* mend;

@@ -416,7 +416,8 @@ __device__ __forceinline__ uint64_t filter_new(const KnnView& v, int gx, int gy,
 }
 
 // Exhaustive scan of the resolved list (sparse phase).
-__device__ __forceinline__ void knn_list(const KnnView& a, WaveLds* L, uint32_t n_res, int x, int y, uint32_t k, int lane, Sel& s) {
+template <class Lds>
+__device__ __forceinline__ void knn_list(const KnnView& a, Lds* L, uint32_t n_res, int x, int y, uint32_t k, int lane, Sel& s) {
     // four chunks of the list per memory round trip
     for (uint32_t base = 0; base < n_res; base += 4 * kWave) {
         uint32_t f[4];
@@ -490,7 +491,8 @@ constexpr int kRingU = 1;
 // order, one tile per lane, the set bits of each tile taken lane-parallel.
 // Stops when k collected points lie closer than any pixel outside the
 // completed rings (every point that close has been collected).
-__device__ __forceinline__ void knn_rings(const KnnView& a, WaveLds* L, int x, int y, uint32_t k, int lane, Sel& s,
+template <class Lds>
+__device__ __forceinline__ void knn_rings(const KnnView& a, Lds* L, int x, int y, uint32_t k, int lane, Sel& s,
                                           uint32_t& iters) {
     const int tx = x >> 3, ty = y >> 3;
     // tiles that can hold points: the grid, plus the ghost margins in tiling mode
@@ -575,8 +577,8 @@ __device__ __forceinline__ void knn_rings(const KnnView& a, WaveLds* L, int x, i
 // order: 4 (256) where latency binds; fewer where the VALU binds, since a
 // dense mask holds k neighbours within the first 64 or so. Returns the
 // number found (<= k).
-template <int KU>
-__device__ __forceinline__ uint32_t knn_table(const KnnView& a, WaveLds* L, int x, int y, uint32_t k, int lane) {
+template <int KU, class Lds>
+__device__ __forceinline__ uint32_t knn_table(const KnnView& a, Lds* L, int x, int y, uint32_t k, int lane) {
     uint32_t found = 0;
     for (uint32_t base = 0; base < a.offtab_n && found < k; base += KU * kWave) {
         int32_t o[KU];
@@ -606,18 +608,21 @@ __device__ __forceinline__ uint32_t knn_table(const KnnView& a, WaveLds* L, int 
     return found < k ? found : k;
 }
 
+// The offset table pays off when about k / density <= 1024 offsets reach k
+// resolved pixels; sparser masks use the ring search.
+__device__ __forceinline__ bool knn_sparse(const KnnView& v, uint32_t k, uint32_t n_res) {
+    return (uint64_t)n_res * 1024ull < (uint64_t)k * v.W * v.H;
+}
+
 // k nearest of (x, y) among the view's resolved pixels (n_res of them), in
 // canonical order, into L->nd; returns the count (<= k). KU: the offset
 // table's offsets per lane per round trip.
-template <int KU = 4>
-__device__ __forceinline__ uint32_t knn_search(const KnnView& v, WaveLds* L, int x, int y, uint32_t k, uint32_t n_res,
+template <int KU = 4, class Lds>
+__device__ __forceinline__ uint32_t knn_search(const KnnView& v, Lds* L, int x, int y, uint32_t k, uint32_t n_res,
                                                int lane, uint32_t& iters, uint32_t& buffered) {
     uint32_t found = 0;
     bool use_sel = n_res <= kBruteMax;
-    // the offset table pays off when about k / density <= 1024 offsets (four
-    // round trips) reach k resolved pixels; sparser masks use the ring search
-    const bool sparse = (uint64_t)n_res * 1024ull < (uint64_t)k * v.W * v.H;
-    if (!use_sel && !sparse) {
+    if (!use_sel && !knn_sparse(v, k, n_res)) {
         found = knn_table<KU>(v, L, x, y, k, lane);
         // fewer than k within the table: search on, unless every point was
         // found (without ghosts there are n_res of them)
@@ -704,6 +709,13 @@ __device__ __forceinline__ float lut4(const float* lut, const uint4& q, uint32_t
     return s;
 }
 
+// Random candidate r of an item: {x | y << 16, map}.
+__device__ __forceinline__ uint2 rand_cand(const BatchArgs& a, uint32_t item, uint32_t r) {
+    const size_t at = (size_t)(item - a.rc_base) * a.m + r;
+    if (a.n_maps == 1) return make_uint2(gld(a.rcands + at), 0u);
+    return gld(reinterpret_cast<const uint2*>(a.rcands) + at);
+}
+
 // Candidate ci of the reference's list: valid coherence candidates in
 // neighbour order, then the random ones (find_candidates, ms.rs:496-599).
 __device__ __forceinline__ void cand_get(const BatchArgs& a, const WaveLds* L, uint32_t rel, uint32_t item,
@@ -717,7 +729,7 @@ __device__ __forceinline__ void cand_get(const BatchArgs& a, const WaveLds* L, u
         xy = e.x;
         ms = e.y;
     } else {
-        uint2 r = gld(a.rcands + (size_t)(item - a.rc_base) * a.m + (ci - n_coh));
+        const uint2 r = rand_cand(a, item, ci - n_coh);
         xy = r.x;
         ms = r.y | 0x80000000u;
     }
@@ -1158,7 +1170,7 @@ __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* ma
                 cmap = e.y;
                 sgn = 1;
             } else {
-                uint2 r = gld(a.rcands + (size_t)(item - a.rc_base) * a.m + (c - n_coh));
+                const uint2 r = rand_cand(a, item, c - n_coh);
                 cxy = r.x;
                 cmap = r.y;
                 sgn = -1;
@@ -1242,7 +1254,7 @@ __device__ __forceinline__ uint4 item_winner(const BatchArgs& a, const MapDesc* 
             cxy = xm->x;
             cmap = xm->y & 0x7fffffffu;
         } else {
-            const uint2 rc = gld(a.rcands + (size_t)(item - a.rc_base) * a.m + (bidx - n_coh));
+            const uint2 rc = rand_cand(a, item, bidx - n_coh);
             cxy = rc.x;
             cmap = rc.y;
         }
@@ -1274,6 +1286,12 @@ __device__ __forceinline__ uint4 mail_record(unsigned long long w0, unsigned lon
 // Neighbour records of an item of a dependency-ordered run, lane j's in lane
 // j (`have`: the lane holds a neighbour, at pixel q): those without a bit in
 // `dep` from the state, the others from the mail once it carries the tag.
+//
+// Polls go past the L2, so the waves waiting far ahead of the front must not
+// flood the fabric: while more than kPollAll records are missing, only one of
+// them is polled, and the rest are read again when it has come. The last few
+// are polled together, so that the item's start costs no extra round trip.
+constexpr uint32_t kPollAll = 4;
 __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs& a, uint64_t dep, uint32_t q,
                                               bool have, int lane) {
     const bool mine = have && ((dep >> lane) & 1ull);
@@ -1282,13 +1300,21 @@ __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs
     bool need = mine;
     unsigned long long w0 = 0, w1 = 0;
     uint32_t polls = 0;
-    for (;;) {
-        if (need) {
+    uint64_t missing = __ballot(need), ask = missing;
+    while (missing) {
+        if ((ask >> lane) & 1ull) {
             w0 = __hip_atomic_load(f.mail + 2 * (size_t)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             w1 = __hip_atomic_load(f.mail + 2 * (size_t)q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             need = (uint32_t)(w0 >> 56) != f.tag || (uint32_t)(w1 >> 56) != f.tag;
         }
-        if (__ballot(need) == 0ull) break;
+        const uint64_t still = __ballot(need);
+        const bool came = still != missing;
+        missing = still;
+        if (missing == 0ull) break;
+        ask = missing;
+        const bool many = (uint32_t)__popcll(missing) > kPollAll;
+        // one lane (the last neighbour missing), unless something came
+        if (many && !came) ask = 1ull << (63 - __clzll((long long)missing));
         ++polls;
         if ((polls & 63u) == 0u) {
             // another wave gave up: end this wait too
@@ -1299,7 +1325,8 @@ __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs
             if (lane == 0) atomicOr(f.overflow, 4u);
             break;
         }
-        __builtin_amdgcn_s_sleep(1);
+        if (many) __builtin_amdgcn_s_sleep(8);
+        else __builtin_amdgcn_s_sleep(1);
     }
     if (mine) st = mail_record(w0, w1);
     return st;
@@ -1408,7 +1435,7 @@ __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc*
         nrs = min(m_r, r0 + per) - r0;
         // the member's first 64 random candidates, loaded ahead of the kNN
         if (!a.ext_cands && !a.knn_only && (uint32_t)lane < nrs)
-            rpre = gld(a.rcands + (size_t)(item - a.rc_base) * a.m + r0 + (uint32_t)lane);
+            rpre = rand_cand(a, item, r0 + (uint32_t)lane);
     }
     // ---- 1. k nearest resolved neighbours (leader) ----
     // With a neighbour list computed ahead every member reads it and derives
@@ -1846,8 +1873,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
         int32_t o = 0;
         if (lane < (int)kf) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
         uint2 rpre = make_uint2(0, 0);
-        const uint2* rc = a.rcands + (size_t)(item - a.rc_base) * a.m;
-        if ((uint32_t)lane < a.m) rpre = gld(rc + lane);
+        if ((uint32_t)lane < a.m) rpre = rand_cand(a, item, (uint32_t)lane);
         const int x = (int)(flat % a.W), y = (int)(flat / a.W);
         if (lane < (int)kf) L->nd[lane] = o;
         uint4 r;
@@ -1960,7 +1986,6 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
         const bool has = lane < (int)kf;
         int32_t o = 0;
         if (has) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
-        const uint2* rc = a.rcands + (size_t)(item - a.rc_base) * a.m;
         const int x = (int)(flat % a.W), y = (int)(flat / a.W);
         if (kf == 0) {
             // no resolved neighbour: alike for every member
@@ -1991,7 +2016,7 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
             if (lane < (int)kSlots) {
                 son = sl < n;
                 if (son) {
-                    const uint2 r = gld(rc + r0 + q * kSlots + sl);
+                    const uint2 r = rand_cand(a, item, r0 + q * kSlots + sl);
                     sxy = r.x;
                     smap = r.y;
                 }
@@ -2161,40 +2186,23 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
 
 // Neighbour lists of items [item0, item1) ahead of their batches, one
 // wavefront per item (the resolve kernels read them instead of searching).
+__device__ __forceinline__ KnnView list_view(const PrefetchArgs& a, uint32_t item, uint32_t n_at) {
+    return KnnView{a.W,    a.H,     a.tiles_x, a.tiles_y,
+                   a.mask, a.rlist, a.offtab,  a.offtab_n,
+                   item < a.redo_end ? nullptr : a.mask_new, a.tile_min, a.rank, n_at};
+}
+
+// With the window's resolved counts per item (the engine and windows of a
+// stage).
 __device__ __forceinline__ void prefetch_item(const PrefetchArgs& a, WaveLds* L, uint32_t item, int lane) {
     const uint32_t rel = item - a.item0;
     const uint32_t flat = gld(a.work + item);
-    uint32_t n_at, bs = 0;
-    if (a.n_at) {
-        n_at = a.n_at[rel];
-    } else {
-        uint32_t lo = 0, hi = a.nb - 1;  // last batch starting at or before the item
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) >> 1;
-            if (a.bounds[mid] <= item) lo = mid;
-            else hi = mid - 1;
-        }
-        n_at = a.bnres[lo];
-        bs = a.bounds[lo];
-    }
-    const KnnView v{a.W,    a.H,      a.tiles_x,  a.tiles_y,
-                    a.mask, a.rlist,  a.offtab,   a.offtab_n,
-                    item < a.redo_end ? nullptr : a.mask_new, a.tile_min, a.rank, n_at};
+    const uint32_t n_at = a.n_at[rel];
+    const KnnView v = list_view(a, item, n_at);
     uint32_t iters, buffered;
     const uint32_t kf = knn_search(v, L, (int)(flat % a.W), (int)(flat / a.W), a.k, n_at, lane, iters, buffered);
     if (lane < (int)kf) gst(a.out_nbrs + (size_t)rel * a.k + lane, L->nd[lane]);
     if (lane == 0) gst(a.out_cnt + rel, kf);
-    if (a.out_dep) {
-        bool d = false;
-        if (lane < (int)kf) {
-            const int32_t o = L->nd[lane];
-            const int X = (int)(flat % a.W) + packed_dx(o), Y = (int)(flat / a.W) + packed_dy(o);
-            const uint32_t r = gld(a.rank + (uint32_t)Y * a.W + (uint32_t)X);
-            d = r >= a.locked && r - a.locked < bs;
-        }
-        const uint64_t dm = __ballot(d);
-        if (lane == 0) a.out_dep[rel] = dm;
-    }
 }
 
 __global__ __launch_bounds__(kWave* kWavesPerWG) void k_knn_prefetch(PrefetchArgs a) {
@@ -2204,6 +2212,114 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) void k_knn_prefetch(PrefetchArg
     const uint32_t item = a.item0 + blockIdx.x * kWavesPerWG + threadIdx.x / kWave;
     if (item >= a.item1) return;
     prefetch_item(a, L, item, lane);
+}
+
+struct ListLds {
+    uint64_t keys[kKeyCap];
+    int32_t nd[kMaxK];
+    uint32_t rk[kMaxK];  // the neighbours' ranks
+};
+constexpr uint32_t kListItems = 8;  // items of a wave, one after another, at most
+constexpr int kListU = 2;           // table offsets per lane per round trip
+
+// Whole stages' neighbour lists and dependency masks, by the batch table
+// (a.bounds, a.bnres). A pixel is resolved at an item's batch start exactly
+// when its rank lies below the batch's resolved count, so the table route
+// reads one word per offset (its rank, which the dependency mask needs
+// anyway) instead of the mask, the picks' mask and then the rank of every
+// pick. Bound by the latency of those reads: the item's batch is found 64 ways
+// at a time, the first round's offsets stay in registers from item to item,
+// and the wave's LDS holds the key buffer and the list only, so that VGPRs
+// rather than LDS set the resident waves (32 per CU against 24).
+__global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(8))) void k_knn_lists(
+    PrefetchArgs a) {
+    __shared__ ListLds lds[kWavesPerWG];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x % kWave;
+    ListLds* L = &lds[wave];
+    int32_t o0[kListU];
+#pragma unroll
+    for (int u = 0; u < kListU; ++u) {
+        const uint32_t t = (uint32_t)(u * kWave + lane);
+        o0[u] = t < a.offtab_n ? gld(a.offtab + t) : 0;
+    }
+    const uint32_t first = a.item0 + (blockIdx.x * kWavesPerWG + (uint32_t)wave) * a.per_wave;
+    for (uint32_t q = 0; q < a.per_wave && first + q < a.item1; ++q) {
+        const uint32_t item = first + q, rel = item - a.item0;
+        // the last batch starting at or before the item
+        uint32_t lo = 0, len = a.nb;
+        while (len > 1) {
+            const uint32_t step = (len + kWave - 1) / kWave, at = lo + (uint32_t)lane * step;
+            const bool below = (uint32_t)lane * step < len && gld(a.bounds + at) <= item;
+            const uint32_t n = (uint32_t)__popcll(__ballot(below));
+            const uint32_t nlo = lo + (n - 1) * step;
+            len = min(step, lo + len - nlo);
+            lo = nlo;
+        }
+        const uint32_t n_at = gld(a.bnres + lo), bs = gld(a.bounds + lo);
+        const uint32_t flat = gld(a.work + item);
+        const int x = (int)(flat % a.W), y = (int)(flat / a.W);
+        const KnnView v = list_view(a, item, n_at);
+        uint32_t found = 0;
+        bool search = n_at <= kBruteMax || knn_sparse(v, a.k, n_at);
+        if (!search) {
+            for (uint32_t base = 0; base < a.offtab_n && found < a.k; base += kListU * kWave) {
+                int32_t o[kListU];
+                uint32_t r[kListU];
+#pragma unroll
+                for (int u = 0; u < kListU; ++u) {
+                    const uint32_t t = base + (uint32_t)(u * kWave + lane);
+                    o[u] = o0[u];
+                    if (base) o[u] = t < a.offtab_n ? gld(a.offtab + t) : 0;
+                    const int X = x + packed_dx(o[u]), Y = y + packed_dy(o[u]);
+                    const bool in = t < a.offtab_n && X >= 0 && Y >= 0 && X < (int)a.W && Y < (int)a.H;
+                    r[u] = in ? gld_at(a.rank, (__umul24((uint32_t)Y, a.W) + (uint32_t)X) * 4u) : 0xffffffffu;
+                }
+#pragma unroll
+                for (int u = 0; u < kListU; ++u) {
+                    const bool hit = r[u] < n_at;
+                    const uint64_t m = __ballot(hit);
+                    const uint32_t at = found + bits_below(m);
+                    if (hit && at < a.k) {
+                        L->nd[at] = o[u];
+                        L->rk[at] = r[u];
+                    }
+                    found += (uint32_t)__popcll(m);
+                }
+            }
+            found = min(found, a.k);
+            // fewer than k within the table, and not every resolved pixel found
+            search = found < a.k && found < n_at;
+            wave_sync();
+        }
+        if (search) {
+            uint32_t iters = 0;
+            Sel s{0u, ~0ull};
+            if (n_at <= kBruteMax) knn_list(v, L, n_at, x, y, a.k, lane, s);
+            else knn_rings(v, L, x, y, a.k, lane, s, iters);
+            wave_sync();
+            s = sel_compact(L->keys, s, a.k, lane);
+            found = s.count;
+            if (lane < (int)found) {
+                const int32_t o = key_to_packed(L->keys[lane]);
+                L->nd[lane] = o;
+                L->rk[lane] = gld(a.rank + (uint32_t)(y + packed_dy(o)) * a.W + (uint32_t)(x + packed_dx(o)));
+            }
+            wave_sync();
+        }
+        bool dep = false;
+        if (lane < (int)found) {
+            gst(a.out_nbrs + (size_t)rel * a.k + lane, L->nd[lane]);
+            const uint32_t r = L->rk[lane];
+            dep = r >= a.locked && r - a.locked < bs;
+        }
+        const uint64_t dm = __ballot(dep);
+        if (lane == 0) {
+            gst(a.out_cnt + rel, found);
+            gst(a.out_dep + rel, dm);
+        }
+        wave_sync();
+    }
 }
 
 __global__ void k_unpack(UnpackArgs a) {
@@ -2369,30 +2485,144 @@ __global__ void k_knn_unpack(const uint32_t* q_flat, const int32_t* packed, cons
 }
 
 // Random candidates of items [item0, item1): Pcg32::seed_from_u64(stage
-// seed + i + 1), m draws of (map, then x and y until the sample mask accepts).
-__device__ __forceinline__ void rand_item(const RandArgs& a, uint32_t item) {
-    Pcg32 g = Pcg32::seed_from_u64(a.stage_seed + (uint64_t)item + 1u);
-    uint2* out = a.out + (size_t)(item - a.item0) * a.m;
-    for (uint32_t r = 0; r < a.m; ++r) {
-        uint32_t map = (uint32_t)range_u64(g, 0, a.n_maps);
-        const MapDesc md = a.maps[map];
-        uint32_t x, y, tries = 0;
-        for (;;) {
-            x = range_u32(g, 0, md.w);
-            y = range_u32(g, 0, md.h);
-            if (md.smask == nullptr || md.smask[y * md.w + x] != 0) break;
-            if (++tries >= (1u << 24)) {
-                atomicOr(a.overflow, 1u);
-                break;
-            }
+// seed + i + 1), m draws of (map, then x and y until the sample mask accepts),
+// one thread per item. Every bounded draw is a rejection loop (half the draws
+// of a power-of-two range are rejected), and 64 lanes in one such loop would
+// all wait for the unluckiest: some seven rounds where two are needed. So a
+// lane's stream is a state machine: each round tests one word for whatever
+// the lane draws next, and lanes drift apart freely. ALU-bound (a 64-bit
+// multiply per round), and for few items bound by the rounds' latency: 1 M
+// items of one map take 0.5 ms (0.70 ms with the loops), 4 K items of m = 50
+// 45 us (80 us).
+
+__device__ __forceinline__ uint32_t pcg_word(uint64_t s) {
+    return rotr32((uint32_t)(((s >> 18) ^ s) >> 27), (uint32_t)(s >> 59));
+}
+__device__ __forceinline__ uint32_t zone_u32(uint32_t range) { return (range << __builtin_clz(range)) - 1u; }
+
+constexpr uint32_t kRandThreads = 256;
+constexpr uint32_t kRing = 8;
+struct RandLds {
+    uint32_t wh[kMapCache];                 // the maps' w | h << 16
+    uint2 ring[kRing][kRandThreads];        // candidates drawn, not yet stored
+};
+
+// With one map, its draw (a u64 of range 1) only rejects high words from
+// 2^31 on; the low word before it is skipped with a two-step advance. Without
+// a mask there is nothing to load.
+__device__ __forceinline__ void rand_one_map(const RandArgs& a, uint32_t w, uint32_t h, uint32_t item) {
+    const Pcg32 g = Pcg32::seed_from_u64(a.stage_seed + (uint64_t)item + 1u);
+    uint32_t* out = a.out + (size_t)(item - a.item0) * a.m;
+    const uint32_t zw = zone_u32(w), zh = zone_u32(h);
+    constexpr uint64_t kMul2 = kPcgMul * kPcgMul;
+    const uint64_t inc2 = g.inc * (kPcgMul + 1);
+    uint64_t s = g.state * kPcgMul + g.inc;
+    uint32_t phase = 0, x = 0, r = 0;  // next word: 0 the map's high word, 1 x, 2 y
+    while (r < a.m) {
+        // both advances beside the test, not after it
+        const uint64_t s1 = s * kPcgMul + g.inc, s2 = s * kMul2 + inc2;
+        const uint32_t v = pcg_word(s);
+        const uint64_t p = (uint64_t)v * (phase == 1 ? w : h);
+        const bool ok = phase == 0 ? v < 0x80000000u : (uint32_t)p <= (phase == 1 ? zw : zh);
+        phase += ok ? 1u : 0u;
+        if (ok && phase == 2) x = (uint32_t)(p >> 32);
+        if (phase == 3) {
+            gst(out + r, x | ((uint32_t)(p >> 32) << 16));
+            ++r;
+            phase = 0;
         }
-        out[r] = make_uint2(x | (y << 16), map);
+        s = phase == 0 ? s2 : s1;
     }
 }
 
-__global__ void k_rand(RandArgs a) {
-    const uint32_t item = a.item0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (item < a.item1) rand_item(a, item);
+// Several maps or a mask: the map's draw tests the 64-bit product of a low
+// and a high word (range 1 included). Loads (the mask) would wait for every
+// store before them, and in each round some lane stores, so candidates
+// collect in LDS until a lane's ring is full, then all are stored at once.
+// L: null in the engine (sides from the maps, candidates stored as drawn).
+__device__ __forceinline__ void rand_maps(const RandArgs& a, RandLds* L, uint32_t item) {
+    const Pcg32 g = Pcg32::seed_from_u64(a.stage_seed + (uint64_t)item + 1u);
+    const uint32_t words = rand_words(a.n_maps);
+    uint32_t* out = a.out + (size_t)(item - a.item0) * a.m * words;
+    const uint32_t range = a.n_maps;
+    const uint64_t zone = ((uint64_t)range << __builtin_clzll((uint64_t)range)) - 1u;
+    uint64_t s = g.state;
+    // next word: 0 and 1 the map's low and high word, 2 x, 3 y
+    uint32_t phase = 0, lo = 0, map = 0, w = 1, h = 1, x = 0, r = 0, held = 0, tries = 0;
+    auto store = [&](uint32_t at, uint32_t xy, uint32_t m) {
+        if (words == 1) gst(out + at, xy);
+        else gst(reinterpret_cast<unsigned long long*>(out) + at, (unsigned long long)m << 32 | xy);
+    };
+    auto flush = [&] {
+        for (uint32_t i = 0; i < kRing; ++i)
+            if (i < held) {
+                const uint2 c = L->ring[i][threadIdx.x];
+                store(r - held + i, c.x, c.y);
+            }
+        held = 0;
+    };
+    bool more = a.m > 0;
+    while (__ballot(more) != 0ull) {
+        if (more) {
+            const uint32_t v = pcg_word(s);
+            s = s * kPcgMul + g.inc;
+            const uint64_t t = (uint64_t)lo * range, u = (uint64_t)v * range + (t >> 32);
+            const bool map_ok = (u << 32 | (uint32_t)t) <= zone;
+            const uint32_t side = phase == 2 ? w : h;
+            const uint64_t p = (uint64_t)v * side;
+            const bool side_ok = (uint32_t)p <= zone_u32(side);
+            const uint32_t next = phase == 0 ? 1u : phase == 1 ? (map_ok ? 2u : 0u) : phase + (side_ok ? 1u : 0u);
+            if (phase == 0) lo = v;
+            if (phase == 2) x = (uint32_t)(p >> 32);
+            if (phase == 1 && map_ok) {
+                map = (uint32_t)(u >> 32);
+                if (L && a.n_maps <= kMapCache) {
+                    const uint32_t wh = L->wh[map];
+                    w = wh & 0xffffu;
+                    h = wh >> 16;
+                } else {
+                    w = a.maps[map].w;
+                    h = a.maps[map].h;
+                }
+            }
+            phase = next;
+            if (next == 4) {
+                const uint32_t y = (uint32_t)(p >> 32);
+                bool take = true;
+                if (a.masked) {
+                    const uint8_t* smask = a.maps[map].smask;
+                    take = smask == nullptr || gld(smask + y * w + x) != 0;
+                    if (!take && ++tries >= (1u << 24)) {
+                        atomicOr(a.overflow, 1u);
+                        take = true;
+                    }
+                }
+                phase = take ? 0u : 2u;
+                if (take) {
+                    if (L) L->ring[held++][threadIdx.x] = make_uint2(x | (y << 16), map);
+                    else store(r, x | (y << 16), map);
+                    ++r;
+                    tries = 0;
+                    more = r < a.m;
+                }
+            }
+        }
+        if (L && __ballot(held == kRing) != 0ull) flush();
+    }
+    if (L) flush();
+}
+
+__global__ __launch_bounds__(kRandThreads) void k_rand(RandArgs a) {
+    const uint32_t item = a.item0 + blockIdx.x * kRandThreads + threadIdx.x;
+    if (item < a.item1) rand_one_map(a, a.maps[0].w, a.maps[0].h, item);
+}
+__global__ __launch_bounds__(kRandThreads) void k_rand_maps(RandArgs a) {
+    __shared__ RandLds lds;
+    if (threadIdx.x < a.n_maps && threadIdx.x < kMapCache)
+        lds.wh[threadIdx.x] = a.maps[threadIdx.x].w | (a.maps[threadIdx.x].h << 16);
+    __syncthreads();
+    const uint32_t item = a.item0 + blockIdx.x * kRandThreads + threadIdx.x;
+    if (item < a.item1) rand_maps(a, &lds, item);
 }
 
 __global__ void k_commit(CommitArgs a) {
@@ -2820,9 +3050,13 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
                            a.score_w, a.gmask);
         } else if (P.kind == Q_RAND) {
             const BatchArgs a = ld_uniform(args + P.arg);
-            const RandArgs ra{a.maps, a.n_maps, a.stage_seed, P.i0, P.i1, a.m, J.rc, J.overflow};
+            const RandArgs ra{a.maps, a.n_maps, a.stage_seed, P.i0, P.i1, a.m, J.rc, J.overflow, 1u};
             const uint32_t i = P.i0 + unit * kQElems + tid;
-            if (tid < kQElems && i < P.i1) rand_item(ra, i);
+            if (tid < kQElems && i < P.i1) {
+                const MapDesc md = ld_uniform(a.maps);
+                if (a.n_maps == 1 && md.smask == nullptr) rand_one_map(ra, md.w, md.h, i);
+                else rand_maps(ra, nullptr, i);
+            }
         } else if (P.kind == Q_RECOLOR) {
             const BatchArgs a = ld_uniform(args + P.arg);
             const uint32_t i = P.i0 + unit * kQElems + tid;
@@ -3009,7 +3243,15 @@ hipError_t launch_knn_prefetch(const PrefetchArgs& a, hipStream_t s) {
     const uint32_t n = a.item1 - a.item0;
     if (n == 0) return hipSuccess;
     if (a.k == 0 || a.k > (uint32_t)kMaxK) return hipErrorInvalidValue;
-    if (!a.n_at && (!a.bounds || !a.bnres || a.nb == 0)) return hipErrorInvalidValue;
+    if (!a.n_at) {
+        if (!a.bounds || !a.bnres || a.nb == 0 || !a.rank || !a.out_dep) return hipErrorInvalidValue;
+        // one item per wave while that leaves waves of the chip (8192) idle
+        PrefetchArgs b = a;
+        b.per_wave = n / 8192u < 1u ? 1u : (n / 8192u > kListItems ? kListItems : n / 8192u);
+        const uint32_t per = kWavesPerWG * b.per_wave;
+        hipLaunchKernelGGL(k_knn_lists, dim3((n + per - 1) / per), dim3(kWave * kWavesPerWG), 0, s, b);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_knn_prefetch, dim3((n + kWavesPerWG - 1) / kWavesPerWG), dim3(kWave * kWavesPerWG),
                        kWavesPerWG * sizeof(WaveLds), s, a);
     return hipGetLastError();
@@ -3229,6 +3471,11 @@ uint32_t flow_max_wgs(uint32_t team, bool guided) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k.fn, (int)k.threads, k.lds) != hipSuccess)
         return 0;
+    // A team run is bound by its chain, not by its waves: 16 waves per CU leave
+    // the second stream room to prepare the later stages meanwhile. (With the
+    // 24 that fit an unguided run, its kernels waited for the run's end:
+    // 2.4 ms of a 1024^2 job's first stage.)
+    if (team > 1) per_cu = per_cu < (int)(16u / team) ? per_cu : (int)(16u / team);
     return (uint32_t)(per_cu * cus);
 }
 
@@ -3267,7 +3514,9 @@ hipError_t launch_resolve(const BatchArgs& a, bool guided, hipStream_t s) {
 hipError_t launch_rand(const RandArgs& a, hipStream_t s) {
     uint32_t n = a.item1 - a.item0;
     if (n == 0 || a.m == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rand, dim3((n + 255) / 256), dim3(256), 0, s, a);
+    const dim3 grid((n + kRandThreads - 1) / kRandThreads), block(kRandThreads);
+    if (a.n_maps == 1 && !a.masked) hipLaunchKernelGGL(k_rand, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(k_rand_maps, grid, block, 0, s, a);
     return hipGetLastError();
 }
 

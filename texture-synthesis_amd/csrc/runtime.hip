@@ -588,6 +588,7 @@ struct tsg_job {
     std::vector<uint32_t> filt;
     std::vector<int> kind;
     bool guided = false;
+    bool masked = false;  // some sampled example has a sample mask
     std::vector<std::pair<uint32_t, uint32_t>> ex_dims, g_dims;
     std::vector<std::unique_ptr<DBuf<uint32_t>>> ex, exg;  // [example] levels x w x h
     std::vector<std::unique_ptr<DBuf<uint8_t>>> smask;    // [example] (null = All)
@@ -606,7 +607,7 @@ struct tsg_job {
     DBuf<uint32_t> rlist;
     // scratch
     DBuf<uint4> result;
-    DBuf<uint2> rc;
+    DBuf<uint32_t> rc;  // rand_words() words per candidate
     // random candidates of whole stages, generated a stage ahead on the side
     // stream (single-job runs): buffer t % 2 holds stage t, in pieces
     // published by events; done[b] marks the end of the stage that read b
@@ -617,7 +618,7 @@ struct tsg_job {
     // moment follows from the pick order alone). `ready` publishes the set;
     // `done` marks the end of the stage that read it.
     struct Ahead {
-        DBuf<uint2> rc;
+        DBuf<uint32_t> rc;
         DBuf<int32_t> nbrs;
         DBuf<uint32_t> cnt, n_at;
         DBuf<uint64_t> mend, mnew;  // resolved mask at the stage end; the stage's picks
@@ -1039,7 +1040,7 @@ int wait_picks(tsg_job* j, int t) {
 // stage, or (deep) one set per stage, and the mail and pick lists of the
 // stages run in dependency order.
 uint64_t ahead_set_bytes(const tsg_job* j, uint64_t S) {
-    return std::max<uint64_t>(1, S) * (j->prm.random_sample_locations * sizeof(uint2) + j->prm.nearest_neighbors * 4 + 16) +
+    return std::max<uint64_t>(1, S) * (j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size()) * 4 + j->prm.nearest_neighbors * 4 + 16) +
            (uint64_t)j->tiles_x * j->tiles_y * 20;
 }
 uint64_t ahead_bytes(const tsg_job* j) { return 2 * ahead_set_bytes(j, stage_size(j, 0)) + j->N * 36; }
@@ -1082,7 +1083,7 @@ int ahead_stage(tsg_job* j) {
     if (j->ahead_deep) {
         // this stage's own set
         const uint64_t n = std::max<uint64_t>(1, S_eff);
-        HIP_TRY(A.rc.reserve(n * m));
+        HIP_TRY(A.rc.reserve(n * m * rand_words(nf)));
         HIP_TRY(A.nbrs.reserve(n * k));
         HIP_TRY(A.cnt.reserve(n));
         HIP_TRY(A.dep.reserve(n));
@@ -1096,7 +1097,8 @@ int ahead_stage(tsg_job* j) {
     // else to run yet
     if (S_eff) {
         hipStream_t rs = t == 0 && j->flow_on ? j->ctx->stream : side;
-        RandArgs ra{j->maps.p + (size_t)level * nf, nf, pss, 0u, (uint32_t)S_eff, m, A.rc.p, j->overflow.p};
+        RandArgs ra{j->maps.p + (size_t)level * nf, nf, pss, 0u, (uint32_t)S_eff, m, A.rc.p, j->overflow.p,
+                    (uint32_t)j->masked};
         HIP_TRY(timed_launch_on(j, rs, K_RAND, S_eff, [&] { return launch_rand(ra, rs); }));
     }
     // picks into the resolved list, their ranks, the stage's picks as a mask
@@ -1413,8 +1415,9 @@ int step_plan_rc(tsg_job* j, uint64_t lo, uint64_t hi, RandArgs* ra, bool* need)
     uint64_t cap_items = std::max<uint64_t>(hi - lo, (uint64_t)j->rc_budget / (8ull * std::max(1u, m)));
     st.rc_lo = lo;
     st.rc_hi = std::min<uint64_t>(st.S_eff, lo + cap_items);
-    HIP_TRY(j->rc.reserve((st.rc_hi - st.rc_lo) * m));
-    *ra = RandArgs{st.a.maps, st.a.n_maps, st.pss, (uint32_t)st.rc_lo, (uint32_t)st.rc_hi, m, j->rc.p, j->overflow.p};
+    HIP_TRY(j->rc.reserve((st.rc_hi - st.rc_lo) * m * rand_words(st.a.n_maps)));
+    *ra = RandArgs{st.a.maps, st.a.n_maps, st.pss, (uint32_t)st.rc_lo, (uint32_t)st.rc_hi, m, j->rc.p, j->overflow.p,
+                   (uint32_t)j->masked};
     st.a.rcands = j->rc.p;
     st.a.rc_base = (uint32_t)st.rc_lo;
     *need = true;
@@ -1725,7 +1728,7 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
         const uint64_t smax = std::max<uint64_t>(1, stage_size(j, 0));
         for (int q = 0; q < 2 && !j->ahead_deep; ++q) {
             tsg_job::Ahead& A = j->ahead[q];
-            HIP_TRY(A.rc.reserve(smax * j->prm.random_sample_locations));
+            HIP_TRY(A.rc.reserve(smax * j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size())));
             HIP_TRY(A.nbrs.reserve(smax * j->prm.nearest_neighbors));
             HIP_TRY(A.cnt.reserve(smax));
             HIP_TRY(A.mend.reserve((size_t)j->tiles_x * j->tiles_y));
@@ -1938,10 +1941,10 @@ size_t job_footprint(const tsg_job* j) {
     for (auto& e : j->smask) b += e->n;
     b += j->tg.n * 4 + j->maps.n * sizeof(MapDesc);
     b += j->N * (sizeof(uint4) + 4 + 4 + 4) + (size_t)j->tiles_x * j->tiles_y * 8 + j->gmask.n * 8;
-    b += j->result.n * sizeof(uint4) + j->rc.n * sizeof(uint2) + j->small_tab.n * 4;
+    b += j->result.n * sizeof(uint4) + j->rc.n * 4 + j->small_tab.n * 4;
     b += j->rank.n * 4 + j->mend.n * 8 + j->tmin.n * 4 + j->pre_n.n * 4 + j->pre_cnt.n * 4 + j->pre_nbrs.n * 4;
     for (const tsg_job::Ahead& A : j->ahead)
-        b += A.rc.n * sizeof(uint2) + A.nbrs.n * 4 + A.cnt.n * 4 + A.n_at.n * 4 + A.mend.n * 8 + A.mnew.n * 8 +
+        b += A.rc.n * 4 + A.nbrs.n * 4 + A.cnt.n * 4 + A.n_at.n * 4 + A.mend.n * 8 + A.mnew.n * 8 +
              A.tmin.n * 4 + A.dep.n * 8;
     b += j->mail.n * 8 + j->flow_ticket.n * 4 + j->unres[0].n * 4 + j->unres[1].n * 4 + j->pick_idx.n * 4 +
          j->pick_link.n * 4 + j->pick_head.n * 4;
@@ -2160,7 +2163,7 @@ int eng_plan(tsg_job* j) {
             const uint64_t cap_items = std::max<uint64_t>(i1 - i0, (uint64_t)j->rc_budget / (8ull * std::max(1u, m)));
             st.rc_lo = i0;
             st.rc_hi = std::min<uint64_t>(st.S_eff, i0 + cap_items);
-            if ((st.rc_hi - st.rc_lo) * m > j->rc.n)
+            if ((st.rc_hi - st.rc_lo) * m * rand_words(st.a.n_maps) > j->rc.n)
                 return fail(TSG_ERR_DEVICE, "random-candidate chunk beyond its buffer");
             eng_push(j, Q_RAND, (uint32_t)st.rc_lo, (uint32_t)st.rc_hi, kQElems, kNoArg);
         }
@@ -2204,7 +2207,7 @@ int eng_begin(tsg_job* j) {
     HIP_TRY(j->eng.luts.reserve((size_t)(P + 1) * 512));
     const uint64_t m = std::max<uint64_t>(1, j->prm.random_sample_locations);
     const uint64_t maxb = j->result.n;
-    HIP_TRY(j->rc.reserve(std::min<uint64_t>(j->N, std::max<uint64_t>(maxb, j->rc_budget / (8 * m))) * m));
+    HIP_TRY(j->rc.reserve(2 * std::min<uint64_t>(j->N, std::max<uint64_t>(maxb, j->rc_budget / (8 * m))) * m));
     const uint64_t win = std::min<uint64_t>(kPrefetchCap, j->N);
     HIP_TRY(j->pre_cnt.reserve(win));
     HIP_TRY(j->pre_nbrs.reserve(win * j->prm.nearest_neighbors));
@@ -2747,6 +2750,7 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
         int kd = sample_kind ? sample_kind[i] : TSG_SAMPLE_ALL;
         j->kind.push_back(kd);
         if (kd != TSG_SAMPLE_IGNORE) j->filt.push_back(i);
+        j->masked = j->masked || kd == TSG_SAMPLE_IMAGE;
     }
     if (inpaint_mask && inpaint_index >= j->filt.size())
         return fail(TSG_ERR_UNSUPPORTED, "inpaint example index beyond the sampled examples (the reference panics)");
@@ -3348,22 +3352,23 @@ int tsg_random_candidates(tsg_ctx* ctx, uint32_t n_maps, const tsg_image* maps, 
         }
     }
     DBuf<MapDesc> dmd;
-    DBuf<uint2> dout;
+    const uint32_t words = rand_words(n_maps);
+    DBuf<uint32_t> dout;
     DBuf<uint32_t> ovf;
     HIP_TRY(dmd.alloc(n_maps));
-    HIP_TRY(dout.alloc((size_t)n * m));
+    HIP_TRY(dout.alloc((size_t)n * m * words));
     HIP_TRY(ovf.alloc(1));
     HIP_TRY(hipMemset(ovf.p, 0, 4));
     HIP_TRY(hipMemcpy(dmd.p, md.data(), n_maps * sizeof(MapDesc), hipMemcpyHostToDevice));
-    RandArgs ra{dmd.p, n_maps, stage_seed, item0, item0 + n, m, dout.p, ovf.p};
+    RandArgs ra{dmd.p, n_maps, stage_seed, item0, item0 + n, m, dout.p, ovf.p, 1u};
     HIP_TRY(launch_rand(ra, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    std::vector<uint2> h((size_t)n * m);
-    HIP_TRY(hipMemcpy(h.data(), dout.p, h.size() * 8, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < h.size(); ++i) {
-        out[i * 3] = h[i].x & 0xffffu;
-        out[i * 3 + 1] = h[i].x >> 16;
-        out[i * 3 + 2] = h[i].y;
+    std::vector<uint32_t> h((size_t)n * m * words);
+    HIP_TRY(hipMemcpy(h.data(), dout.p, h.size() * 4, hipMemcpyDeviceToHost));
+    for (size_t i = 0; i < (size_t)n * m; ++i) {
+        out[i * 3] = h[i * words] & 0xffffu;
+        out[i * 3 + 1] = h[i * words] >> 16;
+        out[i * 3 + 2] = words == 2 ? h[i * words + 1] : 0u;
     }
     return TSG_OK;
 }
