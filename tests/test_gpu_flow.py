@@ -92,3 +92,17 @@ def test_progress_images_are_the_batches_states(ctx):
     assert np.array_equal(g1.image, g0.image) and len(s1) == len(s0)
     for a, b in zip(s1, s0):
         assert a[0] == b[0] and a[1] == b[1] and np.array_equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("t", [1, 8])
+@pytest.mark.parametrize("ex,w,h,k,px", [
+    (40, 23, 20, 12, 0),    # margins of one pixel
+    (40, 61, 47, 50, 5),    # the first five pixels are resolved at random: no ghost copies
+    (40, 19, 19, 30, 0),    # no margin: 5% of 19 is none
+    (64, 330, 270, 50, 0),  # list, ring and table routes, partial edge tiles
+])
+def test_tiling_lists_by_rank(ctx, t, ex, w, h, k, px):
+    sched = dict(ts.default_schedule(), px_per_batch=px)
+    gen, job = run_pair([synth.example(980 + ex, ex, ex)], w, h, sched=sched, seed=w, nearest_neighbors=k,
+                        tiling_mode=True, tuning=team(t))
+    assert_same(gen, job)

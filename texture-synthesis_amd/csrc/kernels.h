@@ -126,6 +126,10 @@ struct PrefetchArgs {
     // work list, below the item's batch start); needs the batch table
     uint64_t* out_dep;            // [item - item0]
     uint32_t per_wave;            // with the batch table: items of a wave (set by the launcher)
+    // tiling mode (with the batch table): pixels of ranks from g_lo on carry
+    // ghost copies within the edge margins (BatchArgs)
+    uint32_t ghosts, g_lo;
+    int32_t xl, xr, yb, yt;
 };
 
 // A dependency-ordered run: consecutive items [a.item0, a.item0 + n) of one

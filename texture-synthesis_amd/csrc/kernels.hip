@@ -312,7 +312,18 @@ struct KnnView {
     int32_t xl, xr, yb, yt;
     const uint64_t* pend;  // more resolved bits (a deferred commit's new pixels), or null
     const int32_t* offc;   // the table's first kOffCache offsets in LDS, or null
+    // a stage's lists in tiling mode (null gmask): pixels of ranks [g_lo, n_at)
+    // carry ghost copies
+    uint32_t ghosts, g_lo;
 };
+
+__device__ __forceinline__ bool has_ghosts(const KnnView& v) { return v.gmask != nullptr || v.ghosts != 0u; }
+// Whether pixel (x, y) carries ghost copies.
+__device__ __forceinline__ bool ghost_at(const KnnView& v, int x, int y) {
+    if (v.gmask) return px_set(v.gmask, v.tiles_x, x, y);
+    const uint32_t r = gld_at(v.rank, (__umul24((uint32_t)y, v.W) + (uint32_t)x) * 4u);
+    return r >= v.g_lo && r < v.n_at;
+}
 
 constexpr uint32_t kOffCache = 256;  // one table round
 
@@ -334,23 +345,35 @@ __device__ __forceinline__ bool view_set(const KnnView& v, int X, int Y) {
     return (mask_word(v, (uint32_t)(Y >> 3) * v.tiles_x + (uint32_t)(X >> 3)) >> (((Y & 7) << 3) | (X & 7))) & 1ull;
 }
 
+// The pixel whose ghost copy would stand at (X, Y) outside the image.
+__device__ __forceinline__ bool ghost_source(const KnnView& v, int X, int Y, int& x0, int& y0) {
+    const bool xin = X >= 0 && X < (int)v.W, yin = Y >= 0 && Y < (int)v.H;
+    x0 = X;
+    y0 = Y;
+    if (xin == yin) return false;  // inside, or diagonal
+    if (!xin) {
+        x0 = X >= (int)v.W ? X - (int)v.W : X + (int)v.W;
+        return (X >= (int)v.W ? x0 < v.xl : x0 > v.xr) && x0 >= 0 && x0 < (int)v.W;
+    }
+    y0 = Y >= (int)v.H ? Y - (int)v.H : Y + (int)v.H;
+    return (Y >= (int)v.H ? y0 < v.yb : y0 > v.yt) && y0 >= 0 && y0 < (int)v.H;
+}
+
 // Whether a point stands at (X, Y), ghosts included (no mask_new).
 __device__ __forceinline__ bool point_at(const KnnView& v, int X, int Y) {
-    const bool xin = X >= 0 && X < (int)v.W, yin = Y >= 0 && Y < (int)v.H;
-    if (xin && yin) return view_set(v, X, Y);
-    if (!v.gmask || (!xin && !yin)) return false;
-    if (!xin) {
-        const int x0 = X >= (int)v.W ? X - (int)v.W : X + (int)v.W;
-        const bool ok = X >= (int)v.W ? x0 < v.xl : x0 > v.xr;
-        return ok && x0 >= 0 && x0 < (int)v.W && px_set(v.gmask, v.tiles_x, x0, Y);
-    }
-    const int y0 = Y >= (int)v.H ? Y - (int)v.H : Y + (int)v.H;
-    const bool ok = Y >= (int)v.H ? y0 < v.yb : y0 > v.yt;
-    return ok && y0 >= 0 && y0 < (int)v.H && px_set(v.gmask, v.tiles_x, X, y0);
+    if (X >= 0 && X < (int)v.W && Y >= 0 && Y < (int)v.H) return view_set(v, X, Y);
+    int x0, y0;
+    return has_ghosts(v) && ghost_source(v, X, Y, x0, y0) && ghost_at(v, x0, y0);
 }
 
 // Ghost flags of pixels (xs + i, Y), i = 0..7, as bits (0 outside [0, W)).
 __device__ __forceinline__ uint32_t ghost_row(const KnnView& v, int Y, int xs) {
+    if (!v.gmask) {
+        uint32_t bits = 0;
+        for (int i = 0; i < 8; ++i)
+            if (xs + i >= 0 && xs + i < (int)v.W && ghost_at(v, xs + i, Y)) bits |= 1u << i;
+        return bits;
+    }
     const int c0 = xs >> 3, off = xs - c0 * 8, sh = (Y & 7) * 8;
     const uint32_t row = (uint32_t)(Y >> 3) * v.tiles_x;
     uint32_t b0 = 0, b1 = 0;
@@ -372,7 +395,7 @@ __device__ __forceinline__ uint64_t tile_points(const KnnView& v, int gx, int gy
     in_grid = gx >= 0 && gy >= 0 && gx < (int)v.tiles_x && gy < (int)v.tiles_y;
     uint64_t w = in_grid ? mask_word(v, (uint32_t)gy * v.tiles_x + (uint32_t)gx) : 0ull;
     const int X0 = gx * 8, Y0 = gy * 8, W = (int)v.W, H = (int)v.H;
-    if (!v.gmask || (X0 >= 0 && Y0 >= 0 && X0 + 8 <= W && Y0 + 8 <= H)) return w;
+    if (!has_ghosts(v) || (X0 >= 0 && Y0 >= 0 && X0 + 8 <= W && Y0 + 8 <= H)) return w;
     for (int j = 0; j < 8; ++j) {
         const int Y = Y0 + j;
         uint32_t bits = 0;
@@ -435,9 +458,9 @@ __device__ __forceinline__ void knn_list(const KnnView& a, Lds* L, uint32_t n_re
             uint64_t key = ~0ull;
             if (v) key = make_key(px - x, py - y);
             sel_push(L->keys, s, k, v, key, lane);
-            if (a.gmask) {
+            if (has_ghosts(a)) {
                 // the point's ghost copies (flush_resolved order: x, then y)
-                const bool g = v && px_set(a.gmask, a.tiles_x, px, py);
+                const bool g = v && ghost_at(a, px, py);
                 const bool gx = g && (px < a.xl || px > a.xr);
                 const bool gy = g && (py < a.yb || py > a.yt);
                 const int sx = px < a.xl ? (int)a.W : -(int)a.W, sy = py < a.yb ? (int)a.H : -(int)a.H;
@@ -497,7 +520,7 @@ __device__ __forceinline__ void knn_rings(const KnnView& a, Lds* L, int x, int y
     const int tx = x >> 3, ty = y >> 3;
     // tiles that can hold points: the grid, plus the ghost margins in tiling mode
     int g_x0 = 0, g_y0 = 0, g_x1 = (int)a.tiles_x - 1, g_y1 = (int)a.tiles_y - 1;
-    if (a.gmask) {
+    if (has_ghosts(a)) {
         g_x0 = (1 - a.xl) >> 3;
         g_y0 = (1 - a.yb) >> 3;
         g_x1 = max(g_x1, ((int)a.W + a.xl - 1) >> 3);
@@ -968,6 +991,17 @@ __device__ __forceinline__ void phase_clock(const BatchArgs& a, uint32_t item, i
 }
 __device__ __forceinline__ void phase_value(const BatchArgs& a, uint32_t item, int slot, uint64_t v, int lane) {
     if (a.dbg_clk && lane == 0) a.dbg_clk[(size_t)item * 16 + slot] = v;
+}
+
+// Pixel of the neighbour at (x + dx, y + dy); in tiling mode (wrap) a ghost
+// neighbour is the pixel it copies (ms.rs:510-512, 1132-1136).
+__device__ __forceinline__ uint32_t wrap_flat(uint32_t W, uint32_t H, bool wrap, int x, int y, int32_t o) {
+    int nx = x + packed_dx(o), ny = y + packed_dy(o);
+    if (wrap) {
+        nx = nx < 0 ? nx + (int)W : (nx >= (int)W ? nx - (int)W : nx);
+        ny = ny < 0 ? ny + (int)H : (ny >= (int)H ? ny - (int)H : ny);
+    }
+    return __umul24((uint32_t)ny, W) + (uint32_t)nx;
 }
 
 // ---- one work item, resolved by a team of T wavefronts (T = 1, 2, 4, 8, 16) ----
@@ -1787,15 +1821,8 @@ __device__ __forceinline__ void flow_args(BatchArgs& a) {
     a.exact = 0;
 }
 
-// Pixel of the neighbour at (x + dx, y + dy); in tiling mode a ghost
-// neighbour is the pixel it copies (ms.rs:510-512, 1132-1136).
 __device__ __forceinline__ uint32_t nbr_flat(const BatchArgs& a, int x, int y, int32_t o) {
-    int nx = x + packed_dx(o), ny = y + packed_dy(o);
-    if (a.gmask) {
-        nx = nx < 0 ? nx + (int)a.W : (nx >= (int)a.W ? nx - (int)a.W : nx);
-        ny = ny < 0 ? ny + (int)a.H : (ny >= (int)a.H ? ny - (int)a.H : ny);
-    }
-    return __umul24((uint32_t)ny, a.W) + (uint32_t)nx;
+    return wrap_flat(a.W, a.H, a.gmask != nullptr, x, y, o);
 }
 
 // Hands a workgroup's waves the items of a run in order: tickets are taken
@@ -2187,9 +2214,16 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
 // Neighbour lists of items [item0, item1) ahead of their batches, one
 // wavefront per item (the resolve kernels read them instead of searching).
 __device__ __forceinline__ KnnView list_view(const PrefetchArgs& a, uint32_t item, uint32_t n_at) {
-    return KnnView{a.W,    a.H,     a.tiles_x, a.tiles_y,
-                   a.mask, a.rlist, a.offtab,  a.offtab_n,
-                   item < a.redo_end ? nullptr : a.mask_new, a.tile_min, a.rank, n_at};
+    KnnView v{a.W,    a.H,     a.tiles_x, a.tiles_y,
+              a.mask, a.rlist, a.offtab,  a.offtab_n,
+              item < a.redo_end ? nullptr : a.mask_new, a.tile_min, a.rank, n_at};
+    v.xl = a.xl;
+    v.xr = a.xr;
+    v.yb = a.yb;
+    v.yt = a.yt;
+    v.ghosts = a.ghosts;
+    v.g_lo = a.g_lo;
+    return v;
 }
 
 // With the window's resolved counts per item (the engine and windows of a
@@ -2231,9 +2265,15 @@ constexpr int kListU = 2;           // table offsets per lane per round trip
 // at a time, the first round's offsets stay in registers from item to item,
 // and the wave's LDS holds the key buffer and the list only, so that VGPRs
 // rather than LDS set the resident waves (32 per CU against 24).
+//
+// GHOSTS: tiling mode. A pixel carries ghost copies from its batch on unless
+// it was resolved at random, which only the items of a batch that starts with
+// nothing resolved are; so the copies follow from the ranks too.
+template <bool GHOSTS>
 __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(8))) void k_knn_lists(
     PrefetchArgs a) {
     __shared__ ListLds lds[kWavesPerWG];
+    if (!GHOSTS) a.ghosts = 0;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int lane = threadIdx.x % kWave;
     ListLds* L = &lds[wave];
@@ -2274,6 +2314,11 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
                     const int X = x + packed_dx(o[u]), Y = y + packed_dy(o[u]);
                     const bool in = t < a.offtab_n && X >= 0 && Y >= 0 && X < (int)a.W && Y < (int)a.H;
                     r[u] = in ? gld_at(a.rank, (__umul24((uint32_t)Y, a.W) + (uint32_t)X) * 4u) : 0xffffffffu;
+                    int gx, gy;
+                    if (GHOSTS && !in && t < a.offtab_n && ghost_source(v, X, Y, gx, gy)) {
+                        r[u] = gld_at(a.rank, (__umul24((uint32_t)gy, a.W) + (uint32_t)gx) * 4u);
+                        if (r[u] < a.g_lo) r[u] = 0xffffffffu;
+                    }
                 }
 #pragma unroll
                 for (int u = 0; u < kListU; ++u) {
@@ -2289,7 +2334,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
             }
             found = min(found, a.k);
             // fewer than k within the table, and not every resolved pixel found
-            search = found < a.k && found < n_at;
+            search = found < a.k && (GHOSTS || found < n_at);
             wave_sync();
         }
         if (search) {
@@ -2303,7 +2348,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
             if (lane < (int)found) {
                 const int32_t o = key_to_packed(L->keys[lane]);
                 L->nd[lane] = o;
-                L->rk[lane] = gld(a.rank + (uint32_t)(y + packed_dy(o)) * a.W + (uint32_t)(x + packed_dx(o)));
+                L->rk[lane] = gld(a.rank + wrap_flat(a.W, a.H, GHOSTS, x, y, o));
             }
             wave_sync();
         }
@@ -3249,7 +3294,9 @@ hipError_t launch_knn_prefetch(const PrefetchArgs& a, hipStream_t s) {
         PrefetchArgs b = a;
         b.per_wave = n / 8192u < 1u ? 1u : (n / 8192u > kListItems ? kListItems : n / 8192u);
         const uint32_t per = kWavesPerWG * b.per_wave;
-        hipLaunchKernelGGL(k_knn_lists, dim3((n + per - 1) / per), dim3(kWave * kWavesPerWG), 0, s, b);
+        const dim3 grid((n + per - 1) / per), block(kWave * kWavesPerWG);
+        if (a.ghosts) hipLaunchKernelGGL(k_knn_lists<true>, grid, block, 0, s, b);
+        else hipLaunchKernelGGL(k_knn_lists<false>, grid, block, 0, s, b);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_knn_prefetch, dim3((n + kWavesPerWG - 1) / kWavesPerWG), dim3(kWave * kWavesPerWG),

@@ -686,6 +686,7 @@ struct tsg_job {
     DBuf<uint32_t> unres[2], pick_idx, pick_link, pick_head;
     const uint32_t* pick_list = nullptr;
     uint64_t pick_left = 0;         // entries of the list
+    uint32_t ghost_lo = 0;          // tiling mode: ranks below carry no ghost copies
     uint32_t flow_tag = 0, flow_launches = 0;
     size_t small_used = 0;
     // host bookkeeping
@@ -1050,6 +1051,15 @@ uint64_t ahead_bytes_deep(const tsg_job* j) {
     return b;
 }
 
+// Tiling mode's ghost margins: 5% of each side (ms.rs:296-331).
+template <class Args>
+void ghost_margins(const tsg_job* j, Args* a) {
+    a->xl = (int32_t)((float)j->W * 0.05f);
+    a->xr = (int32_t)j->W - a->xl;
+    a->yb = (int32_t)((float)j->H * 0.05f);
+    a->yt = (int32_t)j->H - a->yb;
+}
+
 // Prepares stage ahead_next on the side stream (see tsg_job::Ahead). The
 // counts follow the stage driver: a stage opens with `ahead_open` resolved
 // pixels, redoes those past `locked`, and appends its picks.
@@ -1194,6 +1204,14 @@ int ahead_stage(tsg_job* j) {
         pa.out_nbrs = A.nbrs.p;
         pa.out_cnt = A.cnt.p;
         pa.out_dep = A.dep.p;
+        if (j->prm.tiling_mode) {
+            // the only pixels without ghost copies are those resolved at
+            // random: the items of a batch that starts with nothing resolved
+            if (n_open == 0) j->ghost_lo = nb > 1 ? tab[1] : (uint32_t)S_eff;
+            pa.ghosts = 1;
+            pa.g_lo = j->ghost_lo;
+            ghost_margins(j, &pa);
+        }
         HIP_TRY(timed_launch_on(j, side, K_PREFETCH, pre_end, [&] { return launch_knn_prefetch(pa, side); }));
     }
     HIP_TRY(hipEventRecord(A.ready, side));
@@ -1382,12 +1400,8 @@ int step_open_stage(tsg_job* j) {
     a.score_w = j->score.p;
     a.result = j->result.p;
     if (j->prm.tiling_mode) {
-        // ghost margins: 5% of each side (ms.rs:296-331)
         a.gmask = j->gmask.p;
-        a.xl = (int32_t)((float)j->W * 0.05f);
-        a.xr = (int32_t)j->W - a.xl;
-        a.yb = (int32_t)((float)j->H * 0.05f);
-        a.yt = (int32_t)j->H - a.yb;
+        ghost_margins(j, &a);
     }
     if (j->ahead_on) {
         // every item of the stage has its candidates and neighbour list
@@ -1706,7 +1720,8 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     // stage. In dependency order a set per stage is also taken where it holds
     // no more than the two would (at p = 0.5 it never does): the preparation
     // then runs ahead of the stages without waiting for a set to come free.
-    const bool ahead_ok = j->tune.ahead && !j->prm.tiling_mode;
+    // In tiling mode the lists need the batch table's ranks: dependency order only.
+    const bool ahead_ok = j->tune.ahead && (!j->prm.tiling_mode || j->tune.flow);
     const bool two_fit = ahead_bytes(j) <= kAheadBudget;
     const bool deep_fits = j->prm.backtrack_stages + 1 <= 8 && ahead_bytes_deep(j) <= kAheadBudget;
     j->ahead_deep = ahead_ok && deep_fits &&
@@ -2084,10 +2099,7 @@ int eng_open_stage(tsg_job* j) {
     a.rcands = j->rc.p;
     if (j->prm.tiling_mode) {
         a.gmask = j->gmask.p;
-        a.xl = (int32_t)((float)j->W * 0.05f);
-        a.xr = (int32_t)j->W - a.xl;
-        a.yb = (int32_t)((float)j->H * 0.05f);
-        a.yt = (int32_t)j->H - a.yb;
+        ghost_margins(j, &a);
     }
     j->eng.stage_arg = (uint32_t)j->eng.args.size();
     j->eng.args.push_back(a);
