@@ -106,3 +106,12 @@ def test_tiling_lists_by_rank(ctx, t, ex, w, h, k, px):
     gen, job = run_pair([synth.example(980 + ex, ex, ex)], w, h, sched=sched, seed=w, nearest_neighbors=k,
                         tiling_mode=True, tuning=team(t))
     assert_same(gen, job)
+
+
+@pytest.mark.parametrize("t", [2, 4, 8])
+def test_offsets_far_beyond_the_examples(ctx, t):
+    # the first items' neighbours lie several examples away, so that whole
+    # members hold no valid candidate, and the maps differ in size
+    exs = [synth.example(990, 9, 8), synth.example(991, 61, 57)]
+    gen, job = run_pair(exs, 260, 230, seed=3, backtrack_stages=2, tuning=team(t))
+    assert_same(gen, job)

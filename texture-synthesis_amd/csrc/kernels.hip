@@ -694,8 +694,8 @@ __device__ __forceinline__ uint32_t byte_scaled(uint32_t v) {
 // the copy's byte offset slot4 as the addend.
 template <int C>
 constexpr int lut_shift() {
-    static_assert(C == 8 || C == 4, "table copies");
-    return C == 8 ? 5 : 4;
+    static_assert(C == 32 || C == 16 || C == 8 || C == 4, "table copies");
+    return C == 32 ? 7 : C == 16 ? 6 : C == 8 ? 5 : 4;
 }
 __device__ __forceinline__ float lut_sad(const float* lut, uint32_t a, uint32_t b, uint32_t slot4) {
     const uint32_t off = (a > b ? a - b : b - a) + slot4;
@@ -797,9 +797,8 @@ struct NbrRow {
     int dx, dy;
     float w;
 };
-template <bool GUIDED>
+template <bool GUIDED, int C = lut_copies<GUIDED>()>
 __device__ __forceinline__ NbrRow nbr_row(const WaveLds* L, uint32_t j) {
-    constexpr int C = lut_copies<GUIDED>();
     NbrRow r;
     r.q = bytes_scaled<C>(L->pat[j]);
     r.g = GUIDED ? bytes_scaled<C>(L->gpat[j]) : make_uint4(0, 0, 0, 0);
@@ -812,10 +811,9 @@ __device__ __forceinline__ NbrRow nbr_row(const WaveLds* L, uint32_t j) {
 
 // Cost term of a neighbour: (four colour LUT terms, then four guide LUT
 // terms, summed in order) times w_j, as one rounded product.
-template <bool GUIDED>
+template <bool GUIDED, int C = lut_copies<GUIDED>()>
 __device__ __forceinline__ float term_at(const NbrRow& r, const float* lut, const float* glut, uint32_t slot4,
                                          uint32_t p, uint32_t gp) {
-    constexpr int C = lut_copies<GUIDED>();
     float s = lut4<C>(lut, r.q, p, slot4);
     if (GUIDED) s = lut4_add<C>(s, glut, r.g, gp, slot4);
     return __fmul_rn(s, r.w);
@@ -1181,7 +1179,7 @@ __device__ __forceinline__ uint32_t item_neighbours(const BatchArgs& a, const Ma
 
 // Leader: every candidate without pruning, find_best_match's sequential
 // rule, for NaN cost tables and the full-cost test hook.
-template <bool GUIDED, class Lds>
+template <bool GUIDED, int C = lut_copies<GUIDED>(), class Lds>
 __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t rel,
                                            uint32_t kf, uint32_t n_coh, uint32_t n_c, const Lds* L, const float* lut,
                                            const float* glut, int slot, int lane, float& best, uint32_t& bidx) {
@@ -1218,7 +1216,6 @@ __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* ma
                 const bool in = (uint32_t)X2 < md.w && (uint32_t)Y2 < md.h;
                 const uint32_t idx = (uint32_t)Y2 * md.w + (uint32_t)X2;
                 const uint32_t p = in ? gld(md.px + idx) : kOutsidePx;
-                constexpr int C = lut_copies<GUIDED>();
                 float s = lut4<C>(lut, bytes_scaled<C>(L->pat[j]), p, slot4);
                 if (GUIDED) {
                     const bool gin = (uint32_t)X2 < md.gw && (uint32_t)Y2 < md.gh;
@@ -1325,9 +1322,12 @@ __device__ __forceinline__ uint4 mail_record(unsigned long long w0, unsigned lon
 // flood the fabric: while more than kPollAll records are missing, only one of
 // them is polled, and the rest are read again when it has come. The last few
 // are polled together, so that the item's start costs no extra round trip.
+//
+// With `late`, the wait ends once at most kPollAll records are missing, and
+// *late says which.
 constexpr uint32_t kPollAll = 4;
 __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs& a, uint64_t dep, uint32_t q,
-                                              bool have, int lane) {
+                                              bool have, int lane, uint64_t* late = nullptr) {
     const bool mine = have && ((dep >> lane) & 1ull);
     uint4 st = make_uint4(0, 0, 0, 0);
     if (have && !mine) st = gld(a.state + q);
@@ -1335,6 +1335,7 @@ __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs
     unsigned long long w0 = 0, w1 = 0;
     uint32_t polls = 0;
     uint64_t missing = __ballot(need), ask = missing;
+    if (late) *late = 0;
     while (missing) {
         if ((ask >> lane) & 1ull) {
             w0 = __hip_atomic_load(f.mail + 2 * (size_t)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1345,6 +1346,10 @@ __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs
         const bool came = still != missing;
         missing = still;
         if (missing == 0ull) break;
+        if (late && (uint32_t)__popcll(missing) <= kPollAll) {
+            *late = missing;
+            break;
+        }
         ask = missing;
         const bool many = (uint32_t)__popcll(missing) > kPollAll;
         // one lane (the last neighbour missing), unless something came
@@ -1589,11 +1594,10 @@ __device__ __forceinline__ void commit_one(uint32_t W, uint32_t tiles_x, const M
 
 constexpr uint32_t kMapCache = 16;  // map descriptors kept in LDS
 
-template <bool GUIDED>
+template <bool GUIDED, int C = lut_copies<GUIDED>()>
 __device__ __forceinline__ WaveLds* setup_lds(const BatchArgs& a, unsigned char* smem, float*& lut, float*& glut,
                                               MapDesc* smaps, const MapDesc*& maps) {
     lut = reinterpret_cast<float*>(smem);
-    constexpr int C = lut_copies<GUIDED>();
     glut = lut + 256 * C;
     for (int t = threadIdx.x; t < 256 * C; t += blockDim.x) {
         lut[t] = a.lut[t / C];
@@ -1607,7 +1611,7 @@ __device__ __forceinline__ WaveLds* setup_lds(const BatchArgs& a, unsigned char*
     int32_t* oc = offtab_lds();
     for (uint32_t t = threadIdx.x; t < kOffCache && t < a.offtab_n; t += blockDim.x) oc[t] = a.offtab[t];
     __syncthreads();
-    return reinterpret_cast<WaveLds*>(smem + lut_bytes(GUIDED));
+    return reinterpret_cast<WaveLds*>(smem + 256 * C * (GUIDED ? 2 : 1) * sizeof(float));
 }
 
 // Profiling: the launch's execution span on the device clock, as the
@@ -1951,7 +1955,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
 struct TeamLds {
     double dist[kMaxK];
     double avg;
-    unsigned long long best;  // least (cost bits << 32 | candidate index)
+    unsigned long long best[kWavesPerWG];  // per member: least (cost bits << 32 | candidate index)
     uint4 coh[kMaxK];
     int32_t nd[kMaxK];
     float w[kMaxK];
@@ -1965,6 +1969,149 @@ constexpr uint32_t kSlots = 8;  // coherence candidates (and random ones) of a m
 // lanes' float4 reads of their rows cover the banks
 constexpr uint32_t kTermRow = kMaxK + 4;
 constexpr size_t kTeamWaveLds = 2 * kSlots * kTermRow * sizeof(float);
+// Copies of a cost table in a team kernel. At most 16 waves run per CU there
+// (flow_max_wgs), so LDS has room for more copies than in the wave kernels,
+// and a link's term lookups with fewer bank conflicts: with 32 copies a
+// lane's entry lies in a bank of its own.
+template <bool GUIDED, int T>
+constexpr int team_copies() {
+    return (T == 8 ? 32 : T == 4 ? 16 : 8) / (GUIDED ? 2 : 1);
+}
+
+// Least of a 64-bit key over the lanes of each row of 16, in every lane.
+__device__ __forceinline__ unsigned long long row_min(unsigned long long k) {
+#define TSG_ROW_MIN(ctl)                                                                                             \
+    {                                                                                                                \
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)k, ctl, 0xf, 0xf, false);        \
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(k >> 32), ctl, 0xf, 0xf, false); \
+        const unsigned long long o = (unsigned long long)hi << 32 | lo;                                              \
+        k = o < k ? o : k;                                                                                           \
+    }
+    TSG_ROW_MIN(0x128)  // row_ror:8
+    TSG_ROW_MIN(0x124)  // row_ror:4
+    TSG_ROW_MIN(0x122)  // row_ror:2
+    TSG_ROW_MIN(0x121)  // row_ror:1
+#undef TSG_ROW_MIN
+    return k;
+}
+
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t lane_u64(uint64_t v, int l) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+}
+
+// The candidate a lane holds for its team member (lane c: slot c of a round).
+struct SlotCand {
+    bool on;
+    uint32_t xy, map, patch, colour;
+};
+
+// Pattern pixels of a round's candidates (slots L0..L0 + 7 of the lanes' `c`,
+// those that are on; the other slots get some pixels) for each lane's
+// neighbour offset (dx, dy), negated by the caller for mirrored patterns; rad
+// bounds every lane's |dx| and |dy|. No branch per candidate, so that all
+// loads are in flight together: when every candidate lies at least rad from
+// the edges of its map, no bounds test is needed and a pixel is one scalar
+// address plus a lane offset (a slot that is off repeats a candidate that is
+// on); else the addresses are clamped and the pixels outside replaced.
+template <bool GUIDED, bool ONE, int L0>
+__device__ __forceinline__ void gather_slots(const SlotCand& c, const MapDesc& m0, const MapDesc* maps, int dx, int dy,
+                                             int rad, uint32_t (&p)[kSlots], uint32_t (&gp)[kSlots]) {
+    const int cx = (int)(c.xy & 0xffffu), cy = (int)(c.xy >> 16);
+    MapDesc md = m0;
+    if (!ONE) md = maps[c.on ? c.map : 0u];
+    const bool inner = cx >= rad && cy >= rad && cx + rad < (int)md.w && cy + rad < (int)md.h &&
+                       (!GUIDED || (md.gw == md.w && md.gh == md.h));
+    const bool on = c.on && ((threadIdx.x % kWave) & ~(kSlots - 1u)) == (uint32_t)L0;
+    const uint64_t in_m = __ballot(on && inner);
+    if (in_m != 0ull && in_m == __ballot(on)) {
+        const int some = __ffsll((long long)in_m) - 1;
+        const uint32_t at = on ? (uint32_t)(cy - rad) * md.w + (uint32_t)(cx - rad) : 0u;
+        const uint64_t base = (uint64_t)(md.px + at), gbase = GUIDED ? (uint64_t)(md.gpx + at) : 0u;
+        uint32_t off = (__umul24((uint32_t)(dy + rad), m0.w) + (uint32_t)(dx + rad)) * 4u;
+#pragma unroll
+        for (int k = 0; k < (int)kSlots; ++k) {
+            const int l = (in_m >> (L0 + k)) & 1ull ? L0 + k : some;
+            if (!ONE) {
+                const uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)md.w, l);
+                off = (__umul24((uint32_t)(dy + rad), w) + (uint32_t)(dx + rad)) * 4u;
+            }
+            p[k] = gld_at((const uint32_t*)lane_u64(base, l), off);
+            gp[k] = GUIDED ? gld_at((const uint32_t*)lane_u64(gbase, l), off) : kOutsidePx;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < (int)kSlots; ++k) {
+            const int l = L0 + k;
+            const uint32_t xy = (uint32_t)__builtin_amdgcn_readlane((int)c.xy, l);
+            const uint32_t w = ONE ? m0.w : (uint32_t)__builtin_amdgcn_readlane((int)md.w, l);
+            const uint32_t h = ONE ? m0.h : (uint32_t)__builtin_amdgcn_readlane((int)md.h, l);
+            const uint32_t* px = ONE ? m0.px : (const uint32_t*)lane_u64((uint64_t)md.px, l);
+            const uint32_t X = (xy & 0xffffu) + (uint32_t)dx, Y = (xy >> 16) + (uint32_t)dy;
+            const bool in = X < w && Y < h;
+            const uint32_t v = gld_at(px, in ? (__umul24(Y, w) + X) * 4u : 0u);
+            p[k] = in ? v : kOutsidePx;
+            gp[k] = kOutsidePx;
+            if (GUIDED) {
+                const uint32_t gw = ONE ? m0.gw : (uint32_t)__builtin_amdgcn_readlane((int)md.gw, l);
+                const uint32_t gh = ONE ? m0.gh : (uint32_t)__builtin_amdgcn_readlane((int)md.gh, l);
+                const uint32_t* gpx = ONE ? m0.gpx : (const uint32_t*)lane_u64((uint64_t)md.gpx, l);
+                const bool gin = X < gw && Y < gh;
+                const uint32_t g = gld_at(gpx, gin ? (__umul24(Y, gw) + X) * 4u : 0u);
+                gp[k] = gin ? g : kOutsidePx;
+            }
+        }
+    }
+}
+
+// Terms of a round's first n candidates into their rows, one neighbour per
+// lane; zero past the last neighbour (`has`), so that the sums run in whole
+// chunks (adding +0 changes no sum of non-negative terms). Four rows at a
+// time without a branch between them: their table lookups overlap.
+template <bool GUIDED, int C>
+__device__ __forceinline__ void slot_terms(const NbrRow& row, const float* lut, const float* glut, uint32_t slot4,
+                                           uint32_t n, const uint32_t (&p)[kSlots], const uint32_t (&gp)[kSlots],
+                                           bool has, float* rows, int lane) {
+#pragma unroll
+    for (uint32_t g = 0; g < kSlots; g += 4) {
+        if (g < n) {
+            float t[4];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) t[c] = term_at<GUIDED, C>(row, lut, glut, slot4, p[g + c], gp[g + c]);
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) rows[(g + c) * kTermRow + lane] = has ? t[c] : 0.0f;
+        }
+    }
+}
+
+// In-order f32 sum of a candidate's first kf terms (rows are zero from there
+// to the chunk's end), the next chunk read ahead of a chunk's adds.
+__device__ __forceinline__ float row_sum(const float* row, uint32_t kf) {
+    const float4* tp = reinterpret_cast<const float4*>(row);
+    float4 v[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[0][i] = tp[i];
+    float s = 0.0f;
+#pragma unroll
+    for (uint32_t g = 0; g < kMaxK / 16; ++g) {
+        if (16 * g < kf) {
+            if (g + 1 < kMaxK / 16 && 16 * (g + 1) < kf) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[(g + 1) & 1][i] = tp[4 * (g + 1) + i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float4 u = v[g & 1][i];
+                s = __fadd_rn(s, u.x);
+                s = __fadd_rn(s, u.y);
+                s = __fadd_rn(s, u.z);
+                s = __fadd_rn(s, u.w);
+            }
+        }
+    }
+    return s;
+}
 
 // A run with a team of T waves per item (the workgroup), for batches too
 // small to fill the chip, where the dependency chain binds: an item's time
@@ -1973,43 +2120,41 @@ constexpr size_t kTeamWaveLds = 2 * kSlots * kTermRow * sizeof(float);
 // (weights, the random candidates' pixels and colours, the records of the
 // other neighbours), and after it every candidate is evaluated in full: one
 // round trip for the coherence candidates' pixels, during which the random
-// ones' terms are formed, one in-order sum per lane, one 64-bit minimum in
-// LDS. Pruning, duplicate removal and a leader's merge would each add a
-// dependent step that the idle lanes save nothing by. The winner's own lane
-// posts it.
-template <bool GUIDED, int T>
-__global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f) {
+// ones' terms are formed, one in-order sum per lane, the least cost of each
+// member's row, and one barrier to compare the members'. Pruning, duplicate
+// removal and a leader's merge would each add a dependent step that the idle
+// lanes save nothing by. The winner's own lane posts it. ONE: a single map,
+// its descriptor in scalars.
+template <bool GUIDED, int T, bool ONE>
+__global__ __launch_bounds__(kWave* T) __attribute__((amdgpu_waves_per_eu(4))) void k_flow_team(BatchArgs a, FlowArgs f) {
     const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ MapDesc smaps[kMapCache];
     __shared__ TeamLds team[2];
     flow_args(a);
+    constexpr int C = team_copies<GUIDED, T>();
     float *lut, *glut;
     const MapDesc* maps;
     if (threadIdx.x == 0) team[0].next = atomicAdd(f.ticket, 1u);
-    float* rows = reinterpret_cast<float*>(setup_lds<GUIDED>(a, smem, lut, glut, smaps, maps));  // ends with a barrier
-    constexpr int C = lut_copies<GUIDED>();
+    float* rows = reinterpret_cast<float*>(setup_lds<GUIDED, C>(a, smem, lut, glut, smaps, maps));  // ends with a barrier
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int lane = threadIdx.x % kWave;
     rows += (size_t)wave * (2 * kSlots * kTermRow);
     const uint32_t slot4 = (uint32_t)(lane % C) * 4u;
-    MapDesc m0{};
-    if (a.n_maps == 1) m0 = ld_uniform(maps);
+    const MapDesc m0 = ld_uniform(maps);
     const uint32_t rper = (a.m + T - 1) / T;
     const uint32_t r0 = min(a.m, (uint32_t)wave * rper), nrs = min(a.m, r0 + rper) - r0;
-    uint32_t idx = team[0].next;
+    uint32_t idx = uniform(team[0].next);
     for (uint32_t turn = 0; idx < f.n; turn ^= 1u) {
         TeamLds* L = &team[turn];
         const uint32_t item = a.item0 + idx, rel = item - a.pre_base;
+        uint32_t next = 0;  // the ticket is on its way while the item waits
         if (wave == 0) {
             phase_clock(a, item, 0, lane);
-            if (lane == 0) {
-                team[turn ^ 1u].next = atomicAdd(f.ticket, 1u);
-                L->best = ~0ull;
-            }
+            if (lane == 0) next = atomicAdd(f.ticket, 1u);
         }
-        const uint32_t flat = gld(a.work + item);
-        const uint32_t kf = gld(a.pre_cnt + rel);
+        const uint32_t flat = uniform(gld(a.work + item));
+        const uint32_t kf = uniform(gld(a.pre_cnt + rel));
         const bool has = lane < (int)kf;
         int32_t o = 0;
         if (has) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
@@ -2022,50 +2167,47 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
                     const MapDesc& md = maps[r.y & 0xffffu];
                     mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
                     if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+                    team[turn ^ 1u].next = next;
                 }
             }
             __syncthreads();
-            idx = team[turn ^ 1u].next;
+            idx = uniform(team[turn ^ 1u].next);
             continue;
         }
         const int dx = packed_dx(o), dy = packed_dy(o);
         const uint32_t nq = has ? nbr_flat(a, x, y, o) : 0u;
+        // the list is ordered by distance: the last neighbour's bounds every offset
+        const int rad = __builtin_amdgcn_readlane((int)sqrtf((float)(dx * dx + dy * dy)) + 1, (int)kf - 1);
         // a candidate per lane: random ones in lanes 0..7, coherence ones in 8..15
         const uint32_t sl = (uint32_t)lane & (kSlots - 1);
-        uint32_t sxy = 0, smap = 0, scol = 0, spatch = 0, sidx = 0;
-        bool son = false;
+        SlotCand cand{false, 0u, 0u, 0u, 0u};
         uint32_t gp = kOutsidePx;
         if (GUIDED && has) gp = gld(a.tg + nq);
         uint32_t px[kSlots], gpx[kSlots];
+        auto colour_of = [&] {
+            const uint32_t w = ONE ? m0.w : maps[cand.map].w;
+            const uint32_t* mp = ONE ? m0.px : maps[cand.map].px;
+            const uint32_t at = (cand.xy >> 16) * w + (cand.xy & 0xffffu);
+            cand.colour = gld(mp + at);
+            return at;
+        };
         auto random_slots = [&](uint32_t q) {
             // the round's random candidates: pixels of every neighbour, own colour
             const uint32_t n = nrs > q * kSlots ? min(nrs - q * kSlots, kSlots) : 0u;
+            if (n == 0) {
+                if (lane < (int)kSlots) cand.on = false;
+                return n;
+            }
             if (lane < (int)kSlots) {
-                son = sl < n;
-                if (son) {
+                cand.on = sl < n;
+                if (cand.on) {
                     const uint2 r = rand_cand(a, item, r0 + q * kSlots + sl);
-                    sxy = r.x;
-                    smap = r.y;
+                    cand.xy = r.x;
+                    cand.map = r.y;
                 }
             }
-#pragma unroll
-            for (uint32_t c = 0; c < kSlots; ++c) {
-                px[c] = gpx[c] = kOutsidePx;
-                if (c < n) {
-                    const uint32_t cxy = (uint32_t)__builtin_amdgcn_readlane((int)sxy, (int)c);
-                    const uint32_t cm = (uint32_t)__builtin_amdgcn_readlane((int)smap, (int)c);
-                    if (has) {
-                        if (a.n_maps == 1) gather_xy<GUIDED>(m0, cxy, -dx, -dy, px[c], gpx[c]);
-                        else gather_xy<GUIDED>(maps[cm], cxy, -dx, -dy, px[c], gpx[c]);
-                    }
-                }
-            }
-            if (lane < (int)kSlots && son) {
-                const MapDesc& md = maps[smap];
-                const uint32_t f0 = (sxy >> 16) * md.w + (sxy & 0xffffu);
-                scol = gld(md.px + f0);
-                spatch = f0;
-            }
+            gather_slots<GUIDED, ONE, 0>(cand, m0, maps, -dx, -dy, rad, px, gpx);
+            if (lane < (int)kSlots && cand.on) cand.patch = colour_of();
             return n;
         };
         uint32_t n_r = random_slots(0);
@@ -2081,96 +2223,63 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
         if (wave == 0) {
             const uint4 st = flow_records(f, a, f.dep[rel], nq, has, lane);
             phase_clock(a, item, 1, lane);
+            const uint32_t cx = (st.y & 0xffffu) - (uint32_t)dx, cy = (st.y >> 16) - (uint32_t)dy, cm = st.z >> 16;
             bool ok = false;
-            uint32_t cx = 0, cy = 0, cm = 0;
             if (has) {
                 L->pat[lane] = st.x;
-                cx = (st.y & 0xffffu) - (uint32_t)dx;
-                cy = (st.y >> 16) - (uint32_t)dy;
-                cm = st.z >> 16;
-                ok = cm < a.n_maps && coord_ok(maps[cm], (int)cx, (int)cy);
+                ok = cm < a.n_maps && (ONE ? coord_ok(m0, (int)cx, (int)cy) : coord_ok(maps[cm], (int)cx, (int)cy));
             }
             const uint64_t om = __ballot(ok);
             if (ok) L->coh[bits_below(om)] = make_uint4(cx | (cy << 16), cm, st.w, 0u);
-            if (lane == 0) L->n_coh = (uint32_t)__popcll(om);
+            if (lane == 0) {
+                L->n_coh = (uint32_t)__popcll(om);
+                team[turn ^ 1u].next = next;
+            }
         }
         __syncthreads();
-        const uint32_t n_coh = L->n_coh;
+        const uint32_t n_coh = uniform(L->n_coh);
         if (!a.lut_nan && L->avg > 0.0) {
             if (wave == 0) phase_clock(a, item, 2, lane);
+            const uint32_t cper = (n_coh + T - 1) / T;
+            const uint32_t c0 = min(n_coh, (uint32_t)wave * cper), ncs = min(n_coh, c0 + cper) - c0;
             NbrRow row;
             row.q = bytes_scaled<C>(has ? L->pat[lane] : 0u);
             row.g = GUIDED ? bytes_scaled<C>(gp) : make_uint4(0, 0, 0, 0);
             row.w = has ? L->w[lane] : 0.0f;
-            const uint32_t cper = (n_coh + T - 1) / T;
-            const uint32_t c0 = min(n_coh, (uint32_t)wave * cper), ncs = min(n_coh, c0 + cper) - c0;
             // the lane's best candidate so far
             unsigned long long bkey = ~0ull;
-            uint32_t bxy = 0, bmap = 0, bcol = 0, bpatch = 0;
+            SlotCand best{};
             for (uint32_t q = 0;;) {
                 const uint32_t n_c = ncs > q * kSlots ? min(ncs - q * kSlots, kSlots) : 0u;
-                if (lane >= (int)kSlots) {
-                    son = lane < (int)(2 * kSlots) && sl < n_c;
-                    if (son) {
-                        const uint4 e = L->coh[c0 + q * kSlots + sl];
-                        sxy = e.x;
-                        smap = e.y;
-                        spatch = e.z;
-                    }
-                }
-                sidx = lane < (int)kSlots ? n_coh + r0 + q * kSlots + sl : c0 + q * kSlots + sl;
                 uint32_t cpx[kSlots], cgpx[kSlots];
-#pragma unroll
-                for (uint32_t c = 0; c < kSlots; ++c) {
-                    cpx[c] = cgpx[c] = kOutsidePx;
-                    if (c < n_c) {
-                        const uint32_t cxy = (uint32_t)__builtin_amdgcn_readlane((int)sxy, (int)(kSlots + c));
-                        const uint32_t cm = (uint32_t)__builtin_amdgcn_readlane((int)smap, (int)(kSlots + c));
-                        if (has) {
-                            if (a.n_maps == 1) gather_xy<GUIDED>(m0, cxy, dx, dy, cpx[c], cgpx[c]);
-                            else gather_xy<GUIDED>(maps[cm], cxy, dx, dy, cpx[c], cgpx[c]);
-                        }
+                if (lane >= (int)kSlots) {
+                    cand.on = lane < (int)(2 * kSlots) && sl < n_c;
+                    if (cand.on) {
+                        const uint4 e = L->coh[c0 + q * kSlots + sl];
+                        cand.xy = e.x;
+                        cand.map = e.y;
+                        cand.patch = e.z;
                     }
                 }
-                if (lane >= (int)kSlots && son) {
-                    const MapDesc& md = maps[smap];
-                    scol = gld(md.px + (sxy >> 16) * md.w + (sxy & 0xffffu));
+                if (n_c) {
+                    gather_slots<GUIDED, ONE, (int)kSlots>(cand, m0, maps, dx, dy, rad, cpx, cgpx);
+                    if (lane >= (int)kSlots && cand.on) colour_of();
                 }
-                // terms: row c of the round's 16, one neighbour per lane
-#pragma unroll
-                for (uint32_t c = 0; c < kSlots; ++c)
-                    if (c < n_r && has) rows[c * kTermRow + lane] = term_at<GUIDED>(row, lut, glut, slot4, px[c], gpx[c]);
-#pragma unroll
-                for (uint32_t c = 0; c < kSlots; ++c)
-                    if (c < n_c && has)
-                        rows[(kSlots + c) * kTermRow + lane] = term_at<GUIDED>(row, lut, glut, slot4, cpx[c], cgpx[c]);
+                slot_terms<GUIDED, C>(row, lut, glut, slot4, n_r, px, gpx, has, rows, lane);
+                if (n_c)
+                    slot_terms<GUIDED, C>(row, lut, glut, slot4, n_c, cpx, cgpx, has, rows + kSlots * kTermRow, lane);
                 wave_sync();
-                if (son) {
-                    // the reference's sequential f32 sum, terms read ahead of the adds
-                    const float* tp = rows + (uint32_t)lane * kTermRow;
-                    float s = 0.0f;
-                    uint32_t j = 0;
-                    for (; j + 16 <= kf; j += 16) {
-                        const float4 q0 = *reinterpret_cast<const float4*>(tp + j);
-                        const float4 q1 = *reinterpret_cast<const float4*>(tp + j + 4);
-                        const float4 q2 = *reinterpret_cast<const float4*>(tp + j + 8);
-                        const float4 q3 = *reinterpret_cast<const float4*>(tp + j + 12);
-                        s = __fadd_rn(s, q0.x); s = __fadd_rn(s, q0.y); s = __fadd_rn(s, q0.z); s = __fadd_rn(s, q0.w);
-                        s = __fadd_rn(s, q1.x); s = __fadd_rn(s, q1.y); s = __fadd_rn(s, q1.z); s = __fadd_rn(s, q1.w);
-                        s = __fadd_rn(s, q2.x); s = __fadd_rn(s, q2.y); s = __fadd_rn(s, q2.z); s = __fadd_rn(s, q2.w);
-                        s = __fadd_rn(s, q3.x); s = __fadd_rn(s, q3.y); s = __fadd_rn(s, q3.z); s = __fadd_rn(s, q3.w);
-                    }
-                    for (; j < kf; ++j) s = __fadd_rn(s, tp[j]);
+                if (cand.on) {
+                    const float s = row_sum(rows + (uint32_t)lane * kTermRow, kf);
+                    const uint32_t sidx =
+                        lane < (int)kSlots ? n_coh + r0 + q * kSlots + sl : c0 + q * kSlots + sl;
                     // a cost the reference's search cannot take over its start
                     // value counts as that value (find_best_match, ms.rs:1184-1224)
                     const unsigned long long key =
                         (unsigned long long)__float_as_uint(s < FLT_MAX ? s : FLT_MAX) << 32 | sidx;
                     if (key < bkey) {
                         bkey = key;
-                        bxy = sxy;
-                        bmap = smap;
-                        bcol = scol;
-                        bpatch = spatch;
+                        best = cand;
                     }
                 }
                 ++q;
@@ -2179,24 +2288,27 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
                 n_r = random_slots(q);
             }
             if (wave == 0) phase_clock(a, item, 4, lane);
-            if (bkey != ~0ull) atomicMin(&L->best, bkey);
+            // candidates sit in the first row's lanes
+            const unsigned long long rmin = row_min(bkey);
+            const unsigned long long mine = lane_u64(rmin, 0);
+            if (lane == 0) L->best[wave] = mine;
             __syncthreads();
             if (wave == 0) phase_clock(a, item, 5, lane);
-            const unsigned long long best = L->best;
-            if (bkey == best) {
+            const bool beaten = lane < T && L->best[lane < T ? lane : 0] < mine;
+            if (__ballot(beaten) == 0ull && lane < (int)(2 * kSlots) && bkey == mine && mine != ~0ull) {
                 // the winner's lane (indices differ): Generator::update
                 // (ms.rs:334-377), posted; a new pixel keeps its first score
-                const float cost = __uint_as_float((uint32_t)(best >> 32));
-                mail_post(f, flat, bcol, bxy, bmap, bpatch);
+                const float cost = __uint_as_float((uint32_t)(mine >> 32));
+                mail_post(f, flat, best.colour, best.xy, best.map, best.patch);
                 gst(a.item_score + item, cost);
                 if (item >= a.first_new) gst(a.score_w + flat, cost);
             }
         } else {
             if (wave == 0) {
-                float best = FLT_MAX;
+                float cost = FLT_MAX;
                 uint32_t bidx = 0;
-                item_exact<GUIDED>(a, maps, item, 0, kf, n_coh, n_coh + a.m, L, lut, glut, lane % C, lane, best, bidx);
-                const uint4 r = item_winner(a, maps, item, 0, n_coh, L, best, bidx, lane);
+                item_exact<GUIDED, C>(a, maps, item, 0, kf, n_coh, n_coh + a.m, L, lut, glut, lane % C, lane, cost, bidx);
+                const uint4 r = item_winner(a, maps, item, 0, n_coh, L, cost, bidx, lane);
                 if (lane == 0) {
                     const MapDesc& md = maps[r.y & 0xffffu];
                     mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
@@ -2206,7 +2318,312 @@ __global__ __launch_bounds__(kWave* T) void k_flow_team(BatchArgs a, FlowArgs f)
             __syncthreads();
         }
         if (wave == 0) phase_clock(a, item, 6, lane);
-        idx = team[turn ^ 1u].next;
+        idx = uniform(team[turn ^ 1u].next);
+    }
+    launch_span(a, t_start);
+}
+
+// What the eight members of a link team share of one item (two in turn, as
+// TeamLds).
+struct LinkLds {
+    double dist[kMaxK];
+    double avg;
+    unsigned long long best[kWavesPerWG];  // per member: least (cost bits << 32 | candidate order)
+    unsigned long long late;               // neighbours missing when the team started on the item
+    uint4 coh[kMaxK];                      // neighbour j's candidate: xy, map, patch, valid
+    int32_t nd[kMaxK];
+    float w[kMaxK];
+    uint32_t pat[kMaxK];
+    uint32_t gpat[kMaxK];
+    uint32_t next;                         // the workgroup's next item
+};
+
+// A run with a team of eight waves per item, for the smallest batches, whose
+// chain of items is the run's whole time. Evaluating an item takes its CU
+// some 2.5 us of VALU issue (5000 terms), and of 50 neighbours only the last
+// few are ever late. So the team starts once at most kPollAll records are
+// missing, and forms every term that they do not decide while they are on
+// their way; a late neighbour's pixel of each candidate waits in the term's
+// place. When a late record comes, a member adds that neighbour's column for
+// its 16 candidates in one go (a lane per candidate), the late neighbour's
+// own candidate is evaluated by one member, and the sums follow.
+// Member w holds the candidates of neighbours 8 w .. 8 w + 7 and an eighth of
+// the random ones (m <= 64); ties order coherence candidates by neighbour,
+// then the random ones, as the reference's list does.
+template <bool GUIDED, bool ONE>
+__global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(4))) void k_flow_link(BatchArgs a,
+                                                                                                          FlowArgs f) {
+    constexpr int T = kWavesPerWG;
+    const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ MapDesc smaps[kMapCache];
+    __shared__ LinkLds team[2];
+    __shared__ uint32_t late_g[GUIDED ? T : 1][GUIDED ? kPollAll : 1][2 * kSlots];
+    flow_args(a);
+    constexpr int C = team_copies<GUIDED, T>();
+    float *lut, *glut;
+    const MapDesc* maps;
+    if (threadIdx.x == 0) team[0].next = atomicAdd(f.ticket, 1u);
+    float* rows = reinterpret_cast<float*>(setup_lds<GUIDED, C>(a, smem, lut, glut, smaps, maps));  // ends with a barrier
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x % kWave;
+    rows += (size_t)wave * (2 * kSlots * kTermRow);
+    const uint32_t slot4 = (uint32_t)(lane % C) * 4u;
+    const MapDesc m0 = ld_uniform(maps);
+    const uint32_t rper = (a.m + T - 1) / T;
+    const uint32_t r0 = min(a.m, (uint32_t)wave * rper), n_r = min(a.m, r0 + rper) - r0;
+    const uint32_t sl = (uint32_t)lane & (kSlots - 1), c0 = (uint32_t)wave * kSlots;
+    uint32_t idx = uniform(team[0].next);
+    for (uint32_t turn = 0; idx < f.n; turn ^= 1u) {
+        LinkLds* L = &team[turn];
+        const uint32_t item = a.item0 + idx, rel = item - a.pre_base;
+        uint32_t next = 0;  // the ticket is on its way while the item waits
+        if (wave == 0) {
+            phase_clock(a, item, 0, lane);
+            if (lane == 0) next = atomicAdd(f.ticket, 1u);
+        }
+        const uint32_t flat = uniform(gld(a.work + item));
+        const uint32_t kf = uniform(gld(a.pre_cnt + rel));
+        const bool has = lane < (int)kf;
+        int32_t o = 0;
+        if (has) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
+        const int x = (int)(flat % a.W), y = (int)(flat / a.W);
+        if (kf == 0) {
+            // no resolved neighbour: alike for every member
+            if (wave == 0) {
+                const uint4 r = item_at_random(a, maps, item, 0, flat, lane);
+                if (lane == 0) {
+                    const MapDesc& md = maps[r.y & 0xffffu];
+                    mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
+                    if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+                    team[turn ^ 1u].next = next;
+                }
+            }
+            __syncthreads();
+            idx = uniform(team[turn ^ 1u].next);
+            continue;
+        }
+        const int dx = packed_dx(o), dy = packed_dy(o);
+        const uint32_t nq = has ? nbr_flat(a, x, y, o) : 0u;
+        // the list is ordered by distance: the last neighbour's bounds every offset
+        const int rad = __builtin_amdgcn_readlane((int)sqrtf((float)(dx * dx + dy * dy)) + 1, (int)kf - 1);
+        // a candidate per lane: random ones in lanes 0..7, neighbours' in 8..15
+        SlotCand cand{false, 0u, 0u, 0u, 0u};
+        uint32_t gp = kOutsidePx;
+        if (GUIDED && has) gp = gld(a.tg + nq);
+        auto colour_of = [&] {
+            const uint32_t w = ONE ? m0.w : maps[cand.map].w;
+            const uint32_t* mp = ONE ? m0.px : maps[cand.map].px;
+            const uint32_t at = (cand.xy >> 16) * w + (cand.xy & 0xffffu);
+            cand.colour = gld(mp + at);
+            return at;
+        };
+        uint32_t px[kSlots], gpx[kSlots];
+        if (n_r) {
+            if (lane < (int)n_r) {
+                const uint2 r = rand_cand(a, item, r0 + sl);
+                cand.on = true;
+                cand.xy = r.x;
+                cand.map = r.y;
+            }
+            gather_slots<GUIDED, ONE, 0>(cand, m0, maps, -dx, -dy, rad, px, gpx);
+            if (lane < (int)n_r) cand.patch = colour_of();
+        }
+        if (wave == T - 1) {
+            // the weights, from the neighbour offsets alone
+            if (has) {
+                L->nd[lane] = o;
+                if (GUIDED) L->gpat[lane] = gp;
+            }
+            wave_sync();
+            item_geometry(a, x, y, kf, L, lane);
+        }
+        // lane j's candidate from its neighbour's record
+        auto coherent = [&](const uint4& st) {
+            const uint32_t cx = (st.y & 0xffffu) - (uint32_t)dx, cy = (st.y >> 16) - (uint32_t)dy, cm = st.z >> 16;
+            const bool ok = cm < a.n_maps && (ONE ? coord_ok(m0, (int)cx, (int)cy) : coord_ok(maps[cm], (int)cx, (int)cy));
+            return make_uint4(cx | (cy << 16), cm, st.w, ok ? 1u : 0u);
+        };
+        const uint64_t dep = f.dep[rel];
+        uint4 st = make_uint4(0, 0, 0, 0);
+        if (wave == 0) {
+            uint64_t lt;
+            st = flow_records(f, a, dep, nq, has, lane, &lt);
+            phase_clock(a, item, 1, lane);
+            if (has && !((lt >> lane) & 1ull)) {
+                L->pat[lane] = st.x;
+                L->coh[lane] = coherent(st);
+            }
+            if (lane == 0) {
+                L->late = lt;
+                team[turn ^ 1u].next = next;
+            }
+        }
+        __syncthreads();
+        const uint64_t late = lane_u64(L->late, 0);
+        const bool mine_late = (late >> lane) & 1ull;
+        const bool exact = a.lut_nan || !(L->avg > 0.0);
+        if (!exact) {
+            if (wave == 0) phase_clock(a, item, 2, lane);
+            NbrRow row;
+            row.q = bytes_scaled<C>(has ? L->pat[lane] : 0u);
+            row.g = GUIDED ? bytes_scaled<C>(gp) : make_uint4(0, 0, 0, 0);
+            row.w = has ? L->w[lane] : 0.0f;
+            const uint32_t n_c = kf > c0 ? min(kf - c0, kSlots) : 0u;
+            uint32_t cpx[kSlots], cgpx[kSlots];
+            if (n_c) {
+                if (lane >= (int)kSlots && lane < (int)(kSlots + n_c) && !((late >> (c0 + sl)) & 1ull)) {
+                    const uint4 e = L->coh[c0 + sl];
+                    cand.on = e.w != 0u;
+                    cand.xy = e.x;
+                    cand.map = e.y;
+                    cand.patch = e.z;
+                }
+                gather_slots<GUIDED, ONE, (int)kSlots>(cand, m0, maps, dx, dy, rad, cpx, cgpx);
+                if (lane >= (int)kSlots && cand.on) colour_of();
+            }
+            const uint32_t lidx = bits_below(late);  // a late lane's place among the late
+            auto terms = [&](uint32_t n, const uint32_t(&p)[kSlots], const uint32_t(&g)[kSlots], uint32_t s0) {
+#pragma unroll
+                for (uint32_t h = 0; h < kSlots; h += 4) {
+                    if (h < n) {
+                        float t[4];
+#pragma unroll
+                        for (uint32_t c = 0; c < 4; ++c)
+                            t[c] = term_at<GUIDED, C>(row, lut, glut, slot4, p[h + c], g[h + c]);
+#pragma unroll
+                        for (uint32_t c = 0; c < 4; ++c) {
+                            t[c] = has ? t[c] : 0.0f;
+                            rows[(s0 + h + c) * kTermRow + lane] = mine_late ? __uint_as_float(p[h + c]) : t[c];
+                        }
+                        if (GUIDED && late) {
+#pragma unroll
+                            for (uint32_t c = 0; c < 4; ++c)
+                                if (mine_late) late_g[wave][lidx][s0 + h + c] = g[h + c];
+                        }
+                    }
+                }
+            };
+            terms(n_r, px, gpx, 0);
+            terms(n_c, cpx, cgpx, kSlots);
+            if (late) {
+                // the last records, polled by every member
+                const uint4 got = flow_records(f, a, dep & late, nq, mine_late, lane);
+                if (wave == 0) phase_clock(a, item, 7, lane);
+                if (mine_late) row.q = bytes_scaled<C>(got.x);
+                uint4 lc = make_uint4(0, 0, 0, 0);
+                if (mine_late) lc = coherent(got);
+                // this member's late candidates: their pixels first
+                const uint64_t own = (late >> c0) & 0xffull;
+                uint32_t lpx[kPollAll], lgpx[kPollAll];
+                uint64_t rest = own;
+#pragma unroll
+                for (uint32_t i = 0; i < kPollAll; ++i) {
+                    lpx[i] = lgpx[i] = kOutsidePx;
+                    if (rest) {
+                        const int j = __ffsll((long long)rest) - 1, src = (int)c0 + j;
+                        rest &= rest - 1;
+                        const uint32_t xy = (uint32_t)__builtin_amdgcn_readlane((int)lc.x, src);
+                        const uint32_t cm = (uint32_t)__builtin_amdgcn_readlane((int)lc.y, src);
+                        const uint32_t pt = (uint32_t)__builtin_amdgcn_readlane((int)lc.z, src);
+                        const bool on = __builtin_amdgcn_readlane((int)lc.w, src) != 0;
+                        if (lane == (int)kSlots + j) {
+                            cand.on = on;
+                            cand.xy = xy;
+                            cand.map = cm;
+                            cand.patch = pt;
+                            if (on) colour_of();
+                        }
+                        if (on) {
+                            if (ONE) gather_xy<GUIDED>(m0, xy, dx, dy, lpx[i], lgpx[i]);
+                            else gather_xy<GUIDED>(maps[cm], xy, dx, dy, lpx[i], lgpx[i]);
+                        }
+                    }
+                }
+                wave_sync();
+                // the late neighbours' columns, a candidate per lane
+                rest = late;
+                for (uint32_t i = 0; rest; ++i) {
+                    const int j = __ffsll((long long)rest) - 1;
+                    rest &= rest - 1;
+                    NbrRow rj;
+                    rj.q = bytes_scaled<C>((uint32_t)__builtin_amdgcn_readlane((int)got.x, j));
+                    rj.g = GUIDED ? bytes_scaled<C>((uint32_t)__builtin_amdgcn_readlane((int)gp, j))
+                                  : make_uint4(0, 0, 0, 0);
+                    rj.w = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(row.w), j));
+                    if (lane < (int)(2 * kSlots)) {
+                        float* at = rows + (uint32_t)lane * kTermRow + j;
+                        *at = term_at<GUIDED, C>(rj, lut, glut, slot4, __float_as_uint(*at),
+                                                 GUIDED ? late_g[wave][i][lane] : kOutsidePx);
+                    }
+                }
+                wave_sync();
+                rest = own;
+#pragma unroll
+                for (uint32_t i = 0; i < kPollAll; ++i) {
+                    if (rest) {
+                        const int j = __ffsll((long long)rest) - 1;
+                        rest &= rest - 1;
+                        const float t = term_at<GUIDED, C>(row, lut, glut, slot4, lpx[i], lgpx[i]);
+                        rows[(kSlots + j) * kTermRow + lane] = has ? t : 0.0f;
+                    }
+                }
+            }
+            wave_sync();
+            unsigned long long key = ~0ull;
+            if (cand.on) {
+                const float s = row_sum(rows + (uint32_t)lane * kTermRow, kf);
+                // a cost the reference's search cannot take over its start
+                // value counts as that value (find_best_match, ms.rs:1184-1224)
+                key = (unsigned long long)__float_as_uint(s < FLT_MAX ? s : FLT_MAX) << 32 |
+                      (lane < (int)kSlots ? kMaxK + r0 + sl : c0 + sl);
+            }
+            if (wave == 0) phase_clock(a, item, 4, lane);
+            const unsigned long long rmin = row_min(key);  // candidates sit in the first row's lanes
+            const unsigned long long mine = lane_u64(rmin, 0);
+            if (lane == 0) L->best[wave] = mine;
+            __syncthreads();
+            if (wave == 0) phase_clock(a, item, 5, lane);
+            const bool beaten = lane < T && L->best[lane < T ? lane : 0] < mine;
+            if (__ballot(beaten) == 0ull && cand.on && key == mine) {
+                // the winner's lane (orders differ): Generator::update
+                // (ms.rs:334-377), posted; a new pixel keeps its first score
+                const float cost = __uint_as_float((uint32_t)(mine >> 32));
+                mail_post(f, flat, cand.colour, cand.xy, cand.map, cand.patch);
+                gst(a.item_score + item, cost);
+                if (item >= a.first_new) gst(a.score_w + flat, cost);
+            }
+        } else {
+            if (wave == 0) {
+                // the unpruned rule reads the candidates in list order
+                if (late) {
+                    const uint4 got = flow_records(f, a, dep & late, nq, mine_late, lane);
+                    if (mine_late) st = got;
+                }
+                uint4 e = make_uint4(0, 0, 0, 0);
+                if (has) {
+                    L->pat[lane] = st.x;
+                    e = coherent(st);
+                }
+                const uint64_t om = __ballot(e.w != 0u);
+                wave_sync();
+                if (e.w) L->coh[bits_below(om)] = e;
+                wave_sync();
+                const uint32_t n_coh = (uint32_t)__popcll(om);
+                float cost = FLT_MAX;
+                uint32_t bidx = 0;
+                item_exact<GUIDED, C>(a, maps, item, 0, kf, n_coh, n_coh + a.m, L, lut, glut, lane % C, lane, cost, bidx);
+                const uint4 r = item_winner(a, maps, item, 0, n_coh, L, cost, bidx, lane);
+                if (lane == 0) {
+                    const MapDesc& md = maps[r.y & 0xffffu];
+                    mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
+                    if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+                }
+            }
+            __syncthreads();
+        }
+        if (wave == 0) phase_clock(a, item, 6, lane);
+        idx = uniform(team[turn ^ 1u].next);
     }
     launch_span(a, t_start);
 }
@@ -3233,16 +3650,28 @@ struct FlowKernel {
     uint32_t threads;
     size_t lds;
 };
-bool flow_kernel(uint32_t team, bool guided, FlowKernel* k) {
-    if (team == 1) {
-        *k = {guided ? k_flow_wave<true> : k_flow_wave<false>, (uint32_t)(kWave * kWavesPerWG), resolve_lds_bytes(guided)};
-        return true;
+// a guided job's two tables have half the copies each
+template <int T>
+FlowKernel team_kernel(bool guided, bool one) {
+    return {guided ? (one ? k_flow_team<true, T, true> : k_flow_team<true, T, false>)
+                   : (one ? k_flow_team<false, T, true> : k_flow_team<false, T, false>),
+            kWave * T, 256 * team_copies<false, T>() * sizeof(float) + T * kTeamWaveLds};
+}
+bool flow_kernel(uint32_t team, bool guided, bool one, FlowKernel* k) {
+    switch (team) {
+        case 1:
+            *k = {guided ? k_flow_wave<true> : k_flow_wave<false>, (uint32_t)(kWave * kWavesPerWG),
+                  resolve_lds_bytes(guided)};
+            return true;
+        case 2: *k = team_kernel<2>(guided, one); return true;
+        case 4: *k = team_kernel<4>(guided, one); return true;
+        case 8:
+            *k = {guided ? (one ? k_flow_link<true, true> : k_flow_link<true, false>)
+                         : (one ? k_flow_link<false, true> : k_flow_link<false, false>),
+                  kWave * kWavesPerWG, 256 * team_copies<false, 8>() * sizeof(float) + 8 * kTeamWaveLds};
+            return true;
+        default: return false;
     }
-    *k = {nullptr, kWave * team, lut_bytes(guided) + team * kTeamWaveLds};
-    if (team == 2) k->fn = guided ? k_flow_team<true, 2> : k_flow_team<false, 2>;
-    if (team == 4) k->fn = guided ? k_flow_team<true, 4> : k_flow_team<false, 4>;
-    if (team == 8) k->fn = guided ? k_flow_team<true, 8> : k_flow_team<false, 8>;
-    return k->fn != nullptr;
 }
 }  // namespace
 
@@ -3274,12 +3703,13 @@ hipError_t configure_kernels() {
                             (int)resolve_small_lds_bytes(false));
     if (e != hipSuccess) return e;
     for (uint32_t team : {1u, 2u, 4u, 8u})
-        for (bool guided : {false, true}) {
-            FlowKernel k;
-            if (!flow_kernel(team, guided, &k)) return hipErrorInvalidValue;
-            e = hipFuncSetAttribute((const void*)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
-            if (e != hipSuccess) return e;
-        }
+        for (bool guided : {false, true})
+            for (bool one : {false, true}) {
+                FlowKernel k;
+                if (!flow_kernel(team, guided, one, &k)) return hipErrorInvalidValue;
+                e = hipFuncSetAttribute((const void*)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
+                if (e != hipSuccess) return e;
+            }
     return hipFuncSetAttribute((const void*)k_resolve_small<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)resolve_small_lds_bytes(false));
 }
@@ -3512,7 +3942,7 @@ hipError_t launch_resolve_persist(const BatchArgs& a, uint32_t wgs, bool guided,
 
 uint32_t flow_max_wgs(uint32_t team, bool guided) {
     FlowKernel k;
-    if (!flow_kernel(team, guided, &k)) return 0;
+    if (!flow_kernel(team, guided, false, &k)) return 0;
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
@@ -3530,9 +3960,10 @@ hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t w
                                hipStream_t s) {
     if (f.n == 0) return hipSuccess;
     FlowKernel k;
-    if (!flow_kernel(team, guided, &k)) return hipErrorInvalidValue;
+    if (!flow_kernel(team, guided, a.n_maps == 1, &k)) return hipErrorInvalidValue;
     if (wgs == 0 || !f.ticket || !f.dep || !f.mail || !f.overflow || f.tag == 0 || f.tag > 255 || f.spin_limit == 0)
         return hipErrorInvalidValue;
+    if (team == 8 && a.m > kMaxK) return hipErrorInvalidValue;  // eight random candidates per member
     // every item needs its neighbour list; test hooks are not supported
     if (!a.pre_nbrs || a.item0 < a.pre_base || a.item0 + f.n > a.pre_end || a.ext_nbrs || a.ext_cands ||
         a.dbg_nbrs || a.dbg_best || a.knn_only || a.ext_full_cost || a.exact)

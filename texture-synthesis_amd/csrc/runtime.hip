@@ -1638,8 +1638,10 @@ struct Progress {
 uint32_t flow_team_of(const tsg_job* j, uint64_t i0, uint64_t i1) {
     const tsg_tuning& u = j->tune;
     if (i1 - i0 > u.prefetch_max) return 1;
-    if (i0 < u.flow_head) return u.flow_head_team;
-    return std::max(u.flow_team, team_for(i1 - i0, u.team_max, u.team_waves));
+    const uint32_t team =
+        i0 < u.flow_head ? u.flow_head_team : std::max(u.flow_team, team_for(i1 - i0, u.team_max, u.team_waves));
+    // the eight-wave kernel holds 64 random candidates
+    return team == 8 && j->prm.random_sample_locations > kMaxK ? 4u : team;
 }
 
 // The open stage in dependency order (k_flow_team, k_flow_wave): consecutive
