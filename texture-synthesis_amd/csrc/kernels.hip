@@ -118,6 +118,37 @@ __device__ __forceinline__ uint32_t bits_below(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t lane_u64(uint64_t v, int l) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+}
+
+// The less of a lane's key and the key that a DPP control brings it (rows
+// outside the mask keep theirs).
+template <int CTL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_min(unsigned long long k) {
+    const uint32_t l = (uint32_t)k, h = (uint32_t)(k >> 32);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)l, (int)l, CTL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)h, (int)h, CTL, ROWS, 0xf, false);
+    const unsigned long long o = (unsigned long long)hi << 32 | lo;
+    return o < k ? o : k;
+}
+// Least of a 64-bit key over the lanes of each row of 16, in every lane.
+__device__ __forceinline__ unsigned long long row_min(unsigned long long k) {
+    k = dpp_min<0x128, 0xf>(k);  // row_ror:8
+    k = dpp_min<0x124, 0xf>(k);  // row_ror:4
+    k = dpp_min<0x122, 0xf>(k);  // row_ror:2
+    return dpp_min<0x121, 0xf>(k);  // row_ror:1
+}
+// ... and over the wave, in scalars.
+__device__ __forceinline__ unsigned long long wave_min(unsigned long long k) {
+    k = row_min(k);
+    k = dpp_min<0x142, 0xa>(k);  // row_bcast:15 into rows 1 and 3
+    k = dpp_min<0x143, 0xc>(k);  // row_bcast:31 into rows 2 and 3
+    return lane_u64(k, kWave - 1);
+}
+
 // Canonical neighbour order: squared distance, then dy, then dx, ascending.
 __device__ __forceinline__ uint64_t make_key(int dx, int dy) {
     uint64_t d2 = (uint64_t)((int64_t)dx * dx + (int64_t)dy * dy);
@@ -782,6 +813,20 @@ __device__ __forceinline__ void gather_xy(const MapDesc& md, uint32_t xy, int dx
         gp = gin ? gld_at(gpx, (__umul24((uint32_t)Y2, gw) + (uint32_t)X2) * 4u) : kOutsidePx;
     }
 }
+// The same without a branch: the address is clamped into the map.
+template <bool GUIDED>
+__device__ __forceinline__ void gather_clamped(const MapDesc& md, uint32_t xy, int dx, int dy, uint32_t& p, uint32_t& gp) {
+    const uint32_t X = (xy & 0xffffu) + (uint32_t)dx, Y = (xy >> 16) + (uint32_t)dy;
+    const bool in = X < md.w && Y < md.h;
+    const uint32_t v = gld_at(md.px, in ? (__umul24(Y, md.w) + X) * 4u : 0u);
+    p = in ? v : kOutsidePx;
+    gp = kOutsidePx;
+    if (GUIDED) {
+        const bool gin = X < md.gw && Y < md.gh;
+        const uint32_t g = gld_at(md.gpx, gin ? (__umul24(Y, md.gw) + X) * 4u : 0u);
+        gp = gin ? g : kOutsidePx;
+    }
+}
 // Candidate (xy, map word ms): its map, and its mirror bit applied per lane.
 template <bool GUIDED>
 __device__ __forceinline__ void gather_at(const MapDesc* maps, uint32_t xy, uint32_t ms, int dx, int dy,
@@ -886,15 +931,24 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
         const NbrRow row = nbr_row<GUIDED>(L, j0 + (jin ? jj : 0u));
         // all gathers of the chunk first (at most kTermCap / 64 per lane), then
         // the LUT sums. With one example (its descriptor held in scalars) and
-        // one mirror state for the group, the offset's sign is applied once.
+        // one mirror state for the group, the offset's sign is applied once and
+        // the address clamped instead of branched around, so that a pair of
+        // slices is straight-line code; slices past the chunk's end and lanes
+        // past its neighbours do harmless work on stale entries (their terms
+        // are not summed).
         uint32_t px[kTermCap / kWave], gpx[kTermCap / kWave];
         if (n_maps == 1 && g_mir != 2) {
             const int ddx = g_mir ? -row.dx : row.dx, ddy = g_mir ? -row.dy : row.dy;
 #pragma unroll
-            for (int u = 0; u < kTermCap / kWave; ++u) {
-                const uint32_t l = (uint32_t)(u * kWave + lane), ai = l >> sh;
-                px[u] = gpx[u] = 0;
-                if (l < total && jin) gather_xy<GUIDED>(m0, L->act_xy[ai], ddx, ddy, px[u], gpx[u]);
+            for (int u = 0; u < kTermCap / kWave; u += 2) {
+                px[u] = px[u + 1] = gpx[u] = gpx[u + 1] = 0;
+                if ((uint32_t)(u * kWave) < total) {
+#pragma unroll
+                    for (int i = u; i < u + 2; ++i) {
+                        const uint32_t ai = (uint32_t)(i * kWave + lane) >> sh;
+                        gather_clamped<GUIDED>(m0, L->act_xy[ai & (kWave - 1)], ddx, ddy, px[i], gpx[i]);
+                    }
+                }
             }
         } else {
 #pragma unroll
@@ -905,9 +959,13 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
             }
         }
 #pragma unroll
-        for (int u = 0; u < kTermCap / kWave; ++u) {
-            const uint32_t l = (uint32_t)(u * kWave + lane);
-            if (l < total && jin) L->terms[l] = term_at<GUIDED>(row, lut, glut, slot4, px[u], gpx[u]);
+        for (int u = 0; u < kTermCap / kWave; u += 2) {
+            if ((uint32_t)(u * kWave) < total) {
+                const float t0 = term_at<GUIDED>(row, lut, glut, slot4, px[u], gpx[u]);
+                const float t1 = term_at<GUIDED>(row, lut, glut, slot4, px[u + 1], gpx[u + 1]);
+                L->terms[u * kWave + lane] = t0;
+                L->terms[(u + 1) * kWave + lane] = t1;
+            }
         }
         wave_sync();
         const bool act = lane < (int)n_act;
@@ -941,25 +999,17 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
         }
         j0 += jn;
         if (j0 >= kf) {
-            float key = act ? s : INFINITY;
-            uint32_t ki = myidx, kxy = xy, kms = ms;
-            for (int off = kWave / 2; off > 0; off >>= 1) {
-                float ok = __shfl_xor(key, off);
-                uint32_t oi = (uint32_t)__shfl_xor((int)ki, off);
-                uint32_t oxy = (uint32_t)__shfl_xor((int)kxy, off);
-                uint32_t oms = (uint32_t)__shfl_xor((int)kms, off);
-                if (ok < key || (ok == key && oi < ki)) {
-                    key = ok;
-                    ki = oi;
-                    kxy = oxy;
-                    kms = oms;
-                }
-            }
-            if (key < best.B || (key == best.B && best.Bi != kNone && ki < best.Bi)) {
-                best.B = key;
+            // costs are not negative, so their bits order them
+            const unsigned long long key = act ? (unsigned long long)__float_as_uint(s) << 32 | myidx : ~0ull;
+            const unsigned long long k = wave_min(key);
+            const float kB = __uint_as_float((uint32_t)(k >> 32));
+            const uint32_t ki = (uint32_t)k;
+            if (kB < best.B || (kB == best.B && best.Bi != kNone && ki < best.Bi)) {
+                const int l = __ffsll((long long)__ballot(key == k)) - 1;
+                best.B = kB;
                 best.Bi = ki;
-                best.xy = kxy;
-                best.ms = kms;
+                best.xy = (uint32_t)__builtin_amdgcn_readlane((int)xy, l);
+                best.ms = (uint32_t)__builtin_amdgcn_readlane((int)ms, l);
             }
             // publish: another member's complete cost bounds this one's candidates
             if (tb && lane == 0 && best.Bi != kNone)
@@ -1171,7 +1221,8 @@ __device__ __forceinline__ uint32_t item_neighbours(const BatchArgs& a, const Ma
     while (pending) {
         int l = __ffsll((long long)pending) - 1;
         uniq |= 1ull << l;
-        uint32_t kxy = (uint32_t)__shfl((int)xy, l), kms = (uint32_t)__shfl((int)ms, l);
+        const uint32_t kxy = (uint32_t)__builtin_amdgcn_readlane((int)xy, l);
+        const uint32_t kms = (uint32_t)__builtin_amdgcn_readlane((int)ms, l);
         pending &= ~__ballot(v && xy == kxy && ms == kms);
     }
     return n_coh;
@@ -1976,29 +2027,6 @@ constexpr size_t kTeamWaveLds = 2 * kSlots * kTermRow * sizeof(float);
 template <bool GUIDED, int T>
 constexpr int team_copies() {
     return (T == 8 ? 32 : T == 4 ? 16 : 8) / (GUIDED ? 2 : 1);
-}
-
-// Least of a 64-bit key over the lanes of each row of 16, in every lane.
-__device__ __forceinline__ unsigned long long row_min(unsigned long long k) {
-#define TSG_ROW_MIN(ctl)                                                                                             \
-    {                                                                                                                \
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)k, ctl, 0xf, 0xf, false);        \
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(k >> 32), ctl, 0xf, 0xf, false); \
-        const unsigned long long o = (unsigned long long)hi << 32 | lo;                                              \
-        k = o < k ? o : k;                                                                                           \
-    }
-    TSG_ROW_MIN(0x128)  // row_ror:8
-    TSG_ROW_MIN(0x124)  // row_ror:4
-    TSG_ROW_MIN(0x122)  // row_ror:2
-    TSG_ROW_MIN(0x121)  // row_ror:1
-#undef TSG_ROW_MIN
-    return k;
-}
-
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ __forceinline__ uint64_t lane_u64(uint64_t v, int l) {
-    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32 |
-           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
 }
 
 // The candidate a lane holds for its team member (lane c: slot c of a round).
