@@ -196,6 +196,31 @@ struct PickArgs {
 };
 hipError_t launch_picks(const PickArgs& a, hipStream_t s);
 
+// The u[i] = i list of n entries, but u[moves[q].x] = moves[q].y.
+hipError_t launch_list(uint32_t* u, uint32_t n, const uint2* moves, uint32_t n_moves, hipStream_t s);
+
+// A job's maps before the first stage: nothing resolved, colours of `base`
+// (an inpainting's example, of the output's size) or zero.
+struct InitArgs {
+    uint32_t n, W, tiles_x, tiles;
+    const uint32_t* base;    // null: none
+    uint4* state;
+    uint32_t* rank;
+    float* score;
+    uint64_t* mask;
+    uint64_t* gmask;         // tiling mode (else null): as mask
+};
+// A pixel resolved before the stages.
+struct InitPoint {
+    uint32_t flat, colour, xy, maps;
+};
+hipError_t launch_init_fill(const InitArgs& a, hipStream_t s);
+// rlist[0, n): kept pixels of an inpainting, their own source in `map`.
+hipError_t launch_init_kept(const InitArgs& a, const uint32_t* rlist, uint32_t n, uint32_t map, hipStream_t s);
+// n points into resolved-list positions from q0 on.
+hipError_t launch_init_points(const InitArgs& a, const InitPoint* pts, uint32_t n, uint32_t q0, uint32_t* rlist,
+                              hipStream_t s);
+
 // Words of a random candidate: x | y << 16, and its map unless there is but one.
 __host__ __device__ constexpr uint32_t rand_words(uint32_t n_maps) { return n_maps == 1 ? 1u : 2u; }
 
@@ -458,12 +483,30 @@ uint32_t persist_max_wgs(bool guided);
 hipError_t launch_resolve_persist(const BatchArgs& a, uint32_t wgs, bool guided, hipStream_t s);
 hipError_t launch_defer_flush(const DeferFlushArgs& a, hipStream_t s);
 hipError_t launch_recolor(const RecolorArgs& a, hipStream_t s);
-// separable resampling pass: vertical (u8 -> f32) and horizontal (f32 -> u8)
-hipError_t launch_resample_v(const uint32_t* src, uint32_t w, uint32_t h, float4* dst, uint32_t nh,
-                             const uint32_t* left, const uint32_t* cnt, const float* ws, uint32_t stride,
-                             hipStream_t s);
-hipError_t launch_resample_h(const float4* src, uint32_t w, uint32_t h, uint32_t* dst, uint32_t nw,
-                             const uint32_t* left, const uint32_t* cnt, const float* ws, uint32_t stride,
-                             hipStream_t s);
+// One separable resampling pass of one image: vertical (u8 -> f32 rows) or
+// horizontal (f32 rows -> u8), out_w x out_h outputs. Output rows (vertical)
+// or columns (horizontal) o take taps[at + n_o + o] inputs from taps[at + o]
+// on, n_o = the number of rows or columns, weighted by the `stride` floats
+// from taps[at + 2 n_o + o * stride] on.
+struct ResampleUnit {
+    const void* src;
+    void* dst;
+    uint32_t out_w, out_h;
+    uint32_t src_w;
+    uint32_t at, stride;
+    uint32_t block0;       // the launch's first workgroup of this image
+};
+// Workgroups of a pass with w x h outputs.
+inline uint32_t resample_blocks(uint32_t w, uint32_t h) {
+    return w >= 256 ? (w + 255) / 256 * h : (h + 256 / w - 1) / (256 / w);
+}
+hipError_t launch_resample(const ResampleUnit* units, uint32_t n, uint32_t blocks, const uint32_t* taps, bool horizontal,
+                           hipStream_t s);
+// n words of zeros.
+hipError_t launch_zero(uint32_t* p, size_t n, hipStream_t s);
+// RGBA8 to luma (in all three channels, alpha 255) in place; hist[256] += its values.
+hipError_t launch_luma(uint32_t* px, uint32_t n, uint32_t* hist, hipStream_t s);
+// Values of px (luma) moved so that their histogram follows `to`'s; map: 256 words of scratch.
+hipError_t launch_match(uint32_t* px, uint32_t n, const uint32_t* from, const uint32_t* to, uint32_t* map, hipStream_t s);
 
 }  // namespace tsg

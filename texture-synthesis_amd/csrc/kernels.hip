@@ -3173,23 +3173,51 @@ __global__ void k_recolor(RecolorArgs a) {
     reinterpret_cast<uint32_t*>(&a.state[p])[0] = md.px[(st.y >> 16) * md.w + (st.y & 0xffffu)];
 }
 
-// image 0.23 vertical_sample: u8 in, f32 out, taps summed in order.
-__global__ void k_resample_v(const uint32_t* src, uint32_t w, uint32_t h, float4* dst, uint32_t nh,
-                             const uint32_t* left, const uint32_t* cnt, const float* ws, uint32_t stride) {
-    uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t oy = blockIdx.y;
-    if (x >= w || oy >= nh) return;
+// The unit of a workgroup, and the output (x, y) of its thread: rows of 256
+// outputs and more take whole workgroups, shorter rows share one.
+__device__ __forceinline__ bool resample_output(const ResampleUnit* units, uint32_t n, ResampleUnit& u, uint32_t& x,
+                                                uint32_t& y) {
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (units[mid].block0 <= blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    u = units[lo];
+    const uint32_t b = blockIdx.x - u.block0;
+    if (u.out_w >= 256) {
+        const uint32_t per = (u.out_w + 255) / 256;
+        y = b / per;
+        x = (b - y * per) * 256 + threadIdx.x;
+        return x < u.out_w && y < u.out_h;
+    }
+    const uint32_t rows = 256 / u.out_w, r = threadIdx.x / u.out_w;
+    y = b * rows + r;
+    x = threadIdx.x - r * u.out_w;
+    return r < rows && y < u.out_h;
+}
+
+// image 0.23 vertical_sample: u8 in, f32 out. The passes of a job's pyramids
+// run together, so that small levels fill the chip: bound by the L2 reads of
+// the wide levels (six per input pixel and level).
+__global__ void __launch_bounds__(256) k_resample_v(const ResampleUnit* units, uint32_t n_units, const uint32_t* taps) {
+    ResampleUnit u;
+    uint32_t x, oy;
+    if (!resample_output(units, n_units, u, x, oy)) return;
+    const uint32_t* src = static_cast<const uint32_t*>(u.src);
+    const uint32_t* t = taps + u.at;
+    const float* ws = reinterpret_cast<const float*>(t + 2 * (size_t)u.out_h) + (size_t)oy * u.stride;
     float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f, t3 = 0.0f;
-    uint32_t l = left[oy], n = cnt[oy];
+    const uint32_t l = t[oy], n = t[(size_t)u.out_h + oy];
     for (uint32_t i = 0; i < n; ++i) {
-        float wt = ws[oy * stride + i];
-        uint32_t p = src[(size_t)(l + i) * w + x];
+        const float wt = ws[i];
+        const uint32_t p = src[(size_t)(l + i) * u.src_w + x];
         t0 = __fadd_rn(t0, __fmul_rn((float)(p & 255u), wt));
         t1 = __fadd_rn(t1, __fmul_rn((float)((p >> 8) & 255u), wt));
         t2 = __fadd_rn(t2, __fmul_rn((float)((p >> 16) & 255u), wt));
         t3 = __fadd_rn(t3, __fmul_rn((float)(p >> 24), wt));
     }
-    dst[(size_t)oy * w + x] = make_float4(t0, t1, t2, t3);
+    static_cast<float4*>(u.dst)[(size_t)oy * u.out_w + x] = make_float4(t0, t1, t2, t3);
 }
 
 __device__ __forceinline__ uint32_t to_u8(float t) {
@@ -3198,22 +3226,134 @@ __device__ __forceinline__ uint32_t to_u8(float t) {
 }
 
 // image 0.23 horizontal_sample: f32 in, clamped and rounded u8 out.
-__global__ void k_resample_h(const float4* src, uint32_t w, uint32_t h, uint32_t* dst, uint32_t nw,
-                             const uint32_t* left, const uint32_t* cnt, const float* ws, uint32_t stride) {
-    uint32_t ox = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t y = blockIdx.y;
-    if (ox >= nw || y >= h) return;
+__global__ void __launch_bounds__(256) k_resample_h(const ResampleUnit* units, uint32_t n_units, const uint32_t* taps) {
+    ResampleUnit u;
+    uint32_t ox, y;
+    if (!resample_output(units, n_units, u, ox, y)) return;
+    const uint32_t* t = taps + u.at;
+    const float* ws = reinterpret_cast<const float*>(t + 2 * (size_t)u.out_w) + (size_t)ox * u.stride;
     float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f, t3 = 0.0f;
-    uint32_t l = left[ox], n = cnt[ox];
+    const uint32_t l = t[ox], n = t[(size_t)u.out_w + ox];
+    const float4* src = static_cast<const float4*>(u.src) + (size_t)y * u.src_w + l;
     for (uint32_t i = 0; i < n; ++i) {
-        float wt = ws[ox * stride + i];
-        float4 p = src[(size_t)y * w + l + i];
+        const float wt = ws[i];
+        const float4 p = src[i];
         t0 = __fadd_rn(t0, __fmul_rn(p.x, wt));
         t1 = __fadd_rn(t1, __fmul_rn(p.y, wt));
         t2 = __fadd_rn(t2, __fmul_rn(p.z, wt));
         t3 = __fadd_rn(t3, __fmul_rn(p.w, wt));
     }
-    dst[(size_t)y * nw + ox] = to_u8(t0) | (to_u8(t1) << 8) | (to_u8(t2) << 16) | (to_u8(t3) << 24);
+    static_cast<uint32_t*>(u.dst)[(size_t)y * u.out_w + ox] =
+        to_u8(t0) | (to_u8(t1) << 8) | (to_u8(t2) << 16) | (to_u8(t3) << 24);
+}
+
+__global__ void k_zero(uint32_t* p, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+// image 0.23 rgb_to_luma (0.2126 R + 0.7152 G + 0.0722 B in f32, cast to u8)
+// and the histogram of its values.
+__global__ void __launch_bounds__(256) k_luma(uint32_t* px, uint32_t n, uint32_t* hist) {
+    __shared__ uint32_t h[256];
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const uint32_t p = px[i];
+        float l = __fmul_rn(0.2126f, (float)(p & 255u));
+        l = __fadd_rn(l, __fmul_rn(0.7152f, (float)((p >> 8) & 255u)));
+        l = __fadd_rn(l, __fmul_rn(0.0722f, (float)((p >> 16) & 255u)));
+        const uint32_t v = (uint32_t)l & 255u;
+        px[i] = v | (v << 8) | (v << 16) | 0xff000000u;
+        atomicAdd(&h[v], 1u);
+    }
+    __syncthreads();
+    if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
+}
+
+// get_cdf / match_histograms (utils.rs:118-183): each value moves to the
+// position before the first target CDF entry above its own CDF; the u8
+// arithmetic wraps as the release build's does. One workgroup.
+__global__ void __launch_bounds__(256) k_match_map(const uint32_t* from, const uint32_t* to, uint32_t* map) {
+    __shared__ uint32_t h[2][256];
+    __shared__ float c[2][256];
+    const uint32_t v = threadIdx.x;
+    h[0][v] = from[v];
+    h[1][v] = to[v];
+    __syncthreads();
+    if (v < 2) {  // in order: f32 sums
+        float sum = (float)h[v][0];
+        c[v][0] = sum;
+        for (int i = 1; i < 256; ++i) c[v][i] = sum = __fadd_rn(sum, (float)h[v][i]);
+    }
+    __syncthreads();
+    const float m0 = c[0][255], m1 = c[1][255];
+    __syncthreads();
+    c[0][v] = __fdiv_rn(c[0][v], m0);
+    c[1][v] = __fdiv_rn(c[1][v], m1);
+    __syncthreads();
+    int pos = -1;
+    for (int q = 255; q >= 0; --q)
+        if (c[1][q] > c[0][v]) pos = q;
+    map[v] = ((pos >= 0 ? (uint32_t)pos : v + 1u) - 1u) & 255u;
+}
+
+__global__ void k_match_apply(uint32_t* px, uint32_t n, const uint32_t* map) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t v = map[px[i] & 255u];
+    px[i] = v | (v << 8) | (v << 16) | 0xff000000u;
+}
+
+// A job's maps before the first stage. Bound by HBM: 28 bytes written a pixel.
+__global__ void k_init_fill(InitArgs a) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < a.n) {
+        a.state[i] = make_uint4(a.base ? a.base[i] : 0u, 0u, 0u, 0u);
+        a.rank[i] = UINT32_MAX;
+        a.score[i] = 0.0f;
+    }
+    if (i < a.tiles) {  // every tile has a pixel of its own: tiles <= n
+        a.mask[i] = 0;
+        if (a.gmask) a.gmask[i] = 0;
+    }
+}
+
+__device__ __forceinline__ void init_resolved(const InitArgs& a, uint32_t f, uint32_t q) {
+    const uint32_t x = f % a.W, y = f / a.W;
+    a.rank[f] = q;
+    const unsigned long long bit = 1ull << (((y & 7u) << 3) | (x & 7u));
+    const uint32_t t = (y >> 3) * a.tiles_x + (x >> 3);
+    atomicOr(reinterpret_cast<unsigned long long*>(a.mask) + t, bit);
+    // every pixel resolved before the stages starts with its ghost copies (ms.rs:296-331)
+    if (a.gmask) atomicOr(reinterpret_cast<unsigned long long*>(a.gmask) + t, bit);
+}
+
+__global__ void k_init_kept(InitArgs a, const uint32_t* rlist, uint32_t n, uint32_t map) {
+    const uint32_t q = blockIdx.x * 256u + threadIdx.x;
+    if (q >= n) return;
+    const uint32_t f = rlist[q];
+    a.state[f] = make_uint4(a.base[f], (f % a.W) | ((f / a.W) << 16), map, 0u);
+    init_resolved(a, f, q);
+}
+
+__global__ void k_init_points(InitArgs a, const InitPoint* pts, uint32_t n, uint32_t q0, uint32_t* rlist) {
+    const uint32_t q = blockIdx.x * 256u + threadIdx.x;
+    if (q >= n) return;
+    const InitPoint p = pts[q];
+    a.state[p.flat] = make_uint4(p.colour, p.xy, p.maps, p.flat);
+    rlist[q0 + q] = p.flat;
+    init_resolved(a, p.flat, q0 + q);
+}
+
+__global__ void k_list(uint32_t* u, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) u[i] = i;
+}
+
+__global__ void k_list_moves(uint32_t* u, uint32_t n, const uint2* moves, uint32_t n_moves) {
+    const uint32_t q = blockIdx.x * 256u + threadIdx.x;
+    if (q < n_moves && moves[q].x < n) u[moves[q].x] = moves[q].y;
 }
 
 __global__ void k_stats(StatsArgs a) {
@@ -4052,19 +4192,49 @@ hipError_t launch_recolor(const RecolorArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_resample_v(const uint32_t* src, uint32_t w, uint32_t h, float4* dst, uint32_t nh,
-                             const uint32_t* left, const uint32_t* cnt, const float* ws, uint32_t stride,
-                             hipStream_t s) {
-    hipLaunchKernelGGL(k_resample_v, dim3((w + 255) / 256, nh), dim3(256), 0, s, src, w, h, dst, nh, left, cnt, ws,
-                       stride);
+hipError_t launch_init_fill(const InitArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(k_init_fill, dim3((a.n + 255) / 256), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_resample_h(const float4* src, uint32_t w, uint32_t h, uint32_t* dst, uint32_t nw,
-                             const uint32_t* left, const uint32_t* cnt, const float* ws, uint32_t stride,
-                             hipStream_t s) {
-    hipLaunchKernelGGL(k_resample_h, dim3((nw + 255) / 256, h), dim3(256), 0, s, src, w, h, dst, nw, left, cnt, ws,
-                       stride);
+hipError_t launch_init_kept(const InitArgs& a, const uint32_t* rlist, uint32_t n, uint32_t map, hipStream_t s) {
+    hipLaunchKernelGGL(k_init_kept, dim3((n + 255) / 256), dim3(256), 0, s, a, rlist, n, map);
+    return hipGetLastError();
+}
+
+hipError_t launch_init_points(const InitArgs& a, const InitPoint* pts, uint32_t n, uint32_t q0, uint32_t* rlist,
+                              hipStream_t s) {
+    hipLaunchKernelGGL(k_init_points, dim3((n + 255) / 256), dim3(256), 0, s, a, pts, n, q0, rlist);
+    return hipGetLastError();
+}
+
+hipError_t launch_list(uint32_t* u, uint32_t n, const uint2* moves, uint32_t n_moves, hipStream_t s) {
+    if (n) hipLaunchKernelGGL(k_list, dim3((n + 255) / 256), dim3(256), 0, s, u, n);
+    if (n_moves) hipLaunchKernelGGL(k_list_moves, dim3((n_moves + 255) / 256), dim3(256), 0, s, u, n, moves, n_moves);
+    return hipGetLastError();
+}
+
+hipError_t launch_resample(const ResampleUnit* units, uint32_t n, uint32_t blocks, const uint32_t* taps, bool horizontal,
+                           hipStream_t s) {
+    if (n == 0 || blocks == 0) return hipSuccess;
+    if (horizontal) hipLaunchKernelGGL(k_resample_h, dim3(blocks), dim3(256), 0, s, units, n, taps);
+    else hipLaunchKernelGGL(k_resample_v, dim3(blocks), dim3(256), 0, s, units, n, taps);
+    return hipGetLastError();
+}
+
+hipError_t launch_zero(uint32_t* p, size_t n, hipStream_t s) {
+    if (n) hipLaunchKernelGGL(k_zero, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, p, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_luma(uint32_t* px, uint32_t n, uint32_t* hist, hipStream_t s) {
+    hipLaunchKernelGGL(k_luma, dim3(std::min(1024u, (n + 1023) / 1024)), dim3(256), 0, s, px, n, hist);
+    return hipGetLastError();
+}
+
+hipError_t launch_match(uint32_t* px, uint32_t n, const uint32_t* from, const uint32_t* to, uint32_t* map, hipStream_t s) {
+    hipLaunchKernelGGL(k_match_map, dim3(1), dim3(256), 0, s, from, to, map);
+    hipLaunchKernelGGL(k_match_apply, dim3((n + 255) / 256), dim3(256), 0, s, px, n, map);
     return hipGetLastError();
 }
 

@@ -22,6 +22,8 @@
 #include <deque>
 #include <map>
 #include <thread>
+#include <tuple>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/tsgpu.h"
@@ -163,6 +165,16 @@ struct DBuf {
     hipError_t reserve(size_t count) { return count <= n ? hipSuccess : alloc(count); }
 };
 
+// Blocks that no queued work uses any more (their stream was waited for),
+// back to the device's cache.
+template <class... B>
+void give_back(B&... b) {
+    const bool was = g_pool_release;
+    g_pool_release = true;
+    (b.release(), ...);
+    g_pool_release = was;
+}
+
 // ---- image 0.23 separable resampling weights (imageops/sample.rs) ----
 struct Filter {
     float (*kernel)(float);
@@ -196,158 +208,6 @@ float kern_gaussian(float x) {
     const float r = 0.5f;
     float c = 1.0f / (std::sqrt(2.0f * 3.14159265358979323846f) * r);
     return c * std::exp(-(x * x) / (2.0f * (r * r)));
-}
-
-struct Taps {
-    std::vector<uint32_t> left, cnt;
-    std::vector<float> ws;
-    uint32_t stride = 0;
-};
-
-Taps make_taps(uint32_t in_len, uint32_t out_len, const Filter& f) {
-    Taps t;
-    float ratio = (float)in_len / (float)out_len;
-    float sratio = ratio < 1.0f ? 1.0f : ratio;
-    float support = f.support * sratio;
-    std::vector<std::vector<float>> tmp(out_len);
-    t.left.resize(out_len);
-    t.cnt.resize(out_len);
-    for (uint32_t o = 0; o < out_len; ++o) {
-        float in = ((float)o + 0.5f) * ratio;
-        int64_t l = (int64_t)std::floor(in - support);
-        l = std::min<int64_t>(std::max<int64_t>(l, 0), (int64_t)in_len - 1);
-        int64_t r = (int64_t)std::ceil(in + support);
-        r = std::min<int64_t>(std::max<int64_t>(r, l + 1), (int64_t)in_len);
-        in = in - 0.5f;
-        float sum = 0.0f;
-        for (int64_t i = l; i < r; ++i) {
-            float w = f.kernel(((float)i - in) / sratio);
-            tmp[o].push_back(w);
-            sum += w;
-        }
-        for (float& w : tmp[o]) w /= sum;
-        t.left[o] = (uint32_t)l;
-        t.cnt[o] = (uint32_t)(r - l);
-        t.stride = std::max(t.stride, t.cnt[o]);
-    }
-    t.ws.assign((size_t)out_len * t.stride, 0.0f);
-    for (uint32_t o = 0; o < out_len; ++o)
-        for (uint32_t i = 0; i < t.cnt[o]; ++i) t.ws[(size_t)o * t.stride + i] = tmp[o][i];
-    return t;
-}
-
-struct DevTaps {
-    DBuf<uint32_t> left, cnt;
-    DBuf<float> ws;
-    uint32_t stride = 0;
-    hipError_t upload(const Taps& t, hipStream_t s) {
-        hipError_t e;
-        if ((e = left.alloc(t.left.size())) != hipSuccess) return e;
-        if ((e = cnt.alloc(t.cnt.size())) != hipSuccess) return e;
-        if ((e = ws.alloc(t.ws.size())) != hipSuccess) return e;
-        stride = t.stride;
-        if ((e = hipMemcpyAsync(left.p, t.left.data(), t.left.size() * 4, hipMemcpyHostToDevice, s)) != hipSuccess)
-            return e;
-        if ((e = hipMemcpyAsync(cnt.p, t.cnt.data(), t.cnt.size() * 4, hipMemcpyHostToDevice, s)) != hipSuccess)
-            return e;
-        return hipMemcpyAsync(ws.p, t.ws.data(), t.ws.size() * 4, hipMemcpyHostToDevice, s);
-    }
-};
-
-// imageops::resize(img, nw, nh, filter) on the device: vertical then
-// horizontal pass (f32 in between, rounded u8 out).
-int device_resize(const uint32_t* src, uint32_t w, uint32_t h, uint32_t* dst, uint32_t nw, uint32_t nh,
-                  const Filter& f, hipStream_t s) {
-    Taps tv = make_taps(h, nh, f), th = make_taps(w, nw, f);
-    DevTaps dv, dh;
-    DBuf<float4> tmp;
-    HIP_TRY(dv.upload(tv, s));
-    HIP_TRY(dh.upload(th, s));
-    HIP_TRY(tmp.alloc((size_t)w * nh));
-    HIP_TRY(launch_resample_v(src, w, h, tmp.p, nh, dv.left.p, dv.cnt.p, dv.ws.p, dv.stride, s));
-    HIP_TRY(launch_resample_h(tmp.p, w, nh, dst, nw, dh.left.p, dh.cnt.p, dh.ws.p, dh.stride, s));
-    HIP_TRY(hipStreamSynchronize(s));  // taps and tmp die here
-    return TSG_OK;
-}
-
-// transform_to_guide_map (utils.rs:101-116) without a resize: blur with
-// sigma 2 on the device (the resampler at the same size), then grayscale on
-// the host (image 0.23 rgb_to_luma: 0.2126 R + 0.7152 G + 0.0722 B in f32,
-// cast to u8), as RGBA.
-int style_guide(hipStream_t s, const tsg_image& im, std::vector<uint8_t>& out) {
-    const size_t n = (size_t)im.w * im.h;
-    DBuf<uint32_t> src, dst;
-    HIP_TRY(src.alloc(n));
-    HIP_TRY(dst.alloc(n));
-    HIP_TRY(hipMemcpyAsync(src.p, im.rgba, n * 4, hipMemcpyHostToDevice, s));
-    const Filter blur{kern_gaussian_blur2, 4.0f};
-    int rc = device_resize(src.p, im.w, im.h, dst.p, im.w, im.h, blur, s);
-    if (rc) return rc;
-    out.resize(n * 4);
-    HIP_TRY(hipMemcpy(out.data(), dst.p, n * 4, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; ++i) {
-        uint8_t* p = &out[i * 4];
-        float l = 0.2126f * (float)p[0];
-        l = l + 0.7152f * (float)p[1];
-        l = l + 0.0722f * (float)p[2];
-        const uint8_t v = (uint8_t)l;
-        p[0] = p[1] = p[2] = v;
-        p[3] = 255;
-    }
-    return TSG_OK;
-}
-
-// match_histograms / get_histogram / get_cdf (utils.rs:118-183) on the first
-// channel: each value moves to the position before the first target CDF entry
-// above its own CDF; the u8 arithmetic wraps as the release build's does.
-void match_histograms(std::vector<uint8_t>& src, const std::vector<uint8_t>& tgt) {
-    auto cdf_of = [](const std::vector<uint8_t>& im) {
-        std::vector<uint32_t> hist(256, 0);
-        for (size_t i = 0; i < im.size(); i += 4) hist[im[i]] += 1;
-        std::vector<float> c(256, 0.0f);
-        for (int i = 0; i < 256; ++i) c[i] = i ? c[i - 1] + (float)hist[i] : (float)hist[i];
-        const float mx = c[255];
-        for (float& v : c) v /= mx;
-        return c;
-    };
-    const std::vector<float> tc = cdf_of(tgt), sc = cdf_of(src);
-    uint8_t map[256];
-    for (int v = 0; v < 256; ++v) {
-        int pos = -1;
-        for (int q = 0; q < 256; ++q)
-            if (tc[q] > sc[v]) {
-                pos = q;
-                break;
-            }
-        map[v] = (uint8_t)((pos >= 0 ? (uint8_t)pos : (uint8_t)(v + 1)) - 1u);
-    }
-    for (size_t i = 0; i < src.size(); i += 4) {
-        const uint8_t n = map[src[i]];
-        src[i] = src[i + 1] = src[i + 2] = n;
-        src[i + 3] = 255;
-    }
-}
-
-// ImagePyramid::build_gaussian (img_pyramid.rs:20-37): `levels` full-size
-// levels at out, coarsest first; the last is the input itself.
-int device_pyramid(const uint8_t* host_rgba, uint32_t w, uint32_t h, uint32_t levels, uint32_t* out,
-                   hipStream_t s) {
-    const Filter g{kern_gaussian, 3.0f};
-    size_t npx = (size_t)w * h;
-    uint32_t* last = out + (size_t)(levels - 1) * npx;
-    HIP_TRY(hipMemcpyAsync(last, host_rgba, npx * 4, hipMemcpyHostToDevice, s));
-    DBuf<uint32_t> small;
-    for (uint32_t lv = 0; lv + 1 < levels; ++lv) {
-        uint32_t i = levels - 1 - lv;
-        uint32_t pw = w >> i, ph = h >> i;
-        if (pw == 0 || ph == 0) return fail(TSG_ERR_INVALID_ARGUMENT, "image too small for the pyramid depth");
-        HIP_TRY(small.reserve((size_t)pw * ph));
-        int rc = device_resize(last, w, h, small.p, pw, ph, g, s);
-        if (rc) return rc;
-        rc = device_resize(small.p, pw, ph, out + (size_t)lv * npx, w, h, g, s);
-        if (rc) return rc;
-    }
-    return TSG_OK;
 }
 
 const std::vector<int32_t>& offset_table() {
@@ -594,10 +454,8 @@ struct tsg_job {
     std::vector<std::unique_ptr<DBuf<uint8_t>>> smask;    // [example] (null = All)
     DBuf<uint32_t> tg;                                    // levels x W x H
     DBuf<MapDesc> maps;                                   // [level][filtered map]
-    std::vector<std::vector<uint32_t>> h_finest;          // finest example pixels
     // initial state inputs
     bool inpaint = false;
-    std::vector<uint8_t> inpaint_mask_r;
     uint32_t inpaint_index = 0;
     // device state
     DBuf<uint4> state;
@@ -689,8 +547,11 @@ struct tsg_job {
     uint32_t ghost_lo = 0;          // tiling mode: ranks below carry no ghost copies
     uint32_t flow_tag = 0, flow_launches = 0;
     size_t small_used = 0;
-    // host bookkeeping
+    DBuf<uint2> pick_moves;         // entries of the list that are not their own index
+    // host bookkeeping. The unresolved list before the first stage: of an
+    // inpainting in `unresolved`, else entry i is pixel i but for unres_moves
     std::vector<uint32_t> unresolved;
+    std::unordered_map<uint32_t, uint32_t> unres_moves;
     size_t n_res = 0, locked = 0, N0 = 0;
     std::vector<uint64_t> st_items;
     std::vector<std::vector<uint32_t>> picks_keep;
@@ -821,79 +682,297 @@ int check_range(float v, float lo, float hi, const char* name) {
     return TSG_OK;
 }
 
-// Initial state: Generator::new / new_from_inpaint (ms.rs:220-293) and the
-// random init of Session::run (session.rs:42-52).
-int init_state(tsg_job* j) {
-    const size_t N = j->N;
-    std::vector<uint4> st(N, make_uint4(0, 0, 0, 0));
-    std::vector<uint64_t> mask((size_t)j->tiles_x * j->tiles_y, 0);
-    std::vector<uint32_t> rl;
-    rl.reserve(N);
-    auto set_bit = [&](uint32_t f) {
-        uint32_t x = f % j->W, y = f / j->W;
-        mask[(y >> 3) * j->tiles_x + (x >> 3)] |= 1ull << (((y & 7u) << 3) | (x & 7u));
+// Resampling weights of in_len -> out_len by `f`, as words appended to `blob`:
+// left[out_len], count[out_len], then `stride` weights per output.
+struct Taps {
+    uint32_t at = 0, stride = 0;
+};
+
+Taps make_taps(uint32_t in_len, uint32_t out_len, const Filter& f, std::vector<uint32_t>& blob) {
+    const float ratio = (float)in_len / (float)out_len;
+    const float sratio = ratio < 1.0f ? 1.0f : ratio;
+    const float support = f.support * sratio;
+    Taps t;
+    t.at = (uint32_t)blob.size();
+    auto span = [&](uint32_t o, float in, int64_t* l) {
+        *l = std::min<int64_t>(std::max<int64_t>((int64_t)std::floor(in - support), 0), (int64_t)in_len - 1);
+        const int64_t r = std::min<int64_t>(std::max<int64_t>((int64_t)std::ceil(in + support), *l + 1), (int64_t)in_len);
+        return (uint32_t)(r - *l);
     };
-    j->unresolved.clear();
-    if (j->inpaint) {
-        const std::vector<uint32_t>& col = j->h_finest[j->inpaint_index];
-        for (size_t i = 0; i < N; ++i) {
-            st[i].x = col[i];
-            if (j->inpaint_mask_r[i] < 255) {
-                j->unresolved.push_back((uint32_t)i);
-            } else {
-                uint32_t x = (uint32_t)(i % j->W), y = (uint32_t)(i / j->W);
-                st[i] = make_uint4(col[i], x | (y << 16), j->inpaint_index, 0u);
-                set_bit((uint32_t)i);
-                rl.push_back((uint32_t)i);
-            }
-        }
-    } else {
-        j->unresolved.resize(N);
-        for (size_t i = 0; i < N; ++i) j->unresolved[i] = (uint32_t)i;
+    for (uint32_t o = 0; o < out_len; ++o) {
+        int64_t l;
+        t.stride = std::max(t.stride, span(o, ((float)o + 0.5f) * ratio, &l));
     }
-    j->locked = rl.size();
+    blob.resize(t.at + (size_t)out_len * (2 + t.stride));
+    uint32_t* left = blob.data() + t.at;
+    uint32_t* cnt = left + out_len;
+    float* ws = reinterpret_cast<float*>(cnt + out_len);
+    for (uint32_t o = 0; o < out_len; ++o, ws += t.stride) {
+        float in = ((float)o + 0.5f) * ratio;
+        int64_t l;
+        const uint32_t n = span(o, in, &l);
+        left[o] = (uint32_t)l;
+        cnt[o] = n;
+        in = in - 0.5f;
+        float sum = 0.0f;
+        for (uint32_t i = 0; i < n; ++i) {
+            ws[i] = f.kernel(((float)(l + i) - in) / sratio);
+            sum += ws[i];
+        }
+        for (uint32_t i = 0; i < n; ++i) ws[i] /= sum;
+    }
+    return t;
+}
+
+// imageops::resize(src, nw, nh, filter): a vertical pass into f32, then a
+// horizontal one, rounded to u8.
+struct Resize {
+    const uint32_t* src;
+    uint32_t w, h;
+    uint32_t* dst;
+    uint32_t nw, nh;
+    Filter f;
+};
+
+// f32 rows between the passes held at once, unless one resize alone needs more.
+constexpr size_t kResampleBytes = 256u << 20;
+
+// The steps in order, each one's resizes together: two launches per step
+// where their intermediate rows fit kResampleBytes. Waits for the stream.
+int resize_all(tsg_ctx* c, const std::vector<std::vector<Resize>>& steps) {
+    hipStream_t s = c->stream;
+    std::vector<uint32_t> blob;
+    std::map<std::tuple<uint32_t, uint32_t, float (*)(float)>, Taps> seen;
+    auto taps = [&](uint32_t in_len, uint32_t out_len, const Filter& f) {
+        const auto key = std::make_tuple(in_len, out_len, f.kernel);
+        auto it = seen.find(key);
+        if (it == seen.end()) it = seen.emplace(key, make_taps(in_len, out_len, f, blob)).first;
+        return it->second;
+    };
+    struct Group {
+        size_t u0 = 0, n = 0;
+        uint32_t blocks_v = 0, blocks_h = 0;
+    };
+    std::vector<Group> groups;
+    std::vector<ResampleUnit> uv, uh;
+    size_t most = 0;  // rows, in float4
+    for (const std::vector<Resize>& st : steps) {
+        size_t at = 0;
+        bool open = false;
+        for (const Resize& r : st) {
+            const size_t rows = (size_t)r.w * r.nh;
+            if (!open || (at + rows) * sizeof(float4) > kResampleBytes) {
+                groups.push_back(Group{uv.size()});
+                at = 0;
+                open = true;
+            }
+            Group& g = groups.back();
+            const Taps tv = taps(r.h, r.nh, r.f), th = taps(r.w, r.nw, r.f);
+            // (the rows' place is an offset until they are allocated)
+            uv.push_back(ResampleUnit{r.src, reinterpret_cast<void*>(at), r.w, r.nh, r.w, tv.at, tv.stride, g.blocks_v});
+            uh.push_back(ResampleUnit{reinterpret_cast<const void*>(at), r.dst, r.nw, r.nh, r.w, th.at, th.stride, g.blocks_h});
+            g.blocks_v += resample_blocks(r.w, r.nh);
+            g.blocks_h += resample_blocks(r.nw, r.nh);
+            g.n += 1;
+            at += rows;
+            most = std::max(most, at);
+        }
+    }
+    if (uv.empty()) return TSG_OK;
+    DBuf<float4> rows;
+    DBuf<uint32_t> dtaps;
+    DBuf<ResampleUnit> du;
+    HIP_TRY(rows.alloc(most));
+    HIP_TRY(dtaps.alloc(blob.size()));
+    HIP_TRY(du.alloc(2 * uv.size()));
+    for (ResampleUnit& u : uv) u.dst = rows.p + reinterpret_cast<size_t>(u.dst);
+    for (ResampleUnit& u : uh) u.src = rows.p + reinterpret_cast<size_t>(u.src);
+    const size_t nu = uv.size();
+    uv.insert(uv.end(), uh.begin(), uh.end());
+    HIP_TRY(c->staging.upload(dtaps.p, blob.data(), blob.size() * 4, s));
+    HIP_TRY(c->staging.upload(du.p, uv.data(), uv.size() * sizeof(ResampleUnit), s));
+    for (const Group& g : groups) {
+        HIP_TRY(launch_resample(du.p + g.u0, (uint32_t)g.n, g.blocks_v, dtaps.p, false, s));
+        HIP_TRY(launch_resample(du.p + nu + g.u0, (uint32_t)g.n, g.blocks_h, dtaps.p, true, s));
+    }
+    HIP_TRY(hipStreamSynchronize(s));
+    give_back(rows, dtaps, du);
+    return TSG_OK;
+}
+
+// One pyramid in the making: `levels` full-size levels at px, coarsest
+// first; the last is the input itself, which is in place.
+struct Pyramid {
+    uint32_t* px;
+    uint32_t w, h;
+};
+
+int check_pyramid(uint32_t w, uint32_t h, uint32_t levels) {
+    if (levels > 1 && (levels > 32 || (w >> (levels - 1)) == 0 || (h >> (levels - 1)) == 0))
+        return fail(TSG_ERR_INVALID_ARGUMENT, "image too small for the pyramid depth");
+    return TSG_OK;
+}
+
+// ImagePyramid::build_gaussian (img_pyramid.rs:20-37) of several images
+// together: every level of every image is scaled down, then up, in four
+// launches in all. A level at a time, each with its own tables, buffers and
+// wait, took 1.2 ms an image of 512^2 and 14 ms of a guided 1024^2 job.
+int build_pyramids(tsg_ctx* c, const std::vector<Pyramid>& imgs, uint32_t levels) {
+    const Filter g{kern_gaussian, 3.0f};
+    size_t n_small = 0;
+    for (const Pyramid& im : imgs)
+        for (uint32_t i = 1; i < levels; ++i) n_small += (size_t)(im.w >> i) * (im.h >> i);
+    if (!n_small) return TSG_OK;
+    DBuf<uint32_t> small;
+    HIP_TRY(small.alloc(n_small));
+    std::vector<std::vector<Resize>> steps(2);
+    size_t at = 0;
+    for (const Pyramid& im : imgs) {
+        const size_t npx = (size_t)im.w * im.h;
+        const uint32_t* last = im.px + (levels - 1) * npx;
+        for (uint32_t lv = 0; lv + 1 < levels; ++lv) {
+            const uint32_t i = levels - 1 - lv, pw = im.w >> i, ph = im.h >> i;
+            steps[0].push_back(Resize{last, im.w, im.h, small.p + at, pw, ph, g});
+            steps[1].push_back(Resize{small.p + at, pw, ph, im.px + lv * npx, im.w, im.h, g});
+            at += (size_t)pw * ph;
+        }
+    }
+    if (int rc = resize_all(c, steps)) return rc;
+    give_back(small);
+    return TSG_OK;
+}
+
+// Style transfer's guides (transform_to_guide_map, utils.rs:101-116, without
+// a resize, and match_histograms, utils.rs:118-183): every image blurred with
+// sigma 2 (the resampler at the same size) and turned to luma; the others
+// then matched to the first one's histogram.
+int style_guides(tsg_ctx* c, const std::vector<Resize>& blurs) {
+    hipStream_t s = c->stream;
+    if (int rc = resize_all(c, {blurs})) return rc;
+    DBuf<uint32_t> hist, map;
+    HIP_TRY(hist.alloc(blurs.size() * 256));
+    HIP_TRY(map.alloc(blurs.size() * 256));
+    HIP_TRY(launch_zero(hist.p, blurs.size() * 256, s));
+    for (size_t q = 0; q < blurs.size(); ++q)
+        HIP_TRY(launch_luma(blurs[q].dst, blurs[q].nw * blurs[q].nh, hist.p + q * 256, s));
+    for (size_t q = 1; q < blurs.size(); ++q)
+        HIP_TRY(launch_match(blurs[q].dst, blurs[q].nw * blurs[q].nh, hist.p + q * 256, hist.p, map.p + q * 256, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    give_back(hist, map);
+    return TSG_OK;
+}
+
+// Initial state: Generator::new / new_from_inpaint (ms.rs:220-293) and the
+// random init of Session::run (session.rs:42-52). The maps are filled on the
+// device (k_init_fill, 28 bytes a pixel); the host brings the pixels that
+// start resolved: an inpainting's kept pixels by their list, randomly
+// initialised ones as records. Built on the host and uploaded it was 40 bytes
+// a pixel written to fresh pages and copied: 15 ms at 2048^2, now 0.1.
+int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_mask) {
+    const size_t N = j->N;
+    hipStream_t s = j->ctx->stream;
+    Staging& up = j->ctx->staging;
+    const uint32_t* base = nullptr;
+    if (j->inpaint) base = j->ex[j->inpaint_index]->p + (size_t)(j->levels - 1) * N;  // the finest level: the input
+    const InitArgs ia{(uint32_t)N, j->W,       j->tiles_x, j->tiles_x * j->tiles_y, base,
+                      j->state.p,  j->rank.p,  j->score.p, j->mask.p,               j->gmask.p};
+    HIP_TRY(launch_init_fill(ia, s));
+    j->unresolved.clear();
+    j->unres_moves.clear();
+    size_t kept = 0, L = N;
+    if (j->inpaint) {
+        std::vector<uint32_t> rl(N);
+        j->unresolved.resize(N);
+        uint32_t* u = j->unresolved.data();
+        size_t nu = 0;
+        for (size_t i = 0; i < N; ++i) {
+            const bool open = inpaint_mask->rgba[i * 4] < 255;
+            u[nu] = (uint32_t)i;
+            rl[kept] = (uint32_t)i;
+            nu += open;
+            kept += !open;
+        }
+        j->unresolved.resize(nu);
+        L = nu;
+        if (kept) {
+            HIP_TRY(up.upload(j->rlist.p, rl.data(), kept * 4, s));
+            HIP_TRY(launch_init_kept(ia, j->rlist.p, (uint32_t)kept, j->inpaint_index, s));
+        }
+    }
+    j->locked = kept;
     if (j->prm.random_init != UINT64_MAX) {
-        for (uint64_t i = 0; i < j->prm.random_init; ++i) {
-            if (j->unresolved.empty()) continue;
+        // the swap_remove chain on the list, or (every pixel in order) on the entries it moved
+        std::vector<InitPoint> pts;
+        for (uint64_t i = 0; i < j->prm.random_init && L > 0; ++i) {
             Pcg32 g = Pcg32::seed_from_u64(j->prm.seed + i);
-            uint64_t k = range_u64(g, 0, j->unresolved.size());
-            uint32_t f = j->unresolved[k];
-            j->unresolved[k] = j->unresolved.back();
-            j->unresolved.pop_back();
+            const uint32_t k = (uint32_t)range_u64(g, 0, L);
+            --L;
+            uint32_t f;
+            if (j->inpaint) {
+                f = j->unresolved[k];
+                j->unresolved[k] = j->unresolved[L];
+            } else {
+                auto at = [&](uint32_t q) {
+                    auto it = j->unres_moves.find(q);
+                    return it == j->unres_moves.end() ? q : it->second;
+                };
+                f = at(k);
+                j->unres_moves[k] = at((uint32_t)L);
+            }
             uint32_t m, x, y;
             random_source(j->prm.seed + i + (uint64_t)f, j->ex_dims, m, x, y);
-            uint32_t c = j->h_finest[m][(size_t)y * j->ex_dims[m].first + x];
-            st[f] = make_uint4(c, x | (y << 16), m | (m << 16), f);
-            set_bit(f);
-            rl.push_back(f);
+            const uint32_t c = pack_px(examples[m].rgba + ((size_t)y * j->ex_dims[m].first + x) * 4);
+            pts.push_back(InitPoint{f, c, x | (y << 16), m | (m << 16)});
         }
+        if (j->inpaint) j->unresolved.resize(L);
         j->locked += j->prm.random_init;
-        if (j->locked > rl.size()) return fail(TSG_ERR_INVALID_ARGUMENT, "random_init exceeds the pixels to resolve");
+        if (j->locked > kept + pts.size())
+            return fail(TSG_ERR_INVALID_ARGUMENT, "random_init exceeds the pixels to resolve");
+        if (!pts.empty()) {
+            DBuf<InitPoint> d;
+            HIP_TRY(d.alloc(pts.size()));
+            HIP_TRY(up.upload(d.p, pts.data(), pts.size() * sizeof(InitPoint), s));
+            HIP_TRY(launch_init_points(ia, d.p, (uint32_t)pts.size(), (uint32_t)kept, j->rlist.p, s));
+            HIP_TRY(hipStreamSynchronize(s));
+            give_back(d);
+        }
+        kept += pts.size();
     }
-    j->n_res = rl.size();
-    j->N0 = j->unresolved.size();
-    hipStream_t s = j->ctx->stream;
-    HIP_TRY(hipMemcpyAsync(j->state.p, st.data(), N * sizeof(uint4), hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(j->mask.p, mask.data(), mask.size() * 8, hipMemcpyHostToDevice, s));
-    // every pixel resolved before the stages starts with its ghost copies (ms.rs:296-331)
-    if (j->prm.tiling_mode) HIP_TRY(hipMemcpyAsync(j->gmask.p, mask.data(), mask.size() * 8, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemsetAsync(j->score.p, 0, N * sizeof(float), s));
-    if (!rl.empty()) HIP_TRY(hipMemcpyAsync(j->rlist.p, rl.data(), rl.size() * 4, hipMemcpyHostToDevice, s));
-    std::vector<uint32_t> rank(N, UINT32_MAX);
-    for (size_t q = 0; q < rl.size(); ++q) rank[rl[q]] = (uint32_t)q;
-    HIP_TRY(hipMemcpyAsync(j->rank.p, rank.data(), N * 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    j->n_res = kept;
+    j->N0 = L;
+    // moves of entries past the list's end are void
+    for (auto it = j->unres_moves.begin(); it != j->unres_moves.end();) {
+        if (it->first >= L || it->first == it->second) it = j->unres_moves.erase(it);
+        else ++it;
+    }
     return TSG_OK;
+}
+
+// The unresolved list on the host, for runs whose pick orders the host computes.
+void host_unresolved(tsg_job* j) {
+    if (j->inpaint) return;  // held from the start
+    j->unresolved.resize(j->N0);
+    for (size_t i = 0; i < j->N0; ++i) j->unresolved[i] = (uint32_t)i;
+    for (const auto& mv : j->unres_moves) j->unresolved[mv.first] = mv.second;
 }
 
 // The unresolved list of a run whose pick orders are drawn on the device.
 int picks_begin(tsg_job* j) {
     j->pick_left = j->N0;
     j->pick_list = nullptr;
-    if (j->N0 < j->N) {
-        // inpainting or random init: not every pixel in order
-        HIP_TRY(j->unres[0].reserve(j->N0));
-        HIP_TRY(j->ctx->staging.upload(j->unres[0].p, j->unresolved.data(), j->N0 * 4, j->ctx->stream));
+    if (j->inpaint || !j->unres_moves.empty()) {
+        // not every pixel in order
+        hipStream_t s = j->ctx->stream;
+        HIP_TRY(j->unres[0].reserve(std::max<size_t>(1, j->N0)));
+        if (j->inpaint) {
+            HIP_TRY(j->ctx->staging.upload(j->unres[0].p, j->unresolved.data(), j->N0 * 4, s));
+        } else {
+            std::vector<uint2> mv;
+            for (const auto& q : j->unres_moves) mv.push_back(make_uint2(q.first, q.second));
+            HIP_TRY(j->pick_moves.reserve(mv.size()));
+            HIP_TRY(j->ctx->staging.upload(j->pick_moves.p, mv.data(), mv.size() * sizeof(uint2), s));
+            HIP_TRY(launch_list(j->unres[0].p, (uint32_t)j->N0, j->pick_moves.p, (uint32_t)mv.size(), s));
+        }
         j->pick_list = j->unres[0].p;
     }
     return TSG_OK;
@@ -1279,7 +1358,10 @@ int step_begin(tsg_job* j) {
         j->pk_start_res = j->n_res;
         j->pk_state = j->flow_on ? 0 : 1;
     }
-    if (!j->flow_on) j->ctx->picks.submit(j);
+    if (!j->flow_on) {
+        host_unresolved(j);
+        j->ctx->picks.submit(j);
+    }
     j->lut_keep.assign(P + 1, std::vector<float>(512));
     j->small_used = 0;
     j->n_batches = 0;
@@ -2770,33 +2852,22 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
         return fail(TSG_ERR_UNSUPPORTED, "inpaint example index beyond the sampled examples (the reference panics)");
     hipStream_t s = ctx->stream;
     std::lock_guard<std::mutex> lk(ctx->mu);
+    Staging& up = ctx->staging;
     // style transfer (session.rs:385-393, lib.rs:572-581): without example
     // guides the target guide becomes a guide map, and each example's guide
     // is its own guide map matched to the target's histogram
-    std::vector<std::vector<uint8_t>> sg_ex;
-    std::vector<uint8_t> sg_tg;
-    std::vector<tsg_image> sg_imgs;
-    tsg_image sg_target{};
-    if (target_guide && !example_guides) {
-        if ((rc = style_guide(s, *target_guide, sg_tg))) return rc;
-        sg_target = tsg_image{target_guide->w, target_guide->h, sg_tg.data()};
-        sg_ex.resize(n_examples);
-        sg_imgs.resize(n_examples);
-        for (uint32_t i = 0; i < n_examples; ++i) {
-            if ((rc = style_guide(s, examples[i], sg_ex[i]))) return rc;
-            match_histograms(sg_ex[i], sg_tg);
-            sg_imgs[i] = tsg_image{examples[i].w, examples[i].h, sg_ex[i].data()};
-        }
-        example_guides = sg_imgs.data();
-        target_guide = &sg_target;
-    }
+    const bool style = target_guide && !example_guides;
+    std::vector<Pyramid> pyr;
+    const uint32_t top = j->levels - 1;  // the finest level, which is the input
     for (uint32_t i = 0; i < n_examples; ++i) {
         const tsg_image& im = examples[i];
+        const size_t npx = (size_t)im.w * im.h;
         j->ex_dims.push_back({im.w, im.h});
-        j->h_finest.push_back(packed(im));
+        if ((rc = check_pyramid(im.w, im.h, j->levels))) return rc;
         std::unique_ptr<DBuf<uint32_t>> b(new DBuf<uint32_t>());
-        HIP_TRY(b->alloc((size_t)j->levels * im.w * im.h));
-        if ((rc = device_pyramid(im.rgba, im.w, im.h, j->levels, b->p, s))) return rc;
+        HIP_TRY(b->alloc(j->levels * npx));
+        HIP_TRY(up.upload(b->p + top * npx, im.rgba, npx * 4, s));
+        pyr.push_back(Pyramid{b->p, im.w, im.h});
         j->ex.push_back(std::move(b));
         std::unique_ptr<DBuf<uint8_t>> mk(new DBuf<uint8_t>());
         if (j->kind[i] == TSG_SAMPLE_IMAGE) {
@@ -2812,22 +2883,44 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
             if (valid == 0)
                 return fail(TSG_ERR_SAMPLING, "sample mask admits no pixel (the reference loops forever)");
             HIP_TRY(mk->alloc(v.size()));
-            HIP_TRY(hipMemcpy(mk->p, v.data(), v.size(), hipMemcpyHostToDevice));
+            HIP_TRY(up.upload(mk->p, v.data(), v.size(), s));
         }
         j->smask.push_back(std::move(mk));
-        if (example_guides) {
-            const tsg_image& g = example_guides[i];
+        if (j->guided) {
+            const tsg_image& g = style ? im : example_guides[i];
+            const size_t gpx = (size_t)g.w * g.h;
             j->g_dims.push_back({g.w, g.h});
+            if ((rc = check_pyramid(g.w, g.h, j->levels))) return rc;
             std::unique_ptr<DBuf<uint32_t>> gb(new DBuf<uint32_t>());
-            HIP_TRY(gb->alloc((size_t)j->levels * g.w * g.h));
-            if ((rc = device_pyramid(g.rgba, g.w, g.h, j->levels, gb->p, s))) return rc;
+            HIP_TRY(gb->alloc(j->levels * gpx));
+            if (!style) HIP_TRY(up.upload(gb->p + top * gpx, g.rgba, gpx * 4, s));
+            pyr.push_back(Pyramid{gb->p, g.w, g.h});
             j->exg.push_back(std::move(gb));
         }
     }
-    if (target_guide) {
+    if (j->guided) {
+        if ((rc = check_pyramid(out_w, out_h, j->levels))) return rc;
         HIP_TRY(j->tg.alloc((size_t)j->levels * j->N));
-        if ((rc = device_pyramid(target_guide->rgba, out_w, out_h, j->levels, j->tg.p, s))) return rc;
+        pyr.push_back(Pyramid{j->tg.p, out_w, out_h});
+        uint32_t* last = j->tg.p + top * j->N;
+        if (style) {
+            DBuf<uint32_t> raw;
+            HIP_TRY(raw.alloc(j->N));
+            HIP_TRY(up.upload(raw.p, target_guide->rgba, j->N * 4, s));
+            const Filter blur{kern_gaussian_blur2, 4.0f};
+            std::vector<Resize> blurs{Resize{raw.p, out_w, out_h, last, out_w, out_h, blur}};
+            for (uint32_t i = 0; i < n_examples; ++i) {
+                const uint32_t w = examples[i].w, h = examples[i].h;
+                const size_t at = top * (size_t)w * h;
+                blurs.push_back(Resize{j->ex[i]->p + at, w, h, j->exg[i]->p + at, w, h, blur});
+            }
+            if ((rc = style_guides(ctx, blurs))) return rc;
+            give_back(raw);
+        } else {
+            HIP_TRY(up.upload(last, target_guide->rgba, j->N * 4, s));
+        }
     }
+    if ((rc = build_pyramids(ctx, pyr, j->levels))) return rc;
     // map descriptors per level; the guide of filtered map m is the m-th
     // entry of the unfiltered guide list (get_single_guide_level, ms.rs:1566-1573)
     const uint32_t nf = (uint32_t)j->filt.size();
@@ -2848,12 +2941,10 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
             md[(size_t)lv * nf + mi] = d;
         }
     HIP_TRY(j->maps.alloc(md.size()));
-    HIP_TRY(hipMemcpy(j->maps.p, md.data(), md.size() * sizeof(MapDesc), hipMemcpyHostToDevice));
+    HIP_TRY(up.upload(j->maps.p, md.data(), md.size() * sizeof(MapDesc), s));
     if (inpaint_mask) {
         j->inpaint = true;
         j->inpaint_index = inpaint_index;
-        j->inpaint_mask_r.resize(j->N);
-        for (size_t i = 0; i < j->N; ++i) j->inpaint_mask_r[i] = inpaint_mask->rgba[i * 4];
     }
     const uint32_t P = prm->backtrack_stages;
     HIP_TRY(j->state.alloc(j->N));
@@ -2872,10 +2963,9 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
     HIP_TRY(j->rank.alloc(j->N));
     HIP_TRY(j->mend.alloc((size_t)j->tiles_x * j->tiles_y));
     HIP_TRY(j->tmin.alloc((size_t)j->tiles_x * j->tiles_y));
-    HIP_TRY(hipMemset(j->done_counter.p, 0, 4));
     // Generator::new / new_from_inpaint and the random init are content-
     // independent of the stages: upload the initial state now
-    if ((rc = init_state(j.get()))) return rc;
+    if ((rc = init_state(j.get(), examples, inpaint_mask))) return rc;
     j->state_ready = true;
     HIP_TRY(hipStreamSynchronize(s));
     {
@@ -3164,8 +3254,10 @@ int tsg_pyramid_build(tsg_ctx* ctx, const tsg_image* img, uint32_t levels, uint8
     size_t npx = (size_t)img->w * img->h;
     DBuf<uint32_t> d;
     HIP_TRY(d.alloc(L * npx));
-    int rc = device_pyramid(img->rgba, img->w, img->h, L, d.p, ctx->stream);
+    int rc = check_pyramid(img->w, img->h, L);
     if (rc) return rc;
+    HIP_TRY(ctx->staging.upload(d.p + (L - 1) * npx, img->rgba, npx * 4, ctx->stream));
+    if ((rc = build_pyramids(ctx, {Pyramid{d.p, img->w, img->h}}, L))) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipMemcpy(out, d.p, L * npx * 4, hipMemcpyDeviceToHost));
     return TSG_OK;
@@ -3189,10 +3281,11 @@ int tsg_resize(tsg_ctx* ctx, const tsg_image* img, uint32_t nw, uint32_t nh, int
     DBuf<uint32_t> src, dst;
     HIP_TRY(src.alloc(n_in));
     HIP_TRY(dst.alloc(n_out));
-    HIP_TRY(hipMemcpyAsync(src.p, img->rgba, n_in * 4, hipMemcpyHostToDevice, ctx->stream));
-    int rc = device_resize(src.p, img->w, img->h, dst.p, nw, nh, f, ctx->stream);
+    HIP_TRY(ctx->staging.upload(src.p, img->rgba, n_in * 4, ctx->stream));
+    int rc = resize_all(ctx, {{Resize{src.p, img->w, img->h, dst.p, nw, nh, f}}});
     if (rc) return rc;
     HIP_TRY(hipMemcpy(out, dst.p, n_out * 4, hipMemcpyDeviceToHost));
+    give_back(src, dst);
     return TSG_OK;
 }
 
