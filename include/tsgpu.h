@@ -257,7 +257,11 @@ void tsg_job_destroy(tsg_job* job);
 
 /* ---- many syntheses at once (no counterpart in the reference: serving and
  *      batch callers that run many Session::run at the same time) ----
- * A tsg_batch runs its admitted jobs together. Each step (a "round") plans
+ * A tsg_batch runs its admitted jobs together. tsg_batch_run_all runs each
+ * job whole, several at a time on streams of their own, where the
+ * stage-ahead buffers of those in flight fit (16 GiB, or the bytes given to
+ * tsg_batch_set_alone_below). Else, and in steps, which end early enough for
+ * jobs to be submitted and cancelled meanwhile, each step (a "round") plans
  * every job's next phases exactly as a run alone would batch them (random
  * candidates, each Jacobi batch's resolve and commit, stage statistics) and
  * runs all of them in one launch of a persistent work-queue kernel, whose
@@ -287,10 +291,11 @@ int tsg_batch_set_quantum(tsg_batch* b, uint64_t items);
 /* A job that starts while fewer than `jobs` jobs are in the batch (running
  * and waiting, itself included) runs alone instead: to its end, on the
  * single-job path with the whole device (tsg_job_run's launch sequence),
- * before the round's engine launch; a round's alone jobs run smallest first.
- * Its stage-ahead buffers, beyond tsg_footprint_estimate, are used only when
- * they fit ahead_bytes, and are released when its run ends. jobs = 0, the
- * default: every job runs on the engine. Under light load a lone job's chain
+ * before the round's engine launch; where a round has several such jobs,
+ * those with stage-ahead buffers run a few at a time on streams of their own.
+ * The stage-ahead buffers, beyond tsg_footprint_estimate, of the jobs in
+ * flight are used only when they fit ahead_bytes, and are released when a run
+ * ends. jobs = 0, the default: none. Under light load a lone job's chain
  * of small batches is what bounds its latency, and the single-job path
  * shortens that chain; under load the engine's throughput wins. Results do
  * not depend on it. */
@@ -302,7 +307,8 @@ int tsg_batch_run_all(tsg_batch* b);
 /* Finished jobs not yet taken: tickets and their run status (0 = ok). */
 int tsg_batch_poll(tsg_batch* b, uint64_t* tickets, int* status, uint32_t cap, uint32_t* n);
 int tsg_batch_take(tsg_batch* b, uint64_t ticket, tsg_job** job);
-/* Rounds and engine launches so far, engine phases run, and jobs run alone
+/* Rounds and launches (engine launches, or several whole runs together) so
+ * far, engine phases and batches run, and jobs run alone
  * (tsg_batch_set_alone_below); any pointer may be NULL. */
 int tsg_batch_stats(tsg_batch* b, uint64_t* rounds, uint64_t* launches, uint64_t* units, uint64_t* alone);
 /* Cancels a job that has not finished: a waiting job never starts, a

@@ -3804,7 +3804,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
 
 namespace {
 // events the next resolve launch records around its dispatch (profiling)
-hipEvent_t g_ev_start = nullptr, g_ev_stop = nullptr;
+thread_local hipEvent_t g_ev_start = nullptr, g_ev_stop = nullptr;
 }  // namespace
 
 void set_launch_events(hipEvent_t start, hipEvent_t stop) {

@@ -18,6 +18,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <condition_variable>
 #include <deque>
 #include <map>
@@ -418,6 +419,16 @@ static void parallel_copy(void* dst, const void* src, size_t n, unsigned threads
     for (auto& x : th) x.join();
 }
 
+// A stream and its staging for one of the jobs that run at the same time (a
+// batch's, run_on_lanes).
+struct Lane {
+    hipStream_t stream = nullptr;
+    Staging staging;
+    ~Lane() {
+        if (stream) (void)hipStreamDestroy(stream);
+    }
+};
+
 struct tsg_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -428,6 +439,7 @@ struct tsg_ctx {
     DBuf<int32_t> offtab;
     uint32_t offtab_n = 0;
     DBuf<float> dummy_lut;
+    std::vector<std::unique_ptr<Lane>> lanes;  // made on first use
     unsigned char* scratch = nullptr;  // this device's copy of the file-scope scratch array
     std::mutex mu;
     // launch structures stored by the autotuner, by job shape (see tuning_key)
@@ -439,6 +451,17 @@ constexpr unsigned kPickThreads = 12;
 
 struct tsg_job {
     tsg_ctx* ctx = nullptr;
+    // where its run goes: the context's streams, or a lane's one stream
+    hipStream_t stream = nullptr, side = nullptr;
+    Staging *stg = nullptr, *stg_side = nullptr;
+    uint32_t share = 1;  // jobs that run beside it, itself included
+    void on_context() {
+        stream = ctx->stream;
+        side = ctx->side;
+        stg = &ctx->staging;
+        stg_side = &ctx->staging_side;
+        share = 1;
+    }
     tsg_params prm{};
     tsg_schedule sched{};
     tsg_tuning tune{};
@@ -871,8 +894,8 @@ int style_guides(tsg_ctx* c, const std::vector<Resize>& blurs) {
 // build took 18 ms, now 0.7.
 int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_mask) {
     const size_t N = j->N;
-    hipStream_t s = j->ctx->stream;
-    Staging& up = j->ctx->staging;
+    hipStream_t s = j->stream;
+    Staging& up = *j->stg;
     const uint32_t* base = nullptr;
     if (j->inpaint) base = j->ex[j->inpaint_index]->p + (size_t)(j->levels - 1) * N;  // the finest level: the input
     const InitArgs ia{(uint32_t)N, j->W,       j->tiles_x, j->tiles_x * j->tiles_y, base,
@@ -963,15 +986,15 @@ int picks_begin(tsg_job* j) {
     j->pick_list = nullptr;
     if (j->inpaint || !j->unres_moves.empty()) {
         // not every pixel in order
-        hipStream_t s = j->ctx->stream;
+        hipStream_t s = j->stream;
         HIP_TRY(j->unres[0].reserve(std::max<size_t>(1, j->N0)));
         if (j->inpaint) {
-            HIP_TRY(j->ctx->staging.upload(j->unres[0].p, j->unresolved.data(), j->N0 * 4, s));
+            HIP_TRY(j->stg->upload(j->unres[0].p, j->unresolved.data(), j->N0 * 4, s));
         } else {
             std::vector<uint2> mv;
             for (const auto& q : j->unres_moves) mv.push_back(make_uint2(q.first, q.second));
             HIP_TRY(j->pick_moves.reserve(mv.size()));
-            HIP_TRY(j->ctx->staging.upload(j->pick_moves.p, mv.data(), mv.size() * sizeof(uint2), s));
+            HIP_TRY(j->stg->upload(j->pick_moves.p, mv.data(), mv.size() * sizeof(uint2), s));
             HIP_TRY(launch_list(j->unres[0].p, (uint32_t)j->N0, j->pick_moves.p, (uint32_t)mv.size(), s));
         }
         j->pick_list = j->unres[0].p;
@@ -1004,6 +1027,20 @@ constexpr int kKinds = 7;
 constexpr size_t kEngineRcBudget = 4u << 20;  // random-candidate chunk of a job under the engine
 constexpr uint64_t kPrefetchCap = 65536;       // items per prefetched kNN window
 constexpr uint32_t kFlowSpin = 1u << 18;       // polls of one dependency wait before a run gives up
+// Jobs of a batch that run at the same time, and the part of the chip's
+// resident workgroups (one in kLaneShare) that a launch of theirs may take.
+// HIP serves streams from four hardware queues, so five streams keep three or
+// four runs on the device. 48 jobs of 128^2..512^2, ms: 3 lanes 176, 4 lanes
+// 140, 5 lanes 106, 6 103, 7 118, 8 110, 12 109; a launch's part 1/2: 113 (6
+// lanes), 1/3: 103, 1/4: 104, 1/6: 120. A burst of 16 requests: 65 (5 lanes, 1/3),
+// 71 (6), 65 (6, 1/2), 73 (6, 1/4). One job after another: 209 and 90; the
+// engine: 152 (batch).
+constexpr size_t kLanes = 5, kLaneShare = 3;
+// Runs that share the chip give a team to items of batches up to this many,
+// where a run alone does up to prefetch_max: a team's waves finish an item
+// soonest but do more work for it. 48 jobs, ms: 1024 137 (6 lanes, 1/4), 512
+// and fewer 104, 64 106, 32 112.
+constexpr uint64_t kLaneTeamMax = 256;
 constexpr uint32_t kFlowTickets = 256;         // ticket counters of a job's dependency-ordered launches
 
 hipError_t next_event(tsg_job* j, hipEvent_t* e) {
@@ -1055,7 +1092,7 @@ hipError_t timed_launch_on(tsg_job* j, hipStream_t s, int kind, uint64_t items, 
 }
 template <class F>
 hipError_t timed_launch(tsg_job* j, int kind, uint64_t items, F&& launch) {
-    return timed_launch_on(j, j->ctx->stream, kind, items, launch);
+    return timed_launch_on(j, j->stream, kind, items, launch);
 }
 
 constexpr uint64_t kAheadBudget = 16ull << 30;  // device bytes of the stage-ahead buffers
@@ -1148,7 +1185,7 @@ int ahead_stage(tsg_job* j) {
     const int t = j->ahead_next;
     if (t > P) return TSG_OK;
     tsg_job::Ahead& A = j->aset(t);
-    hipStream_t side = j->ctx->side;
+    hipStream_t side = j->side;
     const uint32_t nf = (uint32_t)j->filt.size();
     const uint32_t m = (uint32_t)j->prm.random_sample_locations;
     const uint32_t k = j->prm.nearest_neighbors;
@@ -1186,7 +1223,7 @@ int ahead_stage(tsg_job* j) {
     // level maps); the first stage's on the job's stream, which has nothing
     // else to run yet
     if (S_eff) {
-        hipStream_t rs = t == 0 && j->flow_on ? j->ctx->stream : side;
+        hipStream_t rs = t == 0 && j->flow_on ? j->stream : side;
         RandArgs ra{j->maps.p + (size_t)level * nf, nf, pss, 0u, (uint32_t)S_eff, m, A.rc.p, j->overflow.p,
                     (uint32_t)j->masked};
         HIP_TRY(timed_launch_on(j, rs, K_RAND, S_eff, [&] { return launch_rand(ra, rs); }));
@@ -1231,7 +1268,7 @@ int ahead_stage(tsg_job* j) {
         HIP_TRY(hipMemsetAsync(A.tmin.p, 0xff, tiles * 4, side));
         if (!picks.empty()) {
             const uint32_t lo = (uint32_t)n_open, hi = (uint32_t)(n_open + picks.size());
-            HIP_TRY(j->ctx->staging_side.upload(j->rlist.p + n_open, picks.data(), picks.size() * 4, side));
+            HIP_TRY(j->stg_side->upload(j->rlist.p + n_open, picks.data(), picks.size() * 4, side));
             HIP_TRY(launch_rank(j->rlist.p, lo, hi, j->rank.p, side));
             HIP_TRY(launch_mask_or(j->rlist.p, lo, hi, j->W, j->tiles_x, A.mnew.p, A.tmin.p, side));
             HIP_TRY(launch_mask_or(j->rlist.p, lo, hi, j->W, j->tiles_x, A.mend.p, nullptr, side));
@@ -1259,7 +1296,7 @@ int ahead_stage(tsg_job* j) {
     const uint64_t pre_end = j->ahead_deep || j->flow_on ? S_eff : w_end;
     if (pre_end) {
         HIP_TRY(A.n_at.reserve(tab.size()));
-        HIP_TRY(j->ctx->staging_side.upload(A.n_at.p, tab.data(), tab.size() * 4, side));
+        HIP_TRY(j->stg_side->upload(A.n_at.p, tab.data(), tab.size() * 4, side));
         PrefetchArgs pa{};
         pa.W = j->W;
         pa.H = j->H;
@@ -1333,8 +1370,16 @@ int ahead_poll(tsg_job* j, bool block) {
     return ahead_stage(j);
 }
 
+// Items of the largest batch: a fraction of the resolved count, a fixed size, or the cap.
+uint64_t largest_batch(const tsg_job* j) {
+    uint64_t maxb = j->sched.px_per_batch ? j->sched.px_per_batch
+                                          : (uint64_t)j->N >> std::min(j->sched.redo_shift, j->sched.new_shift);
+    if (j->sched.max_batch) maxb = std::min<uint64_t>(maxb, j->sched.max_batch);
+    return std::min<uint64_t>(std::max<uint64_t>(maxb + 1, small_batch_max()), j->N);
+}
+
 int step_begin(tsg_job* j) {
-    hipStream_t s = j->ctx->stream;
+    hipStream_t s = j->stream;
     if (!j->state_ready) return fail(TSG_ERR_INVALID_ARGUMENT, "job state was not initialised");
     if (j->ran || j->step.active) return fail(TSG_ERR_INVALID_ARGUMENT, "a job runs once (Session::run consumes the session)");
     j->timed.clear();
@@ -1379,13 +1424,8 @@ int step_begin(tsg_job* j) {
         uint64_t per_seg = sh >= 40 ? items : (run_max + 1) << sh;
         bound = std::min<uint64_t>(items, 2ull * (P + 1) * per_seg);
     }
-    if (!j->in_engine) HIP_TRY(j->small_tab.reserve(3 * bound + 4 * (P + 1) + 16));
-    // largest batch: a fraction of the resolved count, a fixed size, or the cap
-    uint64_t maxb = j->sched.px_per_batch ? j->sched.px_per_batch
-                                          : (uint64_t)j->N >> std::min(j->sched.redo_shift, j->sched.new_shift);
-    if (j->sched.max_batch) maxb = std::min<uint64_t>(maxb, j->sched.max_batch);
-    maxb = std::max<uint64_t>(maxb + 1, small_batch_max());
-    HIP_TRY(j->result.reserve(std::min<uint64_t>(maxb, j->N)));
+    if (!j->in_engine && !j->flow_on) HIP_TRY(j->small_tab.reserve(3 * bound + 4 * (P + 1) + 16));
+    HIP_TRY(j->result.reserve(largest_batch(j)));
     j->overall_total = items;
     j->overall_cur = 0;
     j->step = tsg_job::Step{};
@@ -1398,7 +1438,7 @@ int step_begin(tsg_job* j) {
 
 // Stage preamble (ms.rs:786-858): level, recolour, seed, size, alpha, LUTs, picks.
 int step_open_stage(tsg_job* j) {
-    hipStream_t s = j->ctx->stream;
+    hipStream_t s = j->stream;
     tsg_job::Step& st = j->step;
     const int P = (int)j->prm.backtrack_stages;
     const int t = st.t;
@@ -1422,7 +1462,7 @@ int step_open_stage(tsg_job* j) {
     stage_luts(j->prm.cauchy_dispersion, j->guided, alpha_s, j->lut_keep[t].data());
     uint32_t lut_nan = 0;
     for (float v : j->lut_keep[t]) lut_nan |= (uint32_t)std::isnan(v);
-    HIP_TRY(j->ctx->staging.upload(j->lut.p, j->lut_keep[t].data(), 512 * 4, s));
+    HIP_TRY(j->stg->upload(j->lut.p, j->lut_keep[t].data(), 512 * 4, s));
     if (!j->flow_on) {
         int rc = wait_picks(j, t);
         if (rc) return rc;
@@ -1433,7 +1473,7 @@ int step_open_stage(tsg_job* j) {
     } else if (st.S > st.redo) {
         st.S_eff = st.redo + j->picks_keep[t].size();
         if (!j->picks_keep[t].empty() && !j->ahead_on) {
-            HIP_TRY(j->ctx->staging.upload(j->rlist.p + j->locked + st.redo, j->picks_keep[t].data(),
+            HIP_TRY(j->stg->upload(j->rlist.p + j->locked + st.redo, j->picks_keep[t].data(),
                                            j->picks_keep[t].size() * 4, s));
             const uint32_t lo = (uint32_t)(j->locked + st.redo);
             HIP_TRY(launch_rank(j->rlist.p, lo, lo + (uint32_t)j->picks_keep[t].size(), j->rank.p, s));
@@ -1526,7 +1566,7 @@ int step_ensure_rc(tsg_job* j, uint64_t lo, uint64_t hi) {
     bool need;
     int rc = step_plan_rc(j, lo, hi, &ra, &need);
     if (rc || !need) return rc;
-    HIP_TRY(timed_launch(j, K_RAND, ra.item1 - ra.item0, [&] { return launch_rand(ra, j->ctx->stream); }));
+    HIP_TRY(timed_launch(j, K_RAND, ra.item1 - ra.item0, [&] { return launch_rand(ra, j->stream); }));
     return TSG_OK;
 }
 
@@ -1555,7 +1595,7 @@ bool step_wants_prefetch(const tsg_job* j, uint64_t i0, uint64_t i1) {
 // its batch start, i.e. the pixels listed before position n_at(i) of the
 // resolved list. The mask holds the window's pixels too; rank filters them.
 int step_prefetch(tsg_job* j, uint64_t i0) {
-    hipStream_t s = j->ctx->stream;
+    hipStream_t s = j->stream;
     tsg_job::Step& st = j->step;
     std::vector<uint32_t> n_at;
     const bool redo = i0 < st.redo_eff;
@@ -1575,7 +1615,7 @@ int step_prefetch(tsg_job* j, uint64_t i0) {
     HIP_TRY(j->pre_n.reserve(std::min<uint64_t>(kPrefetchCap, j->N)));
     HIP_TRY(j->pre_cnt.reserve(std::min<uint64_t>(kPrefetchCap, j->N)));
     HIP_TRY(j->pre_nbrs.reserve(std::min<uint64_t>(kPrefetchCap, j->N) * k));
-    HIP_TRY(j->ctx->staging.upload(j->pre_n.p, n_at.data(), n * 4, s));
+    HIP_TRY(j->stg->upload(j->pre_n.p, n_at.data(), n * 4, s));
     PrefetchArgs pa{};
     pa.W = j->W;
     pa.H = j->H;
@@ -1625,12 +1665,12 @@ int step_close_stage(tsg_job* j) {
     tsg_job::Step& st = j->step;
     HIP_TRY(timed_launch(j, K_STATS, st.S_eff, [&] {
         return launch_stats_chunks(j->item_score.p, (uint32_t)st.S_eff, j->st_part.p, j->st_part_n.p,
-                                   j->st_sum.p + st.t, j->st_cnt.p + st.t, j->ctx->stream);
+                                   j->st_sum.p + st.t, j->st_cnt.p + st.t, j->stream);
     }));
     if (j->ahead_on) {
         tsg_job::Ahead& A = j->aset(st.t);
         if (!A.done) HIP_TRY(hipEventCreateWithFlags(&A.done, hipEventDisableTiming));
-        HIP_TRY(hipEventRecord(A.done, j->ctx->stream));
+        HIP_TRY(hipEventRecord(A.done, j->stream));
         A.done_recorded = true;
     }
     j->st_items[st.t] = st.S_eff;
@@ -1648,10 +1688,10 @@ int step_end(tsg_job* j) {
     if (j->ahead_on) {
         hipEvent_t e;
         HIP_TRY(next_event(j, &e));
-        HIP_TRY(hipEventRecord(e, j->ctx->side));
-        HIP_TRY(hipStreamWaitEvent(j->ctx->stream, e, 0));
+        HIP_TRY(hipEventRecord(e, j->side));
+        HIP_TRY(hipStreamWaitEvent(j->stream, e, 0));
     }
-    HIP_TRY(hipEventRecord(j->ev_run1, j->ctx->stream));
+    HIP_TRY(hipEventRecord(j->ev_run1, j->stream));
     return TSG_OK;
 }
 
@@ -1704,7 +1744,7 @@ struct Progress {
         if (!due(j, i1)) return TSG_OK;
         last_pct = pct(j, i1);
         snap.resize(j->N * 4);
-        HIP_TRY(hipStreamSynchronize(j->ctx->stream));
+        HIP_TRY(hipStreamSynchronize(j->stream));
         std::vector<uint4> stv(j->N);
         HIP_TRY(hipMemcpy(stv.data(), j->state.p, j->N * sizeof(uint4), hipMemcpyDeviceToHost));
         for (size_t q = 0; q < j->N; ++q) memcpy(&snap[q * 4], &stv[q].x, 4);
@@ -1720,7 +1760,7 @@ struct Progress {
 // larger batches take a wave per item.
 uint32_t flow_team_of(const tsg_job* j, uint64_t i0, uint64_t i1) {
     const tsg_tuning& u = j->tune;
-    if (i1 - i0 > u.prefetch_max) return 1;
+    if (i1 - i0 > (j->share > 1 ? std::min<uint64_t>(u.prefetch_max, kLaneTeamMax) : u.prefetch_max)) return 1;
     const uint32_t team =
         i0 < u.flow_head ? u.flow_head_team : std::max(u.flow_team, team_for(i1 - i0, u.team_max, u.team_waves));
     // the eight-wave kernel holds 64 random candidates
@@ -1734,7 +1774,7 @@ uint32_t flow_team_of(const tsg_job* j, uint64_t i0, uint64_t i1) {
 // end where it is due, and the items so far enter the state (no later item
 // reads them there: its own batch starts after them).
 int flow_stage(tsg_job* j, Progress& pr) {
-    hipStream_t s = j->ctx->stream;
+    hipStream_t s = j->stream;
     tsg_job::Step& st = j->step;
     BatchArgs& a = st.a;
     int rc;
@@ -1755,7 +1795,7 @@ int flow_stage(tsg_job* j, Progress& pr) {
             i1 = b1;
             if ((due = pr.due(j, i1))) break;
         }
-        const uint32_t most = flow_max_wgs(team, j->guided);
+        const uint32_t most = std::max(1u, flow_max_wgs(team, j->guided) / j->share);
         const uint32_t wgs = j->tune.flow_wgs ? std::min(j->tune.flow_wgs, most) : most;
         if (j->flow_launches == kFlowTickets) {
             HIP_TRY(hipMemsetAsync(j->flow_ticket.p, 0, kFlowTickets * 4, s));
@@ -1792,20 +1832,13 @@ int flow_stage(tsg_job* j, Progress& pr) {
     return TSG_OK;
 }
 
-// Single job: with stage-ahead neighbour lists, every stage runs in
-// dependency order (flow_stage). Else runs of small batches go to one
-// single-workgroup launch; other batches get one k_resolve launch,
-// committing in its last workgroup when the batch holds at most fuse_max
-// items.
-int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
-    hipStream_t s = j->ctx->stream;
-    int rc;
-    // content-independent work ahead on the side stream when the buffer
-    // sets fit the budget: one per stage (deep), else two of the largest
-    // stage. In dependency order a set per stage is also taken where it holds
-    // no more than the two would (at p = 0.5 it never does): the preparation
-    // then runs ahead of the stages without waiting for a set to come free.
-    // In tiling mode the lists need the batch table's ranks: dependency order only.
+// Content-independent work ahead on the side stream when the buffer sets fit
+// the budget: one per stage (deep), else two of the largest stage. In
+// dependency order a set per stage is also taken where it holds no more than
+// the two would (at p = 0.5 it never does): the preparation then runs ahead
+// of the stages without waiting for a set to come free. In tiling mode the
+// lists need the batch table's ranks: dependency order only.
+void plan_ahead(tsg_job* j) {
     const bool ahead_ok = j->tune.ahead && (!j->prm.tiling_mode || j->tune.flow);
     const bool two_fit = ahead_bytes(j) <= kAheadBudget;
     const bool deep_fits = j->prm.backtrack_stages + 1 <= 8 && ahead_bytes_deep(j) <= kAheadBudget;
@@ -1814,6 +1847,17 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     j->ahead_on = j->ahead_deep || (ahead_ok && two_fit);
     // dependency order needs the stage-ahead neighbour lists
     j->flow_on = j->ahead_on && j->tune.flow;
+}
+
+// Single job: with stage-ahead neighbour lists, every stage runs in
+// dependency order (flow_stage). Else runs of small batches go to one
+// single-workgroup launch; other batches get one k_resolve launch,
+// committing in its last workgroup when the batch holds at most fuse_max
+// items.
+int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
+    hipStream_t s = j->stream;
+    int rc;
+    plan_ahead(j);
     if ((rc = step_begin(j))) return rc;
     if (j->flow_on) {
         if ((rc = picks_begin(j))) return rc;
@@ -1843,7 +1887,7 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
         hipEvent_t e;
         HIP_TRY(next_event(j, &e));
         HIP_TRY(hipEventRecord(e, s));
-        HIP_TRY(hipStreamWaitEvent(j->ctx->side, e, 0));
+        HIP_TRY(hipStreamWaitEvent(j->side, e, 0));
         if ((rc = ahead_stage(j))) return rc;
     }
     // persistent single-wave batches
@@ -1902,7 +1946,7 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
         if (j->small_used + tab.size() > j->small_tab.n) return fail(TSG_ERR_DEVICE, "small-batch table overflow");
         uint32_t* dt = j->small_tab.p + j->small_used;
         j->small_used += tab.size();
-        HIP_TRY(j->ctx->staging.upload(dt, tab.data(), tab.size() * 4, s));
+        HIP_TRY(j->stg->upload(dt, tab.data(), tab.size() * 4, s));
         const BatchArgs& a = j->step.a;
         if (sb_coop) {
             HIP_TRY(timed_launch(j, K_RUN, sb_bounds.back() - sb_bounds.front(), [&] {
@@ -2064,6 +2108,8 @@ struct tsg_batch {
         int status;
         bool failed;  // status set by the engine (planning error, cancellation)
         bool alone;   // runs (ran) alone on the single-job path; status final once run
+        bool lane = false;        // as alone, beside other jobs, by run_on_lanes
+        uint64_t lane_bytes = 0;  // its stage-ahead buffers
     };
     std::vector<Entry> active, pending, done, taken;
     uint64_t next_ticket = 1;
@@ -2081,7 +2127,9 @@ struct tsg_batch {
     uint64_t quantum = 0;                 // resolve items per job per launch (0: no bound)
     uint32_t alone_below = 0;             // jobs starting while fewer are in the batch run alone (0: never)
     uint64_t alone_ahead = 0;             // device bytes an alone run may add for its stage-ahead sets
+    bool alone_set = false;               // alone_ahead was given
     uint64_t alone_runs = 0;              // jobs run alone so far
+    uint64_t lane_budget() const { return alone_set ? alone_ahead : kAheadBudget; }
     tsg_tuning tune{};
     ~tsg_batch() {
         if (h_blk) (void)hipHostFree(h_blk);
@@ -2119,7 +2167,7 @@ void eng_push(tsg_job* j, uint32_t kind, uint32_t i0, uint32_t i1, uint32_t per_
 // Stage preamble (ms.rs:786-858) as planned work: the recolour phase, the
 // stage's cost tables and picks uploaded, the stage's batch arguments.
 int eng_open_stage(tsg_job* j) {
-    hipStream_t s = j->ctx->stream;
+    hipStream_t s = j->stream;
     tsg_job::Step& st = j->step;
     const int P = (int)j->prm.backtrack_stages;
     const int t = st.t;
@@ -2139,14 +2187,14 @@ int eng_open_stage(tsg_job* j) {
     uint32_t lut_nan = 0;
     for (float v : j->lut_keep[t]) lut_nan |= (uint32_t)std::isnan(v);
     float* lut = j->eng.luts.p + (size_t)t * 512;
-    HIP_TRY(j->ctx->staging.upload(lut, j->lut_keep[t].data(), 512 * 4, s));
+    HIP_TRY(j->stg->upload(lut, j->lut_keep[t].data(), 512 * 4, s));
     int rc = wait_picks(j, t);
     if (rc) return rc;
     st.S_eff = st.S;
     if (st.S > st.redo) {
         st.S_eff = st.redo + j->picks_keep[t].size();
         if (!j->picks_keep[t].empty()) {
-            HIP_TRY(j->ctx->staging.upload(j->rlist.p + j->locked + st.redo, j->picks_keep[t].data(),
+            HIP_TRY(j->stg->upload(j->rlist.p + j->locked + st.redo, j->picks_keep[t].data(),
                                            j->picks_keep[t].size() * 4, s));
             const uint32_t lo = (uint32_t)(j->locked + st.redo);
             HIP_TRY(launch_rank(j->rlist.p, lo, lo + (uint32_t)j->picks_keep[t].size(), j->rank.p, s));
@@ -2337,66 +2385,216 @@ int eng_drop(tsg_batch* b, size_t q, int status) {
     return TSG_OK;
 }
 
-int batch_admit(tsg_batch* b) {
+// A run within `budget` bytes of stage-ahead buffers.
+void ahead_within(tsg_job* j, uint64_t budget) {
+    if (j->tune.ahead >= 2 && ahead_bytes_deep(j) > budget) j->tune.ahead = 1;
+    if (ahead_bytes(j) > budget) j->tune.ahead = 0;
+}
+
+// Whether a job of a batch that may add `budget` bytes of stage-ahead buffers
+// runs in dependency order, and the bytes it takes; if not, it is as it was.
+bool lane_plan(tsg_job* j, uint64_t budget, uint64_t* bytes) {
+    const uint32_t ahead = j->tune.ahead;
+    ahead_within(j, budget);
+    plan_ahead(j);
+    *bytes = j->ahead_deep ? ahead_bytes_deep(j) : ahead_bytes(j);
+    if (j->flow_on && *bytes <= budget) return true;
+    j->tune.ahead = ahead;
+    j->ahead_deep = j->ahead_on = j->flow_on = false;
+    return false;
+}
+
+// Every stage-ahead and dependency-order buffer of the planned run.
+hipError_t lane_reserve(tsg_job* j) {
+    const int P = (int)j->prm.backtrack_stages;
+    const uint64_t words = j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size());
+    const size_t tiles = (size_t)j->tiles_x * j->tiles_y;
+    hipError_t e = j->mail.reserve(2 * j->N);
+    for (DBuf<uint32_t>* d : {&j->unres[0], &j->unres[1], &j->pick_idx, &j->pick_link, &j->pick_head})
+        if (e == hipSuccess) e = d->reserve(std::max<size_t>(1, j->N0));
+    for (int t = 0; t < (j->ahead_deep ? P + 1 : 2) && e == hipSuccess; ++t) {
+        tsg_job::Ahead& A = j->ahead[t];
+        const uint64_t n = std::max<uint64_t>(1, stage_size(j, j->ahead_deep ? P - t : 0));
+        e = A.rc.reserve(n * words);
+        if (e == hipSuccess) e = A.nbrs.reserve(n * j->prm.nearest_neighbors);
+        if (e == hipSuccess) e = A.cnt.reserve(n);
+        if (e == hipSuccess) e = A.dep.reserve(n);
+        if (e == hipSuccess) e = A.mend.reserve(tiles);
+        if (e == hipSuccess) e = A.mnew.reserve(tiles);
+        if (e == hipSuccess) e = A.tmin.reserve(tiles);
+    }
+    return e;
+}
+
+// Gives back what lane_reserve took (nothing of the job is in flight).
+void lane_release(tsg_job* j) {
+    for (tsg_job::Ahead& A : j->ahead) give_back(A.rc, A.nbrs, A.cnt, A.n_at, A.mend, A.mnew, A.tmin, A.dep);
+    give_back(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head, j->pick_moves);
+}
+
+int batch_admit(tsg_batch* b, bool whole) {
     while (b->active.size() < b->max_active && !b->pending.empty()) {
         tsg_batch::Entry e = b->pending.front();
         b->pending.erase(b->pending.begin());
         // few jobs in the batch: this one gets the whole device to itself
         e.alone = b->alone_below && b->active.size() + b->pending.size() + 1 < b->alone_below;
+        int rc = TSG_OK;
+        if (!e.alone && whole && !b->quantum && !b->wgs_cap && !b->engine_flags && b->lane_budget() &&
+            lane_plan(e.job, b->lane_budget(), &e.lane_bytes)) {
+            // the job's run is one of several at a time (run_on_lanes)
+            e.lane = true;
+            const hipError_t he = e.job->result.reserve(largest_batch(e.job));
+            if (he != hipSuccess)
+                rc = fail(he == hipErrorOutOfMemory ? TSG_ERR_OUT_OF_MEMORY : TSG_ERR_DEVICE, hipGetErrorString(he));
+        }
         b->active.push_back(e);
         if (e.alone) continue;
-        const int rc = eng_begin(e.job);
+        if (!e.lane) rc = eng_begin(e.job);
         if (rc) eng_drop(b, b->active.size() - 1, rc);
     }
     return TSG_OK;
 }
 
-// Jobs admitted to run alone: each runs to its end on the single-job path
-// (tsg_job_run's launch sequence), one after another, smallest first, before
-// the round's engine launch. Its stage-ahead sets (which the dependency-
-// ordered runs need) are used only when they fit the bytes the caller allows
-// beyond tsg_footprint_estimate, and are released when the run ends.
-int batch_run_alone(tsg_batch* b) {
-    std::vector<tsg_batch::Entry> runs;
+// One whole single-job run (tsg_job_run's launch sequence) of a batch's job.
+void lane_run_job(tsg_batch::Entry& e) {
+    tsg_job* j = e.job;
+    j->in_engine = false;
+    j->pk_threads = kPickThreads;
+    e.status = run_job(j, nullptr, nullptr);
+    // nothing of the run is in flight any more: its stage-ahead sets go back
+    // to the device cache now, not with the job
+    (void)hipStreamSynchronize(j->stream);
+    if (j->side != j->stream) (void)hipStreamSynchronize(j->side);
+    lane_release(j);
+}
+
+// Runs in dependency order, kLanes at a time, each on a stream and a host
+// thread of its own: a small job's time is that of its chain of dependent
+// items, which leaves most of the chip to the others. Lane 0 and every second
+// one take the largest job left, the others the smallest, so that jobs bound
+// by their chain run beside jobs bound by the vector units. The runs in
+// flight hold at most `budget` bytes of stage-ahead buffers. Jobs whose
+// buffers the device cannot hold are left with e.lane_bytes = UINT64_MAX.
+void run_on_lanes(tsg_batch* b, std::vector<tsg_batch::Entry>& runs, uint64_t budget) {
+    std::stable_sort(runs.begin(), runs.end(),
+                     [](const tsg_batch::Entry& x, const tsg_batch::Entry& y) { return x.job->N > y.job->N; });
+    tsg_ctx* c = b->ctx;
+    const size_t n = std::min(kLanes, runs.size());
+    while (c->lanes.size() < n) {
+        std::unique_ptr<Lane> l(new Lane());
+        if (hipStreamCreateWithFlags(&l->stream, hipStreamNonBlocking) != hipSuccess ||
+            l->staging.init(1u << 20, 4) != hipSuccess)
+            break;
+        c->lanes.push_back(std::move(l));
+    }
+    const size_t lanes = std::max<size_t>(1, std::min(n, c->lanes.size()));
+    std::mutex mu;
+    std::condition_variable cv;
+    size_t head = 0, tail = runs.size(), busy = 0;
+    uint64_t used = 0;
+    auto work = [&](size_t l) {
+        (void)hipSetDevice(c->device);
+        std::unique_lock<std::mutex> lk(mu);
+        for (;;) {
+            size_t q = 0;
+            cv.wait(lk, [&] {
+                if (head == tail) return true;
+                q = l % 2 ? tail - 1 : head;
+                return busy == 0 || used + runs[q].lane_bytes <= budget;
+            });
+            if (head == tail) return;
+            if (l % 2) --tail;
+            else ++head;
+            tsg_batch::Entry& e = runs[q];
+            const uint64_t bytes = e.lane_bytes;
+            used += bytes;
+            ++busy;
+            lk.unlock();
+            tsg_job* j = e.job;
+            if (l < c->lanes.size()) {
+                j->stream = j->side = c->lanes[l]->stream;
+                j->stg = j->stg_side = &c->lanes[l]->staging;
+            }
+            j->share = (uint32_t)std::min(lanes, kLaneShare);
+            if (lane_reserve(j) == hipSuccess) {
+                lane_run_job(e);
+            } else {
+                lane_release(j);
+                e.lane_bytes = UINT64_MAX;
+            }
+            j->on_context();
+            lk.lock();
+            used -= bytes;
+            --busy;
+            cv.notify_all();
+        }
+    };
+    std::vector<std::thread> th;
+    for (size_t l = 1; l < lanes; ++l) {
+        try {
+            th.emplace_back(work, l);
+        } catch (const std::system_error&) {
+            break;  // no more threads: the lanes there are do the work
+        }
+    }
+    work(0);
+    for (std::thread& t : th) t.join();
+}
+
+// The round's jobs that run whole (admitted alone, or to a lane), before its
+// engine launch. Stage-ahead sets, which the dependency-ordered runs need,
+// are used only within the bytes that the batch may add beyond
+// tsg_footprint_estimate, and are released when a run ends. Runs in
+// dependency order go to the lanes, others one after another, smallest first.
+int batch_run_whole(tsg_batch* b) {
+    std::vector<tsg_batch::Entry> runs, rest;
+    const uint64_t budget = b->lane_budget();
+    bool shared = false;
     for (size_t q = 0; q < b->active.size();) {
-        if (!b->active[q].alone) {
+        tsg_batch::Entry& e = b->active[q];
+        if (!e.alone && !e.lane) {
             ++q;
             continue;
         }
-        runs.push_back(b->active[q]);
+        shared = shared || e.lane;
+        const bool lane = e.lane || lane_plan(e.job, budget, &e.lane_bytes);
+        (lane ? runs : rest).push_back(e);
         b->active.erase(b->active.begin() + q);
     }
-    std::stable_sort(runs.begin(), runs.end(),
-                     [](const tsg_batch::Entry& x, const tsg_batch::Entry& y) { return x.job->N < y.job->N; });
+    if (runs.empty() && rest.empty()) return TSG_OK;
+    if (!runs.empty()) run_on_lanes(b, runs, budget);
     for (tsg_batch::Entry& e : runs) {
-        tsg_job* j = e.job;
-        // a single-job run (its small-batch tables, all pick threads); the
-        // random candidates keep the engine's chunk size of the estimate
-        j->in_engine = false;
-        j->pk_threads = kPickThreads;
-        if (j->tune.ahead >= 2 && ahead_bytes_deep(j) > b->alone_ahead) j->tune.ahead = 1;
-        if (ahead_bytes(j) > b->alone_ahead) j->tune.ahead = 0;
-        e.status = run_job(j, nullptr, nullptr);
-        b->alone_runs += 1;
-        // the run has ended (run_job waited for it, and the side stream is
-        // drained here): its stage-ahead sets go back to the device cache
-        // now, not with the job
-        HIP_TRY(hipStreamSynchronize(j->ctx->side));
-        g_pool_release = true;
-        for (tsg_job::Ahead& A : j->ahead) {
-            A.rc.release();
-            A.nbrs.release();
-            A.cnt.release();
-            A.n_at.release();
-            A.mend.release();
-            A.mnew.release();
-            A.tmin.release();
-            A.dep.release();
+        if (e.lane_bytes == UINT64_MAX) {
+            // its buffers did not fit the device after all
+            e.lane_bytes = 0;
+            if (e.alone) {
+                e.job->tune.ahead = 0;  // without them
+                rest.push_back(e);
+            } else {
+                e.lane = false;
+                e.job->in_engine = true;
+                e.job->ahead_deep = e.job->ahead_on = e.job->flow_on = false;
+                b->active.push_back(e);
+                const int rc = eng_begin(e.job);
+                if (rc) eng_drop(b, b->active.size() - 1, rc);
+            }
+            continue;
         }
-        j->mail.release();
-        for (DBuf<uint32_t>* d : {&j->unres[0], &j->unres[1], &j->pick_idx, &j->pick_link, &j->pick_head}) d->release();
-        g_pool_release = false;
+        if (e.alone) b->alone_runs += 1;
+        else b->units_total += e.job->n_batches;
         b->done.push_back(e);
+    }
+    std::stable_sort(rest.begin(), rest.end(),
+                     [](const tsg_batch::Entry& x, const tsg_batch::Entry& y) { return x.job->N < y.job->N; });
+    for (tsg_batch::Entry& e : rest) {
+        ahead_within(e.job, budget);
+        lane_run_job(e);
+        b->alone_runs += 1;
+        b->done.push_back(e);
+    }
+    if (shared) {
+        b->rounds += 1;
+        b->launches += 1;
     }
     return TSG_OK;
 }
@@ -2411,7 +2609,7 @@ double host_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
-int batch_round(tsg_batch* b) {
+int batch_round(tsg_batch* b, bool whole) {
     hipStream_t s = b->ctx->stream;
     double t_mark = host_ms();
     auto lap = [&](int slot) {
@@ -2419,9 +2617,10 @@ int batch_round(tsg_batch* b) {
         b->prof[slot] += t - t_mark;
         t_mark = t;
     };
-    batch_admit(b);
-    batch_run_alone(b);
+    batch_admit(b, whole);
     lap(6);
+    batch_run_whole(b);
+    lap(9);
     if (b->active.empty()) return TSG_OK;
     // plan every job as far as its picks allow; a job that cannot be planned leaves
     for (size_t q = 0; q < b->active.size();) {
@@ -2663,7 +2862,7 @@ int batch_reap(tsg_batch* b, bool wait) {
             ++q;
             continue;
         }
-        if (b->done[q].alone) {
+        if (b->done[q].alone || b->done[q].lane) {
             // run_job has waited for its end and set its state
             j->step.active = false;
             j->ran = true;
@@ -2832,6 +3031,7 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
     HIP_TRY(hipSetDevice(ctx->device));
     std::unique_ptr<tsg_job> j(new tsg_job());
     j->ctx = ctx;
+    j->on_context();
     j->prm = *prm;
     tsg_schedule_default(&j->sched);
     tsg_tuning_default(&j->tune);
@@ -3704,7 +3904,7 @@ int tsg_batch_submit(tsg_batch* b, tsg_job* job, uint64_t* ticket) {
             if (e.job == job) return fail(TSG_ERR_INVALID_ARGUMENT, "job already submitted");
     *ticket = b->next_ticket++;
     job->owner = b;
-    b->pending.push_back({*ticket, job, 0, false});
+    b->pending.push_back({*ticket, job, 0, false, false});
     return TSG_OK;
 }
 
@@ -3749,6 +3949,7 @@ int tsg_batch_set_alone_below(tsg_batch* b, uint32_t jobs, uint64_t ahead_bytes)
     if (!b) return fail(TSG_ERR_INVALID_ARGUMENT, "null batch");
     b->alone_below = jobs;
     b->alone_ahead = ahead_bytes;
+    b->alone_set = true;
     return TSG_OK;
 }
 
@@ -3788,7 +3989,7 @@ int tsg_batch_step(tsg_batch* b, uint32_t max_rounds, uint32_t* in_flight) {
     HIP_TRY(hipSetDevice(b->ctx->device));
     std::lock_guard<std::mutex> lk(b->ctx->mu);
     for (uint32_t r = 0; r < max_rounds && !(b->active.empty() && b->pending.empty()); ++r) {
-        int rc = batch_round(b);
+        int rc = batch_round(b, false);
         if (rc) return rc;
     }
     int rc = batch_reap(b, false);
@@ -3802,7 +4003,9 @@ int tsg_batch_run_all(tsg_batch* b) {
     HIP_TRY(hipSetDevice(b->ctx->device));
     std::lock_guard<std::mutex> lk(b->ctx->mu);
     while (!(b->active.empty() && b->pending.empty())) {
-        int rc = batch_round(b);
+        // nothing can be submitted or cancelled before every job has finished:
+        // jobs need not take part in rounds
+        int rc = batch_round(b, true);
         if (rc) return rc;
     }
     return batch_reap(b, true);

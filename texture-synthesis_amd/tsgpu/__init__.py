@@ -550,9 +550,11 @@ class Session:
 class Batch:
     """Many sessions in flight on one device.
 
-    Each round plans every active session as far as its pick orders allow and
-    runs everything planned in one launch of the work-queue engine; a
-    session's result is identical to Session.run on it alone. No counterpart
+    run_all runs the sessions whole, several at a time, where their
+    stage-ahead buffers fit. Else, and under step, each round plans every
+    active session as far as its pick orders allow and runs everything planned
+    in one launch of the work-queue engine. A session's result is identical to
+    Session.run on it alone. No counterpart
     in the reference, whose Session::run (session.rs:37-66) synthesises one
     image at a time."""
 
@@ -576,7 +578,8 @@ class Batch:
 
     def set_alone(self, below: int, ahead_bytes: int = 0):
         """Sessions starting while fewer than `below` are in the batch run
-        alone; their stage-ahead buffers are used when they fit ahead_bytes."""
+        alone (several such a few at a time); the stage-ahead buffers of those
+        in flight are used when they fit ahead_bytes."""
         self._alone_below = int(below)
         _check(lib().tsg_batch_set_alone_below(self._h, int(below), max(0, int(ahead_bytes))))
 

@@ -8,8 +8,9 @@ estimate fit the memory budget and an engine slot is free: it is then built
 launch of the work-queue engine. Requests that arrive while others run join
 at the next round, and a finished request frees its memory and slot for the
 next in line. Unless ALONE_BELOW or more requests are in flight, a request
-starting runs alone with the whole device instead, which shortens its chain
-of small batches; the engine takes over as requests pile up. A request whose estimate alone exceeds the budget is rejected
+starting runs alone instead, whole (several that start together a few at a
+time), which shortens its chain of small batches; the engine takes over as
+requests pile up. A request whose estimate alone exceeds the budget is rejected
 (AdmissionRejected) rather than held; a request can be cancelled; a request
 that fails (invalid, out of memory) is reported without disturbing others.
 
