@@ -895,8 +895,14 @@ __device__ __forceinline__ void prune_bound(const unsigned long long* tb, const 
 // FIRST_SH: while a pruning bound exists, the first chunk holds 2^FIRST_SH
 // neighbours. 3 (8 neighbours) starts pruning early, which pays where the
 // VALU binds (the multi-job engine); 6 (a full chunk) saves a gather round
-// trip, which pays where latency binds (the single-job kernels). A constant
-// here also lets the compiler keep the loop in fewer registers.
+// trip, which pays where latency binds (the batch kernels); kGrowing (the wave
+// runs, whose waves hide the round trips and are bound by the gathers and
+// terms together): chunks of 2, 8, 32 and 64 neighbours, as most candidates
+// fall in the first. Device time of a run at 1024^2 and 2048^2, ms: full
+// chunks or 8 first 10.5 and 32.5, 4 first 10.1 and 30.7, 2 first 9.9 and
+// 30.0, growing from 2 9.9 and 29.9; guided 1024^2 18.6, -, 17.9, 17.6. A
+// constant here also lets the compiler keep the loop in fewer registers.
+constexpr int kGrowing = 1;
 template <bool GUIDED, int FIRST_SH>
 __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps, WaveLds* L, const float* lut, const float* glut,
                                            int slot, int lane, uint32_t kf, uint32_t n_act, Best& best,
@@ -919,7 +925,12 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
     while (n_act > 0) {
         // chunk of 2^sh neighbours with n_act << sh <= kTermCap; while a bound
         // exists the first chunk holds 2^FIRST_SH
-        uint32_t sh = (j0 == 0 && PBi != kNone) ? (uint32_t)FIRST_SH : 6u;
+        uint32_t sh = 6u;
+        if (FIRST_SH == kGrowing) {
+            if (PBi != kNone) sh = j0 == 0 ? 1u : j0 < 8 ? 3u : j0 < 32 ? 5u : 6u;
+        } else if (j0 == 0 && PBi != kNone) {
+            sh = (uint32_t)FIRST_SH;
+        }
         while (sh > 0 && (n_act << sh) > (uint32_t)kTermCap) --sh;
         const uint32_t jc = 1u << sh;
         const uint32_t jn = min(jc, kf - j0);
@@ -1973,7 +1984,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
                                                            uniq, &st);
             phase_clock(a, item, 2, lane);
             if (!a.lut_nan && L->avg > 0.0) {
-                const Best b = eval_slice<GUIDED, 6>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, 0, a.m, rpre, 0,
+                const Best b = eval_slice<GUIDED, kGrowing>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, 0, a.m, rpre, 0,
                                                      1, true, L, lut, glut, lane % lut_copies<GUIDED>(), lane, nullptr);
                 phase_clock(a, item, 5, lane);
                 const bool have = b.Bi != kNone;
