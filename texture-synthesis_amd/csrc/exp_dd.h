@@ -169,4 +169,24 @@ TSG_HD double exp_dd(double x) {
     return ldexp(z.hi + rest, m);
 }
 
+// (float)exp_dd(x). In plain double arithmetic (the same reduction, e^r - 1
+// to r^5: a truncation below 2^-54) the value is within 3 units in the last
+// place of exp(x), and exp_dd's within one; unless it lies within 16 units of
+// the midpoint of two floats, both round to the same one. One argument in
+// 2^24 takes the long way, and so does every one outside (-80, 0].
+TSG_HD float exp_f32(double x) {
+    if (x <= 0.0 && x > -80.0) {
+        const double n = rint(x * kInvLn2x64);
+        const int ni = (int)n;
+        const int j = ni & 63;
+        const double r = fma(-n, kLn2d64b, fma(-n, kLn2d64a, x));
+        double t = kInvFact[4][0];
+        for (int k = 3; k >= 1; --k) t = fma(t, r, kInvFact[k][0]);
+        const double y = fma(kExp2Tab[j][0], fma(r * r, t, r), kExp2Tab[j][0]);  // in [0.99, 2)
+        const uint32_t low = (uint32_t)__builtin_bit_cast(uint64_t, y) & 0x1fffffffu;
+        if (low - (0x10000000u - 16u) > 32u) return ldexpf((float)y, (ni - j) / 64);
+    }
+    return (float)exp_dd(x);
+}
+
 }  // namespace tsg

@@ -59,6 +59,7 @@ struct BatchArgs {
     const int32_t* pre_nbrs;      // [item - pre_base][k] packed dx | dy << 16
     const uint32_t* pre_cnt;
     uint32_t pre_base, pre_end;
+    const double* pre_avg;        // unguided wave runs: [item - pre_base] mean distance (ListAvgArgs)
     // tiling mode (null gmask: off): per 8x8 tile, the resolved pixels that
     // carry ghost copies one image width / height away, on the far side, while
     // within the edge margins x < xl, x > xr, y < yb, y > yt; neighbour records
@@ -131,6 +132,17 @@ struct PrefetchArgs {
     uint32_t ghosts, g_lo;
     int32_t xl, xr, yb, yt;
 };
+
+// Mean distance of the neighbours of items [i0, n) (ms.rs:405-425).
+struct ListAvgArgs {
+    uint32_t W, H;
+    const uint32_t* work;   // [item]
+    const int32_t* nbrs;    // [item][k]
+    const uint32_t* cnt;
+    uint32_t i0, n, k;
+    double* avg;            // 0 where an item has no neighbours
+};
+hipError_t launch_list_avg(const ListAvgArgs& a, hipStream_t s);
 
 // A dependency-ordered run: consecutive items [a.item0, a.item0 + n) of one
 // stage in one launch of persistent workgroups, redo items and new pixels

@@ -1128,18 +1128,22 @@ __device__ __forceinline__ uint4 item_at_random(const BatchArgs& a, const MapDes
 // Every member: neighbour state (own pattern, distances, weights) into L and
 // the coherence candidates; returns n_coh. Lanes < n_k0 hold candidate
 // lane's (xy, map) in xy/ms; `uniq` marks the first of equal ones.
+// Squared distance of a neighbour in units of the image's sides (ms.rs:405-425).
+__device__ __forceinline__ double neighbour_dist(uint32_t W, uint32_t H, int x, int y, int32_t o) {
+    const int nx = x + packed_dx(o), ny = y + packed_dy(o);
+    const double dimx = (double)W, dimy = (double)H;
+    const double x1 = (double)nx / dimx, y1 = (double)ny / dimy;
+    const double x2 = (double)x / dimx, y2 = (double)y / dimy;
+    return fma(x1 - x2, x1 - x2, (y1 - y2) * (y1 - y2));
+}
+
 // The neighbour weights (ms.rs:405-425, 1198-1203), from the neighbour
 // offsets alone: distances, their average over the 4k duplicated entries
 // summed in order, exp(-d / avg).
 template <class Lds>
 __device__ __forceinline__ void item_geometry(const BatchArgs& a, int x, int y, uint32_t kf, Lds* L, int lane) {
     if (lane < (int)kf) {
-        const int32_t o = L->nd[lane];
-        const int nx = x + packed_dx(o), ny = y + packed_dy(o);
-        const double dimx = (double)a.W, dimy = (double)a.H;
-        const double x1 = (double)nx / dimx, y1 = (double)ny / dimy;
-        const double x2 = (double)x / dimx, y2 = (double)y / dimy;
-        L->dist[lane] = fma(x1 - x2, x1 - x2, (y1 - y2) * (y1 - y2));
+        L->dist[lane] = neighbour_dist(a.W, a.H, x, y, L->nd[lane]);
     }
     wave_sync();
     if (lane == 0) {
@@ -1172,6 +1176,20 @@ __device__ __forceinline__ void item_geometry(const BatchArgs& a, int x, int y, 
     }
     wave_sync();
     if (lane < (int)kf) L->w[lane] = (float)exp_dd(-1.0 * (L->dist[lane] / L->avg));
+    wave_sync();
+}
+
+// The same with the mean distance known (k_list_avg), for the unguided wave
+// runs: lane j's offset in o. The sum above is 200 dependent adds of one lane
+// and exp_dd some 80 instructions, together a quarter of an item's vector
+// instructions. Device time of a run with both out of the item's way: 1024^2
+// 9.92 -> 9.58 ms, 2048^2 29.8 -> 29.2. Guided runs wait on twice the gathers
+// and gain nothing (18.6 -> 19.3 at 1024^2 with the kernel's own time), teams
+// form the weights while their records are on their way.
+template <class Lds>
+__device__ __forceinline__ void item_weights(const BatchArgs& a, int x, int y, int32_t o, uint32_t kf, double avg,
+                                             Lds* L, int lane) {
+    if (lane < (int)kf) L->w[lane] = exp_f32(-1.0 * (neighbour_dist(a.W, a.H, x, y, o) / avg));
     wave_sync();
 }
 
@@ -1973,8 +1991,15 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
         if (kf == 0) {
             r = item_at_random(a, maps, item, 0, flat, lane);
         } else {
-            wave_sync();
-            item_geometry(a, x, y, kf, L, lane);
+            double avg;
+            if constexpr (GUIDED) {
+                wave_sync();
+                item_geometry(a, x, y, kf, L, lane);
+                avg = L->avg;
+            } else {
+                avg = gld(a.pre_avg + rel);
+                item_weights(a, x, y, o, kf, avg, L, lane);
+            }
             const uint4 st = flow_records(f, a, f.dep[rel], lane < (int)kf ? nbr_flat(a, x, y, o) : 0u,
                                           lane < (int)kf, lane);
             phase_clock(a, item, 1, lane);
@@ -1983,7 +2008,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
             const uint32_t n_coh = item_neighbours<GUIDED>(a, maps, item, 0, x, y, kf, 0, L, lane, true, cxy, cms,
                                                            uniq, &st);
             phase_clock(a, item, 2, lane);
-            if (!a.lut_nan && L->avg > 0.0) {
+            if (!a.lut_nan && avg > 0.0) {
                 const Best b = eval_slice<GUIDED, kGrowing>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, 0, a.m, rpre, 0,
                                                      1, true, L, lut, glut, lane % lut_copies<GUIDED>(), lane, nullptr);
                 phase_clock(a, item, 5, lane);
@@ -2883,6 +2908,31 @@ __global__ void k_xform_apply(const uint32_t* coord, uint32_t n, const XformSour
     out[i] = srcs[m].px[(size_t)y * srcs[m].w + x];
 }
 
+// Mean distances, an item per lane: the reference's sum is 4 k dependent adds,
+// which one wave per item leaves to one of its lanes.
+__global__ __launch_bounds__(kWave) void k_list_avg(ListAvgArgs a) {
+    extern __shared__ int32_t offs[];  // rows of an odd length: no bank conflicts
+    const uint32_t lane = threadIdx.x, i0 = a.i0 + blockIdx.x * kWave, row = a.k | 1u;
+    const uint32_t rows = min((uint32_t)kWave, a.n - i0);
+    if (lane < a.k) {
+#pragma unroll 8
+        for (uint32_t r = 0; r < rows; ++r) offs[r * row + lane] = gld(a.nbrs + (size_t)(i0 + r) * a.k + lane);
+    }
+    __syncthreads();
+    if (lane >= rows) return;
+    const uint32_t kf = gld(a.cnt + i0 + lane), flat = gld(a.work + i0 + lane);
+    const int x = (int)(flat % a.W), y = (int)(flat / a.W);
+    double sum = 0.0;
+    for (uint32_t j = 0; j < kf; ++j) {
+        const double d = neighbour_dist(a.W, a.H, x, y, offs[lane * row + j]);
+        sum = sum + d;
+        sum = sum + d;
+        sum = sum + d;
+        sum = sum + d;
+    }
+    gst(a.avg + i0 + lane, kf ? sum / (double)(4u * kf) : 0.0);
+}
+
 // ---- pick orders (PickArgs) ----
 // The chain of swaps is serial only in appearance. Step q moves the list's
 // last entry, position L0 - 1 - q, to position idx[q]; so the content of a
@@ -3485,7 +3535,7 @@ __device__ __forceinline__ void unit_publish(bool spread) {
     if (spread) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
 }
 
-// Weight-exp sweep (test hook): out[i - i0] = (float)exp_dd(-1.0 * x_i), the
+// Weight-exp sweep (test hook): out[i - i0] = exp_f32(-1.0 * x_i), the
 // expression of the neighbour weights in item_geometry, for the arguments
 // x_i = t * 8 when i % 4 != 0, else 8 + t * 56, with t = ((i * 0x9E3779B97F4A7C15)
 // >> 11) * 2^-53 in [0, 1): three quarters of the arguments in [0, 8), where
@@ -3496,7 +3546,7 @@ __global__ void k_exp_sweep(uint64_t i0, uint64_t n, float* out) {
     const uint64_t i = i0 + r;
     const double t = (double)((i * 0x9E3779B97F4A7C15ull) >> 11) * 0x1p-53;
     const double x = (i & 3u) ? t * 8.0 : __dadd_rn(8.0, __dmul_rn(t, 56.0));
-    out[r] = (float)exp_dd(-1.0 * x);
+    out[r] = exp_f32(-1.0 * x);
 }
 
 __global__ void k_xcc_probe(uint32_t* out, uint32_t n) {
@@ -3913,6 +3963,14 @@ hipError_t launch_knn_prefetch(const PrefetchArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_list_avg(const ListAvgArgs& a, hipStream_t s) {
+    if (a.i0 >= a.n) return hipSuccess;
+    if (a.k == 0 || a.k > (uint32_t)kMaxK) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_list_avg, dim3((a.n - a.i0 + kWave - 1) / kWave), dim3(kWave),
+                       kWave * (a.k | 1u) * sizeof(int32_t), s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_unpack(const UnpackArgs& a, hipStream_t s) {
     const uint32_t n = a.n > a.n_res ? a.n : a.n_res;
     if (n == 0) return hipSuccess;
@@ -4144,7 +4202,7 @@ hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t w
         return hipErrorInvalidValue;
     if (team == 8 && a.m > kMaxK) return hipErrorInvalidValue;  // eight random candidates per member
     // every item needs its neighbour list; test hooks are not supported
-    if (!a.pre_nbrs || a.item0 < a.pre_base || a.item0 + f.n > a.pre_end || a.ext_nbrs || a.ext_cands ||
+    if (!a.pre_nbrs || (team == 1 && !guided && !a.pre_avg) || a.item0 < a.pre_base || a.item0 + f.n > a.pre_end || a.ext_nbrs || a.ext_cands ||
         a.dbg_nbrs || a.dbg_best || a.knn_only || a.ext_full_cost || a.exact)
         return hipErrorInvalidValue;
     const uint32_t per = team == 1 ? kTicketItems : 1u, most = (f.n + per - 1) / per;

@@ -577,6 +577,7 @@ struct tsg_job {
         DBuf<uint32_t> cnt, n_at;
         DBuf<uint64_t> mend, mnew;  // resolved mask at the stage end; the stage's picks
         DBuf<uint32_t> tmin;        // per tile: least position of its picks
+        DBuf<double> avg;           // per item of an unguided wave run: mean distance of its neighbours
         DBuf<uint64_t> dep;         // per prefetched item: neighbours that are the stage's picks
         hipEvent_t ready = nullptr, done = nullptr;
         bool done_recorded = false;
@@ -1311,7 +1312,7 @@ int wait_picks(tsg_job* j, int t) {
 // stage, or (deep) one set per stage, and the mail and pick lists of the
 // stages run in dependency order.
 uint64_t ahead_set_bytes(const tsg_job* j, uint64_t S) {
-    return std::max<uint64_t>(1, S) * (j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size()) * 4 + j->prm.nearest_neighbors * 4 + 16) +
+    return std::max<uint64_t>(1, S) * (j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size()) * 4 + j->prm.nearest_neighbors * 4 + 24) +
            (uint64_t)j->tiles_x * j->tiles_y * 20;
 }
 uint64_t ahead_bytes(const tsg_job* j) { return 2 * ahead_set_bytes(j, stage_size(j, 0)) + j->N * 36; }
@@ -1329,6 +1330,8 @@ void ghost_margins(const tsg_job* j, Args* a) {
     a->yb = (int32_t)((float)j->H * 0.05f);
     a->yt = (int32_t)j->H - a->yb;
 }
+
+uint32_t flow_team_of(const tsg_job* j, uint64_t i0, uint64_t i1);
 
 // Prepares stage ahead_next on the side stream (see tsg_job::Ahead). The
 // counts follow the stage driver: a stage opens with `ahead_open` resolved
@@ -1367,6 +1370,7 @@ int ahead_stage(tsg_job* j) {
         HIP_TRY(A.nbrs.reserve(n * k));
         HIP_TRY(A.cnt.reserve(n));
         HIP_TRY(A.dep.reserve(n));
+        HIP_TRY(A.avg.reserve(n));
         HIP_TRY(A.mend.reserve(tiles));
         HIP_TRY(A.mnew.reserve(tiles));
         HIP_TRY(A.tmin.reserve(tiles));
@@ -1432,12 +1436,13 @@ int ahead_stage(tsg_job* j) {
     // (in dependency order, or deep: of every item; else the rest search in-kernel)
     std::vector<uint32_t> tab;  // bounds (nb + 1), then resolved counts (nb)
     std::vector<uint32_t> nres_b;
-    uint64_t i = 0, nres = n_open, w_end = 0;
+    uint64_t i = 0, nres = n_open, w_end = 0, wave0 = S_eff;  // wave0: first item of a wave run
     bool window = true;
     while (i < S_eff) {
         const uint64_t e = batch_end_at(j, t, i, nres, redo, S_eff);
         tab.push_back((uint32_t)i);
         nres_b.push_back((uint32_t)nres);
+        if (j->flow_on && wave0 == S_eff && flow_team_of(j, i, e) == 1) wave0 = i;
         if (window && e - i <= j->tune.prefetch_max) w_end = e;
         else window = false;
         if (e > redo_eff) nres += e - std::max(i, redo_eff);
@@ -1483,6 +1488,9 @@ int ahead_stage(tsg_job* j) {
             ghost_margins(j, &pa);
         }
         HIP_TRY(timed_launch_on(j, side, K_PREFETCH, pre_end, [&] { return launch_knn_prefetch(pa, side); }));
+        if (j->flow_on && !j->guided)
+            HIP_TRY(launch_list_avg({j->W, j->H, pa.work, A.nbrs.p, A.cnt.p, (uint32_t)wave0, (uint32_t)pre_end, k, A.avg.p},
+                                    side));
     }
     HIP_TRY(hipEventRecord(A.ready, side));
     A.stage = t;
@@ -1687,6 +1695,7 @@ int step_open_stage(tsg_job* j) {
         st.rc_hi = st.S_eff;
         a.pre_nbrs = j->aset(t).nbrs.p;
         a.pre_cnt = j->aset(t).cnt.p;
+        a.pre_avg = j->flow_on ? j->aset(t).avg.p : nullptr;
         a.pre_base = 0;
         a.pre_end = (uint32_t)j->aset(t).pre_end;
     }
@@ -2032,6 +2041,7 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
             HIP_TRY(A.mnew.reserve((size_t)j->tiles_x * j->tiles_y));
             HIP_TRY(A.tmin.reserve((size_t)j->tiles_x * j->tiles_y));
             HIP_TRY(A.dep.reserve(smax));
+            HIP_TRY(A.avg.reserve(smax));
             if (!A.ready) HIP_TRY(hipEventCreateWithFlags(&A.ready, hipEventDisableTiming));
         }
         j->ahead_open = j->n_res;
@@ -2242,7 +2252,7 @@ size_t job_footprint(const tsg_job* j) {
     b += j->rank.n * 4 + j->mend.n * 8 + j->tmin.n * 4 + j->pre_n.n * 4 + j->pre_cnt.n * 4 + j->pre_nbrs.n * 4;
     for (const tsg_job::Ahead& A : j->ahead)
         b += A.rc.n * 4 + A.nbrs.n * 4 + A.cnt.n * 4 + A.n_at.n * 4 + A.mend.n * 8 + A.mnew.n * 8 +
-             A.tmin.n * 4 + A.dep.n * 8;
+             A.tmin.n * 4 + A.dep.n * 8 + A.avg.n * 8;
     b += j->mail.n * 8 + j->flow_ticket.n * 4 + j->unres[0].n * 4 + j->unres[1].n * 4 + j->pick_idx.n * 4 +
          j->pick_link.n * 4 + j->pick_head.n * 4;
     b += j->state2.n * sizeof(uint4) + j->stamp.n * 4 + j->pend.n * 8;
@@ -2572,6 +2582,7 @@ hipError_t lane_reserve(tsg_job* j) {
         if (e == hipSuccess) e = A.nbrs.reserve(n * j->prm.nearest_neighbors);
         if (e == hipSuccess) e = A.cnt.reserve(n);
         if (e == hipSuccess) e = A.dep.reserve(n);
+        if (e == hipSuccess) e = A.avg.reserve(n);
         if (e == hipSuccess) e = A.mend.reserve(tiles);
         if (e == hipSuccess) e = A.mnew.reserve(tiles);
         if (e == hipSuccess) e = A.tmin.reserve(tiles);
@@ -2581,7 +2592,7 @@ hipError_t lane_reserve(tsg_job* j) {
 
 // Gives back what lane_reserve took (nothing of the job is in flight).
 void lane_release(tsg_job* j) {
-    for (tsg_job::Ahead& A : j->ahead) give_back(A.rc, A.nbrs, A.cnt, A.n_at, A.mend, A.mnew, A.tmin, A.dep);
+    for (tsg_job::Ahead& A : j->ahead) give_back(A.rc, A.nbrs, A.cnt, A.n_at, A.mend, A.mnew, A.tmin, A.dep, A.avg);
     give_back(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head, j->pick_moves);
 }
 
