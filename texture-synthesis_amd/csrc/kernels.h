@@ -126,7 +126,6 @@ struct PrefetchArgs {
     // earlier batch of the stage resolves (rank - locked, its position in the
     // work list, below the item's batch start); needs the batch table
     uint64_t* out_dep;            // [item - item0]
-    uint32_t per_wave;            // with the batch table: items of a wave (set by the launcher)
     // tiling mode (with the batch table): pixels of ranks from g_lo on carry
     // ghost copies within the edge margins (BatchArgs)
     uint32_t ghosts, g_lo;

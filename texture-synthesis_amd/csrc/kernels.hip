@@ -2764,9 +2764,13 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
         const uint32_t t = (uint32_t)(u * kWave + lane);
         o0[u] = t < a.offtab_n ? gld(a.offtab + t) : 0;
     }
-    const uint32_t first = a.item0 + (blockIdx.x * kWavesPerWG + (uint32_t)wave) * a.per_wave;
-    for (uint32_t q = 0; q < a.per_wave && first + q < a.item1; ++q) {
-        const uint32_t item = first + q, rel = item - a.item0;
+    // A wave's items lie a grid apart: the first items of a first stage search
+    // the longest (few pixels are resolved), and dealt out in runs they kept
+    // the first waves busy long after the others had ended (a 2048^2 job's
+    // runs wait for its first lists: 29.35 -> 28.8 ms on the device).
+    const uint32_t waves = gridDim.x * kWavesPerWG;
+    for (uint32_t item = a.item0 + blockIdx.x * kWavesPerWG + (uint32_t)wave; item < a.item1; item += waves) {
+        const uint32_t rel = item - a.item0;
         // the last batch starting at or before the item
         uint32_t lo = 0, len = a.nb;
         while (len > 1) {
@@ -3950,12 +3954,10 @@ hipError_t launch_knn_prefetch(const PrefetchArgs& a, hipStream_t s) {
     if (!a.n_at) {
         if (!a.bounds || !a.bnres || a.nb == 0 || !a.rank || !a.out_dep) return hipErrorInvalidValue;
         // one item per wave while that leaves waves of the chip (8192) idle
-        PrefetchArgs b = a;
-        b.per_wave = n / 8192u < 1u ? 1u : (n / 8192u > kListItems ? kListItems : n / 8192u);
-        const uint32_t per = kWavesPerWG * b.per_wave;
+        const uint32_t per = kWavesPerWG * (n / 8192u < 1u ? 1u : (n / 8192u > kListItems ? kListItems : n / 8192u));
         const dim3 grid((n + per - 1) / per), block(kWave * kWavesPerWG);
-        if (a.ghosts) hipLaunchKernelGGL(k_knn_lists<true>, grid, block, 0, s, b);
-        else hipLaunchKernelGGL(k_knn_lists<false>, grid, block, 0, s, b);
+        if (a.ghosts) hipLaunchKernelGGL(k_knn_lists<true>, grid, block, 0, s, a);
+        else hipLaunchKernelGGL(k_knn_lists<false>, grid, block, 0, s, a);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_knn_prefetch, dim3((n + kWavesPerWG - 1) / kWavesPerWG), dim3(kWave * kWavesPerWG),
