@@ -8,9 +8,8 @@ reference's criterion benches build outside the timer
 (lib/benches/all-the-things.rs:20-29), so inputs are resident in HBM.
 
 Prints one JSON line: Mpix/s of output, per-step latency p50/p99, the
-roofline of the dominant kernel (the throughput-bound batch launches:
-k_resolve_persist for single-wave items, k_resolve for teams) from the
-launches' device-clock spans in the timed steps, and the CPU oracle timed on
+roofline of the dominant kernel (k_flow_wave, a stage's larger batches) from
+the launches' device-clock spans in the timed steps, and the CPU oracle timed on
 the host's cores.
 
 Beside the main line: "guided" (4 x 300^2 examples with guides -> 1024^2)
@@ -18,7 +17,7 @@ and "plain_2048" (the plain path at 2048^2, with the job's device bytes).
 Two more legs report in the same line:
 * "batched": 256 independent syntheses (examples uniform in {64..512}^2,
   outputs uniform in {128..1024}^2, k in {20, 50}, m = 50, seeds 4000+j)
-  run together through the work-queue engine, against the same 256 run one
+  run together (Batch.run_all), against the same 256 run one
   after another; aggregate output Mpix/s of both with the outputs resident
   (as the main line), the download-inclusive rate apart, and whether every
   batched result equals its sequential twin bit for bit.
@@ -185,7 +184,7 @@ def batched_leg(ts, synth, n, sequential=True):
     alg = sum(sum(int((0.5 ** s_) * o * o) for s_ in range(6)) * (4 * k * (k + M) + 24 * k + 28)
               for _, o, k, _ in specs)
     t_kern = prof["launch_to_done_ms"] / 1e3
-    ec = counters_from_profiles("engine_c4_counters.md", "k_engine")
+    ec = counters_from_profiles("resolve_c2_counters.md", "k_flow_wave")
     return {
         "workload": f"{n} syntheses: examples uniform in {{64,128,256,512}}^2, outputs uniform in "
                     f"{{128,256,512,1024}}^2, k in {{20,50}}, m=50, seeds 4000+j",
@@ -199,13 +198,13 @@ def batched_leg(ts, synth, n, sequential=True):
         "identical_to_alone": (seq == got) if seq is not None else None,
         "launches": st["launches"], "engine_rounds": st["rounds"],
         "engine_workgroup_ms": {k: (round(v, 1) if isinstance(v, float) else v) for k, v in prof.items()},
-        "roofline": {"kernel": "k_engine<false>", "bound": "hbm", "algorithmic_bytes": alg,
+        "roofline": {"kernel": "k_flow_link + k_flow_team + k_flow_wave (whole runs, several at a time)", "bound": "hbm", "algorithmic_bytes": alg,
                      "achieved": round(alg / t_kern / 1e9, 1) if t_kern > 0 else None, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(alg / t_kern / 1e9 / HBM_PEAK_GBS, 4) if t_kern > 0 else None,
-                     "over": "launch to completion of the engine launches (host clock)",
-                     "traffic": (ec or {}).get("hbm_bytes"), "l2_hit": (ec or {}).get("l2_hit"),
+                     "over": "the batch's runs, first launch to the last run's end (host clock)",
+                     "traffic": None, "l2_hit": (ec or {}).get("l2_hit"),
                      "valu_busy": (ec or {}).get("valu_busy"), "waves_per_cu": (ec or {}).get("waves_per_cu"),
-                     "limiter": limiter(ec), "counters_from": "profiles/engine_c4_counters.md"},
+                     "limiter": limiter(ec), "counters_from": "profiles/resolve_c2_counters.md (k_flow_wave alone on the chip)"},
     }
 
 
@@ -338,8 +337,7 @@ def serving_leg(ts, synth, n, qps, budget_gib, quantum=None, rounds_per_pump=1):
 
 
 def traffic_from_profiles():
-    """HBM bytes per batch launch (k_resolve_persist and k_resolve) of this
-    workload, from the committed counter summary (FETCH_SIZE + WRITE_SIZE per
+    """HBM bytes per batch launch (k_resolve, with flow = 0) of this workload, from the committed counter summary (FETCH_SIZE + WRITE_SIZE per
     dispatch, copy-calibrated)."""
     import re
     path = os.path.join(ROOT, "profiles", "resolve_c2_traffic.md")
@@ -471,17 +469,16 @@ def main():
     # profiled run (separate, after the timed region): every kernel's device time
     g = prof.run()
     ks = g.kernel_stats
-    # the dominant kernel: one launch per batch of more than a few items
-    # (k_resolve_persist, or k_resolve for teams; the one-workgroup loop over
-    # the smallest batches is reported apart), over the timed steps; durations
-    # are the launches' device-clock spans
+    # the dominant kernel: a stage's larger batches, one launch per stage
+    # (k_flow_wave; the teams' launches for the smaller batches are reported
+    # apart), over the timed steps; durations are the launches' device-clock spans
     resolves = (res["items"] + ks["resolve_runs"]["items"] * args.steps) // args.steps
     kern_s = res["ms"] / 1e3
     achieved = res["items"] * BYTES_PER_RESOLVE / kern_s / 1e9 if kern_s > 0 else 0.0
     per_launch = res["items"] * BYTES_PER_RESOLVE / max(1, res["launches"])
     ms_per_step = t_all * 1e3 / args.steps
     value = 1024 * 1024 * args.steps / t_all / 1e6
-    rc_ctr = counters_from_profiles("resolve_c2_counters.md", "k_resolve")
+    rc_ctr = counters_from_profiles("resolve_c2_counters.md", "k_flow_wave")
     lat_sorted = sorted(lat)
     p99 = lat_sorted[min(len(lat_sorted) - 1, int(round(0.99 * (len(lat_sorted) - 1))))]
     out = {
@@ -508,11 +505,13 @@ def main():
                            "note": "the same steps with the output image, coordinate and id maps and the "
                                    "resolved list downloaded to host memory"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_from_profiles(),
+                     "frac": round(achieved / HBM_PEAK_GBS, 4),
+                     # (algorithmic bytes: exact pruning skips most of them, and caches serve most of the rest)
+                     "traffic": (rc_ctr or {}).get("hbm_bytes") or traffic_from_profiles(),
                      "l2_hit": (rc_ctr or {}).get("l2_hit"), "lds_bank_conflict": (rc_ctr or {}).get("lds_bank_conflict"),
                      "valu_busy": (rc_ctr or {}).get("valu_busy"), "waves_per_cu": (rc_ctr or {}).get("waves_per_cu"),
                      "limiter": limiter(rc_ctr), "counters_from": "profiles/resolve_c2_counters.md",
-                     "kernel": "k_resolve_persist + k_resolve", "bytes_per_resolve": BYTES_PER_RESOLVE,
+                     "kernel": "k_flow_wave", "bytes_per_resolve": BYTES_PER_RESOLVE,
                      "algorithmic_bytes_per_launch": round(per_launch),
                      "avg_launch_ms": round(res["ms"] / max(1, res["launches"]), 4),
                      "launches": res["launches"], "over": "the timed steps"},

@@ -4187,10 +4187,11 @@ uint32_t flow_max_wgs(uint32_t team, bool guided) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k.fn, (int)k.threads, k.lds) != hipSuccess)
         return 0;
-    // A team run is bound by its chain, not by its waves: 16 waves per CU leave
-    // the second stream room to prepare the later stages meanwhile. (With the
-    // 24 that fit an unguided run, its kernels waited for the run's end:
-    // 2.4 ms of a 1024^2 job's first stage.)
+    // A team run is bound by its chain, not by its waves: at most 16 waves per
+    // CU (the registers of k_flow_link and k_flow_team hold no more). Fewer
+    // leave the second stream room to prepare the later stages meanwhile, but
+    // what that gains the run loses (256^2: 512 workgroups 3.62 ms, 384 4.4,
+    // 256 5.4).
     if (team > 1) per_cu = per_cu < (int)(16u / team) ? per_cu : (int)(16u / team);
     return (uint32_t)(per_cu * cus);
 }
