@@ -49,3 +49,19 @@ def test_inpaint_start(ctx, n, flow):
     gen, job = run_pair([synth.example(70, w, h)], w, h, seed=2, inpaint_mask=mask, inpaint_index=0, sample_kind=[2],
                         sample_masks=[mask], backtrack_stages=3, tuning=dict(flow=flow), **kw)
     assert_same(gen, job)
+
+
+# pixel counts that are not whole words of the mask; a mask larger than its example
+@pytest.mark.parametrize("w,h", [(33, 29), (1, 50), (64, 33)])
+def test_sample_masks(ctx, w, h):
+    ex = synth.example(80, w, h)
+    rng = np.random.default_rng(w)
+    big = np.zeros((h + 3, w + 5, 4), np.uint8)
+    big[:, :, 0] = (rng.random((h + 3, w + 5)) < 0.3) * rng.integers(1, 256, (h + 3, w + 5))
+    mask = np.ascontiguousarray(big[:h, :w])
+    kw = dict(seed=6, sample_kind=[2], backtrack_stages=0, nearest_neighbors=9, random_sample_locations=7)
+    gen, job = run_pair([ex], 40, 31, sample_masks=[mask], **kw)
+    assert_same(gen, job)
+    b = ts.Session.builder().seed(6).backtrack_stages(0).nearest_neighbors(9).random_sample_locations(7)
+    got = b.add_example(ts.Example(ex).set_sample_method(big)).output_size(ts.Dims(40, 31)).build().run()
+    assert np.array_equal(got.image, gen.image) and np.array_equal(got.coord, gen.coord)

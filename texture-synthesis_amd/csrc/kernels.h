@@ -207,6 +207,9 @@ struct PickArgs {
 };
 hipError_t launch_picks(const PickArgs& a, hipStream_t s);
 
+// Sample mask of a w x h example: 1 where the red byte of src (rows of src_w pixels) is not 0.
+hipError_t launch_sample_mask(const uint32_t* src, uint32_t src_w, uint32_t w, uint32_t h, uint8_t* mask, hipStream_t s);
+
 // The u[i] = i list of n entries, but u[moves[q].x] = moves[q].y.
 hipError_t launch_list(uint32_t* u, uint32_t n, const uint2* moves, uint32_t n_moves, hipStream_t s);
 

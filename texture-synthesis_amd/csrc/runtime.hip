@@ -1059,10 +1059,13 @@ int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_m
     j->unres_moves.clear();
     size_t kept = 0, L = N;
     if (j->inpaint) {
-        std::vector<uint32_t> rl(N);
-        j->unresolved.resize(N);
-        uint32_t* u = j->unresolved.data();
+        // (one more entry than each list holds: the writes have no branch)
         size_t nu = 0;
+        for (size_t i = 0; i < N; ++i) nu += inpaint_mask->rgba[i * 4] < 255;
+        std::unique_ptr<uint32_t[]> rl(new uint32_t[N - nu + 1]);
+        j->unresolved.resize(nu + 1);
+        uint32_t* u = j->unresolved.data();
+        nu = 0;
         for (size_t i = 0; i < N; ++i) {
             const bool open = inpaint_mask->rgba[i * 4] < 255;
             u[nu] = (uint32_t)i;
@@ -1073,7 +1076,7 @@ int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_m
         j->unresolved.resize(nu);
         L = nu;
         if (kept) {
-            HIP_TRY(up.upload(j->rlist.p, rl.data(), kept * 4, s));
+            HIP_TRY(up.upload(j->rlist.p, rl.get(), kept * 4, s));
             HIP_TRY(launch_init_kept(ia, j->rlist.p, (uint32_t)kept, j->inpaint_index, s));
         }
     }
@@ -3222,6 +3225,7 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
     // is its own guide map matched to the target's histogram
     const bool style = target_guide && !example_guides;
     std::vector<Pyramid> pyr;
+    std::vector<std::unique_ptr<DBuf<uint32_t>>> mask_px;  // masks as given, until the build ends
     const uint32_t top = j->levels - 1;  // the finest level, which is the input
     for (uint32_t i = 0; i < n_examples; ++i) {
         const tsg_image& im = examples[i];
@@ -3236,18 +3240,19 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
         std::unique_ptr<DBuf<uint8_t>> mk(new DBuf<uint8_t>());
         if (j->kind[i] == TSG_SAMPLE_IMAGE) {
             const tsg_image& sm = sample_masks[i];
-            std::vector<uint8_t> v((size_t)im.w * im.h);
-            size_t valid = 0;
-            for (uint32_t y = 0; y < im.h; ++y)
-                for (uint32_t x = 0; x < im.w; ++x) {
-                    uint8_t r = sm.rgba[((size_t)y * sm.w + x) * 4];
-                    v[(size_t)y * im.w + x] = r != 0;
-                    valid += r != 0;
-                }
-            if (valid == 0)
+            auto admits = [&] {
+                for (uint32_t y = 0; y < im.h; ++y)
+                    for (uint32_t x = 0; x < im.w; ++x)
+                        if (sm.rgba[((size_t)y * sm.w + x) * 4]) return true;
+                return false;
+            };
+            if (!admits())
                 return fail(TSG_ERR_SAMPLING, "sample mask admits no pixel (the reference loops forever)");
-            HIP_TRY(mk->alloc(v.size()));
-            HIP_TRY(up.upload(mk->p, v.data(), v.size(), s));
+            HIP_TRY(mk->alloc(npx));
+            mask_px.emplace_back(new DBuf<uint32_t>());
+            HIP_TRY(mask_px.back()->alloc((size_t)sm.w * im.h));
+            HIP_TRY(up.upload(mask_px.back()->p, sm.rgba, (size_t)sm.w * im.h * 4, s));
+            HIP_TRY(launch_sample_mask(mask_px.back()->p, sm.w, im.w, im.h, mk->p, s));
         }
         j->smask.push_back(std::move(mk));
         if (j->guided) {
@@ -3332,6 +3337,7 @@ int tsg_job_create(tsg_ctx* ctx, const tsg_params* prm, uint32_t n_examples, con
     if ((rc = init_state(j.get(), examples, inpaint_mask))) return rc;
     j->state_ready = true;
     HIP_TRY(hipStreamSynchronize(s));
+    for (auto& m : mask_px) give_back(*m);
     {
         // a launch structure the autotuner stored for this shape (ctx->mu is held)
         auto it = ctx->tunings.find(tuning_key(j.get()));
@@ -3641,7 +3647,7 @@ int tsg_resize(tsg_ctx* ctx, const tsg_image* img, uint32_t nw, uint32_t nh, int
     HIP_TRY(ctx->staging.upload(src.p, img->rgba, n_in * 4, ctx->stream));
     int rc = resize_all(ctx, {{Resize{src.p, img->w, img->h, dst.p, nw, nh, f}}});
     if (rc) return rc;
-    HIP_TRY(hipMemcpy(out, dst.p, n_out * 4, hipMemcpyDeviceToHost));
+    if ((rc = copy_out(ctx, ctx->stream, {{out, dst.p, n_out * 4}}))) return rc;
     give_back(src, dst);
     return TSG_OK;
 }
