@@ -1183,7 +1183,13 @@ enum { K_RESOLVE = 0, K_COMMIT = 1, K_RAND = 2, K_RECOLOR = 3, K_STATS = 4, K_PR
 constexpr int kKinds = 7;
 constexpr size_t kEngineRcBudget = 4u << 20;  // random-candidate chunk of a job under the engine
 constexpr uint64_t kPrefetchCap = 65536;       // items per prefetched kNN window
-constexpr uint32_t kFlowSpin = 1u << 18;       // polls of one dependency wait before a run gives up
+// Polls (0.5 us each and more) of one dependency wait before its run gives up.
+// A wait legitimately lasts as long as the items handed out before its own take
+// one after another: at most three for each of 8192 waves, at up to 1 us a
+// candidate (the unpruned rule's). On top of that 10 s, for a chip shared with
+// others. A fixed 2^18 polls ended runs that were only slow: 256^2 with 4096
+// random candidates and a wave per item.
+uint32_t flow_spin(uint64_t m) { return (uint32_t)(2 * (10000000 + 3 * 8192 * (m + kMaxK))); }
 // Jobs of a batch that run at the same time, and the part of the chip's
 // resident workgroups (one in kLaneShare) that a launch of theirs may take.
 // HIP serves streams from four hardware queues, so five streams keep three or
@@ -1967,8 +1973,8 @@ int flow_stage(tsg_job* j, Progress& pr) {
             j->flow_launches = 0;
         }
         const uint32_t n = (uint32_t)(i1 - i0);
-        const FlowArgs f{j->flow_ticket.p + j->flow_launches++, n, j->aset(st.t).dep.p, j->mail.p, j->flow_tag, kFlowSpin,
-                         j->overflow.p};
+        const FlowArgs f{j->flow_ticket.p + j->flow_launches++, n, j->aset(st.t).dep.p, j->mail.p, j->flow_tag,
+                         flow_spin(j->prm.random_sample_locations), j->overflow.p};
         a.item0 = (uint32_t)i0;
         a.item1 = (uint32_t)i1;
         HIP_TRY(timed_launch(j, team == 1 ? K_RESOLVE : K_RUN, n,
