@@ -477,8 +477,9 @@ hipError_t launch_resolve_small(const BatchArgs& a, const uint32_t* bounds, cons
                                 uint32_t n_batches, bool guided, hipStream_t s);
 hipError_t launch_resolve(const BatchArgs& a, bool guided, hipStream_t s);
 // A dependency-ordered run (FlowArgs) with `team` waves per item (1, 2, 4 or
-// 8) on at most wgs persistent workgroups. flow_max_wgs: as many as are resident.
-uint32_t flow_max_wgs(uint32_t team, bool guided);
+// 8) on at most wgs persistent workgroups. flow_max_wgs: as many as are
+// resident, of the kernel for m random candidates.
+uint32_t flow_max_wgs(uint32_t team, uint32_t m, bool guided);
 hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t wgs, uint32_t team, bool guided,
                                hipStream_t s);
 hipError_t launch_stage_end(const StageEndArgs& a, hipStream_t s);

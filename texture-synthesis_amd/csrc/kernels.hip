@@ -2692,6 +2692,138 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
     launch_span(a, t_start);
 }
 
+// What the members of a slice team share of one item (two in turn, as
+// TeamLds).
+struct SliceLds {
+    uint4 rec[kMaxK];                      // the neighbours' records
+    unsigned long long best[kWavesPerWG];  // per member: least (cost bits << 32 | candidate index)
+    unsigned long long bound;              // least of any member so far
+    uint32_t next;                         // the workgroup's next item
+};
+
+// A run with a team of waves per item (the workgroup) and more than kMaxK
+// random candidates: their terms, not the link's steps, are what an item's time
+// goes to, so each member evaluates its slice with exact pruning, as a wave run
+// does, and the members share the least cost so far. The records go to the
+// members through LDS, the weights from the last member, which forms them while
+// the first one waits. Evaluated in full by k_flow_team, many candidates took
+// longer than with a launch per batch and pruning. Device time of a 256^2 run,
+// ms, a launch per batch / k_flow_team / this (first chunks of 64 neighbours; of
+// 8; growing): m = 65 10.1 / 6.6 / 5.7 (6.5; 7.0), 128 11.2 / 8.4 / 6.5 (7.4;
+// 7.9), 512 18.6 / 26.1 / 12.2 (13.0; 13.5), 4096 79 / 196 / 55 (59; 62);
+// guided 300^2 at m = 512 32 / 53 / 27. Teams of four alone: 256^2 at m = 65
+// 6.1, 512 16.2.
+template <bool GUIDED>
+__global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(4))) void k_flow_slice(BatchArgs a,
+                                                                                                           FlowArgs f) {
+    const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ MapDesc smaps[kMapCache];
+    __shared__ SliceLds team[2];
+    flow_args(a);
+    float *lut, *glut;
+    const MapDesc* maps;
+    if (threadIdx.x == 0) team[0].next = atomicAdd(f.ticket, 1u);
+    WaveLds* wls = setup_lds<GUIDED>(a, smem, lut, glut, smaps, maps);  // ends with a barrier
+    const int T = __builtin_amdgcn_readfirstlane((int)(blockDim.x / kWave));
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x % kWave;
+    WaveLds *L = wls + wave, *last = wls + (T - 1);
+    const uint32_t rper = (a.m + (uint32_t)T - 1) / (uint32_t)T;
+    const uint32_t r0 = min(a.m, (uint32_t)wave * rper), nrs = min(a.m, r0 + rper) - r0;
+    uint32_t idx = uniform(team[0].next);
+    for (uint32_t turn = 0; idx < f.n; turn ^= 1u) {
+        SliceLds* S = &team[turn];
+        const uint32_t item = a.item0 + idx, rel = item - a.pre_base;
+        uint32_t next = 0;  // the ticket is on its way while the item waits
+        if (wave == 0) {
+            phase_clock(a, item, 0, lane);
+            if (lane == 0) next = atomicAdd(f.ticket, 1u);
+        }
+        const uint32_t flat = uniform(gld(a.work + item));
+        const uint32_t kf = uniform(gld(a.pre_cnt + rel));
+        const bool has = lane < (int)kf;
+        int32_t o = 0;
+        if (has) o = gld(a.pre_nbrs + (size_t)rel * a.k + lane);
+        uint2 rpre = make_uint2(0, 0);
+        if ((uint32_t)lane < nrs) rpre = rand_cand(a, item, r0 + (uint32_t)lane);
+        const int x = (int)(flat % a.W), y = (int)(flat / a.W);
+        uint4 r = make_uint4(0, 0, 0, 0);
+        bool post = false;  // in lane 0: r is the item's result
+        if (kf == 0) {
+            // no resolved neighbour: alike for every member
+            if (wave == 0) {
+                r = item_at_random(a, maps, item, 0, flat, lane);
+                post = lane == 0;
+                if (lane == 0) team[turn ^ 1u].next = next;
+            }
+            __syncthreads();
+        } else {
+            if (has) L->nd[lane] = o;
+            wave_sync();
+            if (wave == T - 1) item_geometry(a, x, y, kf, L, lane);
+            if (wave == 0) {
+                const uint4 st = flow_records(f, a, f.dep[rel], has ? nbr_flat(a, x, y, o) : 0u, has, lane);
+                phase_clock(a, item, 1, lane);
+                if (has) S->rec[lane] = st;
+                if (lane == 0) {
+                    S->bound = ~0ull;
+                    team[turn ^ 1u].next = next;
+                }
+            }
+            __syncthreads();
+            const double avg = last->avg;
+            if (has && wave != T - 1) L->w[lane] = last->w[lane];
+            const uint4 st = S->rec[has ? lane : 0];
+            uint32_t cxy, cms;
+            uint64_t uniq;
+            const uint32_t n_coh = item_neighbours<GUIDED>(a, maps, item, 0, x, y, kf, 0, L, lane, true, cxy, cms, uniq,
+                                                           &st);
+            if (wave == 0) phase_clock(a, item, 2, lane);
+            if (!a.lut_nan && avg > 0.0) {
+                const Best b = eval_slice<GUIDED, 6>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, r0, nrs, rpre, wave,
+                                                     T, wave == 0, L, lut, glut, lane % lut_copies<GUIDED>(), lane,
+                                                     &S->bound);
+                const bool have = b.Bi != kNone;
+                const unsigned long long mine =
+                    have ? (unsigned long long)__float_as_uint(b.B) << 32 | b.Bi : ~0ull;
+                if (lane == 0) S->best[wave] = mine;
+                if (wave == 0) phase_clock(a, item, 4, lane);
+                __syncthreads();
+                if (wave == 0) phase_clock(a, item, 5, lane);
+                const bool beaten = lane < T && S->best[lane < T ? lane : 0] < mine;
+                // without a cost below the search's start value the list's
+                // first candidate stays (find_best_match, ms.rs:1184-1224)
+                if (__ballot(beaten) == 0ull && (have || wave == 0)) {
+                    const uint2 xm = make_uint2(b.xy, b.ms);
+                    r = item_winner(a, maps, item, 0, n_coh, L, have ? b.B : FLT_MAX, have ? b.Bi : 0u, lane,
+                                    have ? &xm : nullptr);
+                    post = lane == 0;
+                }
+            } else {
+                if (wave == 0) {
+                    float best = FLT_MAX;
+                    uint32_t bidx = 0;
+                    item_exact<GUIDED>(a, maps, item, 0, kf, n_coh, n_coh + a.m, L, lut, glut,
+                                       lane % lut_copies<GUIDED>(), lane, best, bidx);
+                    r = item_winner(a, maps, item, 0, n_coh, L, best, bidx, lane);
+                    post = lane == 0;
+                }
+                __syncthreads();
+            }
+        }
+        if (post) {
+            // Generator::update (ms.rs:334-377), posted; a new pixel keeps its first score
+            const MapDesc& md = maps[r.y & 0xffffu];
+            mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
+            if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+        }
+        if (wave == 0) phase_clock(a, item, 6, lane);
+        idx = uniform(team[turn ^ 1u].next);
+    }
+    launch_span(a, t_start);
+}
+
 // Neighbour lists of items [item0, item1) ahead of their batches, one
 // wavefront per item (the resolve kernels read them instead of searching).
 __device__ __forceinline__ KnnView list_view(const PrefetchArgs& a, uint32_t item, uint32_t n_at) {
@@ -3905,7 +4037,12 @@ FlowKernel team_kernel(bool guided, bool one) {
                    : (one ? k_flow_team<false, T, true> : k_flow_team<false, T, false>),
             kWave * T, 256 * team_copies<false, T>() * sizeof(float) + T * kTeamWaveLds};
 }
-bool flow_kernel(uint32_t team, bool guided, bool one, FlowKernel* k) {
+bool flow_kernel(uint32_t team, uint32_t m, bool guided, bool one, FlowKernel* k) {
+    if (m > (uint32_t)kMaxK && (team == 2 || team == 4 || team == 8)) {
+        *k = {guided ? k_flow_slice<true> : k_flow_slice<false>, kWave * team,
+              lut_bytes(guided) + team * sizeof(WaveLds)};
+        return true;
+    }
     switch (team) {
         case 1:
             *k = {guided ? k_flow_wave<true> : k_flow_wave<false>, (uint32_t)(kWave * kWavesPerWG),
@@ -3950,14 +4087,15 @@ hipError_t configure_kernels() {
     e = hipFuncSetAttribute((const void*)k_resolve_coop<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)resolve_small_lds_bytes(false));
     if (e != hipSuccess) return e;
-    for (uint32_t team : {1u, 2u, 4u, 8u})
-        for (bool guided : {false, true})
-            for (bool one : {false, true}) {
-                FlowKernel k;
-                if (!flow_kernel(team, guided, one, &k)) return hipErrorInvalidValue;
-                e = hipFuncSetAttribute((const void*)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
-                if (e != hipSuccess) return e;
-            }
+    for (uint32_t team : {1u, 2u, 4u, 8u})  // (of one kernel, the largest team's bytes last)
+        for (uint32_t m : {1u, kMaxK + 1u})
+            for (bool guided : {false, true})
+                for (bool one : {false, true}) {
+                    FlowKernel k;
+                    if (!flow_kernel(team, m, guided, one, &k)) return hipErrorInvalidValue;
+                    e = hipFuncSetAttribute((const void*)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
+                    if (e != hipSuccess) return e;
+                }
     return hipFuncSetAttribute((const void*)k_resolve_small<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)resolve_small_lds_bytes(false));
 }
@@ -4194,9 +4332,9 @@ hipError_t launch_resolve_persist(const BatchArgs& a, uint32_t wgs, bool guided,
     return hipGetLastError();
 }
 
-uint32_t flow_max_wgs(uint32_t team, bool guided) {
+uint32_t flow_max_wgs(uint32_t team, uint32_t m, bool guided) {
     FlowKernel k;
-    if (!flow_kernel(team, guided, false, &k)) return 0;
+    if (!flow_kernel(team, m, guided, false, &k)) return 0;
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
@@ -4215,10 +4353,9 @@ hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t w
                                hipStream_t s) {
     if (f.n == 0) return hipSuccess;
     FlowKernel k;
-    if (!flow_kernel(team, guided, a.n_maps == 1, &k)) return hipErrorInvalidValue;
+    if (!flow_kernel(team, a.m, guided, a.n_maps == 1, &k)) return hipErrorInvalidValue;
     if (wgs == 0 || !f.ticket || !f.dep || !f.mail || !f.overflow || f.tag == 0 || f.tag > 255 || f.spin_limit == 0)
         return hipErrorInvalidValue;
-    if (team == 8 && a.m > kMaxK) return hipErrorInvalidValue;  // eight random candidates per member
     // every item needs its neighbour list; test hooks are not supported
     if (!a.pre_nbrs || (team == 1 && !guided && !a.pre_avg) || a.item0 < a.pre_base || a.item0 + f.n > a.pre_end || a.ext_nbrs || a.ext_cands ||
         a.dbg_nbrs || a.dbg_best || a.knn_only || a.ext_full_cost || a.exact)

@@ -1932,10 +1932,7 @@ struct Progress {
 uint32_t flow_team_of(const tsg_job* j, uint64_t i0, uint64_t i1) {
     const tsg_tuning& u = j->tune;
     if (i1 - i0 > (j->share > 1 ? std::min<uint64_t>(u.prefetch_max, kLaneTeamMax) : u.prefetch_max)) return 1;
-    const uint32_t team =
-        i0 < u.flow_head ? u.flow_head_team : std::max(u.flow_team, team_for(i1 - i0, u.team_max, u.team_waves));
-    // the eight-wave kernel holds 64 random candidates
-    return team == 8 && j->prm.random_sample_locations > kMaxK ? 4u : team;
+    return i0 < u.flow_head ? u.flow_head_team : std::max(u.flow_team, team_for(i1 - i0, u.team_max, u.team_waves));
 }
 
 // The open stage in dependency order (k_flow_team, k_flow_wave): consecutive
@@ -1966,7 +1963,7 @@ int flow_stage(tsg_job* j, Progress& pr) {
             i1 = b1;
             if ((due = pr.due(j, i1))) break;
         }
-        const uint32_t most = std::max(1u, flow_max_wgs(team, j->guided) / j->share);
+        const uint32_t most = std::max(1u, flow_max_wgs(team, a.m, j->guided) / j->share);
         const uint32_t wgs = j->tune.flow_wgs ? std::min(j->tune.flow_wgs, most) : most;
         if (j->flow_launches == kFlowTickets) {
             HIP_TRY(hipMemsetAsync(j->flow_ticket.p, 0, kFlowTickets * 4, s));
