@@ -645,8 +645,9 @@ struct tsg_job {
     uint32_t flow_tag = 0, flow_launches = 0;
     size_t small_used = 0;
     DBuf<uint2> pick_moves;         // entries of the list that are not their own index
-    // host bookkeeping. The unresolved list before the first stage: of an
-    // inpainting in `unresolved`, else entry i is pixel i but for unres_moves
+    // host bookkeeping. The unresolved list before the first stage: in
+    // `unresolved` (listed), else entry i is pixel i but for unres_moves
+    bool listed = false;
     std::vector<uint32_t> unresolved;
     std::unordered_map<uint32_t, uint32_t> unres_moves;
     size_t n_res = 0, locked = 0, N0 = 0;
@@ -1081,15 +1082,26 @@ int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_m
         }
     }
     j->locked = kept;
+    // An inpainting has its list. Else, for up to one point in kListShare
+    // pixels, the entries that the points move are held in a map: a list costs
+    // what filling and uploading it costs, a map some 0.1 us a point, which
+    // grows with it (CPU, 2^20 pixels: 4096 points 0.35 ms against 0.8, 8192
+    // 0.83 against 0.8, 65536 9.7 against 1.8; 2^22: 32768 3.8 against 3.9).
+    constexpr uint64_t kListShare = 128;
+    j->listed = j->inpaint || (j->prm.random_init != UINT64_MAX && j->prm.random_init > N / kListShare);
+    if (j->listed && !j->inpaint) {
+        j->unresolved.resize(N);
+        for (size_t i = 0; i < N; ++i) j->unresolved[i] = (uint32_t)i;
+    }
     if (j->prm.random_init != UINT64_MAX) {
-        // the swap_remove chain on the list, or (every pixel in order) on the entries it moved
+        // the swap_remove chain on the list, or on the entries it moved
         std::vector<InitPoint> pts;
         for (uint64_t i = 0; i < j->prm.random_init && L > 0; ++i) {
             Pcg32 g = Pcg32::seed_from_u64(j->prm.seed + i);
             const uint32_t k = (uint32_t)range_u64(g, 0, L);
             --L;
             uint32_t f;
-            if (j->inpaint) {
+            if (j->listed) {
                 f = j->unresolved[k];
                 j->unresolved[k] = j->unresolved[L];
             } else {
@@ -1105,7 +1117,7 @@ int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_m
             const uint32_t c = pack_px(examples[m].rgba + ((size_t)y * j->ex_dims[m].first + x) * 4);
             pts.push_back(InitPoint{f, c, x | (y << 16), m | (m << 16)});
         }
-        if (j->inpaint) j->unresolved.resize(L);
+        if (j->listed) j->unresolved.resize(L);
         j->locked += j->prm.random_init;
         if (j->locked > kept + pts.size())
             return fail(TSG_ERR_INVALID_ARGUMENT, "random_init exceeds the pixels to resolve");
@@ -1131,7 +1143,7 @@ int init_state(tsg_job* j, const tsg_image* examples, const tsg_image* inpaint_m
 
 // The unresolved list on the host, for runs whose pick orders the host computes.
 void host_unresolved(tsg_job* j) {
-    if (j->inpaint) return;  // held from the start
+    if (j->listed) return;  // held from the start
     j->unresolved.resize(j->N0);
     for (size_t i = 0; i < j->N0; ++i) j->unresolved[i] = (uint32_t)i;
     for (const auto& mv : j->unres_moves) j->unresolved[mv.first] = mv.second;
@@ -1141,11 +1153,11 @@ void host_unresolved(tsg_job* j) {
 int picks_begin(tsg_job* j) {
     j->pick_left = j->N0;
     j->pick_list = nullptr;
-    if (j->inpaint || !j->unres_moves.empty()) {
+    if (j->listed || !j->unres_moves.empty()) {
         // not every pixel in order
         hipStream_t s = j->stream;
         HIP_TRY(j->unres[0].reserve(std::max<size_t>(1, j->N0)));
-        if (j->inpaint) {
+        if (j->listed) {
             HIP_TRY(j->stg->upload(j->unres[0].p, j->unresolved.data(), j->N0 * 4, s));
         } else {
             std::vector<uint2> mv;
