@@ -355,9 +355,13 @@ int tsg_debug_fail_allocs(int64_t count);
  * [i0, i0 + n), n <= 2^28: t = ((i * 0x9E3779B97F4A7C15) mod 2^64 >> 11) *
  * 2^-53, x_i = 8 t when i % 4 != 0, else 8 + 56 t (f64, no contraction).
  * Test hook for comparing with the host C library's exp, as the reference
- * calls it. tsg_debug_exp_sweep_host computes the same on the host. */
+ * calls it. tsg_debug_exp_sweep_host computes the same on the host; the f32
+ * forms do so by the exp of the unguided wave runs, in plain double arithmetic
+ * where that decides the float. */
 int tsg_debug_exp_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, float* out);
 int tsg_debug_exp_sweep_host(uint64_t i0, uint64_t n, float* out);
+int tsg_debug_exp_f32_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, float* out);
+int tsg_debug_exp_f32_sweep_host(uint64_t i0, uint64_t n, float* out);
 
 /* ImagePyramid::new(img, Some(levels)) on the device: writes max(levels,1)
  * full-size RGBA8 levels, coarsest first (img_pyramid.rs:20-37). */

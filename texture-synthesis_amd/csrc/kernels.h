@@ -444,8 +444,9 @@ struct QEngineArgs {
 // Workgroups of the engine launch resident on the device at once.
 uint32_t engine_max_wgs(bool guided);
 hipError_t launch_engine(const QEngineArgs& e, const BatchArgs* args, uint32_t wgs, bool guided, hipStream_t s);
-// (float)exp(-x_i) for the sweep arguments x_i, i in [i0, i0 + n) (test hook).
-hipError_t launch_exp_sweep(uint64_t i0, uint64_t n, float* out, hipStream_t s);
+// (float)exp(-x_i) by exp_dd, or (plain) by exp_f32, for the sweep arguments
+// x_i, i in [i0, i0 + n) (test hook).
+hipError_t launch_exp_sweep(uint64_t i0, uint64_t n, bool plain, float* out, hipStream_t s);
 // XCD of each of n workgroups of a probe launch (test hook: the engine's
 // job placement relies on the hardware XCC id).
 hipError_t launch_xcc_probe(uint32_t* out, uint32_t n, hipStream_t s);

@@ -3686,18 +3686,20 @@ __device__ __forceinline__ void unit_publish(bool spread) {
     if (spread) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
 }
 
-// Weight-exp sweep (test hook): out[i - i0] = exp_f32(-1.0 * x_i), the
-// expression of the neighbour weights in item_geometry, for the arguments
-// x_i = t * 8 when i % 4 != 0, else 8 + t * 56, with t = ((i * 0x9E3779B97F4A7C15)
-// >> 11) * 2^-53 in [0, 1): three quarters of the arguments in [0, 8), where
-// d / mean lies for real neighbour sets, the rest up to 64.
+// Weight-exp sweep (test hook): out[i - i0] = (float)exp_dd(-1.0 * x_i), the
+// expression of the neighbour weights in item_geometry, or (PLAIN) exp_f32(-1.0
+// * x_i), that of item_weights, for the arguments x_i = t * 8 when i % 4 != 0,
+// else 8 + t * 56, with t = ((i * 0x9E3779B97F4A7C15) >> 11) * 2^-53 in [0, 1):
+// three quarters of the arguments in [0, 8), where d / mean lies for real
+// neighbour sets, the rest up to 64.
+template <bool PLAIN>
 __global__ void k_exp_sweep(uint64_t i0, uint64_t n, float* out) {
     const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const uint64_t i = i0 + r;
     const double t = (double)((i * 0x9E3779B97F4A7C15ull) >> 11) * 0x1p-53;
     const double x = (i & 3u) ? t * 8.0 : __dadd_rn(8.0, __dmul_rn(t, 56.0));
-    out[r] = exp_f32(-1.0 * x);
+    out[r] = PLAIN ? exp_f32(-1.0 * x) : (float)exp_dd(-1.0 * x);
 }
 
 __global__ void k_xcc_probe(uint32_t* out, uint32_t n) {
@@ -4226,9 +4228,11 @@ hipError_t launch_engine(const QEngineArgs& e, const BatchArgs* args, uint32_t w
     return hipGetLastError();
 }
 
-hipError_t launch_exp_sweep(uint64_t i0, uint64_t n, float* out, hipStream_t s) {
+hipError_t launch_exp_sweep(uint64_t i0, uint64_t n, bool plain, float* out, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_exp_sweep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, i0, n, out);
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (plain) hipLaunchKernelGGL(k_exp_sweep<true>, grid, dim3(256), 0, s, i0, n, out);
+    else hipLaunchKernelGGL(k_exp_sweep<false>, grid, dim3(256), 0, s, i0, n, out);
     return hipGetLastError();
 }
 

@@ -4088,7 +4088,8 @@ int tsg_batch_submit(tsg_batch* b, tsg_job* job, uint64_t* ticket) {
     return TSG_OK;
 }
 
-int tsg_debug_exp_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, float* out) {
+namespace {
+int exp_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, bool plain, float* out) {
     if (!ctx || (!out && n)) return fail(TSG_ERR_INVALID_ARGUMENT, "null argument");
     if (n > (1ull << 28)) return fail(TSG_ERR_INVALID_ARGUMENT, "at most 2^28 values per call");
     if (n == 0) return TSG_OK;
@@ -4096,22 +4097,28 @@ int tsg_debug_exp_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, float* out) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     DBuf<float> d;
     HIP_TRY(d.alloc(n));
-    HIP_TRY(launch_exp_sweep(i0, n, d.p, ctx->stream));
+    HIP_TRY(launch_exp_sweep(i0, n, plain, d.p, ctx->stream));
     HIP_TRY(hipMemcpyAsync(out, d.p, n * 4, hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return TSG_OK;
 }
 
-int tsg_debug_exp_sweep_host(uint64_t i0, uint64_t n, float* out) {
+int exp_sweep_host(uint64_t i0, uint64_t n, bool plain, float* out) {
     if (!out && n) return fail(TSG_ERR_INVALID_ARGUMENT, "null argument");
     for (uint64_t r = 0; r < n; ++r) {
         const uint64_t i = i0 + r;
         const double t = (double)((i * 0x9E3779B97F4A7C15ull) >> 11) * 0x1p-53;
         const double x = (i & 3u) ? t * 8.0 : 8.0 + t * 56.0;
-        out[r] = (float)exp_dd(-1.0 * x);
+        out[r] = plain ? exp_f32(-1.0 * x) : (float)exp_dd(-1.0 * x);
     }
     return TSG_OK;
 }
+}  // namespace
+
+int tsg_debug_exp_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, float* out) { return exp_sweep(ctx, i0, n, false, out); }
+int tsg_debug_exp_sweep_host(uint64_t i0, uint64_t n, float* out) { return exp_sweep_host(i0, n, false, out); }
+int tsg_debug_exp_f32_sweep(tsg_ctx* ctx, uint64_t i0, uint64_t n, float* out) { return exp_sweep(ctx, i0, n, true, out); }
+int tsg_debug_exp_f32_sweep_host(uint64_t i0, uint64_t n, float* out) { return exp_sweep_host(i0, n, true, out); }
 
 int tsg_batch_engine_profile(tsg_batch* b, double* out11) {
     if (!b || !out11) return fail(TSG_ERR_INVALID_ARGUMENT, "null argument");

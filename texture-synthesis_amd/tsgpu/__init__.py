@@ -172,6 +172,8 @@ def lib():
     L.tsg_batch_engine_profile.argtypes = [vp, vp]
     L.tsg_debug_exp_sweep.argtypes = [vp, u64, u64, vp]
     L.tsg_debug_exp_sweep_host.argtypes = [u64, u64, vp]
+    L.tsg_debug_exp_f32_sweep.argtypes = [vp, u64, u64, vp]
+    L.tsg_debug_exp_f32_sweep_host.argtypes = [u64, u64, vp]
     L.tsg_batch_destroy.argtypes = [vp]
     _lib = L
     return L
@@ -835,6 +837,21 @@ def debug_exp_sweep_host(i0: int, n: int) -> np.ndarray:
     """Test hook: the library's weight exp on the host for the sweep arguments."""
     out = np.empty(n, np.float32)
     _check(lib().tsg_debug_exp_sweep_host(int(i0), int(n), _ptr(out)))
+    return out
+
+
+def debug_exp_f32_sweep(i0: int, n: int, ctx: Optional[Context] = None) -> np.ndarray:
+    """Test hook: debug_exp_sweep by the unguided wave runs' exp (tsg_debug_exp_f32_sweep)."""
+    ctx = ctx or Context.default()
+    out = np.empty(n, np.float32)
+    _check(lib().tsg_debug_exp_f32_sweep(ctx._h, int(i0), int(n), _ptr(out)))
+    return out
+
+
+def debug_exp_f32_sweep_host(i0: int, n: int) -> np.ndarray:
+    """Test hook: debug_exp_f32_sweep on the host."""
+    out = np.empty(n, np.float32)
+    _check(lib().tsg_debug_exp_f32_sweep_host(int(i0), int(n), _ptr(out)))
     return out
 
 
