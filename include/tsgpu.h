@@ -168,6 +168,12 @@ const char* tsg_version(void);
 /* Context: one HIP device and stream. */
 int tsg_ctx_create(int device, tsg_ctx** out);
 void tsg_ctx_destroy(tsg_ctx* ctx);
+/* Frees device blocks that the library keeps for later allocations (at most
+ * 16 GiB a device, shared by its contexts), those given back longest ago
+ * first, until at most `keep` bytes stay; *cached (may be NULL): the bytes that
+ * stay. For programs that share the device with another allocator: only a
+ * failing allocation of the library's own empties the cache by itself. */
+int tsg_ctx_trim(tsg_ctx* ctx, uint64_t keep, uint64_t* cached);
 
 /* SessionBuilder::build (session.rs:336-448) for already-decoded images.
  * examples: finest example images at their final size, in add order
@@ -259,8 +265,8 @@ void tsg_job_destroy(tsg_job* job);
  *      batch callers that run many Session::run at the same time) ----
  * A tsg_batch runs its admitted jobs together. tsg_batch_run_all runs each
  * job whole, several at a time on streams of their own, where the
- * stage-ahead buffers of those in flight fit (16 GiB, or the bytes given to
- * tsg_batch_set_alone_below). Else, and in steps, which end early enough for
+ * stage-ahead buffers of those in flight fit (16 GiB and half of the device's
+ * free memory, or the bytes given to tsg_batch_set_alone_below). Else, and in steps, which end early enough for
  * jobs to be submitted and cancelled meanwhile, each step (a "round") plans
  * every job's next phases exactly as a run alone would batch them (random
  * candidates, each Jacobi batch's resolve and commit, stage statistics) and

@@ -62,20 +62,24 @@ int fail(int code, const std::string& msg) {
         }                                                                                          \
     } while (0)
 
-// Device blocks of destroyed jobs, per device, kept for the next jobs'
-// allocations: a job allocates about a hundred buffers (pyramids, state,
-// stage-ahead sets) and hipMalloc / hipFree cost tens of microseconds each.
-// Only releases made while g_pool_release is set (job destruction, when the
-// job has no device work in flight) enter the cache; any other release may
-// race queued kernels and goes to hipFree, which waits for them. At most
-// kPoolCap bytes per device stay cached (a 2048^2 job holds 5.5 GB; its blocks
-// were freed and allocated anew with each run while the cap was 4 GiB), the
-// latest given back: what is left of other sizes goes first, so that jobs of
-// one kind after another's find their blocks again. A block serves requests
-// of half its size and more. An allocation that fails empties the cache.
+// Device blocks given back, per device, kept for later allocations: a job
+// allocates about a hundred buffers (pyramids, state, stage-ahead sets) and
+// hipMalloc / hipFree cost tens of microseconds each. Only releases made while
+// g_pool_release is set enter the cache: a destroyed job's, which has no device
+// work in flight, and give_back's, of builds, transforms, resizes and runs on
+// lanes whose stream has been waited for; any other release may race queued
+// kernels and goes to hipFree, which waits for them. At most kPoolCap bytes per
+// device stay cached (a 2048^2 job holds 5.5 GB; its blocks were freed and
+// allocated anew with each run while the cap was 4 GiB), the latest given back:
+// what is left of other sizes goes first, so that jobs of one kind after
+// another's find their blocks again. A block serves requests of half its size
+// and more, while g_pool_exact is set only those of its size. An allocation
+// that fails empties the cache; tsg_ctx_trim cuts it down for other
+// allocators of the process.
 constexpr size_t kPoolCap = 16ull << 30;
 constexpr int kPoolDevices = 16;
 thread_local bool g_pool_release = false;
+thread_local bool g_pool_exact = false;
 
 struct DevPool {
     std::mutex mu;
@@ -121,7 +125,7 @@ hipError_t pool_get(size_t bytes, void** p, size_t* got) {
     if (DevPool* pl = pool_here()) {
         std::lock_guard<std::mutex> lk(pl->mu);
         auto it = pl->free.lower_bound(bytes);
-        if (it != pl->free.end() && it->first <= 2 * bytes) {
+        if (it != pl->free.end() && it->first <= (g_pool_exact ? 1 : 2) * bytes) {
             *p = it->second.p;
             *got = it->first;
             pl->cached -= it->first;
@@ -2310,7 +2314,18 @@ struct tsg_batch {
     uint64_t alone_ahead = 0;             // device bytes an alone run may add for its stage-ahead sets
     bool alone_set = false;               // alone_ahead was given
     uint64_t alone_runs = 0;              // jobs run alone so far
-    uint64_t lane_budget() const { return alone_set ? alone_ahead : kAheadBudget; }
+    // bytes of stage-ahead buffers that its runs may add: as given, or the
+    // most that a single run may take, but half of what the device has free
+    uint64_t lane_budget() const {
+        if (alone_set) return alone_ahead;
+        size_t left = 0, total = 0;
+        if (hipMemGetInfo(&left, &total) != hipSuccess) return 0;
+        if (DevPool* pl = pool_here()) {
+            std::lock_guard<std::mutex> lk(pl->mu);
+            left += pl->cached;
+        }
+        return std::min<uint64_t>(kAheadBudget, left / 2);
+    }
     tsg_tuning tune{};
     ~tsg_batch() {
         if (h_blk) (void)hipHostFree(h_blk);
@@ -2585,8 +2600,9 @@ bool lane_plan(tsg_job* j, uint64_t budget, uint64_t* bytes) {
     return false;
 }
 
-// Every stage-ahead and dependency-order buffer of the planned run.
-hipError_t lane_reserve(tsg_job* j) {
+// Every stage-ahead and dependency-order buffer of the planned run; *held: the
+// bytes of the blocks behind them.
+hipError_t lane_reserve(tsg_job* j, uint64_t* held) {
     const int P = (int)j->prm.backtrack_stages;
     const uint64_t words = j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size());
     const size_t tiles = (size_t)j->tiles_x * j->tiles_y;
@@ -2605,6 +2621,9 @@ hipError_t lane_reserve(tsg_job* j) {
         if (e == hipSuccess) e = A.mnew.reserve(tiles);
         if (e == hipSuccess) e = A.tmin.reserve(tiles);
     }
+    auto bytes = [](const auto&... b) { return (0ull + ... + b.bytes); };
+    *held = bytes(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head);
+    for (const tsg_job::Ahead& A : j->ahead) *held += bytes(A.rc, A.nbrs, A.cnt, A.mend, A.mnew, A.tmin, A.dep, A.avg);
     return e;
 }
 
@@ -2614,15 +2633,16 @@ void lane_release(tsg_job* j) {
     give_back(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head, j->pick_moves);
 }
 
-int batch_admit(tsg_batch* b, bool whole) {
+// budget: bytes of stage-ahead buffers that whole runs may add.
+int batch_admit(tsg_batch* b, bool whole, uint64_t budget) {
     while (b->active.size() < b->max_active && !b->pending.empty()) {
         tsg_batch::Entry e = b->pending.front();
         b->pending.erase(b->pending.begin());
         // few jobs in the batch: this one gets the whole device to itself
         e.alone = b->alone_below && b->active.size() + b->pending.size() + 1 < b->alone_below;
         int rc = TSG_OK;
-        if (!e.alone && whole && !b->quantum && !b->wgs_cap && !b->engine_flags && b->lane_budget() &&
-            lane_plan(e.job, b->lane_budget(), &e.lane_bytes)) {
+        if (!e.alone && whole && !b->quantum && !b->wgs_cap && !b->engine_flags && budget &&
+            lane_plan(e.job, budget, &e.lane_bytes)) {
             // the job's run is one of several at a time (run_on_lanes)
             e.lane = true;
             const hipError_t he = e.job->result.reserve(largest_batch(e.job));
@@ -2691,7 +2711,7 @@ void run_on_lanes(tsg_batch* b, std::vector<tsg_batch::Entry>& runs, uint64_t bu
             if (l % 2) --tail;
             else ++head;
             tsg_batch::Entry& e = runs[q];
-            const uint64_t bytes = e.lane_bytes;
+            uint64_t bytes = e.lane_bytes;
             used += bytes;
             ++busy;
             lk.unlock();
@@ -2701,7 +2721,26 @@ void run_on_lanes(tsg_batch* b, std::vector<tsg_batch::Entry>& runs, uint64_t bu
                 j->stg = j->stg_side = &c->lanes[l]->staging;
             }
             j->share = (uint32_t)std::min(lanes, kLaneShare);
-            if (lane_reserve(j) == hipSuccess) {
+            uint64_t held = 0;
+            hipError_t he = lane_reserve(j, &held);
+            if (he == hipSuccess && held > bytes) {
+                // cached blocks larger than what they serve: they count whole
+                // or, beyond the budget, blocks of the sizes asked for are taken
+                lk.lock();
+                const bool fits = used - bytes + held <= budget;
+                if (fits) {
+                    used += held - bytes;
+                    bytes = held;
+                }
+                lk.unlock();
+                if (!fits) {
+                    lane_release(j);
+                    g_pool_exact = true;
+                    he = lane_reserve(j, &held);
+                    g_pool_exact = false;
+                }
+            }
+            if (he == hipSuccess) {
                 lane_run_job(e);
             } else {
                 lane_release(j);
@@ -2731,9 +2770,8 @@ void run_on_lanes(tsg_batch* b, std::vector<tsg_batch::Entry>& runs, uint64_t bu
 // are used only within the bytes that the batch may add beyond
 // tsg_footprint_estimate, and are released when a run ends. Runs in
 // dependency order go to the lanes, others one after another, smallest first.
-int batch_run_whole(tsg_batch* b) {
+int batch_run_whole(tsg_batch* b, uint64_t budget) {
     std::vector<tsg_batch::Entry> runs, rest;
-    const uint64_t budget = b->lane_budget();
     bool shared = false;
     for (size_t q = 0; q < b->active.size();) {
         tsg_batch::Entry& e = b->active[q];
@@ -2802,9 +2840,11 @@ int batch_round(tsg_batch* b, bool whole) {
         b->prof[slot] += t - t_mark;
         t_mark = t;
     };
-    batch_admit(b, whole);
+    // (steps run jobs whole only where the caller gave the bytes)
+    const uint64_t budget = whole || b->alone_set ? b->lane_budget() : 0;
+    batch_admit(b, whole, budget);
     lap(6);
-    batch_run_whole(b);
+    batch_run_whole(b, budget);
     lap(9);
     if (b->active.empty()) return TSG_OK;
     // plan every job as far as its picks allow; a job that cannot be planned leaves
@@ -3133,6 +3173,19 @@ int tsg_ctx_create(int device, tsg_ctx** out) {
     HIP_TRY(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
     c->scratch = static_cast<unsigned char*>(sp);
     *out = c.release();
+    return TSG_OK;
+}
+
+int tsg_ctx_trim(tsg_ctx* ctx, uint64_t keep, uint64_t* cached) {
+    if (!ctx) return fail(TSG_ERR_INVALID_ARGUMENT, "null context");
+    HIP_TRY(hipSetDevice(ctx->device));
+    if (DevPool* pl = pool_here()) {
+        std::lock_guard<std::mutex> lk(pl->mu);
+        while (pl->cached > keep) pl->drop_oldest();
+        if (cached) *cached = pl->cached;
+    } else if (cached) {
+        *cached = 0;
+    }
     return TSG_OK;
 }
 

@@ -129,6 +129,7 @@ def lib():
     L.tsg_schedule_default.argtypes = [P(Schedule)]
     L.tsg_ctx_create.argtypes = [C.c_int, P(vp)]
     L.tsg_ctx_destroy.argtypes = [vp]
+    L.tsg_ctx_trim.argtypes = [vp, u64, P(u64)]
     L.tsg_job_create.argtypes = [vp, P(Params), u32, P(Image), P(C.c_int), P(Image), P(Image), P(Image), P(Image),
                                  u32, u32, u32, P(vp)]
     L.tsg_job_set_schedule.argtypes = [vp, P(Schedule)]
@@ -245,6 +246,13 @@ class Context:
 
     def clear_tunings(self) -> None:
         _check(lib().tsg_ctx_clear_tunings(self._h))
+
+    def trim(self, keep: int = 0) -> int:
+        """Frees device blocks that the library keeps for later allocations
+        until at most `keep` bytes stay; returns the bytes that stay."""
+        v = C.c_uint64()
+        _check(lib().tsg_ctx_trim(self._h, int(keep), C.byref(v)))
+        return v.value
 
     def __del__(self):
         if getattr(self, "_h", None) and _lib is not None:
