@@ -133,7 +133,10 @@ hipError_t pool_get(size_t bytes, void** p, size_t* got) {
             return hipSuccess;
         }
     }
+    // (the runtime keeps a failed call's error until it is asked for, and the
+    // next launch's check would report it)
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
     if (e == hipErrorOutOfMemory) {
         // give the cache back and retry once
         if (DevPool* pl = pool_here()) {
@@ -141,6 +144,7 @@ hipError_t pool_get(size_t bytes, void** p, size_t* got) {
             pl->clear();
         }
         e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
     }
     if (e == hipSuccess) *got = bytes;
     return e;
@@ -2033,6 +2037,39 @@ void plan_ahead(tsg_job* j) {
     j->flow_on = j->ahead_on && j->tune.flow;
 }
 
+// Every stage-ahead and dependency-order buffer of the planned run; *held: the
+// bytes of the blocks behind them.
+hipError_t lane_reserve(tsg_job* j, uint64_t* held) {
+    const int P = (int)j->prm.backtrack_stages;
+    const uint64_t words = j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size());
+    const size_t tiles = (size_t)j->tiles_x * j->tiles_y;
+    hipError_t e = j->mail.reserve(2 * j->N);
+    for (DBuf<uint32_t>* d : {&j->unres[0], &j->unres[1], &j->pick_idx, &j->pick_link, &j->pick_head})
+        if (e == hipSuccess) e = d->reserve(std::max<size_t>(1, j->N0));
+    for (int t = 0; t < (j->ahead_deep ? P + 1 : 2) && e == hipSuccess; ++t) {
+        tsg_job::Ahead& A = j->ahead[t];
+        const uint64_t n = std::max<uint64_t>(1, stage_size(j, j->ahead_deep ? P - t : 0));
+        e = A.rc.reserve(n * words);
+        if (e == hipSuccess) e = A.nbrs.reserve(n * j->prm.nearest_neighbors);
+        if (e == hipSuccess) e = A.cnt.reserve(n);
+        if (e == hipSuccess) e = A.dep.reserve(n);
+        if (e == hipSuccess) e = A.avg.reserve(n);
+        if (e == hipSuccess) e = A.mend.reserve(tiles);
+        if (e == hipSuccess) e = A.mnew.reserve(tiles);
+        if (e == hipSuccess) e = A.tmin.reserve(tiles);
+    }
+    auto bytes = [](const auto&... b) { return (0ull + ... + b.bytes); };
+    *held = bytes(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head);
+    for (const tsg_job::Ahead& A : j->ahead) *held += bytes(A.rc, A.nbrs, A.cnt, A.mend, A.mnew, A.tmin, A.dep, A.avg);
+    return e;
+}
+
+// Gives back what lane_reserve took (nothing of the job is in flight).
+void lane_release(tsg_job* j) {
+    for (tsg_job::Ahead& A : j->ahead) give_back(A.rc, A.nbrs, A.cnt, A.n_at, A.mend, A.mnew, A.tmin, A.dep, A.avg);
+    give_back(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head, j->pick_moves);
+}
+
 // Single job: with stage-ahead neighbour lists, every stage runs in
 // dependency order (flow_stage). Else runs of small batches go to one
 // single-workgroup launch; other batches get one k_resolve launch,
@@ -2042,6 +2079,19 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     hipStream_t s = j->stream;
     int rc;
     plan_ahead(j);
+    if (j->flow_on) {
+        // On a device that cannot hold the sets the job runs without them: a
+        // launch per batch needs a tenth of the bytes.
+        uint64_t held;
+        const hipError_t e = lane_reserve(j, &held);
+        if (e == hipErrorOutOfMemory) {
+            lane_release(j);
+            j->tune.ahead = 0;
+            plan_ahead(j);
+        } else {
+            HIP_TRY(e);
+        }
+    }
     if ((rc = step_begin(j))) return rc;
     if (j->flow_on) {
         if ((rc = picks_begin(j))) return rc;
@@ -2598,39 +2648,6 @@ bool lane_plan(tsg_job* j, uint64_t budget, uint64_t* bytes) {
     j->tune.ahead = ahead;
     j->ahead_deep = j->ahead_on = j->flow_on = false;
     return false;
-}
-
-// Every stage-ahead and dependency-order buffer of the planned run; *held: the
-// bytes of the blocks behind them.
-hipError_t lane_reserve(tsg_job* j, uint64_t* held) {
-    const int P = (int)j->prm.backtrack_stages;
-    const uint64_t words = j->prm.random_sample_locations * rand_words((uint32_t)j->filt.size());
-    const size_t tiles = (size_t)j->tiles_x * j->tiles_y;
-    hipError_t e = j->mail.reserve(2 * j->N);
-    for (DBuf<uint32_t>* d : {&j->unres[0], &j->unres[1], &j->pick_idx, &j->pick_link, &j->pick_head})
-        if (e == hipSuccess) e = d->reserve(std::max<size_t>(1, j->N0));
-    for (int t = 0; t < (j->ahead_deep ? P + 1 : 2) && e == hipSuccess; ++t) {
-        tsg_job::Ahead& A = j->ahead[t];
-        const uint64_t n = std::max<uint64_t>(1, stage_size(j, j->ahead_deep ? P - t : 0));
-        e = A.rc.reserve(n * words);
-        if (e == hipSuccess) e = A.nbrs.reserve(n * j->prm.nearest_neighbors);
-        if (e == hipSuccess) e = A.cnt.reserve(n);
-        if (e == hipSuccess) e = A.dep.reserve(n);
-        if (e == hipSuccess) e = A.avg.reserve(n);
-        if (e == hipSuccess) e = A.mend.reserve(tiles);
-        if (e == hipSuccess) e = A.mnew.reserve(tiles);
-        if (e == hipSuccess) e = A.tmin.reserve(tiles);
-    }
-    auto bytes = [](const auto&... b) { return (0ull + ... + b.bytes); };
-    *held = bytes(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head);
-    for (const tsg_job::Ahead& A : j->ahead) *held += bytes(A.rc, A.nbrs, A.cnt, A.mend, A.mnew, A.tmin, A.dep, A.avg);
-    return e;
-}
-
-// Gives back what lane_reserve took (nothing of the job is in flight).
-void lane_release(tsg_job* j) {
-    for (tsg_job::Ahead& A : j->ahead) give_back(A.rc, A.nbrs, A.cnt, A.n_at, A.mend, A.mnew, A.tmin, A.dep, A.avg);
-    give_back(j->mail, j->unres[0], j->unres[1], j->pick_idx, j->pick_link, j->pick_head, j->pick_moves);
 }
 
 // budget: bytes of stage-ahead buffers that whole runs may add.
