@@ -1560,11 +1560,17 @@ int ahead_poll(tsg_job* j, bool block) {
     return ahead_stage(j);
 }
 
-// Items of the largest batch: a fraction of the resolved count, a fixed size, or the cap.
+// Items of the largest batch that batch_end_at gives: a fixed size (the cap is
+// for the others), or a fraction of the resolved count, by the least of the
+// shifts, the first stage's among them, up to the cap.
 uint64_t largest_batch(const tsg_job* j) {
-    uint64_t maxb = j->sched.px_per_batch ? j->sched.px_per_batch
-                                          : (uint64_t)j->N >> std::min(j->sched.redo_shift, j->sched.new_shift);
-    if (j->sched.max_batch) maxb = std::min<uint64_t>(maxb, j->sched.max_batch);
+    uint64_t maxb = j->sched.px_per_batch;
+    if (!maxb) {
+        uint32_t sh = std::min(j->sched.redo_shift, j->sched.new_shift);
+        if (j->sched.first_new_shift) sh = std::min(sh, j->sched.first_new_shift);
+        maxb = (uint64_t)j->N >> sh;
+        if (j->sched.max_batch) maxb = std::min<uint64_t>(maxb, j->sched.max_batch);
+    }
     return std::min<uint64_t>(std::max<uint64_t>(maxb + 1, small_batch_max()), j->N);
 }
 
