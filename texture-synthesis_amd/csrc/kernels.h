@@ -10,6 +10,8 @@ constexpr int kMaxK = 64;          // nearest_neighbors supported on the device
 constexpr uint32_t kBruteMax = 2048;  // resolved count up to which kNN scans the list
 constexpr int kTableRadius = 64;   // offset table radius of the ring scan
 
+constexpr uint32_t kLutNan = 1, kLutNeg = 2;  // BatchArgs::lut_odd
+
 // One Jacobi batch: items [item0, item1) of the current stage.
 struct BatchArgs {
     uint32_t W, H, tiles_x, tiles_y;
@@ -44,7 +46,11 @@ struct BatchArgs {
     uint32_t* dbg_best;           // [item] winning candidate index (test hook)
     uint32_t knn_only;            // stop after the kNN dump (test hook)
     uint32_t exact;               // force the unpruned lane-per-candidate evaluation
-    uint32_t lut_nan;             // the stage's cost tables hold a NaN (cauchy 0): exact path
+    // what the stage's cost tables hold beside finite, non-negative costs
+    // (kLutNan: cauchy 0; kLutNeg: a guide's weight below zero, once more pixels
+    // are resolved than there were to resolve, as in every guided inpainting of
+    // a smaller part of an image)
+    uint32_t lut_odd;
     // commit fused into the resolve launch (last workgroup) / small-batch kernel
     uint32_t fused_commit;
     uint32_t first_new;           // items >= first_new are new pixels
@@ -479,8 +485,9 @@ hipError_t launch_resolve_small(const BatchArgs& a, const uint32_t* bounds, cons
 hipError_t launch_resolve(const BatchArgs& a, bool guided, hipStream_t s);
 // A dependency-ordered run (FlowArgs) with `team` waves per item (1, 2, 4 or
 // 8) on at most wgs persistent workgroups. flow_max_wgs: as many as are
-// resident, of the kernel for m random candidates.
-uint32_t flow_max_wgs(uint32_t team, uint32_t m, bool guided);
+// resident, of the kernel for m random candidates (neg: and tables with
+// negative costs, which k_flow_slice does not take).
+uint32_t flow_max_wgs(uint32_t team, uint32_t m, bool guided, bool neg);
 hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t wgs, uint32_t team, bool guided,
                                hipStream_t s);
 hipError_t launch_stage_end(const StageEndArgs& a, hipStream_t s);

@@ -864,6 +864,29 @@ __device__ __forceinline__ float term_at(const NbrRow& r, const float* lut, cons
     return __fmul_rn(s, r.w);
 }
 
+// find_best_match's sequential rule (ms.rs:1184-1224) for 64 candidates in
+// list order, one per lane (v): a candidate replaces the best iff none of its
+// partial sums, of which `top` is the largest, reached it. Costs may be NaN.
+__device__ __forceinline__ void scan_best(bool v, float top, float cost, uint32_t base, float& best, uint32_t& bidx) {
+    uint64_t left = __ballot(v);
+    for (;;) {
+        uint64_t m;
+        if (best == best) {
+            m = __ballot(!(top >= best)) & left;
+            if (m == 0ull) break;
+        } else {
+            // every candidate replaces a NaN: on to the first that is none, or the last
+            if (left == 0ull) break;
+            m = __ballot(cost == cost) & left;
+            if (m == 0ull) m = 1ull << (63 - __clzll((long long)left));
+        }
+        const int l = __ffsll((long long)m) - 1;
+        best = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(cost), l));
+        bidx = base + (uint32_t)l;
+        left &= ~((2ull << l) - 1ull);
+    }
+}
+
 struct Best {
     float B;      // lowest complete cost so far (FLT_MAX: none)
     uint32_t Bi;  // its candidate index (kNone: none)
@@ -902,15 +925,23 @@ __device__ __forceinline__ void prune_bound(const unsigned long long* tb, const 
 // chunks or 8 first 10.5 and 32.5, 4 first 10.1 and 30.7, 2 first 9.9 and
 // 30.0, growing from 2 9.9 and 29.9; guided 1024^2 18.6, -, 17.9, 17.6. A
 // constant here also lets the compiler keep the loop in fewer registers.
+//
+// NEG (one member, groups in list order): terms may be negative, so a
+// candidate's largest partial sum (kept in the unused word of L->coh) stands
+// for the one that only grows: the reference drops a candidate once a partial
+// sum reaches the best cost so far, and the candidates left are taken in order.
 constexpr int kGrowing = 1;
-template <bool GUIDED, int FIRST_SH>
+template <bool GUIDED, int FIRST_SH, bool NEG = false>
 __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps, WaveLds* L, const float* lut, const float* glut,
                                            int slot, int lane, uint32_t kf, uint32_t n_act, Best& best,
                                            unsigned long long* tb) {
     const uint32_t slot4 = (uint32_t)slot * 4u;
     MapDesc m0{};
     if (n_maps == 1) m0 = ld_uniform(maps);
-    if (lane < (int)n_act) L->act_sum[lane] = 0.0f;
+    if (lane < (int)n_act) {
+        L->act_sum[lane] = 0.0f;
+        if (NEG) L->coh[lane].w = __float_as_uint(-INFINITY);
+    }
     wave_sync();
     // the group's mirror state: 0 none, 1 all, 2 mixed. A group holds
     // coherence candidates only (never mirrored) or random ones only (always
@@ -980,14 +1011,15 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
         }
         wave_sync();
         const bool act = lane < (int)n_act;
-        float s = 0.0f;
+        float s = 0.0f, top = -INFINITY;
         uint32_t myidx = kNone, xy = 0, ms = 0;
         if (act) {
             s = L->act_sum[lane];
+            if (NEG) top = __uint_as_float(L->coh[lane].w);
             // the terms are loaded 16 at a time ahead of the in-order adds
             const float* tp = &L->terms[lane << sh];
             uint32_t jj = 0;
-            if (sh >= 2) {
+            if (!NEG && sh >= 2) {
                 for (; jj + 16 <= jn; jj += 16) {
                     const float4 q0 = *reinterpret_cast<const float4*>(tp + jj);
                     const float4 q1 = *reinterpret_cast<const float4*>(tp + jj + 4);
@@ -1003,12 +1035,25 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
                     s = __fadd_rn(s, q.x); s = __fadd_rn(s, q.y); s = __fadd_rn(s, q.z); s = __fadd_rn(s, q.w);
                 }
             }
-            for (; jj < jn; ++jj) s = __fadd_rn(s, tp[jj]);
+            for (; jj < jn; ++jj) {
+                s = __fadd_rn(s, tp[jj]);
+                if (NEG) top = fmaxf(top, s);
+            }
             myidx = L->act_idx[lane];
             xy = L->act_xy[lane];
             ms = L->act_ms[lane];
         }
         j0 += jn;
+        if (NEG && j0 >= kf) {
+            uint32_t l = kNone;
+            scan_best(act, top, s, 0u, best.B, l);
+            if (l != kNone) {
+                best.Bi = (uint32_t)__builtin_amdgcn_readlane((int)myidx, (int)l);
+                best.xy = (uint32_t)__builtin_amdgcn_readlane((int)xy, (int)l);
+                best.ms = (uint32_t)__builtin_amdgcn_readlane((int)ms, (int)l);
+            }
+            break;
+        }
         if (j0 >= kf) {
             // costs are not negative, so their bits order them
             const unsigned long long key = act ? (unsigned long long)__float_as_uint(s) << 32 | myidx : ~0ull;
@@ -1029,7 +1074,7 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
             break;
         }
         prune_bound(tb, best, PB, PBi);
-        const bool keep = act && !(s > PB || (s == PB && (PBi == kNone || myidx > PBi)));
+        const bool keep = NEG ? act && !(top >= best.B) : act && !(s > PB || (s == PB && (PBi == kNone || myidx > PBi)));
         const uint64_t km = __ballot(keep);
         const uint32_t pos = bits_below(km);
         wave_sync();
@@ -1038,6 +1083,7 @@ __device__ __forceinline__ void eval_group(const MapDesc* maps, uint32_t n_maps,
             L->act_ms[pos] = ms;
             L->act_idx[pos] = myidx;
             L->act_sum[pos] = s;
+            if (NEG) L->coh[pos].w = __float_as_uint(top);
         }
         n_act = (uint32_t)__popcll(km);
         wave_sync();
@@ -1258,7 +1304,7 @@ __device__ __forceinline__ uint32_t item_neighbours(const BatchArgs& a, const Ma
 }
 
 // Leader: every candidate without pruning, find_best_match's sequential
-// rule, for NaN cost tables and the full-cost test hook.
+// rule, for odd cost tables (lut_odd) and the full-cost test hook.
 template <bool GUIDED, int C = lut_copies<GUIDED>(), class Lds>
 __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t rel,
                                            uint32_t kf, uint32_t n_coh, uint32_t n_c, const Lds* L, const float* lut,
@@ -1289,7 +1335,7 @@ __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* ma
             }
             const MapDesc md = maps[cmap];
             const int cx = (int)(cxy & 0xffffu), cy = (int)(cxy >> 16);
-            float score = 0.0f, lastgood = -INFINITY;
+            float score = 0.0f, top = -INFINITY;
             for (uint32_t j = 0; j < kf; ++j) {
                 const int32_t o = L->nd[j];
                 const int X2 = cx + sgn * packed_dx(o), Y2 = cy + sgn * packed_dy(o);
@@ -1303,41 +1349,13 @@ __device__ __forceinline__ void item_exact(const BatchArgs& a, const MapDesc* ma
                     s = lut4_add<C>(s, glut, bytes_scaled<C>(L->gpat[j]), gp, slot4);
                 }
                 score = __fadd_rn(score, __fmul_rn(s, L->w[j]));
-                if (score == score) lastgood = score;
+                if (score > top) top = score;  // (a NaN passes by)
             }
             F = score;
-            X = (F == F) ? F : lastgood;
+            X = top;
             if (a.ext_full_cost) a.ext_full_cost[(size_t)rel * a.ext_cmax + c] = F;
         }
-        // find_best_match's sequential rule: candidate c replaces the best
-        // iff no partial sum reached it, i.e. !(X_c >= best) (partial sums of
-        // non-negative terms are monotone; X_c is the last non-NaN partial).
-        const bool anynan = __ballot(v && !(F == F)) != 0ull;
-        if (!anynan && best == best) {
-            float key = v ? F : INFINITY;
-            uint32_t ki = c;
-            for (int off = kWave / 2; off > 0; off >>= 1) {
-                float ok = __shfl_xor(key, off);
-                uint32_t oi = (uint32_t)__shfl_xor((int)ki, off);
-                if (ok < key || (ok == key && oi < ki)) {
-                    key = ok;
-                    ki = oi;
-                }
-            }
-            if (key < best) {
-                best = key;
-                bidx = ki;
-            }
-        } else {
-            for (int l = 0; l < kWave; ++l) {
-                if (base + (uint32_t)l >= n_c) break;
-                float Xl = __shfl(X, l), Fl = __shfl(F, l);
-                if (!(Xl >= best)) {
-                    best = Fl;
-                    bidx = base + (uint32_t)l;
-                }
-            }
-        }
+        scan_best(v, X, F, base, best, bidx);
     }
 }
 
@@ -1456,7 +1474,7 @@ __device__ __forceinline__ uint4 flow_records(const FlowArgs& f, const BatchArgs
 // the coherence group alone first (it usually holds the winner and bounds the
 // rest), then the random ones 64 at a time. cxy, cms, uniq: item_neighbours'
 // coherence candidates; rpre: the member's first 64 random candidates.
-template <bool GUIDED, int FIRST_SH>
+template <bool GUIDED, int FIRST_SH, bool NEG = false>
 __device__ __forceinline__ Best eval_slice(const BatchArgs& a, const MapDesc* maps, uint32_t item, uint32_t rel,
                                            uint32_t kf, uint32_t n_coh, uint32_t n_k0, uint32_t cxy, uint32_t cms,
                                            uint64_t uniq, uint32_t r0, uint32_t nrs, uint2 rpre, int member, int T,
@@ -1507,8 +1525,8 @@ __device__ __forceinline__ Best eval_slice(const BatchArgs& a, const MapDesc* ma
             L->act_idx[lane] = ci;
         }
         wave_sync();
-        eval_group<GUIDED, FIRST_SH>(maps, a.n_maps, L, lut, glut, slot, lane, kf, g_hi - g_lo, bst,
-                                     tb);
+        eval_group<GUIDED, FIRST_SH, NEG>(maps, a.n_maps, L, lut, glut, slot, lane, kf, g_hi - g_lo, bst,
+                                          tb);
         if (lead && first) phase_clock(a, item, 4, lane);
         first = false;
         g_lo = g_hi;
@@ -1599,8 +1617,25 @@ __device__ __forceinline__ uint4 resolve_team(const BatchArgs& a, const MapDesc*
             n_c = n_coh + a.m;
         }
         if (lead) phase_clock(a, item, 2, lane);
-        exact = a.exact || a.ext_full_cost || a.lut_nan || !(L->avg > 0.0);
-        if (!exact) {
+        // negative costs: the leader takes every candidate, in list order
+        const bool neg = GUIDED && a.lut_odd == kLutNeg && !a.ext_cands;
+        exact = a.exact || a.ext_full_cost || (a.lut_odd && !neg) || !(L->avg > 0.0);
+        if (!exact && neg) {
+            if constexpr (GUIDED) {
+                Best bst{FLT_MAX, kNone, 0u, 0u};
+                if (lead) {
+                    if ((uint32_t)lane < a.m) rpre = rand_cand(a, item, (uint32_t)lane);
+                    bst = eval_slice<GUIDED, FIRST_SH, true>(a, maps, item, rel, kf, n_coh, n_k0, cxy, cms, uniq, 0, a.m, rpre, 0,
+                                                             1, true, L, lut, glut, slot, lane, nullptr);
+                }
+                if (lane == 0) {
+                    L->t_B = bst.B;
+                    L->t_Bi = bst.Bi;
+                    L->t_xy = bst.xy;
+                    L->t_ms = bst.ms;
+                }
+            }
+        } else if (!exact) {
             // ---- 3. this member's slice, exact pruning ----
             const Best bst = eval_slice<GUIDED, FIRST_SH>(a, maps, item, rel, kf, n_coh, n_k0, cxy, cms, uniq, r0, nrs,
                                                           rpre, member, T, lead, L, lut, glut, slot, lane,
@@ -1951,8 +1986,8 @@ __device__ __forceinline__ uint32_t queue_next(ItemQueue* q, const FlowArgs& f, 
 
 // A run with one wave per item, for batches large enough to fill the chip:
 // persistent workgroups whose waves take items in order and evaluate them
-// with exact pruning, as k_resolve's do.
-template <bool GUIDED>
+// with exact pruning, as k_resolve's do. NEG: tables with negative costs.
+template <bool GUIDED, bool NEG = false>
 __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(6))) void k_flow_wave(BatchArgs a,
                                                                                                           FlowArgs f) {
     const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
@@ -2008,8 +2043,8 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
             const uint32_t n_coh = item_neighbours<GUIDED>(a, maps, item, 0, x, y, kf, 0, L, lane, true, cxy, cms,
                                                            uniq, &st);
             phase_clock(a, item, 2, lane);
-            if (!a.lut_nan && avg > 0.0) {
-                const Best b = eval_slice<GUIDED, kGrowing>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, 0, a.m, rpre, 0,
+            if (!(a.lut_odd & (NEG ? kLutNan : ~0u)) && avg > 0.0) {
+                const Best b = eval_slice<GUIDED, kGrowing, NEG>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, 0, a.m, rpre, 0,
                                                      1, true, L, lut, glut, lane % lut_copies<GUIDED>(), lane, nullptr);
                 phase_clock(a, item, 5, lane);
                 const bool have = b.Bi != kNone;
@@ -2151,12 +2186,14 @@ __device__ __forceinline__ void slot_terms(const NbrRow& row, const float* lut, 
 
 // In-order f32 sum of a candidate's first kf terms (rows are zero from there
 // to the chunk's end), the next chunk read ahead of a chunk's adds.
-__device__ __forceinline__ float row_sum(const float* row, uint32_t kf) {
+// NEG: *top, the largest partial sum.
+template <bool NEG = false>
+__device__ __forceinline__ float row_sum(const float* row, uint32_t kf, float* top = nullptr) {
     const float4* tp = reinterpret_cast<const float4*>(row);
     float4 v[2][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[0][i] = tp[i];
-    float s = 0.0f;
+    float s = 0.0f, t = -INFINITY;
 #pragma unroll
     for (uint32_t g = 0; g < kMaxK / 16; ++g) {
         if (16 * g < kf) {
@@ -2168,12 +2205,17 @@ __device__ __forceinline__ float row_sum(const float* row, uint32_t kf) {
             for (int i = 0; i < 4; ++i) {
                 const float4 u = v[g & 1][i];
                 s = __fadd_rn(s, u.x);
+                if (NEG) t = fmaxf(t, s);
                 s = __fadd_rn(s, u.y);
+                if (NEG) t = fmaxf(t, s);
                 s = __fadd_rn(s, u.z);
+                if (NEG) t = fmaxf(t, s);
                 s = __fadd_rn(s, u.w);
+                if (NEG) t = fmaxf(t, s);
             }
         }
     }
+    if (NEG) *top = t;
     return s;
 }
 
@@ -2188,13 +2230,15 @@ __device__ __forceinline__ float row_sum(const float* row, uint32_t kf) {
 // member's row, and one barrier to compare the members'. Pruning, duplicate
 // removal and a leader's merge would each add a dependent step that the idle
 // lanes save nothing by. The winner's own lane posts it. ONE: a single map,
-// its descriptor in scalars.
-template <bool GUIDED, int T, bool ONE>
+// its descriptor in scalars. NEG: with negative costs the first member takes
+// the candidates in list order by their costs and largest partial sums.
+template <bool GUIDED, int T, bool ONE, bool NEG = false>
 __global__ __launch_bounds__(kWave* T) __attribute__((amdgpu_waves_per_eu(4))) void k_flow_team(BatchArgs a, FlowArgs f) {
     const uint64_t t_start = a.dbg_launch ? wall_clock64() : 0;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ MapDesc smaps[kMapCache];
     __shared__ TeamLds team[2];
+    __shared__ float2 all[NEG ? 2 : 1][NEG ? 2 * kMaxK : 1];  // per candidate: largest partial sum, cost
     flow_args(a);
     constexpr int C = team_copies<GUIDED, T>();
     float *lut, *glut;
@@ -2302,7 +2346,7 @@ __global__ __launch_bounds__(kWave* T) __attribute__((amdgpu_waves_per_eu(4))) v
         }
         __syncthreads();
         const uint32_t n_coh = uniform(L->n_coh);
-        if (!a.lut_nan && L->avg > 0.0) {
+        if (!(a.lut_odd & (NEG ? kLutNan : ~0u)) && L->avg > 0.0) {
             if (wave == 0) phase_clock(a, item, 2, lane);
             const uint32_t cper = (n_coh + T - 1) / T;
             const uint32_t c0 = min(n_coh, (uint32_t)wave * cper), ncs = min(n_coh, c0 + cper) - c0;
@@ -2334,9 +2378,11 @@ __global__ __launch_bounds__(kWave* T) __attribute__((amdgpu_waves_per_eu(4))) v
                     slot_terms<GUIDED, C>(row, lut, glut, slot4, n_c, cpx, cgpx, has, rows + kSlots * kTermRow, lane);
                 wave_sync();
                 if (cand.on) {
-                    const float s = row_sum(rows + (uint32_t)lane * kTermRow, kf);
+                    float top;
+                    const float s = row_sum<NEG>(rows + (uint32_t)lane * kTermRow, kf, &top);
                     const uint32_t sidx =
                         lane < (int)kSlots ? n_coh + r0 + q * kSlots + sl : c0 + q * kSlots + sl;
+                    if (NEG) all[turn][sidx] = make_float2(top, s);
                     // a cost the reference's search cannot take over its start
                     // value counts as that value (find_best_match, ms.rs:1184-1224)
                     const unsigned long long key =
@@ -2352,6 +2398,28 @@ __global__ __launch_bounds__(kWave* T) __attribute__((amdgpu_waves_per_eu(4))) v
                 n_r = random_slots(q);
             }
             if (wave == 0) phase_clock(a, item, 4, lane);
+            if constexpr (NEG) {
+                __syncthreads();
+                if (wave == 0) {
+                    phase_clock(a, item, 5, lane);
+                    float cost = FLT_MAX;
+                    uint32_t bidx = 0;
+                    for (uint32_t base = 0; base < n_coh + a.m; base += kWave) {
+                        const bool v = base + (uint32_t)lane < n_coh + a.m;
+                        const float2 e = all[turn][v ? base + (uint32_t)lane : 0u];
+                        scan_best(v, e.x, e.y, base, cost, bidx);
+                    }
+                    const uint4 r = item_winner(a, maps, item, 0, n_coh, L, cost, bidx, lane);
+                    if (lane == 0) {
+                        const MapDesc& md = maps[r.y & 0xffffu];
+                        mail_post(f, flat, gld(md.px + (r.x >> 16) * md.w + (r.x & 0xffffu)), r.x, r.y & 0xffffu, r.z);
+                        if (item >= a.first_new) gst(a.score_w + flat, __uint_as_float(r.w));
+                    }
+                    phase_clock(a, item, 6, lane);
+                }
+                idx = uniform(team[turn ^ 1u].next);
+                continue;
+            }
             // candidates sit in the first row's lanes
             const unsigned long long rmin = row_min(bkey);
             const unsigned long long mine = lane_u64(rmin, 0);
@@ -2413,8 +2481,10 @@ struct LinkLds {
 // own candidate is evaluated by one member, and the sums follow.
 // Member w holds the candidates of neighbours 8 w .. 8 w + 7 and an eighth of
 // the random ones (m <= 64); ties order coherence candidates by neighbour,
-// then the random ones, as the reference's list does.
-template <bool GUIDED, bool ONE>
+// then the random ones, as the reference's list does. NEG: with negative costs
+// every member takes all candidates in that order by their costs and largest
+// partial sums, and the lane of the one left posts it.
+template <bool GUIDED, bool ONE, bool NEG = false>
 __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per_eu(4))) void k_flow_link(BatchArgs a,
                                                                                                           FlowArgs f) {
     constexpr int T = kWavesPerWG;
@@ -2423,6 +2493,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
     __shared__ MapDesc smaps[kMapCache];
     __shared__ LinkLds team[2];
     __shared__ uint32_t late_g[GUIDED ? T : 1][GUIDED ? kPollAll : 1][2 * kSlots];
+    __shared__ float2 all[NEG ? 2 : 1][NEG ? 2 * kMaxK : 1];  // per candidate: largest partial sum, cost (NaN: none)
     flow_args(a);
     constexpr int C = team_copies<GUIDED, T>();
     float *lut, *glut;
@@ -2526,8 +2597,10 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
         __syncthreads();
         const uint64_t late = lane_u64(L->late, 0);
         const bool mine_late = (late >> lane) & 1ull;
-        const bool exact = a.lut_nan || !(L->avg > 0.0);
-        if (!exact) {
+        const bool exact = (a.lut_odd & (NEG ? kLutNan : ~0u)) || !(L->avg > 0.0);
+        // (told that this is the usual way, the compiler spills 2 VGPRs of a
+        // guided kernel instead of 14: style transfer 640x427 8.4 -> 7.9 ms)
+        if (__builtin_expect(!exact, 1)) {
             if (wave == 0) phase_clock(a, item, 2, lane);
             NbrRow row;
             row.q = bytes_scaled<C>(has ? L->pat[lane] : 0u);
@@ -2634,6 +2707,30 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
                 }
             }
             wave_sync();
+            if constexpr (NEG) {
+                const uint32_t order = lane < (int)kSlots ? kMaxK + r0 + sl : c0 + sl;
+                float top = INFINITY, s = __uint_as_float(0x7fc00000u);
+                if (cand.on) s = row_sum<true>(rows + (uint32_t)lane * kTermRow, kf, &top);
+                if (cand.on || (lane >= (int)kSlots && lane < (int)(2 * kSlots))) all[turn][order] = make_float2(top, s);
+                if (wave == 0) phase_clock(a, item, 4, lane);
+                __syncthreads();
+                if (wave == 0) phase_clock(a, item, 5, lane);
+                const float2 e0 = all[turn][lane], e1 = all[turn][kMaxK + ((uint32_t)lane < a.m ? lane : 0)];
+                const uint64_t coh = __ballot(e0.y == e0.y);
+                float cost = FLT_MAX;
+                // without a cost below the start value the list's first candidate stays
+                uint32_t bidx = coh ? (uint32_t)__ffsll((long long)coh) - 1u : (uint32_t)kMaxK;
+                scan_best(e0.y == e0.y, e0.x, e0.y, 0u, cost, bidx);
+                scan_best((uint32_t)lane < a.m, e1.x, e1.y, kMaxK, cost, bidx);
+                if (cand.on && order == bidx) {
+                    mail_post(f, flat, cand.colour, cand.xy, cand.map, cand.patch);
+                    gst(a.item_score + item, cost);
+                    if (item >= a.first_new) gst(a.score_w + flat, cost);
+                }
+                if (wave == 0) phase_clock(a, item, 6, lane);
+                idx = uniform(team[turn ^ 1u].next);
+                continue;
+            }
             unsigned long long key = ~0ull;
             if (cand.on) {
                 const float s = row_sum(rows + (uint32_t)lane * kTermRow, kf);
@@ -2780,7 +2877,7 @@ __global__ __launch_bounds__(kWave* kWavesPerWG) __attribute__((amdgpu_waves_per
             const uint32_t n_coh = item_neighbours<GUIDED>(a, maps, item, 0, x, y, kf, 0, L, lane, true, cxy, cms, uniq,
                                                            &st);
             if (wave == 0) phase_clock(a, item, 2, lane);
-            if (!a.lut_nan && avg > 0.0) {
+            if (!a.lut_odd && avg > 0.0) {
                 const Best b = eval_slice<GUIDED, 6>(a, maps, item, 0, kf, n_coh, n_coh, cxy, cms, uniq, r0, nrs, rpre, wave,
                                                      T, wave == 0, L, lut, glut, lane % lut_copies<GUIDED>(), lane,
                                                      &S->bound);
@@ -4034,26 +4131,30 @@ struct FlowKernel {
 };
 // a guided job's two tables have half the copies each
 template <int T>
-FlowKernel team_kernel(bool guided, bool one) {
-    return {guided ? (one ? k_flow_team<true, T, true> : k_flow_team<true, T, false>)
-                   : (one ? k_flow_team<false, T, true> : k_flow_team<false, T, false>),
+FlowKernel team_kernel(bool guided, bool one, bool neg) {
+    return {neg      ? (one ? k_flow_team<true, T, true, true> : k_flow_team<true, T, false, true>)
+            : guided ? (one ? k_flow_team<true, T, true> : k_flow_team<true, T, false>)
+                     : (one ? k_flow_team<false, T, true> : k_flow_team<false, T, false>),
             kWave * T, 256 * team_copies<false, T>() * sizeof(float) + T * kTeamWaveLds};
 }
-bool flow_kernel(uint32_t team, uint32_t m, bool guided, bool one, FlowKernel* k) {
+bool flow_kernel(uint32_t team, uint32_t m, bool guided, bool one, bool neg, FlowKernel* k) {
+    if (neg && !guided) return false;  // only a guide's weight falls below zero
     if (m > (uint32_t)kMaxK && (team == 2 || team == 4 || team == 8)) {
+        if (neg) return false;
         *k = {guided ? k_flow_slice<true> : k_flow_slice<false>, kWave * team,
               lut_bytes(guided) + team * sizeof(WaveLds)};
         return true;
     }
     switch (team) {
         case 1:
-            *k = {guided ? k_flow_wave<true> : k_flow_wave<false>, (uint32_t)(kWave * kWavesPerWG),
+            *k = {neg ? k_flow_wave<true, true> : guided ? k_flow_wave<true> : k_flow_wave<false>, (uint32_t)(kWave * kWavesPerWG),
                   resolve_lds_bytes(guided)};
             return true;
-        case 2: *k = team_kernel<2>(guided, one); return true;
-        case 4: *k = team_kernel<4>(guided, one); return true;
+        case 2: *k = team_kernel<2>(guided, one, neg); return true;
+        case 4: *k = team_kernel<4>(guided, one, neg); return true;
         case 8:
-            *k = {guided ? (one ? k_flow_link<true, true> : k_flow_link<true, false>)
+            *k = {neg      ? (one ? k_flow_link<true, true, true> : k_flow_link<true, false, true>)
+                  : guided ? (one ? k_flow_link<true, true> : k_flow_link<true, false>)
                          : (one ? k_flow_link<false, true> : k_flow_link<false, false>),
                   kWave * kWavesPerWG, 256 * team_copies<false, 8>() * sizeof(float) + 8 * kTeamWaveLds};
             return true;
@@ -4092,9 +4193,9 @@ hipError_t configure_kernels() {
     for (uint32_t team : {1u, 2u, 4u, 8u})  // (of one kernel, the largest team's bytes last)
         for (uint32_t m : {1u, kMaxK + 1u})
             for (bool guided : {false, true})
-                for (bool one : {false, true}) {
+                for (int form = 0; form < (guided && (team == 1 || m == 1) ? 4 : 2); ++form) {
                     FlowKernel k;
-                    if (!flow_kernel(team, m, guided, one, &k)) return hipErrorInvalidValue;
+                    if (!flow_kernel(team, m, guided, form & 1, form >= 2, &k)) return hipErrorInvalidValue;
                     e = hipFuncSetAttribute((const void*)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
                     if (e != hipSuccess) return e;
                 }
@@ -4336,9 +4437,9 @@ hipError_t launch_resolve_persist(const BatchArgs& a, uint32_t wgs, bool guided,
     return hipGetLastError();
 }
 
-uint32_t flow_max_wgs(uint32_t team, uint32_t m, bool guided) {
+uint32_t flow_max_wgs(uint32_t team, uint32_t m, bool guided, bool neg) {
     FlowKernel k;
-    if (!flow_kernel(team, m, guided, false, &k)) return 0;
+    if (!flow_kernel(team, m, guided, false, neg, &k)) return 0;
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
@@ -4357,7 +4458,7 @@ hipError_t launch_resolve_flow(const BatchArgs& a, const FlowArgs& f, uint32_t w
                                hipStream_t s) {
     if (f.n == 0) return hipSuccess;
     FlowKernel k;
-    if (!flow_kernel(team, a.m, guided, a.n_maps == 1, &k)) return hipErrorInvalidValue;
+    if (!flow_kernel(team, a.m, guided, a.n_maps == 1, a.lut_odd & kLutNeg, &k)) return hipErrorInvalidValue;
     if (wgs == 0 || !f.ticket || !f.dep || !f.mail || !f.overflow || f.tag == 0 || f.tag > 255 || f.spin_limit == 0)
         return hipErrorInvalidValue;
     // every item needs its neighbour list; test hooks are not supported

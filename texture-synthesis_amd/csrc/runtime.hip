@@ -269,6 +269,13 @@ inline uint32_t pack_px(const uint8_t* p) {
     return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
 }
 
+// BatchArgs::lut_odd of a stage's cost tables.
+uint32_t lut_odd(const std::vector<float>& lut) {
+    uint32_t odd = 0;
+    for (float v : lut) odd |= (std::isnan(v) ? kLutNan : 0u) | (v < 0.0f ? kLutNeg : 0u);
+    return odd;
+}
+
 // metric_cauchy / metric_l2 (ms.rs:1109-1120) for |a-b| = d; the reference's
 // 256x256 tables depend only on |a-b| (exact in f32: the difference of two
 // u8 values is exact and its square removes the sign).
@@ -1656,8 +1663,7 @@ int step_open_stage(tsg_job* j) {
         alpha_s = (b * b) * b;
     }
     stage_luts(j->prm.cauchy_dispersion, j->guided, alpha_s, j->lut_keep[t].data());
-    uint32_t lut_nan = 0;
-    for (float v : j->lut_keep[t]) lut_nan |= (uint32_t)std::isnan(v);
+    const uint32_t odd = lut_odd(j->lut_keep[t]);
     HIP_TRY(j->stg->upload(j->lut.p, j->lut_keep[t].data(), 512 * 4, s));
     if (!j->flow_on) {
         int rc = wait_picks(j, t);
@@ -1710,7 +1716,7 @@ int step_open_stage(tsg_job* j) {
     a.stage_seed = st.pss;
     a.k = j->prm.nearest_neighbors;
     a.item_score = j->item_score.p;
-    a.lut_nan = lut_nan;
+    a.lut_odd = odd;
     a.first_new = (uint32_t)st.redo_eff;
     a.done_counter = j->done_counter.p;
     a.dbg_clk = (j->profile_level >= 2 && t == j->profile_level - 2) ? j->clk.p : nullptr;
@@ -1974,6 +1980,7 @@ int flow_stage(tsg_job* j, Progress& pr) {
     int rc;
     // one tag per stage: a pyramid has at most 16 levels, so a run at most 17 stages
     ++j->flow_tag;
+    const bool neg = a.lut_odd & kLutNeg;
     const uint32_t lock = (uint32_t)j->locked;
     uint64_t q0 = 0;  // items below are in the state
     while (st.i < st.S_eff) {
@@ -1982,14 +1989,15 @@ int flow_stage(tsg_job* j, Progress& pr) {
         uint32_t team = 0;
         bool due = false;
         while (step_peek(j, b0, b1)) {
-            const uint32_t t = flow_team_of(j, b0, b1);
+            // k_flow_slice does not take negative costs
+            const uint32_t t = neg && a.m > kMaxK ? 1u : flow_team_of(j, b0, b1);
             if (team && t != team) break;
             team = t;
             step_advance(j, b0, b1);
             i1 = b1;
             if ((due = pr.due(j, i1))) break;
         }
-        const uint32_t most = std::max(1u, flow_max_wgs(team, a.m, j->guided) / j->share);
+        const uint32_t most = std::max(1u, flow_max_wgs(team, a.m, j->guided, neg) / j->share);
         const uint32_t wgs = j->tune.flow_wgs ? std::min(j->tune.flow_wgs, most) : most;
         if (j->flow_launches == kFlowTickets) {
             HIP_TRY(hipMemsetAsync(j->flow_ticket.p, 0, kFlowTickets * 4, s));
@@ -2436,8 +2444,7 @@ int eng_open_stage(tsg_job* j) {
         alpha_s = (b * b) * b;
     }
     stage_luts(j->prm.cauchy_dispersion, j->guided, alpha_s, j->lut_keep[t].data());
-    uint32_t lut_nan = 0;
-    for (float v : j->lut_keep[t]) lut_nan |= (uint32_t)std::isnan(v);
+    const uint32_t odd = lut_odd(j->lut_keep[t]);
     float* lut = j->eng.luts.p + (size_t)t * 512;
     HIP_TRY(j->stg->upload(lut, j->lut_keep[t].data(), 512 * 4, s));
     int rc = wait_picks(j, t);
@@ -2475,7 +2482,7 @@ int eng_open_stage(tsg_job* j) {
     a.stage_seed = st.pss;
     a.k = j->prm.nearest_neighbors;
     a.item_score = j->item_score.p;
-    a.lut_nan = lut_nan;
+    a.lut_odd = odd;
     a.first_new = (uint32_t)st.redo_eff;
     a.state_w = j->state.p;
     a.mask_w = j->mask.p;
@@ -4067,9 +4074,7 @@ int tsg_score_batch(tsg_ctx* ctx, uint32_t w, uint32_t h, const uint8_t* color, 
     a.ext_cmax = cmax;
     a.ext_full_cost = dfc.p;
     a.dbg_best = dbest.p;
-    bool lut_nan = false;
-    for (float v : lut) lut_nan |= std::isnan(v);
-    a.lut_nan = lut_nan;
+    a.lut_odd = lut_odd(lut);
     HIP_TRY(launch_resolve(a, guided, s));
     HIP_TRY(hipStreamSynchronize(s));
     std::vector<uint4> res(n);
