@@ -307,14 +307,6 @@ struct XformSource {
 hipError_t launch_xform_apply(const uint32_t* coord, uint32_t n, const XformSource* srcs, uint32_t n_src,
                               uint32_t* out, uint32_t* bad, hipStream_t s);
 
-// per-stage statistics: sum and count of non-negative item scores
-struct StatsArgs {
-    const float* item_score;
-    uint32_t n;
-    double* sum;
-    unsigned long long* count;
-};
-
 hipError_t launch_knn_prefetch(const PrefetchArgs& a, hipStream_t s);
 
 // Stage statistics in a fixed order: chunks of kStatsChunk items, each summed
@@ -453,9 +445,6 @@ hipError_t launch_engine(const QEngineArgs& e, const BatchArgs* args, uint32_t w
 // (float)exp(-x_i) by exp_dd, or (plain) by exp_f32, for the sweep arguments
 // x_i, i in [i0, i0 + n) (test hook).
 hipError_t launch_exp_sweep(uint64_t i0, uint64_t n, bool plain, float* out, hipStream_t s);
-// XCD of each of n workgroups of a probe launch (test hook: the engine's
-// job placement relies on the hardware XCC id).
-hipError_t launch_xcc_probe(uint32_t* out, uint32_t n, hipStream_t s);
 // rank[rlist[q]] = q for q in [lo, hi)
 hipError_t launch_rank(const uint32_t* rlist, uint32_t lo, uint32_t hi, uint32_t* rank, hipStream_t s);
 // sets the mask bits of rlist[lo, hi); with tile_min, also the least q per tile
@@ -498,7 +487,6 @@ hipError_t launch_mask_tiles(const uint8_t* mask, uint32_t W, uint32_t H, uint32
 // past each query's count.
 hipError_t launch_knn_unpack(const uint32_t* q_flat, const int32_t* packed, const uint32_t* counts, uint32_t n_q,
                              uint32_t k, uint32_t W, int32_t* pairs, hipStream_t s);
-hipError_t launch_stats(const StatsArgs& a, hipStream_t s);
 hipError_t launch_rand(const RandArgs& a, hipStream_t s);
 hipError_t launch_commit(const CommitArgs& a, hipStream_t s);
 // Single-wave batches on persistent workgroups; persist_max_wgs: resident count.

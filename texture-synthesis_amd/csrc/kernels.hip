@@ -3665,34 +3665,6 @@ __global__ void k_list_moves(uint32_t* u, uint32_t n, const uint2* moves, uint32
     if (q < n_moves && moves[q].x < n) u[moves[q].x] = moves[q].y;
 }
 
-__global__ void k_stats(StatsArgs a) {
-    __shared__ double ssum[256];
-    __shared__ unsigned long long scnt[256];
-    double s = 0.0;
-    unsigned long long c = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
-        float v = a.item_score[i];
-        if (v >= 0.0f) {
-            s += (double)v;
-            c += 1;
-        }
-    }
-    ssum[threadIdx.x] = s;
-    scnt[threadIdx.x] = c;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            ssum[threadIdx.x] += ssum[threadIdx.x + o];
-            scnt[threadIdx.x] += scnt[threadIdx.x + o];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        atomicAdd(a.sum, ssum[0]);
-        atomicAdd(a.count, scnt[0]);
-    }
-}
-
 // Sum and count of the non-negative scores of stage items [lo, hi) (at most
 // kStatsChunk), in a fixed order: threads 0..255 take items t, t + 256, ...
 // in turn, then a tree over the threads. Every thread of the block calls it
@@ -3797,10 +3769,6 @@ __global__ void k_exp_sweep(uint64_t i0, uint64_t n, float* out) {
     const double t = (double)((i * 0x9E3779B97F4A7C15ull) >> 11) * 0x1p-53;
     const double x = (i & 3u) ? t * 8.0 : __dadd_rn(8.0, __dmul_rn(t, 56.0));
     out[r] = PLAIN ? exp_f32(-1.0 * x) : (float)exp_dd(-1.0 * x);
-}
-
-__global__ void k_xcc_probe(uint32_t* out, uint32_t n) {
-    if (threadIdx.x == 0 && blockIdx.x < n) out[blockIdx.x] = xcc_id();
 }
 
 // Persistent workgroups (as many as are resident) that drain the programs of
@@ -4334,20 +4302,6 @@ hipError_t launch_exp_sweep(uint64_t i0, uint64_t n, bool plain, float* out, hip
     const dim3 grid((unsigned)((n + 255) / 256));
     if (plain) hipLaunchKernelGGL(k_exp_sweep<true>, grid, dim3(256), 0, s, i0, n, out);
     else hipLaunchKernelGGL(k_exp_sweep<false>, grid, dim3(256), 0, s, i0, n, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_xcc_probe(uint32_t* out, uint32_t n, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_xcc_probe, dim3(n), dim3(64), 0, s, out, n);
-    return hipGetLastError();
-}
-
-hipError_t launch_stats(const StatsArgs& a, hipStream_t s) {
-    if (a.n == 0) return hipSuccess;
-    uint32_t blocks = (a.n + 255) / 256;
-    if (blocks > 1024) blocks = 1024;
-    hipLaunchKernelGGL(k_stats, dim3(blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
