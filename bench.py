@@ -174,17 +174,21 @@ def batched_leg(ts, synth, n, sequential=True):
     t_bat = time.perf_counter() - t0
     done = dict(batch.poll())
     assert sorted(done) == sorted(tickets) and not any(done.values())
-    got = [digest(batch.take(t)) for t in tickets]
+    taken = [batch.take(t) for t in tickets]
     t_pcie = time.perf_counter() - t0
+    got = [digest(g) for g in taken]
+    del taken
     st = batch.stats()
     prof = batch.engine_profile()
     batch.close()
-    # algorithmic bytes of the engine launches: every job's resolves (its
-    # stage sizes, (0.5^s N) for s = 0..5) at 4k(k+m) + 24k + 28 bytes each
+    # algorithmic bytes of the batch: every job's resolves (its stage sizes,
+    # (0.5^s N) for s = 0..5) at 4k(k+m) + 24k + 28 bytes each; exact pruning
+    # skips most of them
     alg = sum(sum(int((0.5 ** s_) * o * o) for s_ in range(6)) * (4 * k * (k + M) + 24 * k + 28)
               for _, o, k, _ in specs)
     t_kern = prof["launch_to_done_ms"] / 1e3
-    ec = counters_from_profiles("resolve_c2_counters.md", "k_flow_wave")
+    ec = counters_from_profiles("batched_c4_traffic.md", "batch256")
+    moved = ec["hbm_bytes"] if ec and n == 256 else None  # counted for the default mix only
     return {
         "workload": f"{n} syntheses: examples uniform in {{64,128,256,512}}^2, outputs uniform in "
                     f"{{128,256,512,1024}}^2, k in {{20,50}}, m=50, seeds 4000+j",
@@ -198,13 +202,13 @@ def batched_leg(ts, synth, n, sequential=True):
         "identical_to_alone": (seq == got) if seq is not None else None,
         "launches": st["launches"], "engine_rounds": st["rounds"],
         "engine_workgroup_ms": {k: (round(v, 1) if isinstance(v, float) else v) for k, v in prof.items()},
-        "roofline": {"kernel": "k_flow_link + k_flow_team + k_flow_wave (whole runs, several at a time)", "bound": "hbm", "algorithmic_bytes": alg,
-                     "achieved": round(alg / t_kern / 1e9, 1) if t_kern > 0 else None, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(alg / t_kern / 1e9 / HBM_PEAK_GBS, 4) if t_kern > 0 else None,
+        "roofline": {"kernel": "k_flow_link + k_flow_team + k_flow_wave (whole runs, several at a time)", "bound": "hbm",
+                     "achieved": round(moved / t_kern / 1e9, 1) if moved and t_kern > 0 else None, "peak": HBM_PEAK_GBS,
+                     "unit": "GB/s", "frac": round(moved / t_kern / 1e9 / HBM_PEAK_GBS, 4) if moved and t_kern > 0 else None,
+                     "traffic": moved, "algorithmic_bytes": alg,
                      "over": "the batch's runs, first launch to the last run's end (host clock)",
-                     "traffic": None, "l2_hit": (ec or {}).get("l2_hit"),
-                     "valu_busy": (ec or {}).get("valu_busy"), "waves_per_cu": (ec or {}).get("waves_per_cu"),
-                     "limiter": limiter(ec), "counters_from": "profiles/resolve_c2_counters.md (k_flow_wave alone on the chip)"},
+                     "limiter": "the chains of three or four jobs at a time, as many as the hardware queues run",
+                     "counters_from": "profiles/batched_c4_traffic.md"},
     }
 
 
@@ -372,10 +376,11 @@ def limiter(c):
     """The limiter the counters point at."""
     if not c:
         return None
-    if c.get("valu_busy", 0) >= 0.5:
+    if c.get("valu_busy", 0) >= 0.7:
         return "vector ALU (VALU busy %.0f%%), then memory latency" % (100 * c["valu_busy"])
-    return "memory latency: waves wait %.0f%% of their cycles, VALU busy %.0f%%, %.1f resident waves per CU" % (
-        100 * c.get("wait_fraction", 0), 100 * c.get("valu_busy", 0), c.get("waves_per_cu", 0))
+    gather = ", gather units %.0f%%" % (100 * c["gather_busy"]) if "gather_busy" in c else ""
+    return "memory latency: waves wait %.0f%% of their cycles, VALU busy %.0f%%%s, %.1f resident waves per CU" % (
+        100 * c.get("wait_fraction", 0), 100 * c.get("valu_busy", 0), gather, c.get("waves_per_cu", 0))
 
 
 def copy_calibration(mb):
@@ -474,11 +479,14 @@ def main():
     # apart), over the timed steps; durations are the launches' device-clock spans
     resolves = (res["items"] + ks["resolve_runs"]["items"] * args.steps) // args.steps
     kern_s = res["ms"] / 1e3
-    achieved = res["items"] * BYTES_PER_RESOLVE / kern_s / 1e9 if kern_s > 0 else 0.0
     per_launch = res["items"] * BYTES_PER_RESOLVE / max(1, res["launches"])
     ms_per_step = t_all * 1e3 / args.steps
     value = 1024 * 1024 * args.steps / t_all / 1e6
     rc_ctr = counters_from_profiles("resolve_c2_counters.md", "k_flow_wave")
+    # HBM bytes a launch moves (counters), over its span: exact pruning skips
+    # most of the algorithmic bytes, and caches serve most of the rest
+    moved = (rc_ctr or {}).get("hbm_bytes") or traffic_from_profiles()
+    achieved = moved * res["launches"] / kern_s / 1e9 if moved and kern_s > 0 else 0.0
     lat_sorted = sorted(lat)
     p99 = lat_sorted[min(len(lat_sorted) - 1, int(round(0.99 * (len(lat_sorted) - 1))))]
     out = {
@@ -505,10 +513,8 @@ def main():
                            "note": "the same steps with the output image, coordinate and id maps and the "
                                    "resolved list downloaded to host memory"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     # (algorithmic bytes: exact pruning skips most of them, and caches serve most of the rest)
-                     "traffic": (rc_ctr or {}).get("hbm_bytes") or traffic_from_profiles(),
-                     "l2_hit": (rc_ctr or {}).get("l2_hit"), "lds_bank_conflict": (rc_ctr or {}).get("lds_bank_conflict"),
+                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": moved,
+                     "gather_busy": (rc_ctr or {}).get("gather_busy"), "l2_hit": (rc_ctr or {}).get("l2_hit"), "lds_bank_conflict": (rc_ctr or {}).get("lds_bank_conflict"),
                      "valu_busy": (rc_ctr or {}).get("valu_busy"), "waves_per_cu": (rc_ctr or {}).get("waves_per_cu"),
                      "limiter": limiter(rc_ctr), "counters_from": "profiles/resolve_c2_counters.md",
                      "kernel": "k_flow_wave", "bytes_per_resolve": BYTES_PER_RESOLVE,
