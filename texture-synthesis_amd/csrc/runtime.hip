@@ -2093,9 +2093,12 @@ int run_job(tsg_job* j, tsg_progress_fn cb, void* user) {
     hipStream_t s = j->stream;
     int rc;
     plan_ahead(j);
-    if (j->flow_on) {
+    size_t left = 0, total = 0;
+    const uint64_t sets = j->ahead_deep ? ahead_bytes_deep(j) : ahead_bytes(j);
+    if (j->flow_on && (hipMemGetInfo(&left, &total) != hipSuccess || left < sets + sets / 4 + (1u << 30))) {
         // On a device that cannot hold the sets the job runs without them: a
-        // launch per batch needs a tenth of the bytes.
+        // launch per batch needs a tenth of the bytes. (Where there is room
+        // they are allocated as the stages are prepared, beside the run.)
         uint64_t held;
         const hipError_t e = lane_reserve(j, &held);
         if (e == hipErrorOutOfMemory) {
