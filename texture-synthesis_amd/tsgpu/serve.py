@@ -77,7 +77,9 @@ class _Running:
 class Server:
     """Admits requests by device-memory footprint and runs them together.
 
-    hbm_budget: device bytes the admitted requests may hold at once.
+    hbm_budget: device bytes the admitted requests may hold at once, with the
+    stage-ahead buffers of those that run. Idle blocks that the library keeps
+    (at most 16 GiB, Context.trim) are not counted.
     max_active: engine slots (requests advanced per round).
     rounds_per_pump: engine rounds run by each ``pump`` call before finished
     requests are collected and waiting ones admitted.
